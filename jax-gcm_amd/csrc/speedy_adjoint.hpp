@@ -15,8 +15,10 @@
 //   * max/min/clip give 1/2 to each operand at a tie (lax.max / lax.min);
 //   * a reduction max (jnp.max over levels, clouds) splits the gradient evenly
 //     over the tied entries.
-// Each term is recomputed (its forward function fills a tape) right before it
-// is reversed, so only the phase outputs live across the whole adjoint.
+// The forward and its reversal are interleaved (phase_b1_vjp, phase_b2_taped,
+// phase_b2_vjp, phase_a_adj): the surface fluxes and the shortwave are reversed
+// right after they ran, the longwave in the two sweeps that its forward makes, and
+// phase A last, from a recompute of the convection and the clouds.
 #pragma once
 
 #include "speedy_column.hpp"
@@ -25,9 +27,10 @@ namespace speedy {
 
 enum { VJP_RHBL = 0, VJP_TRCNV = 1, VJP_RHLSC = 2, VJP_CO2 = 3, VJP_DRAG = 4, VJP_NPARAM = 5 };
 
-// Floats per column of the longwave tape store used by column_vjp.
+// Floats per column of the longwave tape: per level 1 .. KX-1 and band the flux
+// entering the level from above and the adjoint of the flux leaving it upward.
 template <int KX>
-constexpr int vjp_tape_floats() { return 4 * (KX + 1); }
+constexpr int vjp_tape_floats() { return 8 * (KX - 1); }
 
 // Cotangents of one column's tendencies.  Only level KX-1 of the u and v
 // tendencies is nonzero in the forward (surface stress), so only those matter.
@@ -60,12 +63,9 @@ SPD_HD void settle(R& x) {
 #endif
 }
 
-// The fences are applied where the kernel then fits in registers (up to eight
-// levels: no scratch).  At sixteen levels the accumulators alone are ~100
-// values; forcing them into VGPRs at every fence makes the kernel spill around
-// the fences, and that build gave wrong forward tendencies in the batched
-// forward + VJP kernel on gfx950 (the host build of the same source is right).
-// Sixteen-level kernels therefore keep the unfenced form.
+// The accumulator fences are applied where the kernel fits in registers (up to
+// eight levels).  At sixteen levels the accumulators alone are ~100 values, and
+// forcing them into VGPRs at every fence makes the kernel spill around the fences.
 template <int KX>
 constexpr bool kSettle = KX <= 8;
 
@@ -80,6 +80,15 @@ SPD_HD void settle_adj(ColumnAdj<R, KX>& g) {
 #pragma unroll
   for (int i = 0; i < VJP_NPARAM; ++i) settle(g.prm[i]);
   settle(g.cloudc); settle(g.clstr); settle(g.qcloud); settle(g.precnv); settle(g.precls); settle(g.rps);
+}
+
+// The same after level k of the longwave's up sweep.
+template <typename R, int KX>
+SPD_HD void settle_lw(ColumnAdj<R, KX>& g, int k, R Fu[4], R aD[4], R& a_below) {
+  settle(g.T[k]); settle(g.Q[k]); settle(g.ps); settle(g.cloudc); settle(g.rps); settle(a_below);
+  if (k < KX - 1) settle(g.T[k + 1]);
+#pragma unroll
+  for (int bnd = 0; bnd < 4; ++bnd) { settle(Fu[bnd]); settle(aD[bnd]); }
 }
 
 template <typename R, int KX>
@@ -103,29 +112,41 @@ SPD_HD void verify_ct(uint32_t flags, uint32_t limited, R dt, ColumnCt<R, KX>& c
 #pragma unroll
   for (int k = 0; k < KX; ++k) {
     g_qraw[k] = R(0.0);
-    if ((flags & SPEEDY_FLAG_VERIFY_TENDENCIES) && ((limited >> k) & 1u)) {
-      g_qraw[k] = -ct.dq[k] / dt;
-      ct.dq[k] = R(0.0);
-    }
+    const bool lim = (flags & SPEEDY_FLAG_VERIFY_TENDENCIES) && ((limited >> k) & 1u);
+    g_qraw[k] = sel(lim, -ct.dq[k] / dt, R(0.0));
+    ct.dq[k] = sel(lim, R(0.0), ct.dq[k]);
   }
 }
 
 // verify_state in reverse: where(q < 0, 0, q) passes the gradient only where q >= 0.
 template <typename R>
-SPD_HD R verify_q_grad(R q_raw, R g) { return q_raw < R(0.0) ? R(0.0) : g; }
+SPD_HD R verify_q_grad(R q_raw, R g) { return sel(q_raw < R(0.0), R(0.0), g); }
 
-// d qsat / d ta and d qsat / d ps of qsat_f (humidity.py:95-102).
+// Reciprocal for the adjoint's linear arithmetic: the hardware reciprocal and one
+// Newton step (1 ulp), 3 instructions where a division takes 11.  The forward's
+// values, which decisions depend on, keep mdiv.
+SPD_HD float mrcp(float b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float r = __builtin_amdgcn_rcpf(b);
+  return __builtin_fmaf(__builtin_fmaf(-b, r, 1.0f), r, r);
+#else
+  return 1.0f / b;
+#endif
+}
+SPD_HD double mrcp(double b) { return 1.0 / b; }
+
+// d q / d ta and ps * d q / d ps of q = qsat_f(ta, ps, sig) (humidity.py:95-102), from
+// q itself.  With q = 622 e / D and D = sig ps - 0.378 e, sig ps / D = 1 + 0.378 q / 622, so
+// dq/dta = q (sig ps / D) e'/e with e'/e = c (273.16 - tt) / (ta - tt)^2, and
+// dq/dps = -q (sig ps / D) / ps: no exponential and one reciprocal.
 template <typename R>
-SPD_HD void qsat_grad(R ta, R ps, R sig, R& dq_dt, R& dq_dps) {
+SPD_HD void qsat_grad(R ta, R q, R& dq_dt, R& ps_dq_dps) {
   const bool warm = ta >= R(273.16);
-  const R c = warm ? R(17.269) : R(21.875);
+  const R c = warm ? R(17.269 * (273.16 - 35.86)) : R(21.875 * (273.16 - 7.66));
   const R tt = warm ? R(35.86) : R(7.66);
-  const R e = R(6.108e-3) * mexp(c * (ta - R(273.16)) / (ta - tt));
-  const R D = sig * ps - R(0.378) * e;
-  const R rD = R(1.0) / D;
-  const R de_dt = e * c * (R(273.16) - tt) / sq(ta - tt);
-  dq_dt = R(622.0) * sig * ps * rD * rD * de_dt;
-  dq_dps = -R(622.0) * e * sig * rD * rD;
+  const R gq = q + q * q * R(0.378 / 622.0);
+  dq_dt = gq * c * mrcp(sq(ta - tt));
+  ps_dq_dps = -gq;
 }
 
 // Adjoint of radset4 (longwave_radiation.py:216-225): returns d/d temp of
@@ -145,11 +166,12 @@ SPD_HD R radset4_adj(R temp, R omeps, const R a_fb[4]) {
 // Adjoint of level k's longwave transmissivities tauL[k][:] = exp(-ab * ps * dhs)
 // (shortwave_radiation.py:177-200) and emissions st4a0[k], st4a1[k]
 // (longwave_radiation.py:48-68), applied at once so that no per-level adjoint
-// arrays stay live.  Gradients of the half-level temperatures go to a_Th.
+// arrays stay live.  Gradients of the half-level temperatures above and below the
+// level go to a_Th[0] and a_Th[1].
 template <typename R, int KX>
 SPD_HD void lw_level_adj(int k, const R a_tau[4], R a_s0, R a_s1, const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a,
                          const R tau[4], const SpeedyParams& p, const SpeedyVertical& v, const Uniforms<R>& u,
-                         ColumnAdj<R, KX>& g, R a_Th[KX]) {
+                         ColumnAdj<R, KX>& g, R a_Th[2]) {
   R ab[4];
   lw_absorptivity<R, KX>(k, c, a, p, u, ab);
 #pragma unroll
@@ -158,7 +180,7 @@ SPD_HD void lw_level_adj(int k, const R a_tau[4], R a_s0, R a_s1, const ColumnIn
     g.ps += ax * (-(ab[bnd] * v.dhs[k]));
     const R a_ab = ax * (-(c.ps * v.dhs[k]));
     if (bnd == 0) {
-      if (k >= 2 && k <= KX - 2) g.cloudc += a_ab * ((k > a.icltop) ? p.ablcl1 : p.ablcl2);
+      if (k >= 2 && k <= KX - 2) g.cloudc += a_ab * sel(k > a.icltop, R(p.ablcl1), R(p.ablcl2));
     } else if (bnd == 1) {
       g.prm[VJP_CO2] += a_ab * u.ablco2_d;
     } else if (k >= 1) {
@@ -185,18 +207,18 @@ SPD_HD void lw_level_adj(int k, const R a_tau[4], R a_s0, R a_s1, const ColumnIn
     const R a_grad = a_s1 * R(4.0) * st3a;
     if (k < KX - 1) {
       const R ax = a_grad * R(0.5) * dmax_x(Th(k) - Th(k - 1), R(0.0));
-      a_Th[k] += ax;
-      a_Th[k - 1] += -ax;
+      a_Th[1] += ax;
+      a_Th[0] += -ax;
     } else {
       const R ax = a_grad * dmax_x(c.T[KX - 1] - Th(KX - 2), R(0.0));
       g.T[KX - 1] += ax;
-      a_Th[KX - 2] += -ax;
+      a_Th[0] += -ax;
     }
   } else if (k == 0) {
     const R s0 = R(0.75) * c.T[0] + R(0.25) * Th(0);
     const R as = a_s0 * R(4.0 * SBC) * pow3(s0);
     g.T[0] += R(0.75) * as;
-    a_Th[0] += R(0.25) * as;
+    a_Th[1] += R(0.25) * as;
   } else {
     const R s1 = R(0.50) * c.T[1] + R(0.25) * (Th(0) + Th(1));
     const R as = a_s0 * R(4.0 * SBC) * pow3(s1);
@@ -208,9 +230,9 @@ SPD_HD void lw_level_adj(int k, const R a_tau[4], R a_s0, R a_s1, const ColumnIn
 
 // The column as level k's longwave recompute sees it: the values lw_level(k)
 // reads (T at k-1..k+1, q at k, ps) are passed through an empty asm that also
-// takes `dep`, the adjoint state entering level k, so the recompute cannot be
-// hoisted above the reversal of the previous level (which would keep every
-// level's recomputed values live at once).
+// takes `dep`, the flux entering level k, so the recompute is neither merged with
+// the downward sweep's (which would keep every level's transmissivities live in
+// between) nor hoisted above the previous level.
 template <typename R, int KX>
 SPD_HD ColumnIn<R, KX> column_at_level(const ColumnIn<R, KX>& c, int k, R dep) {
   ColumnIn<R, KX> cc = c;
@@ -225,77 +247,177 @@ SPD_HD ColumnIn<R, KX> column_at_level(const ColumnIn<R, KX>& c, int k, R dep) {
   return cc;
 }
 
-// ---------------------------------------------------------------- longwave up
-// Each level's transmissivities, emissions and band fractions are recomputed
-// here (lw_level) from the column, not taken from the forward.
+// ---------------------------------------------------------------- longwave
+// Cotangent of level k's longwave flux divergence (tlw[k] = dfl[k] grdscp[k] / ps).
+template <typename R, int KX>
+SPD_HD R dfl_ct(const ColumnCt<R, KX>& ct, const SpeedyVertical& v, int k, R rps) {
+  return ct.dt[k] * v.grdscp[k] * rps;
+}
+
+// Longwave down (longwave_radiation.py:13-117) runs from the top down, and so does
+// the adjoint of longwave up; longwave up and the adjoint of longwave down run from
+// the surface up.  So the forward and the reverse of the whole longwave take two
+// sweeps.  The adjoint fluxes need only the cotangents and the transmissivities:
+//   down sweep   Fd (forward) and aU, the adjoint of the upward fluxes; both are kept
+//                per level and band on the tape;
+//   up sweep     Fu (forward) and aD, the adjoint of the downward fluxes; each level
+//                then has all four, and its transmissivities, emissions and band
+//                fractions are reversed once for both directions.
+// One recompute of a level's transmissivities remains (the up sweep's, which the
+// forward kernels make too).  Reversing each direction by itself with a forward
+// recompute before it took six evaluations of every level and 7700 VALU
+// instructions a wave at 8 levels for the whole adjoint.
+//
+// Leaves aF, the adjoint of the flux leaving the surface, and b.dfl, b.rlds as
+// lw_down does.
 template <typename R, int KX, class Store>
-SPD_HD void lw_up_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const PhaseB<R, KX>& b,
-                      const SpeedyParams& p, const SpeedyVertical& v, const Uniforms<R>& u, const Store& Fu,
-                      const R a_dfl[KX], R& a_rlus2, R a_flux_h[2], ColumnAdj<R, KX>& g, R a_Th[KX]) {
-  const R ps = c.ps;
-  const R stratc1 = u.eps1 * ps;
-  LwLevel<R> L0, L1;
-  lw_level<R, KX>(0, c, a, p, v, u, L0);
-  lw_level<R, KX>(1, c, a, p, v, u, L1);
-  // corrections of the two top levels
-  const R a_c1 = -a_dfl[0], a_c2 = -a_dfl[1];
-  const R a_strat1 = a_c1 * v.dhs[0] * L0.st0 + a_c2 * v.dhs[1] * L1.st0;
-  g.ps += a_c1 * c.stratz + a_strat1 * u.eps1;
-  // top level: dfl[0] += (F0 - ft0) + (F1 - ft1), F = Fu[1]
-  R aF[4];
-  {
-    R afb[4] = {R(0.0), R(0.0), R(0.0), R(0.0)};
-    R atau[4] = {R(0.0), R(0.0), R(0.0), R(0.0)};
-    R as0 = a_c1 * v.dhs[0] * stratc1, as1 = R(0.0);
+SPD_HD void lw_down_vjp(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const SpeedyParams& p,
+                        const SpeedyVertical& v, const Uniforms<R>& u, const ColumnCt<R, KX>& ct, PhaseB<R, KX>& b,
+                        Store& tape, R aF[4]) {
+  const R rps = mrcp(c.ps);
+  R Fd[4], Fprev = R(0.0);
 #pragma unroll
-    for (int bnd = 0; bnd < 2; ++bnd) {
-      const R a_ft = -a_dfl[0];
-      const R tau = L0.tau[bnd], em = R(1.0) - tau;
-      aF[bnd] = a_dfl[0] + a_ft * tau;
-      atau[bnd] = a_ft * (Fu.get(4 + bnd) - L0.fb[bnd] * (L0.st0 - R(2.0) * em * L0.st1));
-      afb[bnd] = a_ft * em * (L0.st0 - em * L0.st1);
-      as0 += a_ft * em * L0.fb[bnd];
-      as1 += -a_ft * em * em * L0.fb[bnd];
+  for (int k = 0; k < KX; ++k) {
+    const R a_dfl = dfl_ct<R, KX>(ct, v, k, rps);
+    LwLevel<R> L;
+    lw_level<R, KX>(k, c, a, p, v, u, L);
+    if (k == 0) {
+#pragma unroll
+      for (int bnd = 0; bnd < 4; ++bnd) {
+        const R em = R(1.0) - L.tau[bnd];
+        Fd[bnd] = bnd < 2 ? em * (L.fb[bnd] * (L.st0 + em * L.st1)) : R(0.0);
+        aF[bnd] = bnd < 2 ? a_dfl - a_dfl * L.tau[bnd] : R(0.0);
+      }
+    } else {
+#pragma unroll
+      for (int bnd = 0; bnd < 4; ++bnd) {
+        const R au = aF[bnd] - a_dfl;              // dfl[k] += sum Fu[k+1] - sum Fu[k]
+        tape.put((k - 1) * 8 + bnd, Fd[bnd]);
+        tape.put((k - 1) * 8 + 4 + bnd, au);
+        aF[bnd] = a_dfl + au * L.tau[bnd];
+        const R em = R(1.0) - L.tau[bnd];
+        Fd[bnd] = L.tau[bnd] * Fd[bnd] + em * (L.fb[bnd] * (L.st0 + em * L.st1));
+      }
     }
-    aF[2] = R(0.0); aF[3] = R(0.0);
-    g.T[0] += radset4_adj(c.T[0], u.omeps, afb);
-    lw_level_adj<R, KX>(0, atau, as0, as1, c, a, L0.tau, p, v, u, g, a_Th);
+    const R Fs = ((Fd[0] + Fd[1]) + Fd[2]) + Fd[3];
+    b.dfl[k] = k == 0 ? -Fs : -(Fs - Fprev);
+    Fprev = Fs;
+    if (k == KX - 1) {
+      R rlds = ((p.emisfc * Fd[0] + p.emisfc * Fd[1]) + p.emisfc * Fd[2]) + p.emisfc * Fd[3];
+      const R corlw = u.corlw * L.st0;
+      b.dfl[KX - 1] = b.dfl[KX - 1] + (-corlw);
+      b.rlds = rlds + corlw;
+    }
   }
-  // levels 1 .. KX-1 (the forward ran from KX-1 down to 1)
-#pragma unroll
-  for (int k = 1; k < KX; ++k) {
-    LwLevel<R> Lk;
-    if (k == 1) Lk = L1;
-    else lw_level<R, KX>(k, column_at_level<R, KX>(c, k, aF[0]), a, p, v, u, Lk);
-    R afb[4], atau[4];
-    R as0 = (k == 1) ? a_c2 * v.dhs[1] * stratc1 : R(0.0), as1 = R(0.0);
-    const auto Fk = Fu.after(aF[0]);   // Fu[k+1] read when level k is reversed
+}
+
+// Cotangents of the longwave's surface inputs, from the down sweep's aF and the
+// lowest level's a_dfl.
+template <typename R, int KX>
+SPD_HD void lw_surface_adj(const Uniforms<R>& u, const SpeedyParams& p, R tsfc, R a_dfl, const R aF[4], R& a_rlus2,
+                           R a_flux_h[2]) {
+  R fbt[4];
+  radset4(tsfc, u.omeps, fbt);
+  a_rlus2 = ((aF[0] * fbt[0] + aF[1] * fbt[1]) + (aF[2] * fbt[2] + aF[3] * fbt[3])) + a_dfl * p.epslw;
+  a_flux_h[0] = aF[0] * u.refsfc;
+  a_flux_h[1] = aF[1] * u.refsfc;
+}
+
+// The up sweep: longwave up (longwave_radiation.py:119-202; b.dfl enters holding the
+// longwave-down divergence, b.tlw leaves as lw_up leaves it) and every level's
+// reversal.  b.rlus2, b.tsfc, b.flux_h: the hand-offs of the surface fluxes and the
+// shortwave; a_rlds: cotangent of the downward flux at the surface.
+template <typename R, int KX, class Store>
+SPD_HD void lw_up_vjp(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const SpeedyParams& p,
+                      const SpeedyVertical& v, const Uniforms<R>& u, PhaseB<R, KX>& b, const Store& tape,
+                      const ColumnCt<R, KX>& ct, R a_rlds, ColumnAdj<R, KX>& g) {
+  const R ps = c.ps;
+  const R rps = mdiv(R(1.0), ps), a_rps = mrcp(ps);
+  const R stratc0 = c.stratz * ps, stratc1 = u.eps1 * ps;
+  R Fu[4], aD[4];
+  {
+    R fbt[4];
+    radset4(b.tsfc, u.omeps, fbt);
+    const R flux_h[4] = {b.flux_h[0], b.flux_h[1], R(0.0), R(0.0)};
 #pragma unroll
     for (int bnd = 0; bnd < 4; ++bnd) {
-      const R tau = Lk.tau[bnd], em = R(1.0) - tau;
-      const R a = aF[bnd] - a_dfl[k];            // dfl[k] += sum Fu[k+1] - sum Fu[k]
-      atau[bnd] = a * (Fk.get((k + 1) * 4 + bnd) - Lk.fb[bnd] * (Lk.st0 - R(2.0) * em * Lk.st1));
-      afb[bnd] = a * em * (Lk.st0 - em * Lk.st1);
-      as0 += a * em * Lk.fb[bnd];
-      as1 += -a * em * em * Lk.fb[bnd];
-      aF[bnd] = a_dfl[k] + a * tau;
-    }
-    g.T[k] += radset4_adj(c.T[k], u.omeps, afb);
-    lw_level_adj<R, KX>(k, atau, as0, as1, c, a, Lk.tau, p, v, u, g, a_Th);
-    settle_adj<R, KX>(g);
-    if constexpr (kSettle<KX>) {
-#pragma unroll
-      for (int j = 0; j < KX; ++j) settle(a_Th[j]);
-#pragma unroll
-      for (int bnd = 0; bnd < 4; ++bnd) settle(aF[bnd]);
+      Fu[bnd] = fbt[bnd] * b.rlus2 + u.refsfc * flux_h[bnd];
+      aD[bnd] = a_rlds * p.emisfc;
     }
   }
-  // surface source: Fu[KX] = fbt * rlus2 + refsfc * flux_h; dfl[KX-1] += epslw * rlus2
-  R fbt[4];
-  radset4(b.tsfc, u.omeps, fbt);
-  a_rlus2 += ((aF[0] * fbt[0] + aF[1] * fbt[1]) + (aF[2] * fbt[2] + aF[3] * fbt[3])) + a_dfl[KX - 1] * p.epslw;
-  a_flux_h[0] += aF[0] * u.refsfc;
-  a_flux_h[1] += aF[1] * u.refsfc;
+  b.dfl[KX - 1] = b.dfl[KX - 1] + p.epslw * b.rlus2;
+  R Gnext = ((Fu[0] + Fu[1]) + Fu[2]) + Fu[3];
+  // a_below: cotangent of the half-level temperature under level k, complete once
+  // level k is reversed, and then passed on to T
+  R a_below = R(0.0), corlw2 = R(0.0);
+#pragma unroll
+  for (int k = KX - 1; k >= 0; --k) {
+    const ColumnIn<R, KX> ck = column_at_level<R, KX>(c, k, Fu[0]);
+    const Store tk = tape.after(Fu[0]);
+    LwLevel<R> L;
+    lw_level<R, KX>(k, ck, a, p, v, u, L);
+    const R a_dfl = dfl_ct<R, KX>(ct, v, k, a_rps);
+    R afb[4], atau[4], as0 = R(0.0), as1 = R(0.0);
+    if (k == KX - 1) as0 = (a_rlds - a_dfl) * u.corlw;   // rlds += corlw, dfl[KX-1] -= corlw
+    if (k <= 1) {   // dfl[k] -= dhs[k] stratc1 st4a0[k] (+ stratc0 at k = 0)
+      as0 += -a_dfl * v.dhs[k] * stratc1;
+      g.ps += -a_dfl * v.dhs[k] * L.st0 * u.eps1;
+      if (k == 0) g.ps += -a_dfl * c.stratz;
+    }
+    if (k > 0) {
+#pragma unroll
+      for (int bnd = 0; bnd < 4; ++bnd) {
+        const R tau = L.tau[bnd], em = R(1.0) - tau;
+        const R au = tk.get((k - 1) * 8 + 4 + bnd), fd = tk.get((k - 1) * 8 + bnd);
+        const R ad = aD[bnd] - a_dfl;             // dfl[k] = sum Fd[k-1] - sum Fd[k]
+        aD[bnd] = a_dfl + ad * tau;
+        // up: tau Fu + em fb (st0 - em st1); down: tau Fd + em fb (st0 + em st1).  The flux
+        // and the emission nearly cancel: their difference is formed before the product
+        const R sum = au + ad, dif = ad - au;
+        const R es = em * L.st1, es2 = es + es;
+        atau[bnd] = au * (Fu[bnd] - L.fb[bnd] * (L.st0 - es2)) + ad * (fd - L.fb[bnd] * (L.st0 + es2));
+        afb[bnd] = em * (sum * L.st0 + dif * es);
+        const R ef = em * L.fb[bnd];
+        as0 += sum * ef;
+        as1 += dif * ef * em;
+        Fu[bnd] = L.tau[bnd] * Fu[bnd] + em * (L.fb[bnd] * (L.st0 - em * L.st1));
+      }
+      const R Gk = ((Fu[0] + Fu[1]) + Fu[2]) + Fu[3];
+      b.dfl[k] = b.dfl[k] + (Gnext - Gk);
+      Gnext = Gk;
+      if (k == 1) {
+        corlw2 = v.dhs[1] * stratc1 * L.st0;
+        b.dfl[1] = b.dfl[1] + (-corlw2);
+      }
+    } else {   // the top level absorbs and emits in bands 0 and 1 only (st1 = 0 there)
+      R ft[2];
+#pragma unroll
+      for (int bnd = 0; bnd < 2; ++bnd) {
+        const R em = R(1.0) - L.tau[bnd];
+        const R au = -a_dfl, ad = aD[bnd] - a_dfl;
+        const R sum = au + ad;
+        atau[bnd] = au * (Fu[bnd] - L.fb[bnd] * L.st0) - ad * (L.fb[bnd] * L.st0);
+        afb[bnd] = sum * em * L.st0;
+        as0 += sum * em * L.fb[bnd];
+        ft[bnd] = L.tau[bnd] * Fu[bnd] + em * (L.fb[bnd] * (L.st0 - em * L.st1));
+      }
+      atau[2] = atau[3] = afb[2] = afb[3] = R(0.0);
+      b.dfl[0] = b.dfl[0] + ((Fu[0] - ft[0]) + (Fu[1] - ft[1]));
+      const R corlw1 = v.dhs[0] * stratc1 * L.st0 + stratc0;
+      b.dfl[0] = b.dfl[0] + (-corlw1);
+    }
+    b.tlw[k] = b.dfl[k] * v.grdscp[k] * rps;
+    g.rps += ct.dt[k] * b.dfl[k] * v.grdscp[k];
+    g.T[k] += radset4_adj(ck.T[k], u.omeps, afb);
+    R a_Th[2] = {R(0.0), a_below};   // the half levels above (k - 1) and below (k)
+    lw_level_adj<R, KX>(k, atau, as0, as1, ck, a, L.tau, p, v, u, g, a_Th);
+    if (k < KX - 1) {   // Th[k] = T[k] + wvi1[k] (T[k+1] - T[k])
+      g.T[k] += a_Th[1] * (R(1.0) - u.wvi1[k]);
+      g.T[k + 1] += a_Th[1] * u.wvi1[k];
+    }
+    a_below = a_Th[0];
+    settle_lw<R, KX>(g, k, Fu, aD, a_below);
+  }
 }
 
 // ---------------------------------------------------------------- surface fluxes
@@ -305,7 +427,7 @@ SPD_HD void surface_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const 
                         const ColumnCt<R, KX>& ct, R a_rlus2, R& a_rsds, R& a_rlds, ColumnAdj<R, KX>& g) {
   if (!t.land) return;   // every surface output is zero without lfluxland (Q8)
   const R ps = c.ps;
-  const R rps = R(1.0) / ps;
+  const R rps = mrcp(ps);
   const R fm = c.fmask;
   const R gs = v.grdsig[KX - 1], gc = v.grdscp[KX - 1];
   const R a_ustr2 = ct.du1 * rps * gs, a_vstr2 = ct.dv1 * rps * gs;
@@ -319,13 +441,13 @@ SPD_HD void surface_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const 
   R a_rlus0 = fm * a_rlus2;
   R a_Tb = R(0.0), a_Qb = R(0.0), a_t1_0 = R(0.0), a_t1_1 = R(0.0), a_t2_0 = R(0.0), a_t2_1 = R(0.0);
   R a_den0 = R(0.0), a_den1 = R(0.0), a_den2 = R(0.0), a_tskin = R(0.0), a_qsat00 = R(0.0);
-  R dqt, dqp;
+  R dqt, dqp, a_psq = R(0.0);   // a_psq: sum of the qsat gradients times ps
   // sea
   a_den2 += a_evap1 * s.chs * (t.qsat01 - t.q1_1);
   const R a_qsat01 = a_evap1 * s.chs * t.den2;
   R a_q1_1 = -a_evap1 * s.chs * t.den2;
-  qsat_grad(c.sst, ps, R(1.0), dqt, dqp);
-  g.ps += a_qsat01 * dqp;
+  qsat_grad(c.sst, t.qsat01, dqt, dqp);
+  a_psq += a_qsat01 * dqp;
   a_den2 += a_shf1 * u.chscp * (c.sst - t.t1_1);
   a_t1_1 += -a_shf1 * u.chscp * t.den2;
   // land: sea-side stress and humidity
@@ -341,9 +463,9 @@ SPD_HD void surface_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const 
     const R qs = qsat_f(t.t1_1, ps, R(1.0));
     const R a_qs = a_q1_1 * s.fhum0 * a.rh[KX - 1];
     g.rh[KX - 1] += a_q1_1 * s.fhum0 * qs;
-    qsat_grad(t.t1_1, ps, R(1.0), dqt, dqp);
+    qsat_grad(t.t1_1, qs, dqt, dqp);
     a_t1_1 += a_qs * dqt;
-    g.ps += a_qs * dqp;
+    a_psq += a_qs * dqp;
     a_Qb += a_q1_1 * u.ghum0;
   } else {
     a_Qb += a_q1_1;
@@ -351,8 +473,8 @@ SPD_HD void surface_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const 
   a_den0 += a_den2 * (R(1.0) + t.dths * u.rdth);
   {
     const R a_dths = a_den2 * t.den0 * u.rdth;
-    const R a_ds = (c.sst > t.t2_1) ? a_dths * dmin_x(t.ds, R(s.dtheta))
-                                    : a_dths * dmax_x(u.astab * t.ds, -R(s.dtheta)) * u.astab;
+    const R a_ds = sel(c.sst > t.t2_1, a_dths * dmin_x(t.ds, R(s.dtheta)),
+                       a_dths * dmax_x(u.astab * t.ds, -R(s.dtheta)) * u.astab);
     a_t2_1 += -a_ds;
   }
   // skin-temperature energy-balance correction (surface_flux.py:189-221)
@@ -366,17 +488,17 @@ SPD_HD void surface_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const 
     a_drls += a_rlus0 * t.dtskin;
     a_dtskin += a_rlus0 * t.drls;
     const R Dn = t.clamb + t.drls + (s.chl * t.den1 * (R(CP) + (R(ALHC) * t.qs1)));
-    const R a_hflc = a_dtskin / Dn;
-    const R a_Dn = -a_dtskin * t.dtskin / Dn;
+    const R a_hflc = a_dtskin * mrcp(Dn);
+    const R a_Dn = -a_hflc * t.dtskin;
     a_drls += a_Dn;
     a_den1 += a_Dn * s.chl * (R(CP) + R(ALHC) * t.qs1);
     a_qs1 += a_Dn * s.chl * t.den1 * R(ALHC);
-    if (t.evap0a > R(0.0)) {
-      const R a_qs1p = a_qs1 * c.soilw;
-      a_qsat00 += -a_qs1 * c.soilw;
-      qsat_grad(t.tskin0 + R(1.0), ps, R(1.0), dqt, dqp);
+    {
+      const R a_qs1p = sel(t.evap0a > R(0.0), a_qs1 * c.soilw, R(0.0));
+      a_qsat00 += -a_qs1p;
+      qsat_grad(t.tskin0 + R(1.0), t.qs1p, dqt, dqp);
       a_tskin += a_qs1p * dqt;
-      g.ps += a_qs1p * dqp;
+      a_psq += a_qs1p * dqp;
     }
     a_hfl0 += a_hflc;
     a_tskin += -a_hflc * t.clamb;
@@ -396,16 +518,16 @@ SPD_HD void surface_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const 
     const R a_evx = a_evap0 * s.chl * t.den1 * dmax_x(t.evx, R(0.0));
     a_qsat00 += a_evx * c.soilw;
     const R a_q1_0 = -a_evx;
-    qsat_grad(t.tskin0, ps, R(1.0), dqt, dqp);
+    qsat_grad(t.tskin0, t.qsat00, dqt, dqp);
     a_tskin += a_qsat00 * dqt;
-    g.ps += a_qsat00 * dqp;
+    a_psq += a_qsat00 * dqp;
     if (s.fhum0 > R(0.0)) {
       const R qs = qsat_f(t.t1_0, ps, R(1.0));
       const R a_qs = a_q1_0 * s.fhum0 * a.rh[KX - 1];
       g.rh[KX - 1] += a_q1_0 * s.fhum0 * qs;
-      qsat_grad(t.t1_0, ps, R(1.0), dqt, dqp);
+      qsat_grad(t.t1_0, qs, dqt, dqp);
       a_t1_0 += a_qs * dqt;
-      g.ps += a_qs * dqp;
+      a_psq += a_qs * dqp;
       a_Qb += a_q1_0 * u.ghum0;
     } else {
       a_Qb += a_q1_0;
@@ -424,8 +546,8 @@ SPD_HD void surface_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const 
   a_den0 += a_den1 * (R(1.0) + t.dthl * u.rdth);
   {
     const R a_dthl = a_den1 * t.den0 * u.rdth;
-    const R a_dd = (t.tskin0 > t.t2_0) ? a_dthl * dmin_x(t.dd, R(s.dtheta))
-                                       : a_dthl * dmax_x(u.astab * t.dd, -R(s.dtheta)) * u.astab;
+    const R a_dd = sel(t.tskin0 > t.t2_0, a_dthl * dmin_x(t.dd, R(s.dtheta)),
+                       a_dthl * dmax_x(u.astab * t.dd, -R(s.dtheta)) * u.astab);
     a_tskin += a_dd;
     a_t2_0 += -a_dd;
   }
@@ -438,52 +560,76 @@ SPD_HD void surface_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const 
   // den0 = (p0 * ps / (rgas * t0)) * wind
   R a_t0;
   {
-    const R rho = R(P0) * ps / (R(RGAS) * t.t0);
+    const R rt0 = mrcp(t.t0);
+    const R rho_ps = R(P0 / RGAS) * rt0;
+    const R rho = rho_ps * ps;
     const R a_rho = a_den0 * t.wind;
     const R a_wind = a_den0 * rho;
-    g.ps += a_rho * (R(P0) / (R(RGAS) * t.t0));
-    a_t0 = -a_rho * rho / t.t0;
-    g.u1 += a_wind * t.u0 / t.wind * s.fwind0;
-    g.v1 += a_wind * t.v0 / t.wind * s.fwind0;
+    g.ps += a_rho * rho_ps;
+    a_t0 = -a_rho * rho * rt0;
+    const R aw = a_wind * mrcp(t.wind) * s.fwind0;
+    g.u1 += aw * t.u0;
+    g.v1 += aw * t.v0;
   }
   a_t1_0 += a_t0 * fm;
   a_t1_1 += a_t0 * om;
-  R a_t1_0a = R(0.0), a_t1_1a = R(0.0);
-  if (t.warm) {
-    a_t1_0a = a_t1_0 * s.ftemp0;
-    a_t2_0 += a_t1_0 * u.gtemp0;
-    a_t1_1a = a_t1_1 * s.ftemp0;
-    a_t2_1 += a_t1_1 * u.gtemp0;
-  } else {
-    a_Tb += a_t1_0 + a_t1_1;
-  }
+  const R aw0 = sel(t.warm, a_t1_0, R(0.0)), aw1 = sel(t.warm, a_t1_1, R(0.0));
+  R a_t1_0a = aw0 * s.ftemp0;
+  const R a_t1_1a = aw1 * s.ftemp0;
+  a_t2_0 += aw0 * u.gtemp0;
+  a_t2_1 += aw1 * u.gtemp0;
+  a_Tb += sel(t.warm, R(0.0), a_t1_0 + a_t1_1);
   a_t2_1 += a_t2_0;
   a_Tb += a_t2_1;
   a_t1_0a += a_t1_1a;
-  R a_dt1 = -a_t1_1a * t.phi0 / (R(RGAS288) * v.sigl[KX - 1]);
+  R a_dt1 = -a_t1_1a * t.phi0 * mrcp(R(RGAS288) * v.sigl[KX - 1]);
   a_Tb += a_t1_0a;
   a_dt1 += a_t1_0a;
   a_Tb += a_dt1 * v.wvi[KX - 1][1];
+  g.ps += a_psq * rps;
   g.T[KX - 2] += -a_dt1 * v.wvi[KX - 1][1];
   g.T[KX - 1] += a_Tb;
   g.Q[KX - 1] += a_Qb;
 }
 
 // ---------------------------------------------------------------- shortwave
+// Only the transmissivities are kept from the forward (and a few scalars): the
+// fluxes are their products, 45 instructions to form again against 32 values held
+// across the surface fluxes and their reversal.
 template <typename R, int KX>
 SPD_HD void shortwave_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const PhaseB<R, KX>& b, uint32_t S,
                           const SpeedyParams& p, const SpeedyVertical& v, const Uniforms<R>& u,
-                          const SwTape<R, KX>& t, const ColumnCt<R, KX>& ct, const R a_flux_h[2], R a_rsds,
+                          const SwTape<R, KX>& fwd, const ColumnCt<R, KX>& ct, const R a_flux_h[2], R a_rsds,
                           ColumnAdj<R, KX>& g) {
   const R ps = c.ps;
-  const R rps = R(1.0) / ps;
+  const R rps = mrcp(ps);
+  SwTape<R, KX> t;
+  t.psaz = fwd.psaz;
+  t.acloud = fwd.acloud;
+#pragma unroll
+  for (int k = 0; k < KX; ++k) {
+    t.tau0[k] = fwd.tau0[k];
+    t.tau1[k] = fwd.tau1[k];
+    settle(t.tau0[k]);   // not the forward's registers: its products are not kept for the ones below
+    if (k > 0) settle(t.tau1[k]);
+    t.t22[k] = k == KX - 1 ? p.albcls * a.clstr : sel(((S >> k) & 1u) != 0u, fwd.a_cl, R(0.0));
+  }
+  const R F0 = c.fsol * R(0.95);
+  t.f1[0] = t.tau0[0] * (F0 - c.ozupp * ps);
+  t.f1[1] = t.tau0[1] * (t.f1[0] - c.ozone * ps);
+  t.f2[0] = c.fsol * R(0.05);
+#pragma unroll
+  for (int k = 1; k < KX; ++k) {
+    if (k > 1) t.f1[k] = t.f1[k - 1] * t.tau0[k] * (R(1.0) - t.t22[k]);
+    t.f2[k] = t.f2[k - 1] * t.tau1[k];
+  }
+  t.fu[KX - 1] = t.f1[KX - 1] * b.albsfc;
+#pragma unroll
+  for (int k = KX - 1; k >= 1; --k) t.fu[k - 1] = t.fu[k] * t.tau0[k] + (k > 1 ? t.t22[k] * t.f1[k - 1] : t.t22[k]);
   const bool csw = u.compute_sw != 0u;
   R a_dfabs[KX];
 #pragma unroll
-  for (int k = 0; k < KX; ++k) {
-    a_dfabs[k] = csw ? ct.dt[k] * v.grdscp[k] * rps : R(0.0);
-    if (csw) g.rps += ct.dt[k] * t.dfabs[k] * v.grdscp[k];
-  }
+  for (int k = 0; k < KX; ++k) a_dfabs[k] = sel(csw, ct.dt[k], R(0.0)) * v.grdscp[k] * rps;
   R a_tau0[KX], a_tau1[KX], a_f1[KX], a_f2[KX], a_Rf[KX], a_fu[KX], a_t22[KX];
 #pragma unroll
   for (int k = 0; k < KX; ++k) {
@@ -539,7 +685,6 @@ SPD_HD void shortwave_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, cons
   a_f1[0] += a_f1[1] * t.tau0[1];
   g.ps += -a_f1[1] * t.tau0[1] * c.ozone;
   a_f1[0] += -a_dfabs[0];
-  const R F0 = c.fsol * R(0.95);
   a_tau0[0] += a_f1[0] * (F0 - c.ozupp * ps);
   g.ps += -a_f1[0] * t.tau0[0] * c.ozupp;
   // transmissivities
@@ -547,13 +692,14 @@ SPD_HD void shortwave_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, cons
   a_psaz += a_tau0[0] * t.tau0[0] * (-(v.dhs[0] * p.absdry));
 #pragma unroll
   for (int k = 1; k < KX; ++k) {
-    const R cl = (k <= KX - 2 && k >= a.icltop) ? t.acloud : R(0.0);
+    const bool cloudy = k <= KX - 2 && k >= a.icltop;
+    const R cl = sel(cloudy, t.acloud, R(0.0));
     const R A = u.sw_abs1[k] + p.abswv1 * c.Q[k] + cl;
     const R ax = a_tau0[k] * t.tau0[k];
     a_psaz += ax * (-(v.dhs[k] * A));
     const R a_A = ax * (-(t.psaz * v.dhs[k]));
     g.Q[k] += a_A * p.abswv1;
-    if (k <= KX - 2 && k >= a.icltop) a_acloud += a_A;
+    a_acloud += sel(cloudy, a_A, R(0.0));
     const R bx = a_tau1[k] * t.tau1[k];
     a_psaz += bx * (-(v.dhs[k] * p.abswv2 * c.Q[k]));
     g.Q[k] += bx * (-(t.psaz * v.dhs[k] * p.abswv2));
@@ -568,76 +714,9 @@ SPD_HD void shortwave_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, cons
   R a_acl = R(0.0);
 #pragma unroll
   for (int k = 0; k < KX - 1; ++k)
-    if ((S >> k) & 1u) a_acl += a_t22[k];
+    a_acl += sel(((S >> k) & 1u) != 0u, a_t22[k], R(0.0));
   g.clstr += a_t22[KX - 1] * p.albcls;
-  if (a.icltop < KX) g.cloudc += a_acl * p.albcl;
-}
-
-// ---------------------------------------------------------------- longwave down
-// As lw_up_adj, each level's longwave quantities are recomputed (lw_level).
-template <typename R, int KX, class Store>
-SPD_HD void lw_down_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const SpeedyParams& p,
-                        const SpeedyVertical& v, const Uniforms<R>& u, const Store& Fd, const R a_dfl[KX], R a_rlds,
-                        ColumnAdj<R, KX>& g, R a_Th[KX]) {
-  R aF[4];
-#pragma unroll
-  for (int bnd = 0; bnd < 4; ++bnd) aF[bnd] = a_rlds * p.emisfc;
-#pragma unroll
-  for (int k = KX - 1; k >= 1; --k) {
-    LwLevel<R> Lk;
-    lw_level<R, KX>(k, column_at_level<R, KX>(c, k, aF[0]), a, p, v, u, Lk);
-    R afb[4], atau[4];
-    // rlds = sum_b emisfc * Fd[KX-1][b] + corlw; dfl[KX-1] -= corlw; corlw = corlw_u * st4a0[KX-1]
-    R as0 = (k == KX - 1) ? (a_rlds - a_dfl[KX - 1]) * u.corlw : R(0.0), as1 = R(0.0);
-    const auto Fk = Fd.after(aF[0]);   // Fd[k-1] read when level k is reversed
-#pragma unroll
-    for (int bnd = 0; bnd < 4; ++bnd) {
-      const R tau = Lk.tau[bnd], em = R(1.0) - tau;
-      const R a = aF[bnd] - a_dfl[k];           // dfl[k] = sum Fd[k-1] - sum Fd[k]
-      atau[bnd] = a * (Fk.get((k - 1) * 4 + bnd) - Lk.fb[bnd] * (Lk.st0 + R(2.0) * em * Lk.st1));
-      afb[bnd] = a * em * (Lk.st0 + em * Lk.st1);
-      as0 += a * em * Lk.fb[bnd];
-      as1 += a * em * em * Lk.fb[bnd];
-      aF[bnd] = a_dfl[k] + a * tau;
-    }
-    g.T[k] += radset4_adj(c.T[k], u.omeps, afb);
-    lw_level_adj<R, KX>(k, atau, as0, as1, c, a, Lk.tau, p, v, u, g, a_Th);
-    settle_adj<R, KX>(g);
-    if constexpr (kSettle<KX>) {
-#pragma unroll
-      for (int j = 0; j < KX; ++j) settle(a_Th[j]);
-#pragma unroll
-      for (int bnd = 0; bnd < 4; ++bnd) settle(aF[bnd]);
-    }
-  }
-  {
-    LwLevel<R> L0;
-    lw_level<R, KX>(0, column_at_level<R, KX>(c, 0, aF[0]), a, p, v, u, L0);
-    R afb[4] = {R(0.0), R(0.0), R(0.0), R(0.0)};
-    R atau[4] = {R(0.0), R(0.0), R(0.0), R(0.0)};
-    R as0 = R(0.0), as1 = R(0.0);
-#pragma unroll
-    for (int bnd = 0; bnd < 2; ++bnd) {
-      const R tau = L0.tau[bnd], em = R(1.0) - tau;
-      const R a = aF[bnd] - a_dfl[0];
-      atau[bnd] = -a * L0.fb[bnd] * (L0.st0 + R(2.0) * em * L0.st1);
-      afb[bnd] = a * em * (L0.st0 + em * L0.st1);
-      as0 += a * em * L0.fb[bnd];
-      as1 += a * em * em * L0.fb[bnd];
-    }
-    g.T[0] += radset4_adj(c.T[0], u.omeps, afb);
-    lw_level_adj<R, KX>(0, atau, as0, as1, c, a, L0.tau, p, v, u, g, a_Th);
-  }
-}
-
-// Half-level temperatures Th[k] = T[k] + wvi1[k] * (T[k+1] - T[k]) back to T.
-template <typename R, int KX>
-SPD_HD void half_level_adj(const Uniforms<R>& u, const R a_Th[KX], ColumnAdj<R, KX>& g) {
-#pragma unroll
-  for (int k = 0; k < KX - 1; ++k) {
-    g.T[k] += a_Th[k] * (R(1.0) - u.wvi1[k]);
-    g.T[k + 1] += a_Th[k] * u.wvi1[k];
-  }
+  g.cloudc += sel(a.icltop < KX, a_acl * p.albcl, R(0.0));
 }
 
 // ---------------------------------------------------------------- vertical diffusion
@@ -652,42 +731,35 @@ SPD_HD void vdiff_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const Sp
   for (int k = NL1 - 1; k >= 0; --k) {
     suf = suf + ct.dt[k + 1];
     const R se0 = a.se[k + 1] - p.segrad * (c.PHI[k + 1] - c.PHI[k]);
-    if (a.se[k] < se0) {
-      const R a_fse = ct.dt[k] * u.rsig[k] - suf * u.rsig1[k];
-      const R a_x = a_fse * u.fvdise;
-      g.se[k + 1] += a_x;
-      g.se[k] += -a_x;
-    }
+    const R a_fse = ct.dt[k] * u.rsig[k] - suf * u.rsig1[k];
+    const R a_x = sel(a.se[k] < se0, a_fse * u.fvdise, R(0.0));
+    g.se[k + 1] += a_x;
+    g.se[k] += -a_x;
   }
   // moisture diffusion above the PBL
 #pragma unroll
   for (int k = 2; k < KX - 2; ++k) {
     const R d = a.rh[k + 1] - a.rh[k];
-    if (d >= u.vd_drh0[k] && ((u.vd_on >> k) & 1u)) {
-      const R a_fq = ct.dq[k] * u.rsig[k] - ct.dq[k + 1] * u.rsig[k + 1];
-      g.qsat[k] += a_fq * u.vd_fq[k] * d;
-      const R a_d = a_fq * u.vd_fq[k] * a.qsat[k];
-      g.rh[k + 1] += a_d;
-      g.rh[k] += -a_d;
-    }
+    const bool on = (d >= u.vd_drh0[k]) & (((u.vd_on >> k) & 1u) != 0u);
+    const R a_fq = sel(on, ct.dq[k] * u.rsig[k] - ct.dq[k + 1] * u.rsig[k + 1], R(0.0));
+    g.qsat[k] += a_fq * u.vd_fq[k] * d;
+    const R a_d = a_fq * u.vd_fq[k] * a.qsat[k];
+    g.rh[k + 1] += a_d;
+    g.rh[k] += -a_d;
   }
   // shallow convection / PBL moisture exchange between the two lowest levels
   const R dmse = a.se[KX - 1] - a.se[NL1 - 1] + R(ALHC) * (c.Q[KX - 1] - a.qsat[NL1 - 1]);
   const R drh = a.rh[KX - 1] - a.rh[NL1 - 1];
-  const R fcnv = (icnv > 0 && dmse >= R(0.0)) ? p.redshc : R(1.0);
+  const bool up = dmse >= R(0.0);
+  const R fcnv = sel((icnv > 0) & up, R(p.redshc), R(1.0));
   const R rsA = u.rsig[NL1 - 1], rsB = u.rsig[KX - 1];
-  R a_dmse = R(0.0), a_drh = R(0.0);
   const R a_fq2 = ct.dq[NL1 - 1] * rsA - ct.dq[KX - 1] * rsB;
-  if (dmse >= R(0.0)) {
-    a_dmse = (ct.dt[NL1 - 1] * rsA - ct.dt[KX - 1] * rsB) * fcnv * u.fshcse;
-    if (drh >= R(0.0)) {
-      g.qsat[KX - 1] += a_fq2 * fcnv * u.fshcq * drh;
-      a_drh = a_fq2 * fcnv * u.fshcq * a.qsat[KX - 1];
-    }
-  } else if (drh > u.drh0) {
-    g.qsat[NL1 - 1] += a_fq2 * u.fvdiq2 * drh;
-    a_drh = a_fq2 * u.fvdiq2 * a.qsat[NL1 - 1];
-  }
+  const R a_dmse = sel(up, (ct.dt[NL1 - 1] * rsA - ct.dt[KX - 1] * rsB) * fcnv * u.fshcse, R(0.0));
+  const R a_up = sel(up & (drh >= R(0.0)), a_fq2 * fcnv * u.fshcq, R(0.0));
+  const R a_dn = sel(!up & (drh > u.drh0), a_fq2 * u.fvdiq2, R(0.0));
+  g.qsat[KX - 1] += a_up * drh;
+  g.qsat[NL1 - 1] += a_dn * drh;
+  const R a_drh = a_up * a.qsat[KX - 1] + a_dn * a.qsat[NL1 - 1];
   g.se[KX - 1] += a_dmse;
   g.se[NL1 - 1] += -a_dmse;
   g.Q[KX - 1] += a_dmse * R(ALHC);
@@ -710,13 +782,13 @@ SPD_HD void clouds_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const S
   const R a_cc = g.cloudc - R(1.2) * a_clsx;
   const R a_fsa = a_fstab * dmin_x(mmax(t.fstab_arg, R(0.0)), R(1.0)) * dmax_x(t.fstab_arg, R(0.0));
   const R a_gse = a_fsa * u.rgse;
-  const R rdphi = R(1.0) / (c.PHI[KX - 2] - c.PHI[KX - 1]);
+  const R rdphi = mrcp(c.PHI[KX - 2] - c.PHI[KX - 1]);
   g.se[KX - 2] += a_gse * rdphi;
   g.se[KX - 1] += -a_gse * rdphi;
   g.Q[KX - 2] += g.qcloud;
   const R a_raw = a_cc * dmin_x(t.ccraw, R(1.0));
   const R mx = mmax(R(EPS), t.pr1);
-  const R a_pr1 = a_raw * p.wpcl * (R(0.5) / msqrt_1ulp(mx)) * dmax_x(t.pr1, R(EPS));
+  const R a_pr1 = a_raw * p.wpcl * (R(0.5) * mrcp(msqrt_1ulp(mx))) * dmax_x(t.pr1, R(EPS));
   const R a_sum = a_pr1 * dmin_x(R(86.4) * (a.precnv + a.precls), R(p.pmaxcl)) * R(86.4);
   g.precnv += a_sum;
   g.precls += a_sum;
@@ -725,16 +797,16 @@ SPD_HD void clouds_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const S
   int nt = 0;
 #pragma unroll
   for (int k = 2; k <= KX - 3; ++k) nt += (t.cu[k] == t.cmax) ? 1 : 0;
-  const R share = a_cmax / R(nt > 0 ? nt : 1);
+  const R share = a_cmax * mrcp(R(nt > 0 ? nt : 1));
   R a_cc0 = R(0.0);
 #pragma unroll
   for (int k = 2; k <= KX - 3; ++k) {
-    if (t.cu[k] == t.cmax) {
-      if ((t.mk >> k) & 1u) g.rh[k] += share;
-      else a_cc0 += share;
-    }
+    const R part = sel(t.cu[k] == t.cmax, share, R(0.0));
+    const bool own = ((t.mk >> k) & 1u) != 0u;
+    g.rh[k] += sel(own, part, R(0.0));
+    a_cc0 += sel(own, R(0.0), part);
   }
-  if (t.m0) g.rh[KX - 2] += a_cc0;
+  g.rh[KX - 2] += sel(t.m0, a_cc0, R(0.0));
 }
 
 // ---------------------------------------------------------------- condensation
@@ -747,7 +819,7 @@ SPD_HD void condensation_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, c
 #pragma unroll
   for (int k = 1; k < KX; ++k) {
     const R dqa = u.rhref[k] * a.qsat[k] - c.Q[k];
-    qlsc[k] = dqa < R(0.0) ? dqa * u.rtlsc : R(0.0);
+    qlsc[k] = sel(dqa < R(0.0), dqa * u.rtlsc, R(0.0));
   }
   R sum = R(0.0);
 #pragma unroll
@@ -758,17 +830,16 @@ SPD_HD void condensation_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, c
 #pragma unroll
   for (int k = 1; k < KX; ++k) {
     const R dqa = u.rhref[k] * a.qsat[k] - c.Q[k];
-    if (dqa < R(0.0)) {
-      const R dq = qlsc[k];
-      const R cap = u.dqmax[k] * psa2;
-      const R a_m = ct.dt[k] * R(TFACT);
-      const R a_dq = ct.dq[k] + a_sum * u.pfact[k] - a_m * dmin_x(-dq, cap);
-      a_psa2 += a_m * dmin_x(cap, -dq) * u.dqmax[k];
-      const R a_dqa = a_dq * u.rtlsc;
-      g.qsat[k] += a_dqa * u.rhref[k];
-      g.Q[k] += -a_dqa;
-      g.prm[VJP_RHLSC] += a_dqa * a.qsat[k] * u.rhref_d[k];
-    }
+    const bool on = dqa < R(0.0);
+    const R dq = qlsc[k];
+    const R cap = u.dqmax[k] * psa2;
+    const R a_m = ct.dt[k] * R(TFACT);
+    const R a_dq = ct.dq[k] + a_sum * u.pfact[k] - a_m * dmin_x(-dq, cap);
+    a_psa2 += sel(on, a_m * dmin_x(cap, -dq) * u.dqmax[k], R(0.0));
+    const R a_dqa = sel(on, a_dq * u.rtlsc, R(0.0));
+    g.qsat[k] += a_dqa * u.rhref[k];
+    g.Q[k] += -a_dqa;
+    g.prm[VJP_RHLSC] += a_dqa * a.qsat[k] * u.rhref_d[k];
   }
   g.ps += a_psa2 * R(2.0) * ps;
 }
@@ -780,7 +851,7 @@ SPD_HD void convection_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, con
                            const ColumnCt<R, KX>& ct, ColumnAdj<R, KX>& g) {
   const int iptop = a.iptop_conv;
   const R ps = c.ps;
-  const R rps = R(1.0) / ps;
+  const R rps = mrcp(ps);
   R a_dfse[KX], a_dfqa[KX];
   a_dfse[0] = ct.dt[0];
   a_dfqa[0] = ct.dq[0];
@@ -794,10 +865,13 @@ SPD_HD void convection_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, con
   R a_top_s = R(0.0), a_top_q = R(0.0);
 #pragma unroll
   for (int k = 0; k < KX; ++k)
-    if (iptop - 1 == k) {
-      a_top_s = a_dfse[k]; a_top_q = a_dfqa[k];
-      a_dfse[k] = R(0.0); a_dfqa[k] = R(0.0);
-    }
+  {
+    const bool at = iptop - 1 == k;
+    a_top_s = sel(at, a_dfse[k], a_top_s);
+    a_top_q = sel(at, a_dfqa[k], a_top_q);
+    a_dfse[k] = sel(at, R(0.0), a_dfse[k]);
+    a_dfqa[k] = sel(at, R(0.0), a_dfqa[k]);
+  }
   R a_fm_t = R(0.0), a_fus_t = a_top_s, a_fds_t = -a_top_s, a_fuq_t = a_top_q, a_fdq_t = -a_top_q;
   {
     const R a_pr = g.precnv + R(ALHC) * a_top_s - a_top_q;
@@ -807,11 +881,11 @@ SPD_HD void convection_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, con
     a_fm_t += -a_P * t.qsatb;
     const R a_qsatb = -a_P * t.fm_t;
 #pragma unroll
-    for (int k = 0; k < KX - 1; ++k)
-      if (iptop - 1 == k) {
-        g.qsat[k] += a_qsatb * (R(1.0) - u.wvi1[k]);
-        g.qsat[k + 1] += a_qsatb * u.wvi1[k];
-      }
+    for (int k = 0; k < KX - 1; ++k) {
+      const R aq = sel(iptop - 1 == k, a_qsatb, R(0.0));
+      g.qsat[k] += aq * (R(1.0) - u.wvi1[k]);
+      g.qsat[k + 1] += aq * u.wvi1[k];
+    }
   }
   R a_FM[KX], a_FUS[KX], a_FUQ[KX], a_FDS[KX], a_FDQ[KX];
 #pragma unroll
@@ -828,18 +902,16 @@ SPD_HD void convection_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, con
 #pragma unroll
   for (int k = 0; k < KX - 1; ++k) {
     const R a_fsq = a_dfqa[k] - a_dfqa[KX - 1];
-    if (t.delq[k] > R(0.0)) {
-      a_cbmf += a_fsq * p.smf * t.delq[k];
-      const R a_delq = a_fsq * p.smf * a.cbmf;
-      g.qsat[k] += a_delq * p.rhil;
-      g.Q[k] += -a_delq;
-    }
-    if (k >= iptop) {
-      a_FUS[k + 1] += a_dfse[k]; a_FDS[k + 1] += -a_dfse[k];
-      a_FUS[k] += -a_dfse[k]; a_FDS[k] += a_dfse[k];
-      a_FUQ[k + 1] += a_dfqa[k]; a_FDQ[k + 1] += -a_dfqa[k];
-      a_FUQ[k] += -a_dfqa[k]; a_FDQ[k] += a_dfqa[k];
-    }
+    const R a_s = sel(t.delq[k] > R(0.0), a_fsq * p.smf, R(0.0));
+    a_cbmf += a_s * t.delq[k];
+    const R a_delq = a_s * a.cbmf;
+    g.qsat[k] += a_delq * p.rhil;
+    g.Q[k] += -a_delq;
+    const R as = sel(k >= iptop, a_dfse[k], R(0.0)), aq = sel(k >= iptop, a_dfqa[k], R(0.0));
+    a_FUS[k + 1] += as; a_FDS[k + 1] += -as;
+    a_FUS[k] += -as; a_FDS[k] += as;
+    a_FUQ[k + 1] += aq; a_FDQ[k + 1] += -aq;
+    a_FUQ[k] += -aq; a_FDQ[k] += aq;
   }
   R a_fds = a_dfse[KX - 1] + a_FDS[KX - 1], a_fus = -a_dfse[KX - 1];
   R a_fdq = a_dfqa[KX - 1] + a_FDQ[KX - 1], a_fuq = -a_dfqa[KX - 1];
@@ -864,10 +936,10 @@ SPD_HD void convection_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, con
       const R a_en = pm + pS * a.se[j] + pQ * c.Q[j];
       g.se[j] += pS * t.en[j];
       g.Q[j] += pQ * t.en[j];
-      const bool lm = (j <= KX - 2) && (j >= iptop) && (j >= 1);
-      if (lm) {
-        g.ps += a_en * u.entr[j] * a.cbmf;
-        a_cbmf += a_en * u.entr[j] * ps;
+      if (j >= 1 && j <= KX - 2) {
+        const R ae = sel(j >= iptop, a_en * u.entr[j], R(0.0));
+        g.ps += ae * a.cbmf;
+        a_cbmf += ae * ps;
       }
     }
     a_fmass += pm;
@@ -880,21 +952,22 @@ SPD_HD void convection_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, con
   R a_qmax = a_fuq * t.fmass;
   const R a_sb = a_fds * t.fmass;
   R a_qb = a_fdq * t.fmass;
-  if (iptop < KX) a_fmass += a_cbmf;
+  a_fmass += sel(iptop < KX, a_cbmf, R(0.0));
   // fmass = fm0 * fpsa * min(5, qdif / (qmax - qb))
   R a_qdif;
   {
     const R den = t.qmax - t.qb;
-    const R ratio = t.qdif / den;
+    const R rden = mrcp(den);
+    const R ratio = mdiv(t.qdif, den);
     const R m = mmin(R(5.0), ratio);
     const R a_fpsa = a_fmass * u.fm0 * m;
     const R a_fm0 = a_fmass * t.fpsa * m;
     const R a_ratio = a_fmass * u.fm0 * t.fpsa * dmin_x(ratio, R(5.0));
-    a_qdif = a_ratio / den;
-    const R a_den = -a_ratio * ratio / den;
+    a_qdif = a_ratio * rden;
+    const R a_den = -a_ratio * ratio * rden;
     a_qmax += a_den;
     a_qb += -a_den;
-    g.prm[VJP_TRCNV] += a_fm0 * (-(u.fm0 / p.trcnv));
+    g.prm[VJP_TRCNV] += a_fm0 * (-(u.fm0 * mrcp(R(p.trcnv))));
     const R y = (ps - p.psmin) * u.rdps;
     g.ps += a_fpsa * mmin(R(1.0), y) + a_fpsa * ps * dmin_x(y, R(1.0)) * u.rdps;
   }
@@ -917,51 +990,44 @@ SPD_HD void convection_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, con
     g.qsat[KX - 1] += a_qmax * dmax_x(a.qsat[KX - 1], q1);
   }
   // qdif (diagnose_convection)
-  R a_qthr0 = R(0.0), a_mse0 = R(0.0), a_msthr = R(0.0);
-  if (t.case1) {
-    const R A = c.Q[KX - 1] - t.qthr0;
-    const R B = (t.mse0 - t.msthr) * R(RLHC);
-    const R a_A = a_qdif * dmax_x(A, B), a_B = a_qdif * dmax_x(B, A);
-    g.Q[KX - 1] += a_A;
-    a_qthr0 = -a_A;
-    a_mse0 = a_B * R(RLHC);
-    a_msthr = -a_B * R(RLHC);
-  } else if (t.case2) {
-    g.Q[KX - 1] += a_qdif;
-    a_qthr0 = -a_qdif;
-  }
+  const R A = c.Q[KX - 1] - t.qthr0;
+  const R B = (t.mse0 - t.msthr) * R(RLHC);
+  const R a_A = sel(t.case1, a_qdif * dmax_x(A, B), sel(t.case2, a_qdif, R(0.0)));
+  const R a_B = sel(t.case1, a_qdif * dmax_x(B, A), R(0.0));
+  g.Q[KX - 1] += a_A;
+  const R a_qthr0 = -a_A, a_mse0 = a_B * R(RLHC), a_msthr = -a_B * R(RLHC);
   g.prm[VJP_RHBL] += a_qthr0 * a.qsat[KX - 1];
   g.qsat[KX - 1] += a_qthr0 * p.rhbl;
   g.se[KX - 1] += a_mse0;
   g.Q[KX - 1] += a_mse0 * R(ALHC);
 #pragma unroll
-  for (int k = 2; k <= KX - 4; ++k)
-    if (t.ktop2 == k + 1) {   // msthr = mss2[k], mss = se + alhc * qsat
-      const R w = u.wvi1[k];
-      const R am0 = a_msthr * (R(1.0) - w), am1 = a_msthr * w;
-      g.se[k] += am0;
-      g.qsat[k] += am0 * R(ALHC);
-      g.se[k + 1] += am1;
-      g.qsat[k + 1] += am1 * R(ALHC);
-    }
+  for (int k = 2; k <= KX - 4; ++k) {   // msthr = mss2[k] at k = ktop2 - 1, mss = se + alhc * qsat
+    const R w = u.wvi1[k];
+    const R am = sel(t.ktop2 == k + 1, a_msthr, R(0.0));
+    const R am0 = am * (R(1.0) - w), am1 = am * w;
+    g.se[k] += am0;
+    g.qsat[k] += am0 * R(ALHC);
+    g.se[k + 1] += am1;
+    g.qsat[k + 1] += am1 * R(ALHC);
+  }
 }
 
 // humidity, static energy and 1/ps back to the state.
 template <typename R, int KX>
-SPD_HD void humidity_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const SpeedyVertical& v,
-                         ColumnAdj<R, KX>& g) {
+SPD_HD void humidity_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, ColumnAdj<R, KX>& g) {
+  const R rps = mrcp(c.ps);
+  R a_psq = R(0.0);
 #pragma unroll
   for (int k = 0; k < KX; ++k) {
-    const R rq = R(1.0) / a.qsat[k];
-    g.Q[k] += g.rh[k] * rq;
-    const R a_qs = g.qsat[k] - g.rh[k] * a.rh[k] * rq;
+    const R a_q = g.rh[k] * mrcp(a.qsat[k]);   // rh = Q / qsat
+    g.Q[k] += a_q;
+    const R a_qs = g.qsat[k] - a_q * a.rh[k];
     R dqt, dqp;
-    qsat_grad(c.T[k], c.ps, R(v.fsg[k]), dqt, dqp);
+    qsat_grad(c.T[k], a.qsat[k], dqt, dqp);
     g.T[k] += a_qs * dqt + R(CP) * g.se[k];
-    g.ps += a_qs * dqp;
+    a_psq += a_qs * dqp;
   }
-  const R rps = R(1.0) / c.ps;
-  g.ps += -g.rps * rps * rps;
+  g.ps += a_psq * rps - g.rps * rps * rps;
 }
 
 // Per-column storage for the longwave flux tapes between a term's recompute and
@@ -974,104 +1040,61 @@ struct ArrayStore {
   SPD_HD const ArrayStore& after(R) const { return *this; }
 };
 
-// A copy of the column whose values the optimizer cannot see through: a term
-// recomputed from it is not merged with the same computation elsewhere in the
-// kernel (which would keep that term's intermediates live in between).
+// What phase b2 hands from its forward to its reversal.
 template <typename R, int KX>
-SPD_HD ColumnIn<R, KX> opaque_column(const ColumnIn<R, KX>& c_in) {
-  ColumnIn<R, KX> c = c_in;
-#if defined(__HIP_DEVICE_COMPILE__)
-#pragma unroll
-  for (int k = 0; k < KX; ++k) {
-    asm volatile("" : "+v"(c.T[k]));
-    asm volatile("" : "+v"(c.Q[k]));
-    asm volatile("" : "+v"(c.PHI[k]));
-  }
-  asm volatile("" : "+v"(c.ps));
-#endif
-  return c;
+struct VjpTapeB {
+  SwTape<R, KX> sw;
+  SfcTape<R> sf;
+  R aF[4];       // adjoint of the upward longwave fluxes at the surface
+};
+
+// Forward + VJP of phase b1: the forward of phase_b1 (b.dfl, b.rlds, albedos, vertical
+// diffusion) with the longwave's down sweep.  Clears g.
+template <typename R, int KX, class Store>
+SPD_HD void phase_b1_vjp(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const SpeedyParams& p,
+                         const SpeedyVertical& v, const Uniforms<R>& u, const ColumnCt<R, KX>& ct, PhaseB<R, KX>& b,
+                         ColumnAdj<R, KX>& g, VjpTapeB<R, KX>& t, Store& tape) {
+  adj_zero<R, KX>(g);
+  albedos<R, KX>(c, p, b);
+  lw_down_vjp<R, KX>(c, a, p, v, u, ct, b, tape, t.aF);
+  vdiff<R, KX>(c, a, p, u, b);
 }
 
-// The whole column: given the forward's phase outputs (a: phase A; b: phase B's
-// scalars, the longwave-down divergence in b.dfl and the hand-offs flux_h, rlus2,
-// tsfc) and the cotangents, accumulate the gradients into g.  The longwave
-// transmissivities and emissions are recomputed where the longwave terms are
-// reversed, from their own opaque copies of the column, rather than read from b.
+// The forward of the shortwave and the surface fluxes, with their tapes.
+template <typename R, int KX>
+SPD_HD void phase_b2_taped(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, uint32_t S, const SpeedyParams& p,
+                           const SpeedyVertical& v, const Uniforms<R>& u, uint32_t flags, const ColumnCt<R, KX>& ct,
+                           PhaseB<R, KX>& b, ColumnAdj<R, KX>& g, VjpTapeB<R, KX>& t) {
+  R flux_h[4];
+  shortwave<R, KX, false>(c, a, S, p, v, u, b, flux_h, t.sw);
+#pragma unroll
+  for (int k = 0; k < KX; ++k)   // tsw[k] = dfabs[k] grdscp[k] / ps
+    g.rps += sel(u.compute_sw != 0u, ct.dt[k], R(0.0)) * t.sw.dfabs[k] * v.grdscp[k];
+  R tsfc;
+  surface<R, KX, false>(c, a, p, v, u, flags, b, tsfc, t.sf);
+  b.flux_h[0] = flux_h[0]; b.flux_h[1] = flux_h[1]; b.rlus2 = t.sf.rlus2; b.tsfc = tsfc;
+}
+
+// Reversal of the surface fluxes and the shortwave, then the longwave's up sweep
+// (which also leaves the forward's b.tlw).  ct.dq as verify_ct left it.
 template <typename R, int KX, class Store>
-SPD_HD void column_vjp(const ColumnIn<R, KX>& c_in, const PhaseA<R, KX>& a, const PhaseB<R, KX>& b, uint32_t S,
-                       const SpeedyParams& p, const SpeedyVertical& v, const Uniforms<R>& u, uint32_t flags,
-                       const ColumnCt<R, KX>& ct, ColumnAdj<R, KX>& g, Store& tape) {
-  adj_zero<R, KX>(g);
-  // The terms below recompute the forward from the column; none of the forward's
-  // intermediates stay live across the adjoint (they are equal by construction).
-  const ColumnIn<R, KX> c = opaque_column<R, KX>(c_in);
-  const R rps = R(1.0) / c.ps;
-  R a_dfl[KX], a_Th[KX];
-#pragma unroll
-  for (int k = 0; k < KX; ++k) {
-    a_dfl[k] = ct.dt[k] * v.grdscp[k] * rps;
-    a_Th[k] = R(0.0);
-  }
-  R a_rlus2 = R(0.0), a_flux_h[2] = {R(0.0), R(0.0)}, a_rsds = R(0.0), a_rlds = R(0.0);
-  {
-    const ColumnIn<R, KX> cl = opaque_column<R, KX>(c);
-    PhaseB<R, KX> bb;
-    LwdTape<R, KX> et;
-    lw_transmissivity<R, KX>(cl, a, p, v, u, bb);
-    lw_emissions<R, KX>(cl, u, bb, et);
-#pragma unroll
-    for (int k = 0; k < KX; ++k) bb.dfl[k] = b.dfl[k];
-    bb.rlds = b.rlds;
-    LwuTape<R, KX> lt;
-    const R fh[4] = {b.flux_h[0], b.flux_h[1], R(0.0), R(0.0)};
-    lw_up<R, KX, false>(cl, a, p, v, u, bb, b.rlus2, b.tsfc, fh, lt);
-#pragma unroll
-    for (int k = 0; k < KX; ++k) g.rps += ct.dt[k] * lt.dfl[k] * v.grdscp[k];
-#pragma unroll
-    for (int k = 1; k <= KX; ++k)
-#pragma unroll
-      for (int bnd = 0; bnd < 4; ++bnd) tape.put(k * 4 + bnd, lt.Fu[k][bnd]);
-  }
-  {
-    const ColumnIn<R, KX> ca = opaque_column<R, KX>(c);
-    lw_up_adj<R, KX>(ca, a, b, p, v, u, tape, a_dfl, a_rlus2, a_flux_h, g, a_Th);
-    settle_adj<R, KX>(g);
-    if constexpr (kSettle<KX>) { settle(a_rlus2); settle(a_flux_h[0]); settle(a_flux_h[1]); }
-  }
-  {
-    PhaseB<R, KX> bb = b;
-    SfcTape<R> st;
-    R tsfc;
-    surface<R, KX, false>(c, a, p, v, u, flags, bb, tsfc, st);
-    surface_adj<R, KX>(c, a, b, p, v, u, st, ct, a_rlus2, a_rsds, a_rlds, g);
-    settle_adj<R, KX>(g);
-    if constexpr (kSettle<KX>) { settle(a_rsds); settle(a_rlds); }
-  }
-  {
-    PhaseB<R, KX> bb = b;
-    SwTape<R, KX> st;
-    R fh[4];
-    shortwave<R, KX, false>(c, a, S, p, v, u, bb, fh, st);
-    shortwave_adj<R, KX>(c, a, b, S, p, v, u, st, ct, a_flux_h, a_rsds, g);
-    settle_adj<R, KX>(g);
-  }
-  {
-    const ColumnIn<R, KX> cl = opaque_column<R, KX>(c);
-    PhaseB<R, KX> bb;
-    LwdTape<R, KX> lt;
-    lw_transmissivity<R, KX>(cl, a, p, v, u, bb);
-    lw_down<R, KX>(cl, p, u, bb, lt);
-#pragma unroll
-    for (int k = 0; k < KX - 1; ++k)
-#pragma unroll
-      for (int bnd = 0; bnd < 4; ++bnd) tape.put(k * 4 + bnd, lt.Fd[k][bnd]);
-  }
-  {
-    const ColumnIn<R, KX> ca = opaque_column<R, KX>(c);
-    lw_down_adj<R, KX>(ca, a, p, v, u, tape, a_dfl, a_rlds, g, a_Th);
-    settle_adj<R, KX>(g);
-  }
-  half_level_adj<R, KX>(u, a_Th, g);
+SPD_HD void phase_b2_vjp(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, uint32_t S, const SpeedyParams& p,
+                         const SpeedyVertical& v, const Uniforms<R>& u, const ColumnCt<R, KX>& ct, PhaseB<R, KX>& b,
+                         ColumnAdj<R, KX>& g, const VjpTapeB<R, KX>& t, const Store& tape) {
+  R a_rlus2, a_flux_h[2], a_rsds = R(0.0), a_rlds = R(0.0);
+  lw_surface_adj<R, KX>(u, p, b.tsfc, dfl_ct<R, KX>(ct, v, KX - 1, mrcp(c.ps)), t.aF, a_rlus2, a_flux_h);
+  surface_adj<R, KX>(c, a, b, p, v, u, t.sf, ct, a_rlus2, a_rsds, a_rlds, g);
+  shortwave_adj<R, KX>(c, a, b, S, p, v, u, t.sw, ct, a_flux_h, a_rsds, g);
+  lw_up_vjp<R, KX>(c, a, p, v, u, b, tape, ct, a_rlds, g);
+}
+
+// Reversal of vertical diffusion and phase A.  The cloud and convection
+// intermediates are recomputed (376 of the forward's 2842 instructions; keeping them
+// would hold about 70 values across phase B).
+template <typename R, int KX>
+SPD_HD void phase_a_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const SpeedyParams& p,
+                        const SpeedyVertical& v, const Uniforms<R>& u, const ColumnCt<R, KX>& ct,
+                        ColumnAdj<R, KX>& g) {
   vdiff_adj<R, KX>(c, a, p, u, ct, g);
   settle_adj<R, KX>(g);
   {
@@ -1089,7 +1112,21 @@ SPD_HD void column_vjp(const ColumnIn<R, KX>& c_in, const PhaseA<R, KX>& a, cons
     convection<R, KX>(c, p, v, u, aa, t);
     convection_adj<R, KX>(c, a, p, v, u, t, ct, g);
   }
-  humidity_adj<R, KX>(c, a, v, g);
+  humidity_adj<R, KX>(c, a, g);
+}
+
+// The whole column from the forward's phase A: the gradients into g (the forward of
+// phase B is evaluated again; the kernels run the pieces above in place of it).
+template <typename R, int KX, class Store>
+SPD_HD void column_vjp(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const PhaseB<R, KX>&, uint32_t S,
+                       const SpeedyParams& p, const SpeedyVertical& v, const Uniforms<R>& u, uint32_t flags,
+                       const ColumnCt<R, KX>& ct, ColumnAdj<R, KX>& g, Store& tape) {
+  PhaseB<R, KX> b;
+  VjpTapeB<R, KX> t;
+  phase_b1_vjp<R, KX>(c, a, p, v, u, ct, b, g, t, tape);
+  phase_b2_taped<R, KX>(c, a, S, p, v, u, flags, ct, b, g, t);
+  phase_b2_vjp<R, KX>(c, a, S, p, v, u, ct, b, g, t, tape);
+  phase_a_adj<R, KX>(c, a, p, v, u, ct, g);
 }
 
 }  // namespace speedy

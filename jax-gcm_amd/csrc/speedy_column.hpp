@@ -100,6 +100,17 @@ constexpr double PRG = 1e5 / 9.81;
 constexpr double RGAS288 = 2.0 / 7.0 * 1004.0 * 288.0;
 constexpr double EPS = 1e-9;
 
+// c ? a : b with both sides evaluated first.  The column code has no branch that
+// depends on the column: every lane of a wave runs the same instructions and
+// chooses by selects.  Two reasons.  A branch around a few instructions costs as
+// much as they do.  And in a kernel this full of registers the compiler places
+// copies between registers right before the instruction that turns all lanes back
+// on at the end of such a branch, so lanes that did not take it lose the value
+// (wrong tendencies in some lanes, in whichever kernel the copies happened to fall;
+// tests/test_kernel_resources.py looks for the pattern in the assembly).
+template <typename R>
+SPD_HD R sel(bool c, R a, R b) { return c ? a : b; }
+
 template <typename R>
 SPD_HD R sq(R x) { return x * x; }
 template <typename R>
@@ -169,7 +180,7 @@ SPD_HD R verify_dq(R q, R dq, R dt, bool& limited) {
 #endif
   const R qn = q + dt * dq;
   limited = !(qn >= R(0.0));
-  return limited ? -q / dt : dq;
+  return sel(limited, -q / dt, dq);
 }
 
 // Inputs of one column.
@@ -367,23 +378,22 @@ SPD_HD void convection(const ColumnIn<R, KX>& c, const SpeedyParams& p, const Sp
   int ktop1 = KX, ktop2 = KX;
 #pragma unroll
   for (int k = KX - 4; k >= 2; --k) {   // first unstable level from the top wins
-    if (mss0 > mss2[k]) ktop1 = k + 1;
-    if (mse1 > mss2[k]) ktop2 = k + 1;
+    ktop1 = sel(mss0 > mss2[k], k + 1, ktop1);
+    ktop2 = sel(mse1 > mss2[k], k + 1, ktop2);
   }
   R msthr = mss2[KX - 1];
 #pragma unroll
   for (int k = 2; k <= KX - 4; ++k)
-    if (ktop2 == k + 1) msthr = mss2[k];
+    msthr = sel(ktop2 == k + 1, mss2[k], msthr);
   const R qthr0 = p.rhbl * a.qsat[KX - 1];
   const R qthr1 = p.rhbl * a.qsat[KX - 2];
-  const bool lqthr = (c.Q[KX - 1] > qthr0) && (c.Q[KX - 2] > qthr1);
+  const bool lqthr = (c.Q[KX - 1] > qthr0) & (c.Q[KX - 2] > qthr1);
   const bool mask_psa = c.ps > p.psmin;
-  const bool case1 = mask_psa && (ktop1 < KX) && (ktop2 < KX);
-  const bool case2 = mask_psa && (ktop1 < KX) && !(ktop2 < KX) && lqthr;
-  a.iptop_conv = (case1 || case2) ? ktop1 : KX + 1;
-  R qdif = R(0.0);
-  if (case1) qdif = mmax(c.Q[KX - 1] - qthr0, (mse0 - msthr) * R(RLHC));
-  if (case2) qdif = c.Q[KX - 1] - qthr0;
+  const bool case1 = mask_psa & (ktop1 < KX) & (ktop2 < KX);
+  const bool case2 = mask_psa & (ktop1 < KX) & !(ktop2 < KX) & lqthr;
+  a.iptop_conv = sel(case1 | case2, ktop1, KX + 1);
+  const R dq0 = c.Q[KX - 1] - qthr0;
+  const R qdif = sel(case2, dq0, sel(case1, mmax(dq0, (mse0 - msthr) * R(RLHC)), R(0.0)));
   t.ktop2 = ktop2; t.case1 = case1; t.case2 = case2;
   t.qthr0 = qthr0; t.mse0 = mse0; t.msthr = msthr; t.qdif = qdif;
   // mass fluxes
@@ -413,7 +423,7 @@ SPD_HD void convection(const ColumnIn<R, KX>& c, const SpeedyParams& p, const Sp
 #pragma unroll
   for (int k = 0; k < KX; ++k) {
     const bool lm = (k <= KX - 2) && (k >= iptop);
-    en[k] = (lm && k >= 1) ? u.entr[k] * c.ps * a.cbmf : R(0.0);
+    en[k] = sel(lm && k >= 1, u.entr[k] * c.ps * a.cbmf, R(0.0));
   }
   R* FM = t.FM;
   R* FUS = t.FUS;
@@ -441,12 +451,12 @@ SPD_HD void convection(const ColumnIn<R, KX>& c, const SpeedyParams& p, const Sp
 #pragma unroll
   for (int k = 0; k < KX - 1; ++k) {
     const bool lm = (k >= iptop);
-    dfse[k] = lm ? ((FUS[k + 1] - FDS[k + 1]) - (FUS[k] - FDS[k])) : R(0.0);
-    dfqa[k] = lm ? ((FUQ[k + 1] - FDQ[k + 1]) - (FUQ[k] - FDQ[k])) : R(0.0);
+    dfse[k] = sel(lm, (FUS[k + 1] - FDS[k + 1]) - (FUS[k] - FDS[k]), R(0.0));
+    dfqa[k] = sel(lm, (FUQ[k + 1] - FDQ[k + 1]) - (FUQ[k] - FDQ[k]), R(0.0));
     // secondary moisture flux (:198-202)
-    const R delq = lm ? (p.rhil * a.qsat[k] - c.Q[k]) : R(0.0);
+    const R delq = sel(lm, p.rhil * a.qsat[k] - c.Q[k], R(0.0));
     t.delq[k] = delq;
-    const R fsq = (delq > R(0.0)) ? p.smf * a.cbmf * delq : R(0.0);
+    const R fsq = sel(delq > R(0.0), p.smf * a.cbmf * delq, R(0.0));
     dfqa[k] = dfqa[k] + fsq;
     sumfsq = (k == 0) ? fsq : sumfsq + fsq;
   }
@@ -455,18 +465,25 @@ SPD_HD void convection(const ColumnIn<R, KX>& c, const SpeedyParams& p, const Sp
   R fm_t = R(0.0), fus_t = R(0.0), fuq_t = R(0.0), fds_t = R(0.0), fdq_t = R(0.0), qsatb = R(0.0);
 #pragma unroll
   for (int k = 0; k < KX; ++k) {
-    if (iptop == k) { fm_t = FM[k]; fus_t = FUS[k]; fuq_t = FUQ[k]; fds_t = FDS[k]; fdq_t = FDQ[k]; }
+    const bool at = iptop == k;
+    fm_t = sel(at, FM[k], fm_t);
+    fus_t = sel(at, FUS[k], fus_t);
+    fuq_t = sel(at, FUQ[k], fuq_t);
+    fds_t = sel(at, FDS[k], fds_t);
+    fdq_t = sel(at, FDQ[k], fdq_t);
   }
 #pragma unroll
   for (int k = 0; k < KX - 1; ++k)
-    if (iptop - 1 == k) qsatb = a.qsat[k] + u.wvi1[k] * (a.qsat[k + 1] - a.qsat[k]);
+    qsatb = sel(iptop - 1 == k, a.qsat[k] + u.wvi1[k] * (a.qsat[k + 1] - a.qsat[k]), qsatb);
   t.fm_t = fm_t; t.fus_t = fus_t; t.fuq_t = fuq_t; t.fds_t = fds_t; t.fdq_t = fdq_t; t.qsatb = qsatb;
   a.precnv = mmax(fuq_t - fm_t * qsatb, R(0.0));
   const R top_s = fus_t - fds_t + R(ALHC) * a.precnv;
   const R top_q = fuq_t - fdq_t - a.precnv;
 #pragma unroll
-  for (int k = 0; k < KX; ++k)
-    if (iptop - 1 == k) { dfse[k] = top_s; dfqa[k] = top_q; }
+  for (int k = 0; k < KX; ++k) {
+    dfse[k] = sel(iptop - 1 == k, top_s, dfse[k]);
+    dfqa[k] = sel(iptop - 1 == k, top_q, dfqa[k]);
+  }
   // flux -> tendency (:226-227)
   const R rps = mdiv(R(1.0), c.ps);
   a.tconv[0] = dfse[0];
@@ -489,11 +506,11 @@ SPD_HD void condensation(const ColumnIn<R, KX>& c, const Uniforms<R>& u, PhaseA<
 #pragma unroll
   for (int k = KX - 1; k >= 1; --k) {
     const R dqa = u.rhref[k] * a.qsat[k] - c.Q[k];
-    if (!(dqa >= R(0.0))) first = k;         // argmin(dqa[1:] >= 0) + 1 (Q4 when none)
+    first = sel(dqa >= R(0.0), first, k);    // argmin(dqa[1:] >= 0) + 1 (Q4 when none)
     const bool neg = dqa < R(0.0);
-    const R dq = neg ? dqa * u.rtlsc : R(0.0);
+    const R dq = sel(neg, dqa * u.rtlsc, R(0.0));
     a.qlsc[k] = dq;
-    a.tlsc[k] = neg ? R(TFACT) * mmin(-dq, u.dqmax[k] * psa2) : R(0.0);
+    a.tlsc[k] = sel(neg, R(TFACT) * mmin(-dq, u.dqmax[k] * psa2), R(0.0));
   }
 #pragma unroll
   for (int k = 1; k < KX; ++k) {
@@ -501,8 +518,8 @@ SPD_HD void condensation(const ColumnIn<R, KX>& c, const Uniforms<R>& u, PhaseA<
     precls = (k == 1) ? t : precls + t;
   }
   a.precls = (R(0.0) - precls) * c.ps;
-  const int ipl = first == 0 ? 1 : first;
-  a.iptop = ipl < a.iptop_conv ? ipl : a.iptop_conv;
+  const int ipl = sel(first == 0, 1, first);
+  a.iptop = sel(ipl < a.iptop_conv, ipl, a.iptop_conv);
 }
 
 template <typename R, int KX>
@@ -520,7 +537,7 @@ SPD_HD void clouds(const ColumnIn<R, KX>& c, const SpeedyParams& p, const Unifor
   a.gse = mdiv(a.se[KX - 2] - a.se[KX - 1], c.PHI[KX - 2] - c.PHI[KX - 1]);
   const R rrcl = u.rrcl;
   const bool m0 = a.rh[KX - 2] > p.rhcl1;
-  const R cc0 = m0 ? a.rh[KX - 2] - p.rhcl1 : R(0.0);
+  const R cc0 = sel(m0, a.rh[KX - 2] - p.rhcl1, R(0.0));
   const int icl0 = m0 ? KX - 2 : KX;
   R* cu = t.cu;
   bool mk[KX];
@@ -529,22 +546,22 @@ SPD_HD void clouds(const ColumnIn<R, KX>& c, const SpeedyParams& p, const Unifor
 #pragma unroll
   for (int k = 2; k <= KX - 3; ++k) {
     const R drh = a.rh[k] - p.rhcl1;
-    mk[k] = (drh > cc0) && (c.Q[k] > p.qacl);
-    cu[k] = mk[k] ? drh : cc0;
+    mk[k] = (drh > cc0) & (c.Q[k] > p.qacl);
+    cu[k] = sel(mk[k], drh, cc0);
     cmax = (k == 2) ? cu[k] : mmax(cmax, cu[k]);
-    if (mk[k]) t.mk |= 1u << k;
+    t.mk |= sel(mk[k], 1u << k, 0u);
   }
   int icl = 0;
 #pragma unroll
   for (int k = 2; k <= KX - 3; ++k) {        // Q5: float equality
-    const int cand = (cmax == cu[k]) ? (mk[k] ? k : icl0) : icl0;
-    icl = (k == 2) ? cand : (cand > icl ? cand : icl);
+    const int cand = sel((cmax == cu[k]) & mk[k], k, icl0);
+    icl = (k == 2) ? cand : sel(cand > icl, cand, icl);
   }
   const R pr1 = mmin(p.pmaxcl, R(86.4) * (a.precnv + a.precls));
   const R cl2 = mmin(R(1.0), cmax * rrcl);
   const R ccraw = p.wpcl * msqrt_1ulp(mmax(R(EPS), pr1)) + sq(cl2);
   R cloudc = mmin(R(1.0), ccraw);
-  if (cloudc != cloudc) cloudc = R(1.0);
+  cloudc = sel(cloudc != cloudc, R(1.0), cloudc);
   a.cloudc = cloudc;
   a.icltop = a.iptop < icl ? a.iptop : icl;
   a.qcloud = c.Q[KX - 2];
@@ -600,22 +617,22 @@ SPD_HD int cloud_top(const ColumnIn<R, KX>& c, const SpeedyParams& p, const Spee
     }
     const R qthr0 = p.rhbl * qsat[KX - 1];
     const R qthr1 = p.rhbl * qsat[KX - 2];
-    const bool lqthr = (c.Q[KX - 1] > qthr0) && (c.Q[KX - 2] > qthr1);
+    const bool lqthr = (c.Q[KX - 1] > qthr0) & (c.Q[KX - 2] > qthr1);
     const bool mask_psa = c.ps > p.psmin;
-    const bool case1 = mask_psa && (ktop1 < KX) && (ktop2 < KX);
-    const bool case2 = mask_psa && (ktop1 < KX) && !(ktop2 < KX) && lqthr;
-    iptop_conv = (case1 || case2) ? ktop1 : KX + 1;
+    const bool case1 = mask_psa & (ktop1 < KX) & (ktop2 < KX);
+    const bool case2 = mask_psa & (ktop1 < KX) & !(ktop2 < KX) & lqthr;
+    iptop_conv = sel(case1 | case2, ktop1, KX + 1);
   }
   int first = 0;
 #pragma unroll
   for (int k = KX - 1; k >= 1; --k) {
     const R dqa = u.rhref[k] * qsat[k] - c.Q[k];
-    if (!(dqa >= R(0.0))) first = k;
+    first = sel(dqa >= R(0.0), first, k);
   }
   const int ipl = first == 0 ? 1 : first;
   const int iptop = ipl < iptop_conv ? ipl : iptop_conv;
   const bool m0 = rh[KX - 2] > p.rhcl1;
-  const R cc0 = m0 ? rh[KX - 2] - p.rhcl1 : R(0.0);
+  const R cc0 = sel(m0, rh[KX - 2] - p.rhcl1, R(0.0));
   const int icl0 = m0 ? KX - 2 : KX;
   R cu[KX];
   bool mk[KX];
@@ -623,15 +640,15 @@ SPD_HD int cloud_top(const ColumnIn<R, KX>& c, const SpeedyParams& p, const Spee
 #pragma unroll
   for (int k = 2; k <= KX - 3; ++k) {
     const R drh = rh[k] - p.rhcl1;
-    mk[k] = (drh > cc0) && (c.Q[k] > p.qacl);
-    cu[k] = mk[k] ? drh : cc0;
+    mk[k] = (drh > cc0) & (c.Q[k] > p.qacl);
+    cu[k] = sel(mk[k], drh, cc0);
     cmax = (k == 2) ? cu[k] : mmax(cmax, cu[k]);
   }
   int icl = 0;
 #pragma unroll
   for (int k = 2; k <= KX - 3; ++k) {
-    const int cand = (cmax == cu[k]) ? (mk[k] ? k : icl0) : icl0;
-    icl = (k == 2) ? cand : (cand > icl ? cand : icl);
+    const int cand = sel((cmax == cu[k]) & mk[k], k, icl0);
+    icl = (k == 2) ? cand : sel(cand > icl, cand, icl);
   }
   return iptop < icl ? iptop : icl;
 }
@@ -685,8 +702,8 @@ SPD_HD void lw_absorptivity(int k, const ColumnIn<R, KX>& c, const PhaseA<R, KX>
   ab[0] = p.ablwin; ab[1] = u.ablco2; ab[2] = p.ablwv1 * c.Q[k]; ab[3] = p.ablwv2 * c.Q[k];
   if (k == 0) { ab[2] = R(0.0); ab[3] = R(0.0); }
   if (k >= 2 && k <= KX - 2) {
-    ab[0] = ab[0] + ((k > a.icltop) ? a.cloudc * p.ablcl1 : a.cloudc * p.ablcl2);
     const R ac2 = a.cloudc * p.ablcl2;
+    ab[0] = ab[0] + sel(k > a.icltop, a.cloudc * p.ablcl1, ac2);
     ab[2] = mmax(ab[2], ac2);
     ab[3] = mmax(ab[3], ac2);
   }
@@ -821,28 +838,23 @@ SPD_HD void vdiff(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const Speedy
   for (int k = 0; k < KX; ++k) { tt[k] = R(0.0); qt[k] = R(0.0); }
   const R dmse = a.se[KX - 1] - a.se[NL1 - 1] + R(ALHC) * (c.Q[KX - 1] - a.qsat[NL1 - 1]);
   const R drh = a.rh[KX - 1] - a.rh[NL1 - 1];
-  const R fcnv = (icnv > 0 && dmse >= R(0.0)) ? p.redshc : R(1.0);
+  const bool up = dmse >= R(0.0);
+  const R fcnv = sel((icnv > 0) & up, R(p.redshc), R(1.0));
   const R rsA = u.rsig[NL1 - 1], rsB = u.rsig[KX - 1];
-  if (dmse >= R(0.0)) {
-    const R fluxse = fcnv * u.fshcse * dmse;
-    tt[NL1 - 1] = fluxse * rsA;
-    tt[KX - 1] = -fluxse * rsB;
-    if (drh >= R(0.0)) {
-      const R fluxq = fcnv * u.fshcq * a.qsat[KX - 1] * drh;
-      qt[NL1 - 1] = fluxq * rsA;
-      qt[KX - 1] = -fluxq * rsB;
-    }
-  } else if (dmse < R(0.0) && drh > u.drh0) {
-    const R fluxq = u.fvdiq2 * a.qsat[NL1 - 1] * drh;
-    qt[NL1 - 1] = fluxq * rsA;
-    qt[KX - 1] = -fluxq * rsB;
-  }
+  const R fluxse = fcnv * u.fshcse * dmse;
+  tt[NL1 - 1] = sel(up, fluxse * rsA, R(0.0));
+  tt[KX - 1] = sel(up, -fluxse * rsB, R(0.0));
+  // shallow convection's moisture flux, or the diffusive one of a stable layer
+  const R fluxq = sel(up, fcnv * u.fshcq * a.qsat[KX - 1] * drh, u.fvdiq2 * a.qsat[NL1 - 1] * drh);
+  const bool mix = (up & (drh >= R(0.0))) | ((dmse < R(0.0)) & (drh > u.drh0));
+  qt[NL1 - 1] = sel(mix, fluxq * rsA, R(0.0));
+  qt[KX - 1] = sel(mix, -fluxq * rsB, R(0.0));
   // moisture diffusion above the PBL (:99-118)
   R fq[KX];
 #pragma unroll
   for (int k = 2; k < KX - 2; ++k) {
     const R d = a.rh[k + 1] - a.rh[k];
-    fq[k] = (d >= u.vd_drh0[k] && ((u.vd_on >> k) & 1u)) ? u.vd_fq[k] * a.qsat[k] * d : R(0.0);
+    fq[k] = sel((d >= u.vd_drh0[k]) & (((u.vd_on >> k) & 1u) != 0u), u.vd_fq[k] * a.qsat[k] * d, R(0.0));
   }
 #pragma unroll
   for (int k = 2; k < KX - 2; ++k) qt[k] = qt[k] + fq[k] * u.rsig[k];
@@ -853,7 +865,7 @@ SPD_HD void vdiff(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const Speedy
 #pragma unroll
   for (int k = 0; k < NL1; ++k) {
     const R se0 = a.se[k + 1] - p.segrad * (c.PHI[k + 1] - c.PHI[k]);
-    fse[k] = (a.se[k] < se0) ? u.fvdise * (se0 - a.se[k]) : R(0.0);
+    fse[k] = sel(a.se[k] < se0, u.fvdise * (se0 - a.se[k]), R(0.0));
     tt[k] = tt[k] + fse[k] * u.rsig[k];
   }
   R cum = R(0.0);
@@ -908,10 +920,10 @@ SPD_HD void shortwave(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, uint32_t
                       SwTape<R, KX>& t) {
   const R ps = c.ps;
   const R rps = mdiv(R(1.0), ps);
-  const R a_cl = (a.icltop < KX) ? p.albcl * a.cloudc : R(0.0);
+  const R a_cl = sel(a.icltop < KX, p.albcl * a.cloudc, R(0.0));
   R* t22 = t.t22;
 #pragma unroll
-  for (int k = 0; k < KX - 1; ++k) t22[k] = ((S >> k) & 1u) ? a_cl : R(0.0);   // Q1
+  for (int k = 0; k < KX - 1; ++k) t22[k] = sel(((S >> k) & 1u) != 0u, a_cl, R(0.0));   // Q1
   t22[KX - 1] = p.albcls * a.clstr;
   const R psaz = ps * c.zenit;
   const R acloud = a.cloudc * mmin(p.abscl1 * a.qcloud, p.abscl2);
@@ -921,7 +933,7 @@ SPD_HD void shortwave(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, uint32_t
   tau0[0] = exp_tr(-psaz * v.dhs[0] * p.absdry);
 #pragma unroll
   for (int k = 1; k < KX - 1; ++k) {
-    const R cl = (k >= a.icltop) ? acloud : R(0.0);
+    const R cl = sel(k >= a.icltop, acloud, R(0.0));
     tau0[k] = exp_tr(-psaz * v.dhs[k] * (u.sw_abs1[k] + p.abswv1 * c.Q[k] + cl));
   }
   tau0[KX - 1] = exp_tr(-psaz * v.dhs[KX - 1] * (u.sw_abs1[KX - 1] + p.abswv1 * c.Q[KX - 1]));
@@ -968,7 +980,7 @@ SPD_HD void shortwave(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, uint32_t
   const R ftoa = tau0[0] * fu[0] + Rf[0];
   const bool csw = u.compute_sw != 0u;
 #pragma unroll
-  for (int k = 0; k < KX; ++k) b.tsw[k] = csw ? dfabs[k] * v.grdscp[k] * rps : R(0.0);
+  for (int k = 0; k < KX; ++k) b.tsw[k] = sel(csw, dfabs[k] * v.grdscp[k] * rps, R(0.0));
   flux_h[0] = ftoa; flux_h[1] = f2[KX - 1]; flux_h[2] = R(0.0); flux_h[3] = R(0.0);   // Q2
   b.rsds = rsds;
   if (DIAG) {
@@ -1015,20 +1027,15 @@ SPD_HD void surface(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const Spee
     const R t2_0 = t2_1 - R(RCP) * phi0;
     t.phi0 = phi0; t.dt1 = dt1; t.t1_0a = t1_0; t.t1_1a = t1_1; t.t2_0 = t2_0; t.t2_1 = t2_1;
     t.warm = Tb > c.T[KX - 2];
-    if (Tb > c.T[KX - 2]) {
-      t1_0 = s.ftemp0 * t1_0 + u.gtemp0 * t2_0;
-      t1_1 = s.ftemp0 * t1_1 + u.gtemp0 * t2_1;
-    } else {
-      t1_0 = Tb;
-      t1_1 = Tb;
-    }
+    t1_0 = sel(t.warm, s.ftemp0 * t1_0 + u.gtemp0 * t2_0, Tb);
+    t1_1 = sel(t.warm, s.ftemp0 * t1_1 + u.gtemp0 * t2_1, Tb);
     const R t0 = t1_1 + c.fmask * (t1_0 - t1_1);
     const R wind = msqrt_1ulp(u0 * u0 + v0 * v0 + R(s.vgust) * s.vgust);
     den0 = mdiv(R(P0) * ps, R(RGAS) * t0) * wind;
     tskin = c.stl + s.ctday * c.sqcoa * b.rsds * (R(1.0) - b.alb_l) * ps;
     t.t1_0 = t1_0; t.t1_1 = t1_1; t.t0 = t0; t.wind = wind; t.den0 = den0; t.tskin0 = tskin;
     const R dd = tskin - t2_0;
-    const R dthl = (tskin > t2_0) ? mmin(R(s.dtheta), dd) : mmax(-R(s.dtheta), u.astab * dd);
+    const R dthl = sel(tskin > t2_0, mmin(R(s.dtheta), dd), mmax(-R(s.dtheta), u.astab * dd));
     const R den1 = den0 * (R(1.0) + dthl * u.rdth);
     const R forog = R(1.0) + u.rhdrag * (R(1.0) - exp_tr(-mmax(c.phis0, R(0.0)) * u.rhdrag));
     const R cdldv = u.cdl * den0 * forog;
@@ -1052,7 +1059,7 @@ SPD_HD void surface(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const Spee
       const R clamb = s.clambda + (b.snowc * (R(s.clambsn) - s.clambda));
       hfl0 = hfl0 - (clamb * (tskin - c.stl));
       const R qs1p = qsat_f(tskin + R(1.0), ps, R(1.0));
-      const R qs1 = (evap0 > R(0.0)) ? c.soilw * (qs1p - qsat00) : R(0.0);
+      const R qs1 = sel(evap0 > R(0.0), c.soilw * (qs1p - qsat00), R(0.0));
       const R dtskin = mdiv(hfl0, clamb + drls + (s.chl * den1 * (R(CP) + (R(ALHC) * qs1))));
       t.clamb = clamb; t.qs1p = qs1p; t.qs1 = qs1; t.dtskin = dtskin;
       tskin = tskin + dtskin;
@@ -1062,7 +1069,7 @@ SPD_HD void surface(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const Spee
       hfl0 = clamb * (tskin - c.stl);
     }
     const R ds = c.sst - t2_1;
-    const R dths = (c.sst > t2_1) ? mmin(R(s.dtheta), ds) : mmax(-R(s.dtheta), u.astab * ds);
+    const R dths = sel(c.sst > t2_1, mmin(R(s.dtheta), ds), mmax(-R(s.dtheta), u.astab * ds));
     den2 = den0 * (R(1.0) + dths * u.rdth);
     q1_1 = Qb;
     if (s.fhum0 > R(0.0)) q1_1 = s.fhum0 * (a.rh[KX - 1] * qsat_f(t1_1, ps, R(1.0))) + u.ghum0 * Qb;

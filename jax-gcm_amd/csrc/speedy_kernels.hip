@@ -176,8 +176,7 @@ __device__ __forceinline__ void store_uv_zeros(const KArgs& a, uint32_t m, uint3
 // known.  The phase-A and vertical-diffusion tendencies then die early instead of
 // staying live across phases b1 and b2 (16 fewer registers in the forward, and
 // no scratch at two waves per SIMD).  The sixteen-level kernels keep the sums at
-// the stores: they spill, and the early form gave wrong 16-level fused forward
-// tendencies on gfx950 (the host build of the same order is right).
+// the stores.
 template <int KX>
 constexpr bool kEarlySums = KX <= 8;
 
@@ -202,14 +201,12 @@ __device__ __forceinline__ void tend_after_b1(uint32_t tm, const PhaseB<float, K
   }
 }
 
-// Returns the levels whose q tendency verify_tendencies limited (bit k).
 // at, aq: the partial sums of tend_after_a / tend_after_b1.
-template <int KX, bool DIAG, bool EXTRA, bool UV_ALL>
-__device__ __forceinline__ uint32_t store_outputs(const KArgs& a, uint32_t m, uint32_t c,
-                                                  const ColumnIn<float, KX>& col, const PhaseA<float, KX>& pa,
-                                                  const PhaseB<float, KX>& pb, const float at[KX], const float aq[KX],
-                                                  double colsum[2]) {
-  uint32_t limited = 0u;
+template <int KX, bool DIAG, bool EXTRA>
+__device__ __forceinline__ void store_outputs(const KArgs& a, uint32_t m, uint32_t c,
+                                              const ColumnIn<float, KX>& col, const PhaseA<float, KX>& pa,
+                                              const PhaseB<float, KX>& pb, const float at[KX], const float aq[KX],
+                                              double colsum[2]) {
   const bool budget = EXTRA && a.f.budget != nullptr;
   const double dpg = (double)col.ps * (double)(P0 / GRAV);   // p0 ps / g; times dhs_k: dp_k / g
   colsum[0] = 0.0;
@@ -240,9 +237,8 @@ __device__ __forceinline__ uint32_t store_outputs(const KArgs& a, uint32_t m, ui
     if (EXTRA && (a.flags & SPEEDY_FLAG_VERIFY_TENDENCIES)) {
       bool lim;
       q = verify_dq(gld(a.f.q, base3 + k * ncol), q, a.u.dt_step, lim);   // the unclamped q (re-read, L2)
-      limited |= (lim ? 1u : 0u) << k;
     }
-    if (UV_ALL || k == KX - 1) {   // without UV_ALL the levels above were zeroed by store_uv_zeros
+    if (k == KX - 1) {   // the levels above were zeroed by store_uv_zeros
       gst(a.f.du, base3 + k * ncol, du);
       gst(a.f.dv, base3 + k * ncol, dv);
     }
@@ -291,31 +287,21 @@ __device__ __forceinline__ uint32_t store_outputs(const KArgs& a, uint32_t m, ui
 #pragma unroll
       for (int k = 0; k < KX; ++k) W(pb.tauL[k][b]);
   }
-  return limited;
 }
 
 // ---------------------------------------------------------------- level set S
-// OR over the 64 lanes of a wave (all active).  DPP: six data-parallel-primitive
-// ORs within the register file (quad swaps, half-row and row mirrors give every
-// lane its row's OR; the row-15 and row-31 broadcasts fold rows into row 3), then
-// lane 63 is read: no LDS round trip (the forward kernels).  Otherwise a
-// butterfly of lane shuffles: the forward + VJP kernels keep it, because their
-// register allocation (several KB of spills per lane at 16 levels) changed with
-// another form and gave wrong gradients on gfx950.
-template <bool DPP>
+// OR over the 64 lanes of a wave (all active): six data-parallel-primitive ORs
+// within the register file (quad swaps, half-row and row mirrors give every lane
+// its row's OR; the row-15 and row-31 broadcasts fold rows into row 3), then lane
+// 63 is read: no LDS round trip.
 __device__ __forceinline__ uint32_t wave_or(uint32_t v) {
-  if (DPP) {
-    v |= __builtin_amdgcn_update_dpp(0u, v, 0xB1, 0xF, 0xF, false);    // quad_perm [1,0,3,2]
-    v |= __builtin_amdgcn_update_dpp(0u, v, 0x4E, 0xF, 0xF, false);    // quad_perm [2,3,0,1]
-    v |= __builtin_amdgcn_update_dpp(0u, v, 0x141, 0xF, 0xF, false);   // row_half_mirror
-    v |= __builtin_amdgcn_update_dpp(0u, v, 0x140, 0xF, 0xF, false);   // row_mirror
-    v |= __builtin_amdgcn_update_dpp(0u, v, 0x142, 0xA, 0xF, false);   // row_bcast:15 into rows 1, 3
-    v |= __builtin_amdgcn_update_dpp(0u, v, 0x143, 0xC, 0xF, false);   // row_bcast:31 into rows 2, 3
-    return __builtin_amdgcn_readlane(v, 63);
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v |= __shfl_xor(v, o, 64);
-  return v;
+  v |= __builtin_amdgcn_update_dpp(0u, v, 0xB1, 0xF, 0xF, false);    // quad_perm [1,0,3,2]
+  v |= __builtin_amdgcn_update_dpp(0u, v, 0x4E, 0xF, 0xF, false);    // quad_perm [2,3,0,1]
+  v |= __builtin_amdgcn_update_dpp(0u, v, 0x141, 0xF, 0xF, false);   // row_half_mirror
+  v |= __builtin_amdgcn_update_dpp(0u, v, 0x140, 0xF, 0xF, false);   // row_mirror
+  v |= __builtin_amdgcn_update_dpp(0u, v, 0x142, 0xA, 0xF, false);   // row_bcast:15 into rows 1, 3
+  v |= __builtin_amdgcn_update_dpp(0u, v, 0x143, 0xC, 0xF, false);   // row_bcast:31 into rows 2, 3
+  return __builtin_amdgcn_readlane(v, 63);
 }
 
 __device__ __forceinline__ uint32_t gen_tag(uint32_t g) { return (g & 0x7fffu) | 0x8000u; }
@@ -327,41 +313,29 @@ __device__ __forceinline__ uint32_t clip_bit(int icl, int kx) {
 }
 
 // Fused path: OR of the level bits of member m over the published words of the
-// blocks covering it, polled until every word carries `tag` (one wave).
-// Bounded: after kSpinLimit polls it flags the error word and returns.
-template <bool DPP>
-__device__ __forceinline__ uint32_t collect_fused_t(const KArgs& a, uint32_t tag, uint32_t m) {
+// blocks covering it, polled until every word carries `tag` (one wave, all lanes
+// active throughout: lanes past the last word read it again, since OR is
+// idempotent).  Bounded: after kSpinLimit polls it flags the error word and returns.
+__device__ __forceinline__ uint32_t collect_fused(const KArgs& a, uint32_t tag, uint32_t m) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t b0 = (m * a.ncol) / kBlock, b1 = (m * a.ncol + a.ncol - 1u) / kBlock;
   for (uint32_t spins = 0;; ++spins) {
     uint32_t acc = 0;
     int stale = 0;
-    for (uint32_t b = b0 + lane; b <= b1; b += 64u) {
+    for (uint32_t bb = b0; bb <= b1; bb += 64u) {
+      const uint32_t b = min(bb + lane, b1);
       const uint32_t j = m - divq(b * kBlock, a.dcol);
       const uint32_t w = __hip_atomic_load(&a.partial[2u * b + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       stale |= (w >> 16) != tag;
       acc |= w & 0xffffu;
     }
-    if (!__any(stale)) return wave_or<DPP>(acc);
+    if (!__any(stale)) return wave_or(acc);
     if (spins >= kSpinLimit) {
-      if (lane == 0) __hip_atomic_fetch_or(a.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return wave_or<DPP>(acc);
+      __hip_atomic_store(a.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return wave_or(acc);
     }
     __builtin_amdgcn_s_sleep(1);
   }
-}
-
-// The forward + VJP kernels' form (an outlined call, shuffle OR).
-__device__ uint32_t collect_fused(const KArgs& a, uint32_t tag, uint32_t m) { return collect_fused_t<false>(a, tag, m); }
-
-// Two-kernel path: OR over the level-set chunks that cover member m, by one wave
-// (the forward + VJP kernels' form).
-__device__ uint32_t collect_chunks(const KArgs& a, uint32_t m) {
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t b0 = divq(m * a.ncol, a.dchunk), b1 = divq(m * a.ncol + a.ncol - 1u, a.dchunk);
-  uint32_t acc = 0;
-  for (uint32_t b = b0 + lane; b <= b1; b += 64u) acc |= gld(a.partial, b * a.jmax + (m - divq(b * a.chunk, a.dcol)));
-  return wave_or<false>(acc);
 }
 
 // Two-kernel path: member m's word of level-set chunk b (levelset_batch_kernel output).
@@ -573,9 +547,8 @@ __device__ __forceinline__ void block_budget_partials(const KArgs& a, uint32_t b
   }
 }
 
-// Forward (and, with VJP, the fused forward + VJP).  FUSED: single launch with
-// the split grid barrier (all blocks co-resident); otherwise S comes from the
-// level-set kernel of the same batch.
+// The forward.  FUSED: single launch with the split grid barrier (all blocks
+// co-resident); otherwise S comes from the level-set kernel of the same batch.
 // EXTRA: the optional verify steps and float64 budgets are compiled in (their
 // flags and pointers are then read at run time); the plain forward omits them.
 // The batched forward kernels up to eight levels keep the longwave
@@ -583,9 +556,8 @@ __device__ __forceinline__ void block_budget_partials(const KArgs& a, uint32_t b
 // column, [slot][thread]) instead of recomputing them per level (T425: 153 fewer
 // VALU instructions a wave, ~1 % faster).  The fused kernels recompute: at one
 // wave per SIMD the dependent LDS reads in the longwave-up sweep cost more than
-// the exponentials (T85 forward ~2 % slower with the store).  The forward + VJP
-// kernels' LDS holds the adjoint's tapes, and the sixteen-level kernels keep their
-// tested code.
+// the exponentials (T85 forward ~2 % slower with the store).  The sixteen-level
+// kernels keep their tested code.
 template <bool ON>
 __device__ __forceinline__ auto tau_store(float* s) {
   if constexpr (ON)
@@ -594,185 +566,251 @@ __device__ __forceinline__ auto tau_store(float* s) {
     return NoTauStore{};
 }
 
-template <int KX, bool DIAG, bool FUSED, bool VJP, bool EXTRA>
-__device__ __forceinline__ void fwd_body(const KArgs& a, uint32_t bid) {
-  __shared__ uint32_t s_s[2];
-  constexpr bool kTau = !VJP && !FUSED && KX <= 8;
-  __shared__ float s_tau[kTau ? 4 * KX * kBlock : 1];
-  const auto ts = tau_store<kTau>(s_tau);
-  const uint32_t gid = bid * kBlock + threadIdx.x;
-  const bool active = gid < a.ntot;
-  const uint32_t g0 = gid < a.ntot ? gid : a.ntot - 1u;   // inactive lanes shadow a valid column
-  const uint32_t m = divq(g0, a.dcol);
-  const uint32_t c = g0 - m * a.ncol;
+// Where a block's columns lie and what it knows of its members' level sets.
+// Threads past the last column take the last column and do all its work, its
+// stores included (the same values to the same addresses), so no store needs a
+// branch; only the block sums leave them out.
+struct BlockPos {
+  uint32_t gid, m, c;       // global column, member and column of this thread
+  bool active, wide;        // wide: a member is at least a block, so a block spans at most two members
+  uint32_t m_first, nm;     // the block's first member and how many it spans
+  uint32_t wave;            // this wave's index in the block, as a scalar: branches on it keep all lanes on
+  uint32_t gen, tag;        // fused: the generation word and the call's tag
+  uint32_t lw0, lw1;        // two launches: this thread's share of the members' chunk words
+};
+
+// The thread's position, and the loads the level set needs, issued first so that
+// their round trip overlaps the state's: the generation word (fused), or the level-set
+// chunk words (a member wider than a block: each thread ORs its share of the
+// chunks of the block's members; narrower: the <= 2 chunks covering its own).
+template <bool FUSED>
+__device__ __forceinline__ BlockPos block_pos(const KArgs& a, uint32_t bid) {
+  BlockPos b;
+  b.gid = bid * kBlock + threadIdx.x;
+  b.active = b.gid < a.ntot;
+  const uint32_t g0 = b.gid < a.ntot ? b.gid : a.ntot - 1u;
+  b.m = divq(g0, a.dcol);
+  b.c = g0 - b.m * a.ncol;
   const uint32_t blk0 = bid * kBlock;
-  const uint32_t m_first = divq(blk0, a.dcol);
-  const uint32_t nm = divq(min(blk0 + kBlock, a.ntot) - 1u, a.dcol) - m_first + 1u;   // <= 2 when fused
+  b.m_first = divq(blk0, a.dcol);
+  b.nm = divq(min(blk0 + kBlock, a.ntot) - 1u, a.dcol) - b.m_first + 1u;   // <= 2 when fused
+  b.wide = a.ncol >= (uint32_t)kBlock;
+  b.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  b.gen = b.tag = b.lw0 = b.lw1 = 0u;
   const bool need_s = a.level_set < 0;
-  // The call's generation tag, read first so that its latency overlaps the state
-  // loads; wave 0 publishes and gathers, so each of its lanes holds the tag.
-  uint32_t tag = 0u;
-  if (FUSED && need_s && threadIdx.x < 64u)
-    tag = gen_tag(__hip_atomic_load(a.gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-  // Two-kernel path: the level-set chunk words are loaded first too, so their
-  // round trip overlaps the state's.  A member wider than a block: each thread
-  // ORs its share of the chunks of the block's (at most two) members; narrower:
-  // the <= 2 chunks covering the thread's own member.
-  const bool wide = a.ncol >= (uint32_t)kBlock;   // a block spans at most two members
-  uint32_t lw0 = 0u, lw1 = 0u;
-  if (!FUSED && !VJP && need_s) {
-    if (wide) {
-      lw0 = chunk_share(a, m_first);
-      if (nm > 1u) lw1 = chunk_share(a, m_first + 1u);
+  if (FUSED && need_s) {
+    b.gen = __hip_atomic_load(a.gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    b.tag = gen_tag(b.gen);
+  }
+  if (!FUSED && need_s) {
+    if (b.wide) {
+      b.lw0 = chunk_share(a, b.m_first);
+      if (b.nm > 1u) b.lw1 = chunk_share(a, b.m_first + 1u);
     } else {
-      const uint32_t b0 = divq(m * a.ncol, a.dchunk), b1 = divq(m * a.ncol + a.ncol - 1u, a.dchunk);
-      lw0 = chunk_word(a, b0, m) | chunk_word(a, b1, m);
+      const uint32_t b0 = divq(b.m * a.ncol, a.dchunk), b1 = divq(b.m * a.ncol + a.ncol - 1u, a.dchunk);
+      b.lw0 = chunk_word(a, b0, b.m) | chunk_word(a, b1, b.m);
     }
   }
-  ColumnIn<float, KX> col;
-  load_state<KX, EXTRA>(a, m, c, col);
-  if (!VJP) {
-    load_zonal<KX>(a, c, col);   // S-independent; its loads travel with the state's
-    if (active) store_uv_zeros<KX>(a, m, c);
+  return b;
+}
+
+// Fused: publish this block's word(s) for the call's level set, a wave-level OR
+// per member slot (a fused block spans at most two members), then one word per slot.
+__device__ __forceinline__ void publish_level_bits(const KArgs& a, uint32_t bid, const BlockPos& b, int icltop, int kx) {
+  __shared__ uint32_t s_wor[kBlock / 64][2];
+  const uint32_t bit = b.active ? clip_bit(icltop, kx) : 0u;
+  const uint32_t o0 = wave_or(b.m == b.m_first ? bit : 0u), o1 = wave_or(b.m != b.m_first ? bit : 0u);
+  s_wor[threadIdx.x >> 6][0] = o0;   // the wave's value, from every lane
+  s_wor[threadIdx.x >> 6][1] = o1;
+  __syncthreads();
+  if (b.wave == 0u) {
+    for (uint32_t j = 0; j < b.nm; ++j) {
+      uint32_t w = 0u;
+#pragma unroll
+      for (int i = 0; i < kBlock / 64; ++i) w |= s_wor[i][j];
+      __hip_atomic_store(&a.partial[2u * bid + j], (b.tag << 16) | w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
+}
+
+// The level set of this thread's member: gathered from the published words
+// (fused) or from the chunk words (two launches), or the call's own.
+template <bool FUSED>
+__device__ __forceinline__ uint32_t gather_level_set(const KArgs& a, uint32_t bid, const BlockPos& b) {
+  if (a.level_set >= 0) return (uint32_t)a.level_set;
+  if (FUSED) {
+    __shared__ uint32_t s_s[2];
+    if (b.wave == 0u) {   // wave 0 gathers S for the block's member(s)
+      for (uint32_t j = 0; j < b.nm; ++j) s_s[j] = collect_fused(a, b.tag, b.m_first + j);
+      if (bid == 0) {
+        // every member's S for speedy_read_level_sets; this also waits for every
+        // block's word, i.e. every block has read the generation
+        for (uint32_t mm = 0; mm < a.nmember; ++mm) gst(a.last_s, mm, collect_fused(a, b.tag, mm));
+        __hip_atomic_store(a.gen, b.gen + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    __syncthreads();
+    return s_s[b.m - b.m_first];
+  }
+  uint32_t S = b.lw0;
+  if (b.wide) {   // the block's OR per member slot
+    __shared__ uint32_t s_lw[kBlock / 64][2];
+    const uint32_t o0 = wave_or(b.lw0), o1 = wave_or(b.lw1);
+    s_lw[threadIdx.x >> 6][0] = o0;   // the wave's value, from every lane
+    s_lw[threadIdx.x >> 6][1] = o1;
+    __syncthreads();
+    S = 0u;
+#pragma unroll
+    for (int i = 0; i < kBlock / 64; ++i) S |= s_lw[i][b.m - b.m_first];
+  }
+  // every member's S for speedy_read_level_sets: the same word from each of its columns
+  gst(a.last_s, b.m, S);
+  return S;
+}
+
+// The float64 column budgets of this block (a.f.budget is set; block-uniform).
+template <int KX>
+__device__ __forceinline__ void column_budgets(const KArgs& a, uint32_t bid, const BlockPos& b, const PhaseA<float, KX>& pa,
+                                               const PhaseB<float, KX>& pb, const double colsum[2]) {
+  const uint32_t j = b.c - divq(b.c, a.dlat) * a.nlat;
+  const double w = (double)gld(a.f.coa, j);
+  const double E = (double)pb.evap2, P = (double)pa.precnv + (double)pa.precls;
+  const double res = colsum[1] - (E - P);
+  const double v[kBudParts] = {w * colsum[0], w * colsum[1], w * E, w * P, w * res, fabs(res), w};
+  block_budget_partials(a, bid, b.gid, b.active, b.m - b.m_first, v);
+}
+
+template <int KX, bool DIAG, bool FUSED, bool EXTRA>
+__device__ __forceinline__ void fwd_body(const KArgs& a, uint32_t bid) {
+  constexpr bool kTau = !FUSED && KX <= 8;
+  __shared__ float s_tau[kTau ? 4 * KX * kBlock : 1];
+  const auto ts = tau_store<kTau>(s_tau);
+  const BlockPos b = block_pos<FUSED>(a, bid);
+  ColumnIn<float, KX> col;
+  load_state<KX, EXTRA>(a, b.m, b.c, col);
+  load_zonal<KX>(a, b.c, col);   // S-independent; its loads travel with the state's
+  store_uv_zeros<KX>(a, b.m, b.c);
   PhaseA<float, KX> pa;
   phase_a<float, KX>(col, a.p, a.v, a.u, pa);
   float tend_t[KX], tend_q[KX];
   tend_after_a<KX>(a.term_mask, pa, tend_t, tend_q);
-  if (FUSED && need_s) {
-    // publish this block's word(s) for the call's level set: a wave-level OR per
-    // member slot (a fused block spans at most two members), then one word per slot
-    __shared__ uint32_t s_wor[kBlock / 64][2];
-    const uint32_t bit = active ? clip_bit(pa.icltop, KX) : 0u;
-    const uint32_t o0 = wave_or<!VJP>(m == m_first ? bit : 0u), o1 = wave_or<!VJP>(m != m_first ? bit : 0u);
-    if ((threadIdx.x & 63u) == 0) { s_wor[threadIdx.x >> 6][0] = o0; s_wor[threadIdx.x >> 6][1] = o1; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      for (uint32_t j = 0; j < nm; ++j) {
-        uint32_t w = 0u;
-#pragma unroll
-        for (int i = 0; i < kBlock / 64; ++i) w |= s_wor[i][j];
-        __hip_atomic_store(&a.partial[2u * bid + j], (tag << 16) | w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-  }
+  if (FUSED && a.level_set < 0) publish_level_bits(a, bid, b, pa.icltop, KX);
   PhaseB<float, KX> pb;
   phase_b1<float, KX>(col, pa, a.p, a.v, a.u, pb, ts);
   tend_after_b1<KX>(a.term_mask, pb, tend_q);
-  uint32_t S = (uint32_t)a.level_set;
-  if (VJP && need_s) {
-    // the forward + VJP kernels: wave 0 gathers S for the block's member(s)
-    if (threadIdx.x < 64u) {
-      for (uint32_t j = 0; wide && j < nm; ++j) {
-        const uint32_t v = FUSED ? collect_fused(a, tag, m_first + j) : collect_chunks(a, m_first + j);
-        if (threadIdx.x == 0) s_s[j] = v;
-      }
-      if (bid == 0) {
-        // every member's S for speedy_read_level_sets; in the fused path this also
-        // waits for every block's word, i.e. every block has read the generation
-        for (uint32_t mm = 0; mm < a.nmember; ++mm) {
-          const uint32_t v = FUSED ? collect_fused(a, tag, mm) : collect_chunks(a, mm);
-          if (threadIdx.x == 0) gst(a.last_s, mm, v);
-        }
-        if (FUSED && threadIdx.x == 0) {
-          const uint32_t g = __hip_atomic_load(a.gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          __hip_atomic_store(a.gen, g + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
-    }
-    __syncthreads();
-    if (wide) {
-      S = s_s[m - m_first];
-    } else {   // two-kernel path, members narrower than a block: each spans <= 2 chunks
-      S = 0u;
-      const uint32_t b0 = divq(m * a.ncol, a.dchunk), b1 = divq(m * a.ncol + a.ncol - 1u, a.dchunk);
-      for (uint32_t b = b0; b <= b1; ++b) S |= gld(a.partial, b * a.jmax + (m - divq(b * a.chunk, a.dcol)));
-    }
-  } else if (FUSED && need_s) {
-    if (threadIdx.x < 64u) {   // wave 0 gathers S for the block's member(s)
-      for (uint32_t j = 0; j < nm; ++j) {
-        const uint32_t v = collect_fused_t<true>(a, tag, m_first + j);
-        if (threadIdx.x == 0) s_s[j] = v;
-      }
-      if (bid == 0) {
-        // every member's S for speedy_read_level_sets; this also waits for every
-        // block's word, i.e. every block has read the generation
-        for (uint32_t mm = 0; mm < a.nmember; ++mm) {
-          const uint32_t v = collect_fused_t<true>(a, tag, mm);
-          if (threadIdx.x == 0) gst(a.last_s, mm, v);
-        }
-        if (threadIdx.x == 0) {
-          const uint32_t g = __hip_atomic_load(a.gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          __hip_atomic_store(a.gen, g + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
-    }
-    __syncthreads();
-    S = s_s[m - m_first];
-  } else if (need_s) {
-    if (wide) {   // the block's OR per member slot
-      __shared__ uint32_t s_lw[kBlock / 64][2];
-      const uint32_t o0 = wave_or<true>(lw0), o1 = wave_or<true>(lw1);
-      if ((threadIdx.x & 63u) == 0) { s_lw[threadIdx.x >> 6][0] = o0; s_lw[threadIdx.x >> 6][1] = o1; }
-      __syncthreads();
-      S = 0u;
-#pragma unroll
-      for (int i = 0; i < kBlock / 64; ++i) S |= s_lw[i][m - m_first];
-    } else {
-      S = lw0;
-    }
-    // every member's S for speedy_read_level_sets, from its first column
-    if (active && c == 0u) gst(a.last_s, m, S);
-  }
-  // The forward + VJP kernels keep the zonal loads and all output stores here:
-  // moving them earlier changed their register allocation and, at 16 levels,
-  // gave wrong gradients on gfx950 (the kernels spill ~4 KB per lane).
-  if (VJP) load_zonal<KX>(a, c, col);
+  const uint32_t S = gather_level_set<FUSED>(a, bid, b);
   phase_b2<float, KX, DIAG>(col, pa, S, a.p, a.v, a.u, a.flags, pb, ts);
-  uint32_t limited = 0u;
   double colsum[2] = {0.0, 0.0};
-  if (active) limited = store_outputs<KX, DIAG, EXTRA, VJP>(a, m, c, col, pa, pb, tend_t, tend_q, colsum);
-  if (EXTRA && a.f.budget) {   // float64 column budgets (block-uniform branch)
-    const uint32_t j = c - divq(c, a.dlat) * a.nlat;
-    const double w = (double)gld(a.f.coa, j);
-    const double E = (double)pb.evap2, P = (double)pa.precnv + (double)pa.precls;
-    const double res = colsum[1] - (E - P);
-    const double v[kBudParts] = {w * colsum[0], w * colsum[1], w * E, w * P, w * res, fabs(res), w};
-    block_budget_partials(a, bid, gid, active, m - m_first, v);
+  store_outputs<KX, DIAG, EXTRA>(a, b.m, b.c, col, pa, pb, tend_t, tend_q, colsum);
+  if (EXTRA && a.f.budget) column_budgets<KX>(a, bid, b, pa, pb, colsum);
+}
+
+// Forward + VJP (all terms; the optional verify steps and budgets by run-time
+// flags).  The forward's phase B and its reversal are interleaved
+// (speedy_adjoint.hpp: the longwave's two sweeps; the surface fluxes and the
+// shortwave reversed from their own tapes): nothing of phase B is computed twice
+// but the up sweep's transmissivities, and the tendencies are the forward
+// kernels' bit for bit.  The longwave tape lies in LDS, [slot][thread].
+template <int KX, bool FUSED>
+__device__ __forceinline__ void vjp_body(const KArgs& a, uint32_t bid) {
+  // Values of phase A that phase B does not read wait in LDS (tvd, qsat and, up to
+  // eight levels, rh above the top level) or are read again from memory (phi, dL/ddq), in
+  // the kernels whose registers are short: the batched ones (two waves per SIMD at 7 and 8
+  // levels, 79 floats a column with the tape: two blocks fill a CU's 160 KB).
+  constexpr int kTape = vjp_tape_floats<KX>();
+  constexpr bool kStash = !FUSED;
+  constexpr int kStashRh = KX <= 8 ? KX - 1 : 0;
+  __shared__ float s_tape[(kTape + (kStash ? 2 * KX + kStashRh : 0)) * kBlock];
+  LdsStore tape{s_tape + threadIdx.x};
+  const BlockPos b = block_pos<FUSED>(a, bid);
+  const size_t ncol = a.ncol;
+  const size_t base3 = (size_t)b.m * KX * ncol + b.c;
+  ColumnIn<float, KX> col;
+  load_state<KX, true>(a, b.m, b.c, col);
+  load_zonal<KX>(a, b.c, col);
+  store_uv_zeros<KX>(a, b.m, b.c);
+  PhaseA<float, KX> pa;
+  phase_a<float, KX>(col, a.p, a.v, a.u, pa);
+  if (FUSED && a.level_set < 0) publish_level_bits(a, bid, b, pa.icltop, KX);
+  // the term-ordered sums (speedy_physics.py:123-125), each term added as it exists
+  float tend_t[KX], tend_q[KX];
+#pragma unroll
+  for (int k = 0; k < KX; ++k) {
+    tend_t[k] = (0.0f + pa.tconv[k]) + pa.tlsc[k];
+    tend_q[k] = (0.0f + pa.qconv[k]) + pa.qlsc[k];
   }
-  if (VJP && a.adj.g_t != nullptr) {   // batches mix forward-only and VJP segments
-    ColumnCt<float, KX> ct;
-    load_cotangents<KX>(a, m, c, ct);
-    float g_qraw[KX];
-    verify_ct<float, KX>(EXTRA ? a.flags : 0u, limited, a.u.dt_step, ct, g_qraw);
-    ColumnAdj<float, KX> g;
-    // longwave flux tapes in LDS, [slot][thread]: the kernel runs one block per CU
-    // (up to eight levels, KX more slots hold g_qraw across the adjoint, where it
-    // would otherwise take KX registers)
-    constexpr int kQraw = KX <= 8 ? KX : 0;
-    __shared__ float s_tape[(vjp_tape_floats<KX>() + kQraw) * kBlock];
-    LdsStore tape{s_tape + threadIdx.x};
-    if constexpr (kQraw > 0) {
+  ColumnCt<float, KX> ct;
+  load_cotangents<KX>(a, b.m, b.c, ct);
+  PhaseB<float, KX> pb;
+  ColumnAdj<float, KX> g;
+  VjpTapeB<float, KX> t;
+  phase_b1_vjp<float, KX>(col, pa, a.p, a.v, a.u, ct, pb, g, t, tape);
+  if constexpr (kStash) {
 #pragma unroll
-      for (int k = 0; k < KX; ++k) tape.put(vjp_tape_floats<KX>() + k, g_qraw[k]);
+    for (int k = 0; k < KX; ++k) {
+      tape.put(kTape + k, pb.tvd[k]);
+      tape.put(kTape + KX + k, pa.qsat[k]);
+      if (k > 0 && kStashRh > 0) tape.put(kTape + 2 * KX + k - 1, pa.rh[k]);
     }
-    column_vjp<float, KX>(col, pa, pb, S, a.p, a.v, a.u, a.flags, ct, g, tape);
-    if (EXTRA && (a.flags & SPEEDY_FLAG_VERIFY_STATE)) {
-      const size_t base3 = (size_t)m * KX * a.ncol + c;
-#pragma unroll
-      for (int k = 0; k < KX; ++k) g.Q[k] = verify_q_grad(gld(a.f.q, base3 + k * (size_t)a.ncol), g.Q[k]);
-    }
-    if constexpr (kQraw > 0) {
-      const LdsStore t = tape.after(g.Q[0]);
-#pragma unroll
-      for (int k = 0; k < KX; ++k) g.Q[k] += t.get(vjp_tape_floats<KX>() + k);
-    } else {
-#pragma unroll
-      for (int k = 0; k < KX; ++k) g.Q[k] += g_qraw[k];
-    }
-    if (active) store_grads<KX>(a, m, c, g);
-    block_param_partials(a, bid, gid, active, m - m_first, g.prm);
   }
+  const uint32_t S = gather_level_set<FUSED>(a, bid, b);
+  phase_b2_taped<float, KX>(col, pa, S, a.p, a.v, a.u, a.flags, ct, pb, g, t);
+  const bool budget = a.f.budget != nullptr;
+  const double dpg = (double)col.ps * (double)(P0 / GRAV);   // p0 ps / g; times dhs_k: dp_k / g
+  double colsum[2] = {0.0, 0.0};
+  uint32_t limited = 0u;
+#pragma unroll
+  for (int k = 0; k < KX; ++k) {
+    tend_t[k] = tend_t[k] + pb.tsw[k];
+    float q = tend_q[k];
+    if (k == KX - 1) { tend_t[k] = tend_t[k] + pb.dts1; q = q + pb.dqs1; }
+    q = q + pb.qvd[k];
+    if (a.flags & SPEEDY_FLAG_VERIFY_TENDENCIES) {
+      bool lim;
+      q = verify_dq(gld(a.f.q, base3 + k * ncol), q, a.u.dt_step, lim);   // the unclamped q (re-read, L2)
+      limited |= (lim ? 1u : 0u) << k;
+      ct.dq[k] = sel(lim, 0.0f, ct.dq[k]);   // its cotangent goes to the unclamped q alone (below)
+    }
+    gst(a.f.dq, base3 + k * ncol, q);
+    if (budget) colsum[1] += (double)q * ((double)a.v.dhs[k] * dpg);
+  }
+  gst(a.f.du, base3 + (KX - 1) * ncol, 0.0f + pb.du1);
+  gst(a.f.dv, base3 + (KX - 1) * ncol, 0.0f + pb.dv1);
+  phase_b2_vjp<float, KX>(col, pa, S, a.p, a.v, a.u, ct, pb, g, t, tape);
+  if constexpr (kStash) {
+    uint32_t zero = 0u;   // an offset known only once the longwave is reversed: the reads below stay below
+    asm volatile("" : "+v"(zero) : "v"(g.T[0]));
+    const LdsStore st = tape.after(g.T[0]);
+#pragma unroll
+    for (int k = 0; k < KX; ++k) {
+      const size_t e = base3 + k * ncol + zero;
+      col.PHI[k] = gld(a.f.phi, e);
+      ct.dq[k] = sel(((limited >> k) & 1u) != 0u, 0.0f, gld(a.adj.ct_dq, e));
+      pb.tvd[k] = st.get(kTape + k);
+      pa.qsat[k] = st.get(kTape + KX + k);
+      pa.rh[k] = (k > 0 && kStashRh > 0) ? st.get(kTape + 2 * KX + k - 1) : mdiv(col.Q[k], pa.qsat[k]);
+      pa.se[k] = (float)CP * col.T[k] + col.PHI[k];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < KX; ++k) {
+    const float tt = (tend_t[k] + pb.tlw[k]) + pb.tvd[k];
+    gst(a.f.dt, base3 + k * ncol, tt);
+    if (budget) colsum[0] += (double)CP * (double)tt * ((double)a.v.dhs[k] * dpg);
+  }
+  if (budget) column_budgets<KX>(a, bid, b, pa, pb, colsum);
+  phase_a_adj<float, KX>(col, pa, a.p, a.v, a.u, ct, g);
+  if (a.flags & SPEEDY_FLAG_VERIFY_STATE) {
+#pragma unroll
+    for (int k = 0; k < KX; ++k) g.Q[k] = verify_q_grad(gld(a.f.q, base3 + k * ncol), g.Q[k]);
+  }
+  if (a.flags & SPEEDY_FLAG_VERIFY_TENDENCIES) {   // verify_ct's g_qraw (the cotangent re-read, L2)
+#pragma unroll
+    for (int k = 0; k < KX; ++k)
+      g.Q[k] += sel(((limited >> k) & 1u) != 0u, -gld(a.adj.ct_dq, base3 + k * ncol) / a.u.dt_step, 0.0f);
+  }
+  store_grads<KX>(a, b.m, b.c, g);
+  block_param_partials(a, bid, b.gid, b.active, b.m - b.m_first, g.prm);
 }
 
 
@@ -874,7 +912,14 @@ __global__ __launch_bounds__(kBlock) void param_reduce_kernel(KArgs a) { member_
 
 template <int KX, bool DIAG, bool FUSED, bool VJP, bool EXTRA>
 __global__ __launch_bounds__(kBlock) void fwd_kernel(KArgs a) {
-  fwd_body<KX, DIAG, FUSED, VJP, EXTRA>(a, blockIdx.x);
+  // The forward + VJP reads its arguments through a pointer to the argument segment:
+  // as by-value arguments they are all loaded at entry, and the scalar registers spill
+  // into vector-register lanes (9039 -> 7629 VALU instructions at 8 levels).  The
+  // forward keeps by-value arguments: its loads at entry hide behind the state's.
+  if constexpr (VJP)
+    vjp_body<KX, FUSED>(*(const KArgs*)__builtin_amdgcn_kernarg_segment_ptr(), blockIdx.x);
+  else
+    fwd_body<KX, DIAG, FUSED, EXTRA>(a, blockIdx.x);
 }
 
 // ---------------------------------------------------------------- batches
@@ -899,7 +944,7 @@ template <int KX>
 __global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_only_batch_kernel(const KArgs* __restrict__ segs,
                                                                 const uint32_t* __restrict__ table) {
   const uint32_t e = __builtin_amdgcn_readfirstlane(table[blockIdx.x]);
-  fwd_body<KX, false, false, false, true>(segs[e >> kSegShift], e & kSegLocalMask);
+  fwd_body<KX, false, false, true>(segs[e >> kSegShift], e & kSegLocalMask);
 }
 
 // Forward-only segments of a batch in which none needs the verify steps or the
@@ -911,7 +956,7 @@ template <int KX>
 __global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_plain_batch_kernel(const KArgs* __restrict__ segs,
                                                                  const uint32_t* __restrict__ table) {
   const uint32_t e = __builtin_amdgcn_readfirstlane(table[blockIdx.x]);
-  fwd_body<KX, false, false, false, false>(segs[e >> kSegShift], e & kSegLocalMask);
+  fwd_body<KX, false, false, false>(segs[e >> kSegShift], e & kSegLocalMask);
 }
 
 // Forward-only segments that also write the PhysicsData diagnostics: single
@@ -920,18 +965,22 @@ template <int KX>
 __global__ __launch_bounds__(kBlock) void fwd_diag_batch_kernel(const KArgs* __restrict__ segs,
                                                                 const uint32_t* __restrict__ table) {
   const uint32_t e = __builtin_amdgcn_readfirstlane(table[blockIdx.x]);
-  fwd_body<KX, true, false, false, true>(segs[e >> kSegShift], e & kSegLocalMask);
+  fwd_body<KX, true, false, true>(segs[e >> kSegShift], e & kSegLocalMask);
 }
 
-// Forward + VJP segments of a batch.  Built for two waves per SIMD at 7 and 8
-// levels (at most 256 registers a lane, 132 B of scratch a lane at 8 levels and
-// none at 7, 45 KB of LDS a block): 521 -> 412 us at T425 x 8 levels, against one
-// wave per SIMD without scratch.  The fused forward + VJP kernel keeps one wave
-// per SIMD and no scratch.
+// Forward + VJP segments of a batch.  Bound by VALU issue.  Built for two waves per
+// SIMD at 7 and 8 levels (at most 256 registers a lane; 56 B of scratch at 8 levels,
+// none at 7; 80 KB of LDS a block), one at 16 (512 registers, 156 KB of LDS, 232 B
+// of scratch).  T425 x 8 levels: 412 -> 195 us, and 64 members of T31 x 16 levels:
+// 2710 -> 275 us, against reversing every term from a recompute of its own
+// (speedy_adjoint.hpp).  The descriptor is __restrict__, so uniforms are scalar
+// loads next to their use (without it, vector loads: 310 us at T425).  The fused
+// kernel keeps one wave per SIMD and no scratch.
 template <int KX>
-__global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_batch_kernel(const KArgs* segs, const uint32_t* table) {
+__global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_batch_kernel(const KArgs* __restrict__ segs,
+                                                                        const uint32_t* __restrict__ table) {
   const uint32_t e = __builtin_amdgcn_readfirstlane(table[blockIdx.x]);
-  fwd_body<KX, false, false, true, true>(segs[e >> kSegShift], e & kSegLocalMask);
+  vjp_body<KX, false>(segs[e >> kSegShift], e & kSegLocalMask);
 }
 
 __global__ __launch_bounds__(kBlock) void param_reduce_batch_kernel(const KArgs* __restrict__ segs,
@@ -1184,11 +1233,8 @@ int launch_fwd(const KArgs& a, hipStream_t s) {
   const int64_t cap = init.cap;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   (void)hipStreamIsCapturing(s, &cs);
-  // Sixteen-level forward + VJP calls always take the batch route: at sixteen
-  // levels no one-thread-per-column kernel fits the register file, and the fused
-  // sixteen-level forward + VJP kernel (3.3 KB of scratch per lane) gave wrong
-  // gradients on gfx950 in a case whose host build is right; the batch kernel
-  // passes every sixteen-level case (cause of the fused kernel's error not found).
+  // Sixteen-level forward + VJP calls always take the batch route, whose kernel
+  // keeps phase A in LDS and spills less.
   const bool fused = a.level_set < 0 && (int64_t)a.nblk <= cap && a.ncol >= (uint32_t)kBlock && !(VJP && KX == 16) &&
                      !(a.flags & kFlagBatchRoute);
   const int kind = VJP ? 2 : 1;
@@ -1277,11 +1323,8 @@ int launch_fwd_kx(const KArgs& a, hipStream_t s) {
   return a.f.diag ? launch_fwd<KX, true, false, false>(a, s) : launch_fwd<KX, false, false, false>(a, s);
 }
 
-// The forward + VJP always runs the instantiation that carries the optional
-// verify / budget code (run-time flags).  The instantiation without it gave
-// wrong state and parameter gradients at 16 levels on gfx950 (deterministic;
-// the same source as a host build, and the instantiation with the optional
-// code, agree with the float64 adjoint), so it is not built.
+// The forward + VJP has one instantiation, with the optional verify / budget code
+// (run-time flags).
 template <int KX>
 int launch_fwd_vjp_kx(const KArgs& a, hipStream_t s) {
   return launch_fwd<KX, false, true, true>(a, s);

@@ -134,3 +134,35 @@ def test_term_census(kernels_asm):
         print(f"{k:18s} {v:5d}  {100.0 * v / fused:5.1f} %")
     print(f"{'terms':18s} {total:5d}  {100.0 * total / fused:5.1f} % of fwd_kernel<8> ({fused} VALU)")
     assert 0.75 * fused <= total <= fused
+
+
+def test_no_vector_write_before_all_lanes_are_back(kernels_asm):
+    """Where a branch that some lanes skip ends, the block's first act must be to turn
+    all lanes back on.  A vector register, accumulation register or scratch write
+    placed before that reaches only the lanes that took the branch; the compiler puts
+    register copies there when registers are short, and the other lanes then lose the
+    copied value (wrong tendencies in part of the lanes).  The column code has no such
+    branch, and no kernel of the library shows the pattern."""
+    write = re.compile(r"(v_(?!readlane|readfirstlane|writelane|cmp|cmpx)\w+|scratch_store\w*|buffer_store\w*)\s")
+    found, seen = {}, 0
+    for m in re.finditer(r"\.amdhsa_kernel (\S+)\n", kernels_asm):
+        name = m.group(1)
+        begin = kernels_asm.index("\n" + name + ":")
+        lines = kernels_asm[begin:m.start()].split("\n")
+        start = 0
+        for i, line in enumerate(lines):
+            ins = line.strip()
+            if ins.startswith((".LBB", "; %bb.")):
+                start = i
+            elif re.match(r"s_or_b64 exec, exec|s_(or|andn2)_saveexec", ins):
+                seen += 1
+                early = [x.strip() for x in lines[start + 1:i] if write.match(x.strip())]
+                if early:
+                    found.setdefault(name, []).append(early)
+    assert seen, "no lane-mask restore found: the pattern no longer matches the assembly"
+    assert not found, found
+    column = [m.group(1) for m in re.finditer(r"\.amdhsa_kernel (\S*fwd_plain_batch_kernel\S*)\n", kernels_asm)]
+    assert len(column) == 3
+    for name in column:   # the plain forward has no branch of that kind at all
+        begin = kernels_asm.index("\n" + name + ":")
+        assert "saveexec" not in kernels_asm[begin:kernels_asm.index(".end_amdhsa_kernel", begin)], name
