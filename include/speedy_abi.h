@@ -54,17 +54,18 @@ enum {
  * unclamped q and dt = SpeedyDate.dt_seconds (verify_tendencies, :321-342). */
 #define SPEEDY_FLAG_VERIFY_STATE 0x2u
 #define SPEEDY_FLAG_VERIFY_TENDENCIES 0x4u
-/* PLAIN_LAUNCH (no counterpart in the reference): an uncaptured call whose grid
- * fits on the GPU at once makes a plain launch of the single-launch kernel
- * instead of a cooperative one, as calls under graph capture always do.  The
- * cooperative launch guarantees that all workgroups are resident together,
- * which the kernel's grid-wide level-set exchange needs; it costs about 10 us
- * per call on the GPU at T85.  With this flag, co-residency holds only when no
- * other work shares the GPU.  The exchange's wait is bounded, so the kernel
- * always ends, but if it gave up, speedy_workspace_status reports it and the
- * call's results are invalid.  Ignored by speedy_fwd_batch. */
+/* PLAIN_LAUNCH (no counterpart in the reference): accepted and without effect.
+ * The single-launch kernel is always launched plainly: a workgroup whose
+ * level-set exchange misses another's word (not running yet, because other work
+ * holds the GPU) forms that word itself, so the call does not rely on all
+ * workgroups being resident together. */
 #define SPEEDY_FLAG_PLAIN_LAUNCH 0x8u
-#define SPEEDY_FLAGS_ALL 0xFu
+/* NO_WAIT (no counterpart in the reference): in the single-launch kernel a
+ * workgroup forms every word of the level-set exchange itself instead of waiting
+ * for the others'.  The same results; slower unless the GPU is shared with long
+ * work that keeps part of the call's workgroups from starting. */
+#define SPEEDY_FLAG_NO_WAIT 0x10u
+#define SPEEDY_FLAGS_ALL 0x1Fu
 
 /* term_mask bit i selects the tendency of term i (speedy_physics.py:67-80)
  * for the sum; every term always runs, so the data handed between terms are
@@ -180,7 +181,7 @@ int speedy_diag_names(int32_t kx, char *buf, size_t buf_len);
  * level_set < 0: the Q1 cloud-top level set (shortwave_radiation.py:63-70) is
  * computed per member over all its columns; >= 0: used as given (bit k =
  * level k), for parity tests.  A grid whose workgroups fit on the GPU at once
- * runs as one cooperative launch; other grids (and a given level set) run as a
+ * runs as one launch; other grids (and a given level set) run as a
  * one-segment batch, described in the workspace, in two to four launches.
  * Stream-ordered and safe to capture in a HIP graph; no allocation. */
 int speedy_fwd(const SpeedyFields *fields, const SpeedyVertical *vert, const SpeedyParams *params,

@@ -9,13 +9,17 @@
 // top (end of phase A) and the shortwave (phase B).  Two paths:
 //
 //   fused (the grid fits on the GPU at once, e.g. T85 = 128 blocks):
-//     one cooperative launch.  Right after the cloud top every block publishes
-//     its columns' OR of level bits as one tagged word in its own slot (tag =
-//     the call's generation), computes the S-independent work (longwave
-//     transmissivity, longwave down, vertical diffusion), then polls only the
-//     slots of the blocks covering its member until every tag is current.
-//     Block 0 then advances the generation.  No read-modify-write atomics:
-//     contended same-address atomics cost microseconds per call on this GPU.
+//     one launch.  Right after the cloud top every block publishes its columns' OR
+//     of level bits as one tagged word in its own slot (tag = the call's
+//     generation), computes the S-independent work (longwave transmissivity,
+//     longwave down, vertical diffusion), then polls only the slots of the blocks
+//     covering its member until every tag is current.  A word that stays away
+//     (its block is not running yet: other work holds the GPU) is formed by the
+//     waiting block itself from the state, so no block depends on another one being
+//     resident, and a plain launch is enough (a cooperative one took 20 us more).
+//     Block 0 advances the generation once every block has published.  No
+//     read-modify-write atomics: contended same-address atomics cost microseconds
+//     per call on this GPU.
 //   two launches (larger grids, members narrower than a block, a given S, and
 //     every batch): a level-set kernel, a fixed number of blocks each covering a
 //     contiguous chunk of columns, writes per-(chunk, member) ORs; the forward
@@ -43,7 +47,13 @@ constexpr int kBlock = 256;
 // Internal flag (above the public SPEEDY_FLAG_* bits): take the one-segment batch
 // route even where the fused launch could run (speedy_fwd_noalloc).
 constexpr uint32_t kFlagBatchRoute = 1u << 31;
-constexpr uint32_t kSpinLimit = 4u << 20;   // barrier wait bound (~seconds): a wave always exits
+// Polls (about 1 us each) before a block forms the words it misses itself.  In a
+// GPU without other work the words are there after one or two; each word formed
+// takes one wave about 10 us, so waiting out a short kernel of another stream is
+// cheaper than replacing the blocks it holds up.
+constexpr uint32_t kHelpAfter = 256;
+// Bound of block 0's wait for the last block to publish (hours: a wave always exits).
+constexpr uint32_t kSpinLimit = 1u << 31;
 
 struct Divisor {          // n / d for n < 2^32 by multiply-high + one correction step
   uint32_t d, m;          // m = floor(2^32 / d) (unused when d == 1)
@@ -312,30 +322,96 @@ __device__ __forceinline__ uint32_t clip_bit(int icl, int kx) {
   return 1u << (icl < 0 ? 0 : (icl > kx - 1 ? kx - 1 : icl));
 }
 
-// Fused path: OR of the level bits of member m over the published words of the
-// blocks covering it, polled until every word carries `tag` (one wave, all lanes
-// active throughout: lanes past the last word read it again, since OR is
-// idempotent).  Bounded: after kSpinLimit polls it flags the error word and returns.
-__device__ __forceinline__ uint32_t collect_fused(const KArgs& a, uint32_t tag, uint32_t m) {
+// Level bits of member m over the columns of block b (cloud tops from the state),
+// by one wave with all lanes active: lanes on columns outside the member or the
+// grid take the member's last column.
+template <int KX>
+__device__ __forceinline__ uint32_t block_level_bits(const KArgs& a, uint32_t b, uint32_t m) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t last = m * a.ncol + a.ncol - 1u;
+  uint32_t bits = 0u;
+  for (uint32_t i = 0; i < (uint32_t)kBlock; i += 64u) {
+    const uint32_t gid = b * kBlock + i + lane;
+    const bool mine = gid >= m * a.ncol && gid <= last;
+    const uint32_t c = sel(mine, gid, last) - m * a.ncol;
+    const size_t base3 = (size_t)m * KX * a.ncol + c;
+    ColumnIn<float, KX> col;
+#pragma unroll
+    for (int k = 1; k < KX; ++k) {
+      col.T[k] = gld(a.f.t, base3 + k * (size_t)a.ncol);
+      const float q = gld(a.f.q, base3 + k * (size_t)a.ncol);
+      col.Q[k] = sel((a.flags & SPEEDY_FLAG_VERIFY_STATE) != 0u, verify_q(q), q);
+      col.PHI[k] = gld(a.f.phi, base3 + k * (size_t)a.ncol);
+    }
+    col.ps = gld(a.f.ps, (size_t)m * a.ncol + c);
+    bits |= clip_bit(cloud_top<float, KX>(col, a.p, a.v, a.u), KX);
+  }
+  return bits;   // the member's last column is one of its own: its bit belongs to S
+}
+
+// One poll of the published words of the blocks covering member m: the OR of their
+// level bits, and whether any word is not of this call yet.  By one wave, all lanes
+// active throughout: lanes past the last word read it again (OR is idempotent).
+__device__ __forceinline__ uint32_t poll_words(const KArgs& a, uint32_t tag, uint32_t m, bool& missing) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t b0 = (m * a.ncol) / kBlock, b1 = (m * a.ncol + a.ncol - 1u) / kBlock;
-  for (uint32_t spins = 0;; ++spins) {
-    uint32_t acc = 0;
-    int stale = 0;
-    for (uint32_t bb = b0; bb <= b1; bb += 64u) {
-      const uint32_t b = min(bb + lane, b1);
-      const uint32_t j = m - divq(b * kBlock, a.dcol);
-      const uint32_t w = __hip_atomic_load(&a.partial[2u * b + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      stale |= (w >> 16) != tag;
-      acc |= w & 0xffffu;
-    }
-    if (!__any(stale)) return wave_or(acc);
-    if (spins >= kSpinLimit) {
-      __hip_atomic_store(a.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return wave_or(acc);
-    }
+  uint32_t acc = 0;
+  int stale = 0;
+  for (uint32_t bb = b0; bb <= b1; bb += 64u) {
+    const uint32_t b = min(bb + lane, b1);
+    const uint32_t j = m - divq(b * kBlock, a.dcol);
+    const uint32_t w = __hip_atomic_load(&a.partial[2u * b + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    stale |= (w >> 16) != tag;
+    acc |= w & 0xffffu;
+  }
+  missing = __any(stale);
+  return wave_or(acc);
+}
+
+// Fused path: member m's level set, by one wave.  Polls the published words; after
+// kHelpAfter polls (at once with SPEEDY_FLAG_NO_WAIT) every word still missing is
+// formed here instead.
+template <int KX>
+__device__ __forceinline__ uint32_t collect_fused(const KArgs& a, uint32_t tag, uint32_t m) {
+  const uint32_t patience = (a.flags & SPEEDY_FLAG_NO_WAIT) ? 0u : kHelpAfter;
+  for (uint32_t spins = 0; spins < patience; ++spins) {
+    bool missing;
+    const uint32_t acc = poll_words(a, tag, m, missing);
+    if (!missing) return acc;
     __builtin_amdgcn_s_sleep(1);
   }
+  const uint32_t b0 = (m * a.ncol) / kBlock, b1 = (m * a.ncol + a.ncol - 1u) / kBlock;
+  uint32_t acc = 0u;
+  for (uint32_t b = b0; b <= b1; ++b) {   // uniform: every lane reads the same word
+    const uint32_t j = m - divq(b * kBlock, a.dcol);
+    const uint32_t w = __builtin_amdgcn_readfirstlane(
+        __hip_atomic_load(&a.partial[2u * b + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if ((w >> 16) == tag && patience != 0u)
+      acc |= w & 0xffffu;
+    else
+      acc |= block_level_bits<KX>(a, b, m);
+  }
+  return wave_or(acc);
+}
+
+// Block 0: every member's S to last_s (speedy_read_level_sets), then the next
+// generation, once every block of the call has published (and so read this one).
+__device__ __forceinline__ void finish_generation(const KArgs& a, uint32_t gen, uint32_t tag) {
+  for (uint32_t m = 0; m < a.nmember; ++m) {
+    bool missing;
+    uint32_t v = poll_words(a, tag, m, missing);
+    for (uint32_t spins = 0; missing; ++spins) {
+      if (spins >= kSpinLimit) {
+        __hip_atomic_store(a.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        break;
+      }
+      if (spins < kHelpAfter) __builtin_amdgcn_s_sleep(1);
+      else __builtin_amdgcn_s_sleep(100);
+      v = poll_words(a, tag, m, missing);
+    }
+    gst(a.last_s, m, v);
+  }
+  __hip_atomic_store(a.gen, gen + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Two-kernel path: member m's word of level-set chunk b (levelset_batch_kernel output).
@@ -635,19 +711,15 @@ __device__ __forceinline__ void publish_level_bits(const KArgs& a, uint32_t bid,
 
 // The level set of this thread's member: gathered from the published words
 // (fused) or from the chunk words (two launches), or the call's own.
-template <bool FUSED>
+template <int KX, bool FUSED>
 __device__ __forceinline__ uint32_t gather_level_set(const KArgs& a, uint32_t bid, const BlockPos& b) {
   if (a.level_set >= 0) return (uint32_t)a.level_set;
   if (FUSED) {
     __shared__ uint32_t s_s[2];
     if (b.wave == 0u) {   // wave 0 gathers S for the block's member(s)
-      for (uint32_t j = 0; j < b.nm; ++j) s_s[j] = collect_fused(a, b.tag, b.m_first + j);
-      if (bid == 0) {
-        // every member's S for speedy_read_level_sets; this also waits for every
-        // block's word, i.e. every block has read the generation
-        for (uint32_t mm = 0; mm < a.nmember; ++mm) gst(a.last_s, mm, collect_fused(a, b.tag, mm));
-        __hip_atomic_store(a.gen, b.gen + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
+      for (uint32_t j = 0; j < b.nm; ++j) s_s[j] = collect_fused<KX>(a, b.tag, b.m_first + j);
+    } else if (b.wave == 1u && bid == 0u) {
+      finish_generation(a, b.gen, b.tag);   // no other block waits for this one here: it has published
     }
     __syncthreads();
     return s_s[b.m - b.m_first];
@@ -680,6 +752,15 @@ __device__ __forceinline__ void column_budgets(const KArgs& a, uint32_t bid, con
   block_budget_partials(a, bid, b.gid, b.active, b.m - b.m_first, v);
 }
 
+// The launch's by-value argument block, read again from the argument segment: what
+// follows loads its uniforms anew (scalar loads) where the scalar registers could not
+// hold them from kernel entry and would spill them lane by lane into vector registers.
+__device__ __forceinline__ const KArgs& reread() {
+  typedef const __attribute__((address_space(4))) KArgs* ConstPtr;
+  ConstPtr p = (ConstPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const KArgs*)p;
+}
 template <int KX, bool DIAG, bool FUSED, bool EXTRA>
 __device__ __forceinline__ void fwd_body(const KArgs& a, uint32_t bid) {
   constexpr bool kTau = !FUSED && KX <= 8;
@@ -698,11 +779,15 @@ __device__ __forceinline__ void fwd_body(const KArgs& a, uint32_t bid) {
   PhaseB<float, KX> pb;
   phase_b1<float, KX>(col, pa, a.p, a.v, a.u, pb, ts);
   tend_after_b1<KX>(a.term_mask, pb, tend_q);
-  const uint32_t S = gather_level_set<FUSED>(a, bid, b);
-  phase_b2<float, KX, DIAG>(col, pa, S, a.p, a.v, a.u, a.flags, pb, ts);
+  const uint32_t S = gather_level_set<KX, FUSED>(a, bid, b);
+  // with every output compiled in, the uniforms of phase b2 and the stores are read
+  // again (T85 with diagnostics and verify: 17.2 -> 16.2 us; the plain forward is
+  // 0.4 us slower that way)
+  const KArgs& o = FUSED && DIAG && EXTRA ? reread() : a;
+  phase_b2<float, KX, DIAG>(col, pa, S, o.p, o.v, o.u, o.flags, pb, ts);
   double colsum[2] = {0.0, 0.0};
-  store_outputs<KX, DIAG, EXTRA>(a, b.m, b.c, col, pa, pb, tend_t, tend_q, colsum);
-  if (EXTRA && a.f.budget) column_budgets<KX>(a, bid, b, pa, pb, colsum);
+  store_outputs<KX, DIAG, EXTRA>(o, b.m, b.c, col, pa, pb, tend_t, tend_q, colsum);
+  if (EXTRA && a.f.budget) column_budgets<KX>(o, bid, b, pa, pb, colsum);
 }
 
 // Forward + VJP (all terms; the optional verify steps and budgets by run-time
@@ -753,7 +838,7 @@ __device__ __forceinline__ void vjp_body(const KArgs& a, uint32_t bid) {
       if (k > 0 && kStashRh > 0) tape.put(kTape + 2 * KX + k - 1, pa.rh[k]);
     }
   }
-  const uint32_t S = gather_level_set<FUSED>(a, bid, b);
+  const uint32_t S = gather_level_set<KX, FUSED>(a, bid, b);
   phase_b2_taped<float, KX>(col, pa, S, a.p, a.v, a.u, a.flags, ct, pb, g, t);
   const bool budget = a.f.budget != nullptr;
   const double dpg = (double)col.ps * (double)(P0 / GRAV);   // p0 ps / g; times dhs_k: dp_k / g
@@ -1231,8 +1316,6 @@ int launch_fwd(const KArgs& a, hipStream_t s) {
   if (init.err != hipSuccess)
     return fail(SPEEDY_ERR_HIP, std::string("speedy: stack limit: ") + hipGetErrorString(init.err));
   const int64_t cap = init.cap;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  (void)hipStreamIsCapturing(s, &cs);
   // Sixteen-level forward + VJP calls always take the batch route, whose kernel
   // keeps phase A in LDS and spills less.
   const bool fused = a.level_set < 0 && (int64_t)a.nblk <= cap && a.ncol >= (uint32_t)kBlock && !(VJP && KX == 16) &&
@@ -1241,18 +1324,8 @@ int launch_fwd(const KArgs& a, hipStream_t s) {
   hipError_t e = hipSuccess;
   if (fused) {
     const int slot = timer_begin(s, kind);
-    if (cs == hipStreamCaptureStatusNone && !(a.flags & SPEEDY_FLAG_PLAIN_LAUNCH)) {
-      void* args[] = {const_cast<KArgs*>(&a)};
-      e = hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&fwd_kernel<KX, DIAG, true, VJP, EXTRA>),
-                                     dim3(a.nblk),
-                                     dim3(kBlock), args, 0, s);
-    } else {
-      // Graph capture (or SPEEDY_FLAG_PLAIN_LAUNCH): a plain launch of a grid
-      // that fits on the device; the level-set poll is bounded, so the kernel
-      // terminates in every case.
-      hipLaunchKernelGGL((fwd_kernel<KX, DIAG, true, VJP, EXTRA>), dim3(a.nblk), dim3(kBlock), 0, s, a);
-      e = hipGetLastError();
-    }
+    hipLaunchKernelGGL((fwd_kernel<KX, DIAG, true, VJP, EXTRA>), dim3(a.nblk), dim3(kBlock), 0, s, a);
+    e = hipGetLastError();
     timer_end(s, slot);
   } else {
     // Grids the fused launch cannot take (beyond one co-resident launch, members

@@ -17,6 +17,7 @@ FLAG_LFLUXLAND = 0x1
 FLAG_VERIFY_STATE = 0x2
 FLAG_VERIFY_TENDENCIES = 0x4
 FLAG_PLAIN_LAUNCH = 0x8
+FLAG_NO_WAIT = 0x10
 TERMS = ("set_physics_flags", "set_forcing", "spec_hum_to_rel_hum", "get_convection_tendencies",
          "get_large_scale_condensation_tendencies", "get_clouds", "get_shortwave_rad_fluxes",
          "get_downward_longwave_rad_fluxes", "get_surface_fluxes", "get_upward_longwave_rad_fluxes",

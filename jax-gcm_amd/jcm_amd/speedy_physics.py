@@ -187,11 +187,8 @@ class SpeedyPhysics(Physics):
     def __init__(self, parameters: Parameters | None = None, checkpoint_terms: bool = True,
                  with_diagnostics: bool = False, device: str | torch.device | None = None,
                  plain_launch: bool = False, check_barrier: bool = False):
-        """plain_launch: uncaptured single-launch calls use a plain launch instead of a
-        cooperative one (about 10 us less per call at T85).  Only for a process that
-        has the GPU to itself: the grid-wide level-set exchange then relies on all
-        workgroups being resident together.  barrier_status() reports a call whose
-        exchange gave up (its results are invalid) and resets the workspace.
+        """plain_launch: kept for its callers; single-launch calls are always launched
+        plainly.
         check_barrier: after every call, synchronize and raise SpeedyError if the
         call's level-set exchange gave up, resetting the workspace (costs a
         synchronization per call)."""
@@ -470,7 +467,7 @@ class SpeedyPhysics(Physics):
         _native.check(self._lib.speedy_workspace_status(ws.data_ptr(), ws.numel(), ctypes.byref(st), stream),
                       "speedy_workspace_status")
         if st.value:
-            raise _native.SpeedyError("the call's level-set exchange gave up (not all workgroups were resident); "
+            raise _native.SpeedyError("the call's level-set exchange gave up (a workgroup never started); "
                                       "its results are invalid and the workspace has been reset")
 
     def level_sets(self, nlon: int, nlat: int, nmember: int = 1) -> list:

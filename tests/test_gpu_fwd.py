@@ -800,3 +800,42 @@ def test_fwd_fused_equals_batch_route(kx, variant):
             assert torch.equal(d_f._diag, d_b._diag), f"kx{kx} {variant}: diagnostics differ"
         if budgets:
             assert torch.equal(b_f, b_b), f"kx{kx} {variant}: budgets {b_f} vs {b_b}"
+
+
+@pytest.mark.parametrize("kx", [7, 8, 16])
+@pytest.mark.parametrize("nlon,nlat,nmember,verify", [(64, 32, 1, False), (100, 50, 3, True), (256, 128, 1, False),
+                                                      (23, 13, 1, True)])
+def test_level_set_words_formed_instead_of_awaited(kx, nlon, nlat, nmember, verify):
+    """SPEEDY_FLAG_NO_WAIT makes every workgroup form the level-set words it would
+    otherwise wait for (what a waiting workgroup does when another one is not running):
+    tendencies, gradients and recorded level sets equal the waiting call's bit for bit,
+    on members that share workgroups and a last workgroup that is partly empty, and a
+    waiting call on the same workspace afterwards still does."""
+    import torch
+    from jcm_amd import _native
+    from jcm_amd.physics_interface import PhysicsTendency
+    from jcm_amd.speedy_physics import SpeedyPhysics
+    case = synthetic.make_case(nlon, nlat, kx, seed=5, land=True, nmember=nmember, member_t_sigma=0.5)
+    st, fo, ge, da = case
+    st = st.copy(specific_humidity=st.specific_humidity * np.float32(1.15))   # columns that condense at various levels
+    phys = SpeedyPhysics(parameters=synthetic.draw_vjp_parameters(2))
+    g = torch.Generator(device="cuda").manual_seed(1)
+    cot = PhysicsTendency(*[torch.randn(st.temperature.shape, generator=g, device="cuda") for _ in range(4)])
+
+    def both():
+        t, _ = phys.compute_tendencies(st, fo, ge, da, verify=verify)
+        s = phys.level_sets(nlon, nlat, nmember)
+        tv, sg, pg = phys.compute_tendencies_vjp(st, fo, ge, da, cot, verify=verify)
+        torch.cuda.synchronize()
+        assert phys.level_sets(nlon, nlat, nmember) == s and phys.barrier_status(nlon, nlat, nmember) == 0
+        return s, [getattr(t, f) for f in FIELDS] + [getattr(tv, f) for f in FIELDS] + [
+            getattr(sg, f) for f in FIELDS + ("normalized_surface_pressure",)] + [pg[k] for k in sorted(pg)]
+
+    sets, want = both()
+    phys._launch_flags |= _native.FLAG_NO_WAIT
+    sets_own, got = both()
+    phys._launch_flags &= ~_native.FLAG_NO_WAIT
+    sets_again, again = both()
+    assert sets == sets_own == sets_again
+    for a, b, c in zip(want, got, again):
+        assert torch.equal(a, b) and torch.equal(a, c)
