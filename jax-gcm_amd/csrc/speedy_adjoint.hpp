@@ -122,9 +122,10 @@ SPD_HD void verify_ct(uint32_t flags, uint32_t limited, R dt, ColumnCt<R, KX>& c
 template <typename R>
 SPD_HD R verify_q_grad(R q_raw, R g) { return sel(q_raw < R(0.0), R(0.0), g); }
 
-// Reciprocal for the adjoint's linear arithmetic: the hardware reciprocal and one
+// Reciprocal for gradients of the fields alone: the hardware reciprocal and one
 // Newton step (1 ulp), 3 instructions where a division takes 11.  The forward's
-// values, which decisions depend on, keep mdiv.
+// values, which decisions depend on, and what the parameter gradients pass through
+// keep mdiv: those are sums of many columns that nearly cancel.
 SPD_HD float mrcp(float b) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const float r = __builtin_amdgcn_rcpf(b);
@@ -181,9 +182,8 @@ SPD_HD void lw_level_adj(int k, const R a_tau[4], R a_s0, R a_s1, const ColumnIn
     const R a_ab = ax * (-(c.ps * v.dhs[k]));
     if (bnd == 0) {
       if (k >= 2 && k <= KX - 2) g.cloudc += a_ab * sel(k > a.icltop, R(p.ablcl1), R(p.ablcl2));
-    } else if (bnd == 1) {
-      g.prm[VJP_CO2] += a_ab * u.ablco2_d;
-    } else if (k >= 1) {
+    } else if (bnd >= 2 && k >= 1) {   // band 1 (CO2): the caller's
+
       const R wv = (bnd == 2) ? p.ablwv1 : p.ablwv2;
       if (k >= 2 && k <= KX - 2) {
         const R x = wv * c.Q[k], ac2 = a.cloudc * p.ablcl2;
@@ -274,7 +274,7 @@ template <typename R, int KX, class Store>
 SPD_HD void lw_down_vjp(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const SpeedyParams& p,
                         const SpeedyVertical& v, const Uniforms<R>& u, const ColumnCt<R, KX>& ct, PhaseB<R, KX>& b,
                         Store& tape, R aF[4]) {
-  const R rps = mrcp(c.ps);
+  const R rps = mdiv(R(1.0), c.ps);
   R Fd[4], Fprev = R(0.0);
 #pragma unroll
   for (int k = 0; k < KX; ++k) {
@@ -323,16 +323,21 @@ SPD_HD void lw_surface_adj(const Uniforms<R>& u, const SpeedyParams& p, R tsfc, 
   a_flux_h[1] = aF[1] * u.refsfc;
 }
 
+// The gradient of the CO2 multiplier is the one sum that cancels both between the
+// directions and over the columns, so each direction's part is formed by itself (it
+// waits on the tape, in the place of the level's band-1 fluxes) and added in the order
+// of the levels, upward flux first.
+//
 // The up sweep: longwave up (longwave_radiation.py:119-202; b.dfl enters holding the
 // longwave-down divergence, b.tlw leaves as lw_up leaves it) and every level's
 // reversal.  b.rlus2, b.tsfc, b.flux_h: the hand-offs of the surface fluxes and the
 // shortwave; a_rlds: cotangent of the downward flux at the surface.
 template <typename R, int KX, class Store>
 SPD_HD void lw_up_vjp(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const SpeedyParams& p,
-                      const SpeedyVertical& v, const Uniforms<R>& u, PhaseB<R, KX>& b, const Store& tape,
+                      const SpeedyVertical& v, const Uniforms<R>& u, PhaseB<R, KX>& b, Store& tape,
                       const ColumnCt<R, KX>& ct, R a_rlds, ColumnAdj<R, KX>& g) {
   const R ps = c.ps;
-  const R rps = mdiv(R(1.0), ps), a_rps = mrcp(ps);
+  const R rps = mdiv(R(1.0), ps);
   const R stratc0 = c.stratz * ps, stratc1 = u.eps1 * ps;
   R Fu[4], aD[4];
   {
@@ -349,14 +354,14 @@ SPD_HD void lw_up_vjp(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const Sp
   R Gnext = ((Fu[0] + Fu[1]) + Fu[2]) + Fu[3];
   // a_below: cotangent of the half-level temperature under level k, complete once
   // level k is reversed, and then passed on to T
-  R a_below = R(0.0), corlw2 = R(0.0);
+  R a_below = R(0.0), corlw2 = R(0.0), up0 = R(0.0), dn0 = R(0.0);
 #pragma unroll
   for (int k = KX - 1; k >= 0; --k) {
     const ColumnIn<R, KX> ck = column_at_level<R, KX>(c, k, Fu[0]);
-    const Store tk = tape.after(Fu[0]);
+    auto&& tk = tape.after(Fu[0]);
     LwLevel<R> L;
     lw_level<R, KX>(k, ck, a, p, v, u, L);
-    const R a_dfl = dfl_ct<R, KX>(ct, v, k, a_rps);
+    const R a_dfl = dfl_ct<R, KX>(ct, v, k, rps);
     R afb[4], atau[4], as0 = R(0.0), as1 = R(0.0);
     if (k == KX - 1) as0 = (a_rlds - a_dfl) * u.corlw;   // rlds += corlw, dfl[KX-1] -= corlw
     if (k <= 1) {   // dfl[k] -= dhs[k] stratc1 st4a0[k] (+ stratc0 at k = 0)
@@ -374,8 +379,14 @@ SPD_HD void lw_up_vjp(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const Sp
         // up: tau Fu + em fb (st0 - em st1); down: tau Fd + em fb (st0 + em st1).  The flux
         // and the emission nearly cancel: their difference is formed before the product
         const R sum = au + ad, dif = ad - au;
-        const R es = em * L.st1, es2 = es + es;
-        atau[bnd] = au * (Fu[bnd] - L.fb[bnd] * (L.st0 - es2)) + ad * (fd - L.fb[bnd] * (L.st0 + es2));
+        const R es = em * L.st1;
+        const R up = au * (Fu[bnd] - L.fb[bnd] * (L.st0 - R(2.0) * em * L.st1));
+        const R dn = ad * (fd - L.fb[bnd] * (L.st0 + R(2.0) * em * L.st1));
+        atau[bnd] = up + dn;
+        if (bnd == 1) {
+          tk.put((k - 1) * 8 + 5, up * tau * (-(ck.ps * v.dhs[k])));
+          tk.put((k - 1) * 8 + 1, dn * tau * (-(ck.ps * v.dhs[k])));
+        }
         afb[bnd] = em * (sum * L.st0 + dif * es);
         const R ef = em * L.fb[bnd];
         as0 += sum * ef;
@@ -396,7 +407,12 @@ SPD_HD void lw_up_vjp(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const Sp
         const R em = R(1.0) - L.tau[bnd];
         const R au = -a_dfl, ad = aD[bnd] - a_dfl;
         const R sum = au + ad;
-        atau[bnd] = au * (Fu[bnd] - L.fb[bnd] * L.st0) - ad * (L.fb[bnd] * L.st0);
+        const R up = au * (Fu[bnd] - L.fb[bnd] * L.st0), dn = -ad * L.fb[bnd] * L.st0;
+        atau[bnd] = up + dn;
+        if (bnd == 1) {
+          up0 = up * L.tau[1] * (-(ck.ps * v.dhs[0]));
+          dn0 = dn * L.tau[1] * (-(ck.ps * v.dhs[0]));
+        }
         afb[bnd] = sum * em * L.st0;
         as0 += sum * em * L.fb[bnd];
         ft[bnd] = L.tau[bnd] * Fu[bnd] + em * (L.fb[bnd] * (L.st0 - em * L.st1));
@@ -418,6 +434,13 @@ SPD_HD void lw_up_vjp(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const Sp
     a_below = a_Th[0];
     settle_lw<R, KX>(g, k, Fu, aD, a_below);
   }
+  auto&& tc = tape.after(up0);
+  g.prm[VJP_CO2] += up0 * u.ablco2_d;
+#pragma unroll
+  for (int k = 1; k < KX; ++k) g.prm[VJP_CO2] += tc.get((k - 1) * 8 + 5) * u.ablco2_d;
+#pragma unroll
+  for (int k = KX - 1; k >= 1; --k) g.prm[VJP_CO2] += tc.get((k - 1) * 8 + 1) * u.ablco2_d;
+  g.prm[VJP_CO2] += dn0 * u.ablco2_d;
 }
 
 // ---------------------------------------------------------------- surface fluxes
@@ -427,7 +450,7 @@ SPD_HD void surface_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const 
                         const ColumnCt<R, KX>& ct, R a_rlus2, R& a_rsds, R& a_rlds, ColumnAdj<R, KX>& g) {
   if (!t.land) return;   // every surface output is zero without lfluxland (Q8)
   const R ps = c.ps;
-  const R rps = mrcp(ps);
+  const R rps = mdiv(R(1.0), ps);
   const R fm = c.fmask;
   const R gs = v.grdsig[KX - 1], gc = v.grdscp[KX - 1];
   const R a_ustr2 = ct.du1 * rps * gs, a_vstr2 = ct.dv1 * rps * gs;
@@ -488,7 +511,7 @@ SPD_HD void surface_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const 
     a_drls += a_rlus0 * t.dtskin;
     a_dtskin += a_rlus0 * t.drls;
     const R Dn = t.clamb + t.drls + (s.chl * t.den1 * (R(CP) + (R(ALHC) * t.qs1)));
-    const R a_hflc = a_dtskin * mrcp(Dn);
+    const R a_hflc = mdiv(a_dtskin, Dn);
     const R a_Dn = -a_hflc * t.dtskin;
     a_drls += a_Dn;
     a_den1 += a_Dn * s.chl * (R(CP) + R(ALHC) * t.qs1);
@@ -602,7 +625,7 @@ SPD_HD void shortwave_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, cons
                           const SwTape<R, KX>& fwd, const ColumnCt<R, KX>& ct, const R a_flux_h[2], R a_rsds,
                           ColumnAdj<R, KX>& g) {
   const R ps = c.ps;
-  const R rps = mrcp(ps);
+  const R rps = mdiv(R(1.0), ps);
   SwTape<R, KX> t;
   t.psaz = fwd.psaz;
   t.acloud = fwd.acloud;
@@ -782,13 +805,13 @@ SPD_HD void clouds_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const S
   const R a_cc = g.cloudc - R(1.2) * a_clsx;
   const R a_fsa = a_fstab * dmin_x(mmax(t.fstab_arg, R(0.0)), R(1.0)) * dmax_x(t.fstab_arg, R(0.0));
   const R a_gse = a_fsa * u.rgse;
-  const R rdphi = mrcp(c.PHI[KX - 2] - c.PHI[KX - 1]);
+  const R rdphi = mdiv(R(1.0), c.PHI[KX - 2] - c.PHI[KX - 1]);
   g.se[KX - 2] += a_gse * rdphi;
   g.se[KX - 1] += -a_gse * rdphi;
   g.Q[KX - 2] += g.qcloud;
   const R a_raw = a_cc * dmin_x(t.ccraw, R(1.0));
   const R mx = mmax(R(EPS), t.pr1);
-  const R a_pr1 = a_raw * p.wpcl * (R(0.5) * mrcp(msqrt_1ulp(mx))) * dmax_x(t.pr1, R(EPS));
+  const R a_pr1 = a_raw * p.wpcl * mdiv(R(0.5), msqrt_1ulp(mx)) * dmax_x(t.pr1, R(EPS));
   const R a_sum = a_pr1 * dmin_x(R(86.4) * (a.precnv + a.precls), R(p.pmaxcl)) * R(86.4);
   g.precnv += a_sum;
   g.precls += a_sum;
@@ -797,7 +820,7 @@ SPD_HD void clouds_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const S
   int nt = 0;
 #pragma unroll
   for (int k = 2; k <= KX - 3; ++k) nt += (t.cu[k] == t.cmax) ? 1 : 0;
-  const R share = a_cmax * mrcp(R(nt > 0 ? nt : 1));
+  const R share = mdiv(a_cmax, R(nt > 0 ? nt : 1));
   R a_cc0 = R(0.0);
 #pragma unroll
   for (int k = 2; k <= KX - 3; ++k) {
@@ -851,7 +874,7 @@ SPD_HD void convection_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, con
                            const ColumnCt<R, KX>& ct, ColumnAdj<R, KX>& g) {
   const int iptop = a.iptop_conv;
   const R ps = c.ps;
-  const R rps = mrcp(ps);
+  const R rps = mdiv(R(1.0), ps);
   R a_dfse[KX], a_dfqa[KX];
   a_dfse[0] = ct.dt[0];
   a_dfqa[0] = ct.dq[0];
@@ -957,17 +980,16 @@ SPD_HD void convection_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, con
   R a_qdif;
   {
     const R den = t.qmax - t.qb;
-    const R rden = mrcp(den);
     const R ratio = mdiv(t.qdif, den);
     const R m = mmin(R(5.0), ratio);
     const R a_fpsa = a_fmass * u.fm0 * m;
     const R a_fm0 = a_fmass * t.fpsa * m;
     const R a_ratio = a_fmass * u.fm0 * t.fpsa * dmin_x(ratio, R(5.0));
-    a_qdif = a_ratio * rden;
-    const R a_den = -a_ratio * ratio * rden;
+    a_qdif = mdiv(a_ratio, den);
+    const R a_den = mdiv(-a_ratio * ratio, den);
     a_qmax += a_den;
     a_qb += -a_den;
-    g.prm[VJP_TRCNV] += a_fm0 * (-(u.fm0 * mrcp(R(p.trcnv))));
+    g.prm[VJP_TRCNV] += a_fm0 * (-mdiv(u.fm0, R(p.trcnv)));
     const R y = (ps - p.psmin) * u.rdps;
     g.ps += a_fpsa * mmin(R(1.0), y) + a_fpsa * ps * dmin_x(y, R(1.0)) * u.rdps;
   }
@@ -1037,7 +1059,7 @@ struct ArrayStore {
   R v[N];
   SPD_HD void put(int i, R x) { v[i] = x; }
   SPD_HD R get(int i) const { return v[i]; }
-  SPD_HD const ArrayStore& after(R) const { return *this; }
+  SPD_HD ArrayStore& after(R) { return *this; }
 };
 
 // What phase b2 hands from its forward to its reversal.
@@ -1080,9 +1102,9 @@ SPD_HD void phase_b2_taped(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, uin
 template <typename R, int KX, class Store>
 SPD_HD void phase_b2_vjp(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, uint32_t S, const SpeedyParams& p,
                          const SpeedyVertical& v, const Uniforms<R>& u, const ColumnCt<R, KX>& ct, PhaseB<R, KX>& b,
-                         ColumnAdj<R, KX>& g, const VjpTapeB<R, KX>& t, const Store& tape) {
+                         ColumnAdj<R, KX>& g, const VjpTapeB<R, KX>& t, Store& tape) {
   R a_rlus2, a_flux_h[2], a_rsds = R(0.0), a_rlds = R(0.0);
-  lw_surface_adj<R, KX>(u, p, b.tsfc, dfl_ct<R, KX>(ct, v, KX - 1, mrcp(c.ps)), t.aF, a_rlus2, a_flux_h);
+  lw_surface_adj<R, KX>(u, p, b.tsfc, dfl_ct<R, KX>(ct, v, KX - 1, mdiv(R(1.0), c.ps)), t.aF, a_rlus2, a_flux_h);
   surface_adj<R, KX>(c, a, b, p, v, u, t.sf, ct, a_rlus2, a_rsds, a_rlds, g);
   shortwave_adj<R, KX>(c, a, b, S, p, v, u, t.sw, ct, a_flux_h, a_rsds, g);
   lw_up_vjp<R, KX>(c, a, p, v, u, b, tape, ct, a_rlds, g);
