@@ -6,6 +6,7 @@ fallback: if the shared library is missing or a GPU is absent the calls raise.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 
 KX_MAX = 16
@@ -90,6 +91,29 @@ class SpeedyError(RuntimeError):
 
 _lib = None
 
+# The native call preparation (csrc/host_calls.cpp): one C++ function per entry point
+# that does a plain call's host work.  It links torch's libraries, so torch comes first.
+import torch  # noqa: E402,F401
+
+try:
+    from . import _host_calls as host
+except ModuleNotFoundError:   # not built: load() says so
+    host = None
+
+
+def address(fn) -> int:
+    """Address of a ctypes function."""
+    return ctypes.cast(fn, ctypes.c_void_p).value
+
+
+def _bind_host(lib):
+    from .params import _GROUPS, Parameters
+    p = Parameters.default()
+    ints = {n for n, t in SpeedyParams._fields_ if t is ctypes.c_int32}
+    slots = [(g, n, getattr(SpeedyParams, n).offset, n in ints)
+             for g, grp in enumerate(_GROUPS) for n in vars(getattr(p, grp))]
+    host.bind_physics(address(lib.speedy_fwd), address(lib.speedy_fwd_vjp), address(lib.speedy_diag_rows), _GROUPS, slots)
+
 
 def load(path: str | None = None):
     """Load the library once; raise SpeedyError if it is missing (no fallback)."""
@@ -99,6 +123,8 @@ def load(path: str | None = None):
     p = path or LIB_PATH
     if not os.path.exists(p):
         raise SpeedyError(f"{p} not found: build it with __graft_entry__.build() (there is no CPU fallback)")
+    if host is None:
+        raise SpeedyError("_host_calls.so not found: build it with __graft_entry__.build()")
     lib = ctypes.CDLL(p)
     lib.speedy_abi_version.restype = ctypes.c_int
     lib.speedy_workspace_bytes.restype = ctypes.c_size_t
@@ -146,6 +172,7 @@ def load(path: str | None = None):
     lib.speedy_last_error.restype = ctypes.c_char_p
     if lib.speedy_abi_version() != ABI_VERSION:
         raise SpeedyError("libspeedy_hip ABI version mismatch")
+    _bind_host(lib)
     _lib = lib
     return lib
 
@@ -158,6 +185,11 @@ def check(rc: int, what: str):
 
 def diag_names(kx: int) -> list[str]:
     """Row names of the diagnostic output; 3-D fields expand to kx rows 'name[k]'."""
+    return list(_diag_names(kx))
+
+
+@functools.lru_cache(maxsize=None)
+def _diag_names(kx: int) -> tuple:
     lib = load()
     buf = ctypes.create_string_buffer(8192)
     check(lib.speedy_diag_names(kx, buf, len(buf)), "speedy_diag_names")
@@ -167,7 +199,7 @@ def diag_names(kx: int) -> list[str]:
             out.extend(f"{n[:-2]}[{k}]" for k in range(kx))
         else:
             out.append(n)
-    return out
+    return tuple(out)
 
 
 KERNEL_KINDS = ("levelset", "fwd", "fwd_vjp", "param_reduce")

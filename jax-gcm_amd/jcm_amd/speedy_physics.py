@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import copy
 import ctypes
+import functools
 from types import SimpleNamespace
 from typing import Any, Tuple
 
@@ -32,6 +33,7 @@ VERIFY_FLAGS = _native.FLAG_VERIFY_STATE | _native.FLAG_VERIFY_TENDENCIES
 # torch's raw current-stream query (the one its compiled kernels use): about 0.2 us,
 # against about 2 us for torch.cuda.current_stream(device).cuda_stream
 _RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_VJP_NAMES = tuple(f"{g}.{n}" for g, n in VJP_PARAMS)
 _STATE_FIELDS = (("u_wind", "u"), ("v_wind", "v"), ("temperature", "t"), ("specific_humidity", "q"),
                  ("geopotential", "phi"))
 
@@ -66,8 +68,11 @@ class PhysicsData:
         self._names = names
         self._kx = kx
         self._hshape = tuple(hshape)
-        self._index = {n: i for i, n in enumerate(names)}
         self.date = date           # PhysicsData.date (physics_data.py), read by the term calls
+
+    @functools.cached_property
+    def _index(self):
+        return {n: i for i, n in enumerate(self._names)}
 
     def _row(self, name):
         i = self._index[name]
@@ -261,6 +266,15 @@ class SpeedyPhysics(Physics):
             return ctypes.c_void_p(_RAW_STREAM(torch.cuda.current_device() if idx is None else idx))
         return ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
 
+    def _where(self):
+        """(device index, raw stream or None for the default stream) of a call, as the
+        workspace keys hold them."""
+        idx = self.device.index
+        if idx is None:
+            idx = torch.cuda.current_device()
+        s = _RAW_STREAM(idx) if _RAW_STREAM is not None else torch.cuda.current_stream(idx).cuda_stream
+        return idx, s or None
+
     def _climatology(self, arr) -> torch.Tensor:
         """climatology_rows(arr) on the device, made once per array (per version of a
         tensor, so in-place updates are seen); the calls then read the day's row."""
@@ -365,6 +379,18 @@ class SpeedyPhysics(Physics):
         SPEEDY_NBUDGET) into ``self.last_budgets``: a float64 tensor (nmember, 6) whose
         columns are named by ``_native.BUDGET_NAMES``."""
         self._require_gpu()
+        if _native.host is not None and not budgets and not self.check_barrier:
+            r = _native.host.fwd(self._consts, self._workspaces, self.parameters, *self._where(), state, forcing, geometry,
+                                 date, (VERIFY_FLAGS if verify else 0) | self._launch_flags, term_mask, level_set,
+                                 self.with_diagnostics is True)
+            if r.__class__ is tuple:
+                data = None
+                if r[4] is not None:
+                    kx, ix, il = geometry.nodal_shape
+                    data = PhysicsData(r[4], _native._diag_names(kx), kx, (ix, il), date)
+                return PhysicsTendency(r[0], r[1], r[2], r[3]), data
+            if r is not None:
+                _native.check(r, "speedy_fwd")
         keep: list = []
         f, t, nmember = self._fields(state, forcing, geometry, date, keep)
         kx, ix, il = geometry.nodal_shape
@@ -390,7 +416,7 @@ class SpeedyPhysics(Physics):
         _native.check(rc, "speedy_fwd")
         if self.check_barrier:
             self._raise_on_barrier(ix, il, nmember, stream)
-        data = PhysicsData(diag, _native.diag_names(kx), kx, (ix, il), date) if diag is not None else None
+        data = PhysicsData(diag, _native._diag_names(kx), kx, (ix, il), date) if diag is not None else None
         return PhysicsTendency(*out), data
 
     @property
@@ -448,6 +474,15 @@ class SpeedyPhysics(Physics):
         param_grads maps the five VJP parameters (params.VJP_PARAMS) to per-member sums.
         verify: as in compute_tendencies (the gradients then include the two steps)."""
         self._require_gpu()
+        if _native.host is not None and not self.check_barrier:
+            r = _native.host.fwd_vjp(self._consts, self._workspaces, self.parameters, *self._where(), state, forcing,
+                                     geometry, date, (VERIFY_FLAGS if verify else 0) | self._launch_flags, level_set,
+                                     cotangent)
+            if r.__class__ is tuple:
+                return (PhysicsTendency(r[0], r[1], r[2], r[3]), PhysicsState(r[4], r[5], r[6], r[7], None, r[8]),
+                        dict(zip(_VJP_NAMES, r[9:])))
+            if r is not None:
+                _native.check(r, "speedy_fwd_vjp")
         keep: list = []
         f, adj, outputs, (ix, il, nmember), flags = self.prepare_vjp(state, forcing, geometry, date, cotangent, keep)
         flags |= (VERIFY_FLAGS if verify else 0) | self._launch_flags

@@ -26,6 +26,7 @@ from typing import Dict, Optional
 
 import numpy as np
 
+from ._native import address, host
 from .physics_interface import PhysicsState, PhysicsTendency
 
 LIB_NAME = "libspeedy_sht.so"
@@ -101,6 +102,10 @@ def load(path: Optional[str] = None):
                                         ctypes.POINTER(_Spectral), CFP, sz, CFP]
         lib.speedy_sht_last_error.restype = ctypes.c_char_p
         lib.speedy_sht_last_error.argtypes = []
+        if host is not None:
+            host.bind_transforms(*(address(getattr(lib, n)) for n in (
+                "speedy_sht_workspace_bytes", "speedy_dynamics_to_physics", "speedy_physics_to_dynamics",
+                "speedy_physics_tendency_to_dynamics")))
         _lib = lib
         return lib
 
@@ -310,10 +315,26 @@ def _device_of(*xs):
     return torch.device("cuda", torch.cuda.current_device())
 
 
+def _native_call(name: str, field, *args):
+    """The native preparation of a conversion (csrc/host_calls.cpp) on the GPU of `field`:
+    its outputs, or None when the general path is to be taken."""
+    torch = _torch()
+    if host is None or _lib is None or not isinstance(field, torch.Tensor) or not field.is_cuda:
+        return None
+    idx = field.get_device()
+    r = getattr(host, name)(args[0], idx, torch._C._cuda_getCurrentRawStream(idx), *args[1:])
+    if r.__class__ is int:
+        _check(r, name)
+    return r
+
+
 def dynamics_state_to_physics_state(state: DynamicsState, dynamics: PrimitiveEquations) -> PhysicsState:
     """physics_interface.py:196-234 on the GPU: winds from vorticity/divergence,
     temperature plus the reference, humidity in g/kg, geopotential from
     orography and temperature, surface pressure exp(log_surface_pressure)."""
+    r = _native_call("dynamics_to_physics", state.vorticity, dynamics, state)
+    if r is not None:
+        return PhysicsState(*r)
     torch = _torch()
     g = dynamics.coords.horizontal
     dev = _device_of(state.vorticity, state.divergence, state.temperature_variation)
@@ -377,6 +398,9 @@ def _nodal_to_spectral(u, v, t, q, sp, dynamics, tendency):
 
 def physics_state_to_dynamics_state(physics_state: PhysicsState, dynamics: PrimitiveEquations) -> DynamicsState:
     """physics_interface.py:237-273 on the GPU (the geopotential is not read)."""
+    r = _native_call("to_dynamics", physics_state.u_wind, dynamics, physics_state, False)
+    if r is not None:
+        return DynamicsState(r[0], r[1], r[2], r[3], {"specific_humidity": r[4]})
     vor, div, tm, lsp, qm = _nodal_to_spectral(physics_state.u_wind, physics_state.v_wind, physics_state.temperature,
                                                physics_state.specific_humidity,
                                                physics_state.normalized_surface_pressure, dynamics, False)
@@ -387,6 +411,9 @@ def physics_tendency_to_dynamics_tendency(physics_tendency: PhysicsTendency,
                                           dynamics: PrimitiveEquations) -> DynamicsState:
     """physics_interface.py:275-303 on the GPU: the log-surface-pressure
     tendency is zeros shaped like one level of the temperature tendency."""
+    r = _native_call("to_dynamics", physics_tendency.u_wind, dynamics, physics_tendency, True)
+    if r is not None:
+        return DynamicsState(r[0], r[1], r[2], r[3], {"specific_humidity": r[4]}, sim_time=0.0)
     vor, div, tm, lsp, qm = _nodal_to_spectral(physics_tendency.u_wind, physics_tendency.v_wind,
                                                physics_tendency.temperature, physics_tendency.specific_humidity,
                                                None, dynamics, True)
