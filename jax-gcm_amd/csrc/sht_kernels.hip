@@ -420,10 +420,18 @@ __global__ __launch_bounds__(kThreads) void fourier_synthesis_generic(FourierArg
 }
 
 // The same two passes with both factors known at compile time (the nlon of the
-// Grid.T<N> table): each pass is a short dense DFT in registers whose roots are
-// literals (Roots<n>, evaluated by the compiler), with the line tile read from
-// and written to memory directly; only the pass-1 results and the N roots of
-// unity for the twiddles w^(i1 k2) go through LDS.
+// Grid.T<N> table): each pass is a short FFT in registers (fft, rfft, c2r below: radix
+// 2, 3, 4 and 5 steps with literal roots), with the line tile read from and written to
+// memory directly; only the pass-1 results and the N roots of unity for the twiddles
+// w^(i1 k2) go through LDS.
+//
+// The real side of each stage uses the Hermitian symmetry in k2: a thread takes the
+// pair (k2, N2 - k2), so half the pass-1 results are exchanged and the real FFTs do
+// half the work.  Bound by latency: of the launch's single wave of workgroups at T85, of
+// the few workgroups a CU holds at T213.  With dense sums for the short DFTs (n1 and n2
+// terms per output) T85 analysis and synthesis took 8.7 and 12.3 us, now 7.3 and 11.6;
+// T213 x 41 fields synthesis 115 us, now 53; a T425 conversion of 41 fields 1977 us in
+// the generic kernels, now 617.
 constexpr double kPiD = 3.14159265358979323846;
 constexpr double ct_sin(double x) {   // |x| <= pi, Taylor series to 1e-16
   double term = x, sum = x;
@@ -455,30 +463,241 @@ struct Roots {
   }
 };
 
-template <int N1, int N2>
-__global__ __launch_bounds__(kThreads) void fourier_analysis_kernel(FourierArgs a) {
-  constexpr int N = N1 * N2, NH = N2 / 2 + 1;
-  constexpr Roots<N1> R1{};
-  constexpr Roots<N2> R2{};
-  extern __shared__ float lds[];
-  const int tl = a.tl, b = blockIdx.y, j0 = blockIdx.x * tl;
-  float* twr = lds;
-  float* twi = twr + N;
-  float* zr = twi + N;            // [NH][N1][tl]
-  float* zi = zr + NH * N1 * tl;
+// First radix of a length: 4 where it divides, else the smallest of 2, 3, 5.
+constexpr int radix(int n) { return n % 4 == 0 ? 4 : n % 2 == 0 ? 2 : n % 3 == 0 ? 3 : n % 5 == 0 ? 5 : n; }
+
+// X_k = sum_j x_j w_n^(jk), in place and in natural order.  The inverse (conjugated
+// roots) is the same with real and imaginary parts exchanged: fft(im, re).
+template <int n>
+__device__ __forceinline__ void fft(float (&re)[n], float (&im)[n]) {
+  static_assert(n == 1 || radix(n) < n || n <= 5, "lengths of factors 2, 3 and 5");
+  if constexpr (n == 2) {
+    const float r = re[1], i = im[1];
+    re[1] = re[0] - r; im[1] = im[0] - i;
+    re[0] += r; im[0] += i;
+  } else if constexpr (n == 3) {
+    constexpr float s = 0.866025403784438647f;
+    const float tr = re[1] + re[2], ti = im[1] + im[2];
+    const float ar = re[0] - 0.5f * tr, ai = im[0] - 0.5f * ti;
+    const float br = s * (im[1] - im[2]), bi = s * (re[2] - re[1]);
+    re[0] += tr; im[0] += ti;
+    re[1] = ar + br; im[1] = ai + bi;
+    re[2] = ar - br; im[2] = ai - bi;
+  } else if constexpr (n == 4) {
+    const float ar = re[0] + re[2], ai = im[0] + im[2], br = re[0] - re[2], bi = im[0] - im[2];
+    const float cr = re[1] + re[3], ci = im[1] + im[3], dr = re[1] - re[3], di = im[1] - im[3];
+    re[0] = ar + cr; im[0] = ai + ci;
+    re[2] = ar - cr; im[2] = ai - ci;
+    re[1] = br + di; im[1] = bi - dr;
+    re[3] = br - di; im[3] = bi + dr;
+  } else if constexpr (n == 5) {
+    constexpr float c1 = 0.309016994374947424f, c2 = -0.809016994374947424f;
+    constexpr float s1 = 0.951056516295153572f, s2 = 0.587785252292473129f;
+    const float ar = re[1] + re[4], ai = im[1] + im[4], br = re[2] + re[3], bi = im[2] + im[3];
+    const float cr = re[1] - re[4], ci = im[1] - im[4], dr = re[2] - re[3], di = im[2] - im[3];
+    const float er = re[0] + c1 * ar + c2 * br, ei = im[0] + c1 * ai + c2 * bi;
+    const float fr = re[0] + c2 * ar + c1 * br, fi = im[0] + c2 * ai + c1 * bi;
+    const float gr = s1 * ci + s2 * di, gi = s1 * cr + s2 * dr;
+    const float hr = s2 * ci - s1 * di, hi = s2 * cr - s1 * dr;
+    re[0] += ar + br; im[0] += ai + bi;
+    re[1] = er + gr; im[1] = ei - gi;
+    re[4] = er - gr; im[4] = ei + gi;
+    re[2] = fr + hr; im[2] = fi - hi;
+    re[3] = fr - hr; im[3] = fi + hi;
+  } else if constexpr (n > 1) {
+    // j = j1 + b j2, k = k1 + a k2: a-point transforms over j2, twiddles, b-point over j1
+    constexpr int a = radix(n), b = n / a;
+    constexpr Roots<n> w{};
+    float tr[a][b], ti[a][b];
+#pragma unroll
+    for (int j = 0; j < b; ++j) {
+      float xr[a], xi[a];
+#pragma unroll
+      for (int i = 0; i < a; ++i) { xr[i] = re[j + b * i]; xi[i] = im[j + b * i]; }
+      fft<a>(xr, xi);
+#pragma unroll
+      for (int k = 0; k < a; ++k) {
+        const float c = w.c[(j * k) % n], s = w.s[(j * k) % n];
+        tr[k][j] = j * k == 0 ? xr[k] : xr[k] * c - xi[k] * s;
+        ti[k][j] = j * k == 0 ? xi[k] : xr[k] * s + xi[k] * c;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < a; ++k) {
+      fft<b>(tr[k], ti[k]);
+#pragma unroll
+      for (int q = 0; q < b; ++q) { re[k + a * q] = tr[k][q]; im[k + a * q] = ti[k][q]; }
+    }
+  }
+}
+
+// X_k for k <= n / 2 of a real x (the others are their conjugates).
+template <int n>
+__device__ __forceinline__ void rfft(const float (&x)[n], float (&re)[n / 2 + 1], float (&im)[n / 2 + 1]) {
+  if constexpr (n == 1) {
+    re[0] = x[0]; im[0] = 0.0f;
+  } else if constexpr (n == 2) {
+    re[0] = x[0] + x[1]; im[0] = 0.0f;
+    re[1] = x[0] - x[1]; im[1] = 0.0f;
+  } else if constexpr (n == 3) {
+    const float t = x[1] + x[2];
+    re[0] = x[0] + t; im[0] = 0.0f;
+    re[1] = x[0] - 0.5f * t; im[1] = 0.866025403784438647f * (x[2] - x[1]);
+  } else if constexpr (n == 5) {
+    constexpr float c1 = 0.309016994374947424f, c2 = -0.809016994374947424f;
+    constexpr float s1 = 0.951056516295153572f, s2 = 0.587785252292473129f;
+    const float a = x[1] + x[4], b = x[2] + x[3], c = x[1] - x[4], d = x[2] - x[3];
+    re[0] = x[0] + (a + b); im[0] = 0.0f;
+    re[1] = x[0] + c1 * a + c2 * b; im[1] = -(s1 * c + s2 * d);
+    re[2] = x[0] + c2 * a + c1 * b; im[2] = -(s2 * c - s1 * d);
+  } else if constexpr (n % 4 == 2) {
+    // n = 2 b, b odd: j = b j1 + 2 j2 mod n takes no twiddles (Good-Thomas)
+    constexpr int b = n / 2;
+    float p[b], q[b], pr[b / 2 + 1], pi[b / 2 + 1], qr[b / 2 + 1], qi[b / 2 + 1];
+#pragma unroll
+    for (int j = 0; j < b; ++j) {
+      p[j] = x[2 * j] + x[(2 * j + b) % n];
+      q[j] = x[2 * j] - x[(2 * j + b) % n];
+    }
+    rfft<b>(p, pr, pi);
+    rfft<b>(q, qr, qi);
+#pragma unroll
+    for (int k = 0; k <= b; ++k) {   // X_k = P (even k) or Q (odd k) at k mod b
+      const int m = k % b, c = m <= b / 2 ? m : b - m;
+      const float sg = m <= b / 2 ? 1.0f : -1.0f;
+      re[k] = k % 2 == 0 ? pr[c] : qr[c];
+      im[k] = sg * (k % 2 == 0 ? pi[c] : qi[c]);
+    }
+  } else {
+    static_assert(n % 4 == 0, "rfft lengths");
+    constexpr int b = n / 4;
+    constexpr Roots<n> w{};
+    float t0[b], t1r[b], t1i[b], t2r[b], t2i[b];
+#pragma unroll
+    for (int j = 0; j < b; ++j) {   // four-point transforms of real values: X_0 and X_2 real
+      const float p = x[j] + x[j + 2 * b], q = x[j + b] + x[j + 3 * b];
+      const float r = x[j] - x[j + 2 * b], s = x[j + 3 * b] - x[j + b];
+      const float c1 = w.c[j], s1 = w.s[j], c2 = w.c[(2 * j) % n], s2 = w.s[(2 * j) % n];
+      t0[j] = p + q;
+      t1r[j] = j == 0 ? r : r * c1 - s * s1;
+      t1i[j] = j == 0 ? s : r * s1 + s * c1;
+      t2r[j] = j == 0 ? p - q : (p - q) * c2;
+      t2i[j] = j == 0 ? 0.0f : (p - q) * s2;
+    }
+    float zr[b / 2 + 1], zi[b / 2 + 1];
+    rfft<b>(t0, zr, zi);
+    fft<b>(t1r, t1i);
+    fft<b>(t2r, t2i);
+#pragma unroll
+    for (int q = 0; q < b; ++q) {
+      if (q <= b / 2) { re[4 * q] = zr[q]; im[4 * q] = zi[q]; }
+      const int k = 1 + 4 * q;   // k or its mirror image n - k
+      if (k <= n / 2) { re[k] = t1r[q]; im[k] = t1i[q]; }
+      else { re[n - k] = t1r[q]; im[n - k] = -t1i[q]; }
+      if (2 + 4 * q <= n / 2) { re[2 + 4 * q] = t2r[q]; im[2 + 4 * q] = t2i[q]; }
+    }
+  }
+}
+
+// x_j = sum over the whole spectrum of X_k conj(w_n^(jk)), real, from X_k for k <= n / 2
+// (the imaginary parts of X_0 and X_{n/2} are not read).
+template <int n>
+__device__ __forceinline__ void c2r(const float (&re)[n / 2 + 1], const float (&im)[n / 2 + 1], float (&x)[n]) {
+  if constexpr (n == 1) {
+    x[0] = re[0];
+  } else if constexpr (n == 2) {
+    x[0] = re[0] + re[1];
+    x[1] = re[0] - re[1];
+  } else if constexpr (n == 3) {
+    const float a = re[0] - re[1], b = 1.73205080756887729f * im[1];
+    x[0] = re[0] + 2.0f * re[1];
+    x[1] = a - b;
+    x[2] = a + b;
+  } else if constexpr (n == 5) {
+    constexpr float c1 = 0.618033988749894848f, c2 = -1.618033988749894848f;   // twice the cosines
+    constexpr float s1 = 1.902113032590307144f, s2 = 1.175570504584946258f;
+    const float e = re[0] + c1 * re[1] + c2 * re[2], f = re[0] + c2 * re[1] + c1 * re[2];
+    const float g = s1 * im[1] + s2 * im[2], h = s2 * im[1] - s1 * im[2];
+    x[0] = re[0] + 2.0f * (re[1] + re[2]);
+    x[1] = e - g;
+    x[4] = e + g;
+    x[2] = f - h;
+    x[3] = f + h;
+  } else if constexpr (n % 4 == 2) {
+    constexpr int b = n / 2;
+    float p[b], q[b], pr[b / 2 + 1], pi[b / 2 + 1], qr[b / 2 + 1], qi[b / 2 + 1];
+#pragma unroll
+    for (int k = 0; k <= b; ++k) {
+      const int m = k % b, c = m <= b / 2 ? m : b - m;
+      const float sg = m <= b / 2 ? 1.0f : -1.0f;
+      if (k % 2 == 0) { pr[c] = re[k]; pi[c] = sg * im[k]; }
+      else { qr[c] = re[k]; qi[c] = sg * im[k]; }
+    }
+    c2r<b>(pr, pi, p);
+    c2r<b>(qr, qi, q);
+#pragma unroll
+    for (int j = 0; j < b; ++j) {
+      x[2 * j] = p[j] + q[j];
+      x[(2 * j + b) % n] = p[j] - q[j];
+    }
+  } else {
+    static_assert(n % 4 == 0, "c2r lengths");
+    constexpr int b = n / 4;
+    constexpr Roots<n> w{};
+    float zr[b / 2 + 1], zi[b / 2 + 1], t0[b], t1r[b], t1i[b], t2r[b], t2i[b];
+#pragma unroll
+    for (int q = 0; q < b; ++q) {
+      if (q <= b / 2) { zr[q] = re[4 * q]; zi[q] = im[4 * q]; }
+      const int k = 1 + 4 * q, m = 2 + 4 * q;
+      t1r[q] = k <= n / 2 ? re[k] : re[n - k];
+      t1i[q] = k <= n / 2 ? im[k] : -im[n - k];
+      t2r[q] = m <= n / 2 ? re[m] : re[n - m];
+      t2i[q] = m == n / 2 ? 0.0f : m < n / 2 ? im[m] : -im[n - m];
+    }
+    c2r<b>(zr, zi, t0);
+    fft<b>(t1i, t1r);   // inverse
+    fft<b>(t2i, t2r);
+#pragma unroll
+    for (int j = 0; j < b; ++j) {
+      const float c1 = w.c[j], s1 = -w.s[j], c2 = w.c[(2 * j) % n], s2 = -w.s[(2 * j) % n];
+      const float ar = j == 0 ? t1r[j] : t1r[j] * c1 - t1i[j] * s1;
+      const float ai = j == 0 ? t1i[j] : t1r[j] * s1 + t1i[j] * c1;
+      const float d = j == 0 ? t2r[j] : t2r[j] * c2 - t2i[j] * s2;   // real: its own mirror image
+      const float p = t0[j] + d, q = t0[j] - d;
+      x[j] = p + 2.0f * ar;
+      x[j + 2 * b] = p - 2.0f * ar;
+      x[j + b] = q - 2.0f * ai;
+      x[j + 3 * b] = q + 2.0f * ai;
+    }
+  }
+}
+
+// Threads of a compiled Fourier kernel with tl latitudes: one per (i1, latitude) on the
+// longitude side and one per (pair of k2, latitude) on the wavenumber side.
+constexpr int fourier_threads(int n1, int n2, int tl) {
+  return ((n1 > n2 / 2 ? n1 : n2 / 2) * tl + 63) / 64 * 64;
+}
+
+template <int N1, int N2, int TL>
+__global__ __launch_bounds__(fourier_threads(N1, N2, TL)) void fourier_analysis_kernel(FourierArgs a) {
+  constexpr int N = N1 * N2, NH = N2 / 2 + 1, T = fourier_threads(N1, N2, TL);
+  __shared__ float2 tw[N], z[NH * N1 * TL];   // z: [k2][i1][lat]
+  const int b = blockIdx.y, j0 = blockIdx.x * TL;
   const Seg sg = a.seg.s[find_seg(a.seg, b)];
   const float* src = sg.src + (size_t)(b - sg.first) * N * a.nlat;
   const float lvl = sg.level ? sg.level[(b - sg.first) % sg.period] : 0.0f;
-  load_roots(a, twr, twi);
-  // pass 1: thread (i1, lat): Z[i1][k2] = sum_i2 x[i1 + N1 i2] w_N2^(i2 k2), k2 <= N2 / 2
-  for (int e = threadIdx.x; e < N1 * tl; e += kThreads) {
-    const int i1 = e / tl, jj = e - i1 * tl, j = j0 + jj;
-    const bool in = j < a.nlat;
-    const int jc = in ? j : 0;
-    const float cs = in ? sg.mul * a.w[jc] * ((sg.op & kOpSecLat) ? a.sec[jc] : 1.0f) : 0.0f;
-    float x[N2];
+  const int row = threadIdx.x / TL, jj = threadIdx.x % TL, j = j0 + jj;
+  const bool in = j < a.nlat;
+  const int jc = in ? j : 0;
+  float x[N2];
+  if (row < N1) {
 #pragma unroll
-    for (int i2 = 0; i2 < N2; ++i2) x[i2] = src[(size_t)(i1 + N1 * i2) * a.nlat + jc];
+    for (int i2 = 0; i2 < N2; ++i2) x[i2] = src[(size_t)(row + N1 * i2) * a.nlat + jc];
+  }
+  for (int i = threadIdx.x; i < N; i += T) tw[i] = make_float2(a.twr[i], a.twi[i]);
+  // pass 1: thread (i1, lat): Z[i1][k2] = sum_i2 x[i1 + N1 i2] w_N2^(i2 k2), k2 <= N2 / 2
+  if (row < N1) {
+    const float cs = in ? sg.mul * a.w[jc] * ((sg.op & kOpSecLat) ? a.sec[jc] : 1.0f) : 0.0f;
 #pragma unroll
     for (int i2 = 0; i2 < N2; ++i2) {
       float v = x[i2];
@@ -486,156 +705,128 @@ __global__ __launch_bounds__(kThreads) void fourier_analysis_kernel(FourierArgs 
       if (sg.op & kOpSubLevel) v -= lvl;
       x[i2] = in ? v * cs : 0.0f;
     }
+    float re[NH], im[NH];
+    rfft<N2>(x, re, im);
 #pragma unroll
-    for (int k2 = 0; k2 < NH; ++k2) {
-      float re = 0.0f, im = 0.0f;
-#pragma unroll
-      for (int i2 = 0; i2 < N2; ++i2) {
-        re += x[i2] * R2.c[(i2 * k2) % N2];
-        im += x[i2] * R2.s[(i2 * k2) % N2];
-      }
-      zr[(k2 * N1 + i1) * tl + jj] = re;
-      zi[(k2 * N1 + i1) * tl + jj] = im;
-    }
+    for (int k2 = 0; k2 < NH; ++k2) z[(k2 * N1 + row) * TL + jj] = make_float2(re[k2], im[k2]);
   }
   __syncthreads();
-  // pass 2: thread (k2, lat): X_{k2 + N2 k1} = sum_i1 (Z[i1][k2] w^(i1 k2)) w_N1^(i1 k1)
-  float* Y = a.out + (size_t)b * a.mm * a.nlat;
-  for (int e = threadIdx.x; e < N2 * tl; e += kThreads) {
-    const int k2 = e / tl, jj = e - k2 * tl, j = j0 + jj;
-    const bool cj = k2 >= NH;        // Z[i1][k2] = conj(Z[i1][N2 - k2])
-    const int kz = cj ? N2 - k2 : k2;
-    float pr[N1], pi[N1];
+  // pass 2: thread (k2 and N2 - k2, lat): X_{k2 + N2 k1} = sum_i1 (Z[i1][k2] w^(i1 k2)) w_N1^(i1 k1);
+  // thread row 0 takes k2 = 0 and N2 / 2
+  if (row >= N2 / 2) return;
+  float* Y = a.out + (size_t)b * a.mm * a.nlat + j;
+#pragma unroll
+  for (int side = 0; side < 2; ++side) {
+    const int k2 = side == 0 ? row : (row == 0 ? N2 / 2 : N2 - row);
+    const int kz = side == 0 || row == 0 ? k2 : row;   // the row of z: Z[N2 - k2] = conj(Z[k2])
+    const float cj = side == 0 || row == 0 ? 1.0f : -1.0f;
+    float re[N1], im[N1];
 #pragma unroll
     for (int i1 = 0; i1 < N1; ++i1) {
-      const int z = (kz * N1 + i1) * tl + jj;
-      const float a_r = zr[z], a_i = cj ? -zi[z] : zi[z];
-      const int q = (i1 * k2) % N;
-      const float t_r = twr[q], t_i = twi[q];
-      pr[i1] = a_r * t_r - a_i * t_i;
-      pi[i1] = a_r * t_i + a_i * t_r;
+      const float2 v = z[(kz * N1 + i1) * TL + jj], t = tw[i1 * k2];
+      const float vi = cj * v.y;
+      re[i1] = v.x * t.x - vi * t.y;
+      im[i1] = v.x * t.y + vi * t.x;
     }
+    fft<N1>(re, im);
 #pragma unroll
     for (int k1 = 0; k1 < N1; ++k1) {
       if (N2 * k1 >= a.n_m) break;   // uniform; k < n_m is masked per lane below
       const int k = k2 + N2 * k1;
-      float re = 0.0f, im = 0.0f;
-#pragma unroll
-      for (int i1 = 0; i1 < N1; ++i1) {
-        const float c = R1.c[(i1 * k1) % N1], s = R1.s[(i1 * k1) % N1];
-        re += pr[i1] * c - pi[i1] * s;
-        im += pr[i1] * s + pi[i1] * c;
-      }
-      if (j < a.nlat && k < a.n_m) {
+      if (in && k < a.n_m) {
         if (k == 0) {
-          Y[j] = re * kRsqrt2Pi;
+          Y[0] = re[k1] * kRsqrt2Pi;
         } else {
-          Y[(size_t)(2 * k - 1) * a.nlat + j] = re * kRsqrtPi;
-          Y[(size_t)(2 * k) * a.nlat + j] = -im * kRsqrtPi;
+          Y[(size_t)(2 * k - 1) * a.nlat] = re[k1] * kRsqrtPi;
+          Y[(size_t)(2 * k) * a.nlat] = -im[k1] * kRsqrtPi;
         }
       }
     }
   }
 }
 
-template <int N1, int N2>
-__global__ __launch_bounds__(kThreads) void fourier_synthesis_kernel(FourierArgs a) {
-  constexpr int N = N1 * N2;
-  constexpr Roots<N1> R1{};
-  constexpr Roots<N2> R2{};
-  extern __shared__ float lds[];
-  const int tl = a.tl, h = a.nlat >> 1, b = blockIdx.y, j0 = blockIdx.x * tl;
-  float* twr = lds;
-  float* twi = twr + N;
-  float* wr = twi + N;             // [N1][N2][tl]
-  float* wi = wr + N * tl;
+template <int N1, int N2, int TL>
+__global__ __launch_bounds__(fourier_threads(N1, N2, TL)) void fourier_synthesis_kernel(FourierArgs a) {
+  constexpr int N = N1 * N2, NH = N2 / 2 + 1, T = fourier_threads(N1, N2, TL);
+  __shared__ float2 tw[N], hs[N1 * NH * TL];   // hs: [i1][k2][lat]
+  const int h = a.nlat >> 1, b = blockIdx.y, j0 = blockIdx.x * TL;
   const Seg sg = a.seg.s[find_seg(a.seg, b)];
-  load_roots(a, twr, twi);
-  __syncthreads();
   const float* E = a.in + (size_t)b * a.mm * h;
   const size_t odd = (size_t)a.nfield * a.mm * h;
-  // pass 1: thread (k2, lat): W[i1][k2] = conj(w^(i1 k2)) sum_k1 c_{k2 + N2 k1} conj(w_N1^(i1 k1)),
-  // c_0 = Y_0 / sqrt(2 pi), c_k = (Y_{2k-1} - i Y_{2k}) / sqrt(pi); Y from E + O (south), E - O (north)
-  for (int e = threadIdx.x; e < N2 * tl; e += kThreads) {
-    const int k2 = e / tl, jj = e - k2 * tl, j = j0 + jj;
-    const bool in = j < a.nlat;
-    const int jh = !in ? 0 : (j < h ? j : a.nlat - 1 - j);
-    const float so = j < h ? 1.0f : -1.0f;
-    // the wavenumbers k = k2 + N2 k1 < n_m: k1 < ceil(n_m / N2) for every lane
-    // (a uniform bound), the last one masked per lane; loads at clamped modes
-    // (in bounds) issue back to back, all before any use
-    float ec[N1], oc[N1], es[N1], os[N1];
+  const int row = threadIdx.x / TL, jj = threadIdx.x % TL, j = j0 + jj;
+  const bool in = j < a.nlat;
+  const int jh = !in ? 0 : (j < h ? j : a.nlat - 1 - j);
+  const float so = j < h ? 1.0f : -1.0f;
+  for (int i = threadIdx.x; i < N; i += T) tw[i] = make_float2(a.twr[i], a.twi[i]);
+  __syncthreads();
+  // pass 1: thread (k2 and N2 - k2, lat): W[i1][k2] = conj(w^(i1 k2)) sum_k1 c_{k2 + N2 k1} conj(w_N1^(i1 k1)),
+  // c_0 = Y_0 / sqrt(2 pi), c_k = (Y_{2k-1} - i Y_{2k}) / sqrt(pi); Y from E + O (south), E - O
+  // (north).  The line is the real part of W's transform over k2, so the Hermitian part
+  // (W[k2] + conj(W[N2 - k2])) / 2 is all that pass 2 reads; the halves are in c here.
+  if (row < N2 / 2) {
+    float re[2][N1], im[2][N1];
 #pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) {
-      if (N2 * k1 >= a.n_m) break;
-      const int k = k2 + N2 * k1;
-      const int kc = k < a.n_m ? k : 0;
-      const float* pc = E + (size_t)(kc == 0 ? 0 : 2 * kc - 1) * h + jh;
-      const float* ps = E + (size_t)(kc == 0 ? 0 : 2 * kc) * h + jh;
-      ec[k1] = pc[0]; oc[k1] = pc[odd]; es[k1] = ps[0]; os[k1] = ps[odd];
-    }
-    float cr[N1], ci[N1];
+    for (int side = 0; side < 2; ++side) {
+      const int k2 = side == 0 ? row : (row == 0 ? N2 / 2 : N2 - row);
+      // the wavenumbers k = k2 + N2 k1 < n_m: k1 < ceil(n_m / N2) for every lane (a
+      // uniform bound), the last one masked per lane; loads at clamped modes (in bounds)
 #pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) {
-      cr[k1] = 0.0f;
-      ci[k1] = 0.0f;
-      if (N2 * k1 >= a.n_m) continue;
-      const int k = k2 + N2 * k1;
-      const bool use = in && k < a.n_m;
-      const float y_c = ec[k1] + so * oc[k1], y_s = es[k1] + so * os[k1];
-      cr[k1] = use ? y_c * (k == 0 ? kRsqrt2Pi : kRsqrtPi) : 0.0f;
-      ci[k1] = use && k > 0 ? -y_s * kRsqrtPi : 0.0f;
-    }
-    // k1 outermost with the uniform bound: only the ceil(n_m / N2) wavenumbers
-    // that exist are summed (6 of 16 at T85), in ascending k1 as before
-    float re[N1], im[N1];
-#pragma unroll
-    for (int i1 = 0; i1 < N1; ++i1) {
-      re[i1] = 0.0f;
-      im[i1] = 0.0f;
+      for (int k1 = 0; k1 < N1; ++k1) {
+        re[side][k1] = im[side][k1] = 0.0f;
+        if (N2 * k1 >= a.n_m) continue;
+        const int k = k2 + N2 * k1;
+        const int kc = k < a.n_m ? k : 0;
+        const float* pc = E + (size_t)(kc == 0 ? 0 : 2 * kc - 1) * h + jh;
+        const float* ps = E + (size_t)(2 * kc) * h + jh;
+        const float y_c = pc[0] + so * pc[odd], y_s = ps[0] + so * ps[odd];
+        const bool use = in && k < a.n_m;
+        re[side][k1] = use ? y_c * (k == 0 ? 0.5f * kRsqrt2Pi : 0.5f * kRsqrtPi) : 0.0f;
+        im[side][k1] = use && k > 0 ? -y_s * (0.5f * kRsqrtPi) : 0.0f;
+      }
     }
 #pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) {
-      if (N2 * k1 >= a.n_m) break;
+    for (int side = 0; side < 2; ++side) {
+      const int k2 = side == 0 ? row : (row == 0 ? N2 / 2 : N2 - row);
+      fft<N1>(im[side], re[side]);   // inverse
 #pragma unroll
       for (int i1 = 0; i1 < N1; ++i1) {
-        const float c = R1.c[(i1 * k1) % N1], s = -R1.s[(i1 * k1) % N1];
-        re[i1] += cr[k1] * c - ci[k1] * s;
-        im[i1] += cr[k1] * s + ci[k1] * c;
+        const float2 t = tw[i1 * k2];   // conjugated below
+        const float r = re[side][i1], m = im[side][i1];
+        re[side][i1] = r * t.x + m * t.y;
+        im[side][i1] = m * t.x - r * t.y;
       }
     }
 #pragma unroll
     for (int i1 = 0; i1 < N1; ++i1) {
-      const int q = (i1 * k2) % N;
-      const float t_r = twr[q], t_i = -twi[q];
-      wr[(i1 * N2 + k2) * tl + jj] = re[i1] * t_r - im[i1] * t_i;
-      wi[(i1 * N2 + k2) * tl + jj] = re[i1] * t_i + im[i1] * t_r;
+      float2* o = &hs[i1 * NH * TL + jj];
+      if (row == 0) {
+        o[0] = make_float2(2.0f * re[0][i1], 0.0f);
+        o[(N2 / 2) * TL] = make_float2(2.0f * re[1][i1], 0.0f);
+      } else {
+        o[row * TL] = make_float2(re[0][i1] + re[1][i1], im[0][i1] - im[1][i1]);
+      }
     }
   }
   __syncthreads();
-  // pass 2: thread (i1, lat): x[i1 + N1 i2] = Re sum_k2 W[i1][k2] conj(w_N2^(i2 k2)), then the epilogue
-  float* dst = sg.dst + (size_t)(b - sg.first) * N * a.nlat;
+  // pass 2: thread (i1, lat): x[i1 + N1 i2] = sum_k2 H[i1][k2] conj(w_N2^(i2 k2)), then the epilogue
+  if (row >= N1 || !in) return;
+  float* dst = sg.dst + (size_t)(b - sg.first) * N * a.nlat + j;
   const float lvl = sg.level ? sg.level[(b - sg.first) % sg.period] : 0.0f;
-  for (int e = threadIdx.x; e < N1 * tl; e += kThreads) {
-    const int i1 = e / tl, jj = e - i1 * tl, j = j0 + jj;
-    const int jc = j < a.nlat ? j : 0;
-    float pr[N2], pi[N2];
+  const float sc = ((sg.op & kOpSecLat) ? a.sec[j] : 1.0f);
+  float re[NH], im[NH], x[N2];
 #pragma unroll
-    for (int k2 = 0; k2 < N2; ++k2) {
-      pr[k2] = wr[(i1 * N2 + k2) * tl + jj];
-      pi[k2] = wi[(i1 * N2 + k2) * tl + jj];
-    }
+  for (int k2 = 0; k2 < NH; ++k2) {
+    const float2 v = hs[(row * NH + k2) * TL + jj];
+    re[k2] = v.x;
+    im[k2] = v.y;
+  }
+  c2r<N2>(re, im, x);
 #pragma unroll
-    for (int i2 = 0; i2 < N2; ++i2) {
-      float v = 0.0f;
-#pragma unroll
-      for (int k2 = 0; k2 < N2; ++k2) v += pr[k2] * R2.c[(i2 * k2) % N2] + pi[k2] * R2.s[(i2 * k2) % N2];
-      if (sg.op & kOpSecLat) v *= a.sec[jc];
-      v = v * sg.mul;
-      if (sg.op & kOpAddLevel) v += lvl;
-      if (sg.op & kOpExp) v = expf(v);
-      if (j < a.nlat) dst[(size_t)(i1 + N1 * i2) * a.nlat + j] = v;
-    }
+  for (int i2 = 0; i2 < N2; ++i2) {
+    float v = x[i2] * sc * sg.mul;
+    if (sg.op & kOpAddLevel) v += lvl;
+    if (sg.op & kOpExp) v = expf(v);
+    dst[(size_t)(row + N1 * i2) * a.nlat] = v;
   }
 }
 
@@ -903,17 +1094,19 @@ FourierArgs fourier_args(const SpeedyShtPlan* p, int32_t nfield, int32_t tl, con
   return f;
 }
 
-// The Fourier kernels of one factor pair nlon = n1 * n2: compiled for the nlon
-// of the Grid.T<N> table up to T213 (nlon 640), the generic LDS kernels
-// otherwise (at n1 = 32 the register passes would spill to scratch).
+// The Fourier kernels of one factor pair nlon = n1 * n2, compiled for the nlon of the
+// Grid.T<N> table, each with the latitudes a workgroup takes: 16 (64-byte rows) where
+// the exchange fits 64 KiB of LDS, which is everywhere but T340 and T425.  Other nlon
+// take the generic LDS kernels.
 typedef void (*FourierKernel)(FourierArgs);
 struct FourierPair {
-  int n1, n2;
+  int n1, n2, tl;
   FourierKernel analysis, synthesis;
 };
-#define SHT_PAIR(a, b) {a, b, fourier_analysis_kernel<a, b>, fourier_synthesis_kernel<a, b>}
-const FourierPair kPairs[] = {SHT_PAIR(8, 8),   SHT_PAIR(8, 12),  SHT_PAIR(8, 16),  SHT_PAIR(16, 16),
-                              SHT_PAIR(16, 20), SHT_PAIR(18, 20), SHT_PAIR(16, 32), SHT_PAIR(20, 32)};
+#define SHT_PAIR(a, b, t) {a, b, t, fourier_analysis_kernel<a, b, t>, fourier_synthesis_kernel<a, b, t>}
+const FourierPair kPairs[] = {SHT_PAIR(8, 8, 16),   SHT_PAIR(8, 12, 16),  SHT_PAIR(8, 16, 16),  SHT_PAIR(16, 16, 16),
+                              SHT_PAIR(16, 20, 16), SHT_PAIR(18, 20, 16), SHT_PAIR(16, 32, 16), SHT_PAIR(20, 32, 16),
+                              SHT_PAIR(32, 32, 8),  SHT_PAIR(32, 40, 8)};
 #undef SHT_PAIR
 
 const FourierPair* find_pair(int n1, int n2) {
@@ -922,15 +1115,12 @@ const FourierPair* find_pair(int n1, int n2) {
   return nullptr;
 }
 
-// LDS bytes of the Fourier kernels (roots, line tile, pass-1 result)
+// LDS bytes of the generic Fourier kernels (roots, line tile, pass-1 result)
 constexpr size_t kFourierLds = 64 * 1024;
-size_t analysis_lds(bool fixed, int N, int n1, int n2, int tl) {
-  const size_t z = 2 * (size_t)n1 * (n2 / 2 + 1) * tl;
-  return 4 * (2 * (size_t)N + z + (fixed ? 0 : (size_t)N * tl));
+size_t analysis_lds(int N, int n1, int n2, int tl) {
+  return 4 * (2 * (size_t)N + 2 * (size_t)n1 * (n2 / 2 + 1) * tl + (size_t)N * tl);
 }
-size_t synthesis_lds(bool fixed, int N, int mm, int tl) {
-  return 4 * (2 * (size_t)N + 2 * (size_t)N * tl + (fixed ? 0 : (size_t)mm * tl));
-}
+size_t synthesis_lds(int N, int mm, int tl) { return 4 * (2 * (size_t)N + 2 * (size_t)N * tl + (size_t)mm * tl); }
 
 int tiles(int M, int N) { return ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN); }
 
@@ -940,7 +1130,8 @@ hipError_t run_analysis(const SpeedyShtPlan* p, int32_t nfield, const SegTable& 
   f.out = y;
   const FourierPair* fp = find_pair(p->n1, p->n2);
   hipLaunchKernelGGL(fp ? fp->analysis : fourier_analysis_generic, dim3((p->nlat + p->tl_a - 1) / p->tl_a, nfield),
-                     dim3(kThreads), analysis_lds(fp != nullptr, p->nlon, p->n1, p->n2, p->tl_a), s, f);
+                     dim3(fp ? fourier_threads(p->n1, p->n2, p->tl_a) : kThreads),
+                     fp ? 0 : analysis_lds(p->nlon, p->n1, p->n2, p->tl_a), s, f);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   StageArgs a = stage_args(p, nfield);
@@ -964,7 +1155,8 @@ hipError_t run_synthesis(const SpeedyShtPlan* p, int32_t nfield, const SegTable&
   f.in = y;
   const FourierPair* fp = find_pair(p->n1, p->n2);
   hipLaunchKernelGGL(fp ? fp->synthesis : fourier_synthesis_generic, dim3((p->nlat + p->tl_s - 1) / p->tl_s, nfield),
-                     dim3(kThreads), synthesis_lds(fp != nullptr, p->nlon, p->mm, p->tl_s), s, f);
+                     dim3(fp ? fourier_threads(p->n1, p->n2, p->tl_s) : kThreads),
+                     fp ? 0 : synthesis_lds(p->nlon, p->mm, p->tl_s), s, f);
   return hipGetLastError();
 }
 
@@ -1021,20 +1213,20 @@ int speedy_sht_create(int32_t n_m, int32_t n_l, int32_t nlon, int32_t nlat, doub
   if (int rc = check_grid(n_m, n_l, nlon, nlat)) return rc;
   if (!(radius > 0.0)) return fail(SPEEDY_ERR_ARG, "speedy_sht_create: radius must be positive");
   const int mm = 2 * n_m - 1;
-  // nlon = n1 * n2 with n1 the largest divisor <= sqrt(nlon); the widest latitude
-  // tile (16, 8, .., 1) whose LDS fits
+  // nlon = n1 * n2 with n1 the largest divisor <= sqrt(nlon); the latitude tile of the
+  // compiled pair, or for the generic kernels the widest (16, 15, .., 1) whose LDS fits
   int n1 = 1;
   for (int d = 1; (int64_t)d * d <= nlon; ++d)
     if (nlon % d == 0) n1 = d;
   const int n2 = nlon / n1;
-  // compiled pairs: a thread per (i1 or k2, latitude) in each pass, so at most
-  // kThreads / max(n1, n2) latitudes; generic kernels: 16
-  const bool fixed = find_pair(n1, n2) != nullptr;
-  int tl_a = fixed ? std::min(16, kThreads / std::max(n1, n2)) : 16, tl_s = tl_a;
-  while (tl_a > 1 && analysis_lds(fixed, nlon, n1, n2, tl_a) > kFourierLds) --tl_a;
-  while (tl_s > 1 && synthesis_lds(fixed, nlon, mm, tl_s) > kFourierLds) --tl_s;
-  if (analysis_lds(fixed, nlon, n1, n2, tl_a) > kFourierLds || synthesis_lds(fixed, nlon, mm, tl_s) > kFourierLds)
-    return fail(SPEEDY_ERR_ARG, "speedy_sht_create: nlon too large for the Fourier stages' 64 KiB of LDS");
+  const FourierPair* fp = find_pair(n1, n2);
+  int tl_a = fp ? fp->tl : 16, tl_s = tl_a;
+  if (!fp) {
+    while (tl_a > 1 && analysis_lds(nlon, n1, n2, tl_a) > kFourierLds) --tl_a;
+    while (tl_s > 1 && synthesis_lds(nlon, mm, tl_s) > kFourierLds) --tl_s;
+    if (analysis_lds(nlon, n1, n2, tl_a) > kFourierLds || synthesis_lds(nlon, mm, tl_s) > kFourierLds)
+      return fail(SPEEDY_ERR_ARG, "speedy_sht_create: nlon too large for the Fourier stages' 64 KiB of LDS");
+  }
   std::vector<double> x(nlat), w(nlat);
   gauss_nodes(nlat, x.data(), w.data());
   std::vector<float> P((size_t)n_m * nlat * n_l), wf(nlat), sec(nlat), tw(2 * (size_t)nlon);
