@@ -1,24 +1,19 @@
 // Dynamics <-> physics transforms for gfx950: spherical-harmonic analysis and
-// synthesis on a Gaussian grid as batched fp32 MFMA GEMMs, with the unit
-// conversions, the modal vorticity/divergence <-> wind operators and the
-// hydrostatic geopotential fused around them.
+// synthesis on a Gaussian grid, fp32 matrix instructions over l or latitude and
+// short FFTs over longitude, with the unit conversions, the modal
+// vorticity/divergence <-> wind operators and the hydrostatic geopotential fused
+// into them: two launches a conversion.
 //
 // Reference behaviour: jcm/physics_interface.py:196-303 over dinosaur's
 // RealSphericalHarmonics (Grid.T<N>, jcm/utils.py:28-54).
 //
-// Data flow of one conversion (B stacked fields, Mm = 2*n_m-1 modes):
-//   to_nodal:  modal [B][Mm][L] --Legendre--> Y [B][Mm][nlat] --Fourier--> nodal [B][nlon][nlat]
-//   to_modal:  nodal [B][nlon][nlat] --Fourier--> Y [B][Mm][nlat] --Legendre--> modal [B][Mm][L]
-// Each Legendre arrow is one launch of sht_gemm_kernel<STAGE>: a 64x64 output
-// tile per workgroup of four waves, each wave 32x32 as 2x2
-// v_mfma_f32_16x16x4f32, K in steps of 32 staged through two LDS stages,
-// batched over modes (the basis P[m] is shared by every field).  Each Fourier
-// arrow is one launch of fourier_analysis_kernel / fourier_synthesis_kernel: a
-// real DFT over longitude factored into two short passes in LDS, batched over
-// fields and latitude tiles.  Per-field pre/post operations (1/cos(lat), unit
-// scales, reference temperature, log/exp of surface pressure) ride in the
-// Fourier stages' loads and stores; the l +- 1 modal operators are one
-// elementwise kernel on either side.
+// Data flow of one conversion (B stacked fields, modes Mm = 2*n_m-1):
+//   to_nodal:  modal [B][Mm][L] --Legendre--> Y [B][n_m][nlat] --Fourier--> nodal [B][nlon][nlat]
+//   to_modal:  nodal [B][nlon][nlat] --Fourier--> Y [B][n_m][nlat] --Legendre--> modal [B][Mm][L]
+// with Y a float2 of the cosine and the sine mode.  The modal operators run on the
+// Legendre kernels' rows; per-field pre/post operations (1/cos(lat), unit scales,
+// reference temperature, log/exp of surface pressure) ride in the Fourier kernels'
+// loads and stores.
 
 #include <hip/hip_runtime.h>
 
@@ -37,8 +32,9 @@ struct SpeedyShtPlan {
   int device;
   int32_t n1, n2;      // nlon = n1 * n2 (the Fourier stages' two passes)
   int32_t tl_a, tl_s;  // latitudes per workgroup of the Fourier analysis / synthesis
-  float* P;     // [n_m][nlat][n_l]
-  float* w;     // [nlat] Gauss weights * 2 pi / nlon
+  float* Ps;    // Legendre operand blocks of the synthesis
+  float* Pa;    // and of the analysis (LegendreArgs says how they are laid out)
+  int32_t* blk; // [n_m] first block of order m
   float* sec;   // [nlat] 1 / cos(lat)
   float* tw;    // [2][nlon]: cos(2 pi j / nlon), -sin(2 pi j / nlon)
 };
@@ -52,10 +48,9 @@ int fail(int code, const std::string& msg) {
   return code;
 }
 
-constexpr int kThreads = 256, kBM = 64, kBN = 64, kBK = 32, kPad = 4;
+constexpr int kThreads = 256;
 constexpr int kMaxSeg = 8;
 
-enum Stage { kLegendreAnalysis = 1, kLegendreSynthesis = 2 };
 enum : int32_t { kOpLog = 1, kOpExp = 2, kOpSecLat = 4, kOpSubLevel = 8, kOpAddLevel = 16 };
 
 // A run of stacked fields that share a source (Fourier analysis) or a
@@ -72,13 +67,6 @@ struct SegTable {
   int32_t n;
 };
 
-struct StageArgs {
-  int32_t nlon, nlat, mm, nl, nfield;
-  const float* P;
-  const float* in;    // LA: Y, LS: modal X
-  float* out;         // LA: modal, LS: Y halves
-};
-
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ int find_seg(const SegTable& t, int f) {
@@ -88,152 +76,397 @@ __device__ __forceinline__ int find_seg(const SegTable& t, int f) {
   return k;
 }
 
-// C[M x N] = A[M x K] * B[K x N] for one batch entry (blockIdx.y); element
-// (r, c) of X at X[r * x_r + c * x_c].
-template <int STAGE>
-__global__ __launch_bounds__(kThreads) void sht_gemm_kernel(StageArgs a) {
-  // blockIdx.y = 2 * mode + parity.  Gaussian latitudes are
-  // symmetric (x_{nlat-1-j} = -x_j) and P_l^m(-x) = (-1)^(l+m) P_l^m(x), so each
-  // mode splits into the l with l+m even (parity 0) and odd (parity 1), each over
-  // the southern half of the latitudes: half the work and half the K of a full
-  // contraction.  Analysis reads Y_j +- Y_{nlat-1-j}; synthesis writes the even
-  // and odd partial sums E, O for the southern half ([parity][field][mode][h]),
-  // which the Fourier synthesis combines as E + O (south) and E - O (north).
-  const int b = (int)(blockIdx.y >> 1);
-  const int par = (int)(blockIdx.y & 1u);
-  const int h = a.nlat >> 1;
-  int M, N, K;
-  const float* A;
-  const float* B;
-  float* C;
-  long a_m, a_k, b_k, b_n, c_m, c_n = 1;
-  const int mode_m = (b + 1) >> 1;    // order m of mode b
-  const int lofs = (mode_m + par) & 1;   // first l of this parity (l = lofs + 2c)
-  const int npar = (a.nl - lofs + 1) >> 1;
-  if (STAGE == kLegendreAnalysis) {
-    // Z[:, b, lofs + 2c] [nfield x npar] = (Y_j +- Y_{nlat-1-j})[:, b, :h] [nfield x h] * P_m[:h, lofs + 2c]
-    M = a.nfield; N = npar; K = h;
-    A = a.in + (size_t)b * a.nlat; a_m = (long)a.mm * a.nlat; a_k = 1;
-    B = a.P + (size_t)mode_m * a.nlat * a.nl + lofs; b_k = a.nl; b_n = 2;
-    C = a.out + (size_t)b * a.nl + lofs; c_m = (long)a.mm * a.nl; c_n = 2;
-  } else {
-    // E|O[par][:, b, :h] [nfield x h] = X[:, b, lofs + 2c] [nfield x npar] * P_m[:h, lofs + 2c]^T
-    M = a.nfield; N = h; K = npar;
-    A = a.in + (size_t)b * a.nl + lofs; a_m = (long)a.mm * a.nl; a_k = 2;
-    B = a.P + (size_t)mode_m * a.nlat * a.nl + lofs; b_k = 2; b_n = a.nl;
-    C = a.out + (size_t)par * a.nfield * a.mm * h + (size_t)b * h; c_m = (long)a.mm * h;
+// eps(m, l) = sqrt((l^2 - m^2) / (4 l^2 - 1)) for m <= l, l >= 1; else 0:
+// x P_l^m = eps(m, l+1) P_{l+1}^m + eps(m, l) P_{l-1}^m (unit-norm functions).
+__device__ __forceinline__ float eps_ml(int m, int l) {
+  if (l <= 0 || m > l) return 0.0f;
+  const float fl = (float)l, fm = (float)m;
+  return sqrtf((fl * fl - fm * fm) / (4.0f * fl * fl - 1.0f));
+}
+
+// Modal coefficient (mode 0, l 0) of the constant 1: 1 / (F_0 P_0^0) = 2 sqrt(pi).
+constexpr float kConstCoef = 3.5449077018110318f;
+
+// ------------------------------------------------------------ Legendre stages
+// One workgroup takes one order m and eight fields: 16 rows, the cosine and the sine
+// mode of each (row 2 f and 2 f + 1; m = 0 has no sine mode and its rows are zero).
+// The modal operators of the conversions couple l with l +- 1 and the cosine with the
+// sine mode, both inside the workgroup, so they run on the 16 rows in LDS.
+//
+// Gaussian latitudes are symmetric and P_l^m(-x) = (-1)^(l+m) P_l^m(x): the l with l+m
+// even (parity 0) and odd (parity 1) are separate sums over the southern half of the
+// latitudes.  P_l^m is zero for l < m, and those l are not summed: l = m + par + 2 c.
+// The operand P is laid out for the matrix instructions: blocks of 16 c x 16 southern
+// latitudes j, 1 KiB each, [m][par][c / 16][j / 16], zero outside; lane (g = lane / 16,
+// n = lane % 16) reads the 16 bytes it feeds to the four k substeps of a block: q = 0 .. 3
+// is c = 4 q + g at j = n (synthesis) or j = 4 g + q at c = n (analysis).  The synthesis
+// so sums in ascending l: the terms of a wind's m = 0 cancel from one l to the next at
+// the poles, and other orders leave a larger error there.  The Fourier basis's
+// 1 / sqrt(2 pi) (m = 0) and 1 / sqrt(pi) are in the analysis's P, with the Gauss weights
+// 2 pi w / nlon; the synthesis multiplies its sums by them, and by the 1 / 2 of the
+// Fourier stage's Hermitian pairs (in P they made the error at the poles 1.5 times as
+// large, by rounding the P of neighbouring l apart).
+//
+// Bound by the latency of its three dependent steps (modal input, matrix products, Y),
+// at T213 too (more or fewer workgroups on a CU, or operand blocks in flight, change
+// nothing; the matrix instructions take 5 of 23 us).  Chunks of one order run on one XCD
+// (workgroups go round the 8 XCDs), so that P comes into its L2 once.  Before, dense
+// batched products per mode and parity over all l >= 0 with the modal operators as a
+// kernel of their own: 4.9 + 11.5 us (T85 x 41 fields synthesis) and 7.5 + 3.5 us (T85 x
+// 32 fields analysis), now 8.2 and 6.1; T213 x 41 synthesis 14 + 53 us, now 23.
+struct LegendreArgs {
+  int32_t n_m, nl, nlat, kx;
+  int32_t winds, plain, geo;   // levels of winds, other fields, geopotential levels
+  int32_t nfield;              // fields of Y: the plain ones past it are zero (analysis)
+  int32_t kt;                  // 16-wide tiles of the summed index staged at a time
+  const float* P;
+  const int32_t* blk;
+  float2* y;                   // [field][m][nlat]: cosine and sine mode
+  float* z;                    // analysis: [workgroup][16][nl], if not in LDS
+  float inv_radius, radius2, gravity;
+  const float* vor;            // [kx][mm][nl]
+  const float* div;
+  float* vor_out;
+  float* div_out;
+  const float* src[4];         // the plain fields, a run of `count` [mm][nl] each
+  float* dst[4];
+  int32_t count[4];
+  // geopotential: phi_j = g orography + sum_k W[j][k] (T_var_k + reference_k as a constant)
+  const float* tvar;
+  const float* orography;
+  const float* reference;
+  float geo_w[SPEEDY_SHT_KX_MAX][SPEEDY_SHT_KX_MAX];
+};
+
+enum ChunkKind { kWinds, kPlain, kGeo };
+struct Chunk {
+  int m, id, kind, f0;   // f0: first level (winds, geo) or field (plain)
+};
+
+__host__ __device__ constexpr int chunks(int winds, int plain, int geo) {
+  return (winds + 3) / 4 + (plain + 7) / 8 + (geo + 7) / 8;
+}
+
+__device__ __forceinline__ Chunk find_chunk(const LegendreArgs& a) {
+  const int n = chunks(a.winds, a.plain, a.geo), q = (int)blockIdx.x >> 3;
+  Chunk c;
+  c.id = q % n;
+  c.m = q / n * 8 + ((int)blockIdx.x & 7);
+  int k = c.id;
+  c.kind = kWinds;
+  c.f0 = 4 * k;
+  k -= (a.winds + 3) / 4;
+  if (k >= 0) {
+    c.kind = kPlain;
+    c.f0 = 8 * k;
+    k -= (a.plain + 7) / 8;
+    if (k >= 0) {
+      c.kind = kGeo;
+      c.f0 = 8 * k;
+    }
   }
-  const float sgn = par ? -1.0f : 1.0f;
-  constexpr bool kBNContig = STAGE != kLegendreSynthesis;
-  constexpr int kLoads = kBM * kBK / kThreads;
+  return c;
+}
 
-  const int tiles_n = (N + kBN - 1) / kBN;
-  const int tiles_m = (M + kBM - 1) / kBM;
-  if ((int)blockIdx.x >= tiles_m * tiles_n) return;    // uniform per workgroup
-  const int m0 = (blockIdx.x / tiles_n) * kBM, n0 = (blockIdx.x % tiles_n) * kBN;
-
-  // two LDS stages: the global loads of K-step s+1 are in flight (in registers)
-  // while the MFMAs of step s read the other stage; one barrier per step.  Tiles
-  // are stored [row][k] (row stride kLdk floats).  Within a step the k order is
-  // permuted: lane group g = lane / 16 takes k = 8 g + q at substep q, for A and B
-  // alike, so each MFMA still pairs equal k and a lane's eight operands of a step
-  // are consecutive: two 16-byte LDS reads per operand row, conflict-free at this
-  // stride (16 lanes x 4 banks cover all banks once).
-  static_assert(kBK == 32, "the k permutation assumes 32-wide K steps");
-  constexpr int kLdk = kBK + kPad;
-  __shared__ __align__(16) float As[2][kBM][kLdk];
-  __shared__ __align__(16) float Bs[2][kBN][kLdk];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
-  floatx4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-
-  float ra[kLoads], rb[kLoads];
-  auto load = [&](int k0) {
-#pragma unroll
-    for (int r = 0; r < kLoads; ++r) {
-      const int e = t + kThreads * r;
-      const int mm = e / kBK;
-      const int kk = e % kBK;
-      // clamped indices (always in bounds), no condition: the loads issue back to
-      // back; elements outside the matrix are zeroed when they go to LDS
-      const long row = min(m0 + mm, M - 1) * a_m;
-      const int ck = min(k0 + kk, K - 1);
-      if (STAGE == kLegendreAnalysis)
-        ra[r] = A[row + ck] + sgn * A[row + (a.nlat - 1 - ck)];
-      else
-        ra[r] = A[row + ck * a_k];
-    }
-#pragma unroll
-    for (int r = 0; r < kLoads; ++r) {
-      const int e = t + kThreads * r;
-      const int nn = kBNContig ? (e % kBN) : (e / kBK);
-      const int kk = kBNContig ? (e / kBN) : (e % kBK);
-      const int ck = min(k0 + kk, K - 1), cn = min(n0 + nn, N - 1);
-      rb[r] = B[ck * b_k + cn * b_n];
-    }
-  };
-  auto store = [&](int st, int k0) {
-#pragma unroll
-    for (int r = 0; r < kLoads; ++r) {
-      const int e = t + kThreads * r;
-      const int am = e / kBK;
-      const int ak = e % kBK;
-      As[st][am][ak] = (m0 + am < M && k0 + ak < K) ? ra[r] : 0.0f;
-      const int nn = kBNContig ? (e % kBN) : (e / kBK);
-      const int kk = kBNContig ? (e / kBN) : (e % kBK);
-      Bs[st][nn][kk] = (k0 + kk < K && n0 + nn < N) ? rb[r] : 0.0f;
-    }
-  };
-  load(0);
-  store(0, 0);
-  __syncthreads();
-  int st = 0;
-  for (int k0 = 0; k0 < K; k0 += kBK) {
-    const bool more = k0 + kBK < K;
-    if (more) load(k0 + kBK);
-    // all operands of this step out of LDS first, then the MFMAs
-    const int g8 = (lane >> 4) * 8, r16 = lane & 15;
-    float4 av[2][2], bv[2][2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) av[i][h] = *reinterpret_cast<const float4*>(&As[st][wm + 16 * i + r16][g8 + 4 * h]);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) bv[j][h] = *reinterpret_cast<const float4*>(&Bs[st][wn + 16 * j + r16][g8 + 4 * h]);
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q)
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][q >> 2][q & 3], bv[j][q >> 2][q & 3], acc[i][j],
-                                                           0, 0, 0);
-    // keep the LDS reads ahead of the MFMAs
-    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
-    __builtin_amdgcn_sched_group_barrier(0x008, 32, 0);
-    if (more) store(st ^ 1, k0 + kBK);
-    __syncthreads();
-    st ^= 1;
+// Stacked field of a chunk's slot (0 .. 7), or -1.  The winds of a level are two slots.
+__device__ __forceinline__ int slot_field(const LegendreArgs& a, const Chunk& c, int slot) {
+  if (c.kind == kWinds) {
+    const int k = c.f0 + (slot >> 1);
+    return k < a.winds ? (slot & 1) * a.winds + k : -1;
   }
-  // lane holds C[16 i + 4 (lane >> 4) + r][16 j + (lane & 15)] of its wave's 32 x 32
+  const int f = c.f0 + slot;
+  if (c.kind == kPlain) return f < a.plain ? 2 * a.winds + f : -1;
+  return f < a.geo ? 2 * a.winds + a.plain + f : -1;
+}
+
+// Run and place in it of plain field f < a.plain.
+__device__ __forceinline__ int plain_run(const LegendreArgs& a, int& f) {
+  int r = 0;
+  for (; r < 3 && f >= a.count[r]; ++r) f -= a.count[r];
+  return r;
+}
+
+constexpr int lds_row(int kt) { return 16 * kt + 4; }   // 4 mod 64 banks: 16 rows' 16-byte reads cover all banks
+// Place of c in its row of the synthesis: the lane group c % 4 reads four in one.
+__host__ __device__ constexpr int place(int c) { return (c & ~15) | (c & 3) << 2 | (c >> 2 & 3); }
+constexpr int kAhead = 4;                               // operand blocks in flight per parity
+
+__global__ __launch_bounds__(kThreads) void legendre_synthesis_kernel(LegendreArgs a) {
+  extern __shared__ __align__(16) float lds[];   // [par][16][ld]
+  const Chunk c = find_chunk(a);
+  if (c.m >= a.n_m) return;
+  const int m = c.m, nl = a.nl, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, r16 = lane & 15;
+  const int h = a.nlat >> 1, jts = (h + 15) >> 4, cts = ((nl - m + 1) / 2 + 15) >> 4;
+  const int ld = lds_row(a.kt), par1 = 16 * ld;
+  const size_t per = (size_t)(2 * a.n_m - 1) * nl;
+  const size_t oc = (size_t)(m == 0 ? 0 : 2 * m - 1) * nl, os = oc + (m == 0 ? 0 : nl);   // cosine, sine rows
+  const floatx4* P = reinterpret_cast<const floatx4*>(a.P) + (size_t)a.blk[m] * 64 + lane;
+  const float scale = m == 0 ? 0.5f * 0.3989422804014327f : 0.5f * 0.5641895835477563f;
+
+  for (int k0 = 0; k0 < cts; k0 += a.kt) {
+    const int k1 = min(k0 + a.kt, cts);
+    floatx4 next[2][kAhead];
+    auto load = [&](int jt, int ct) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+      for (int u = 0; u < kAhead; ++u)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int gn = n0 + wn + 16 * j + (lane & 15);
-      if (gn >= N) continue;
+        for (int par = 0; par < 2; ++par)
+          next[par][u] = P[(size_t)((par * cts + min(ct + u, k1 - 1)) * jts + jt) * 64];
+    };
+    if (wave < jts) load(wave, k0);
+    if (k0) __syncthreads();
+    // the modal rows: coefficient l = m + i at [i & 1][row][place(i / 2)]; loads at clamped l (no
+    // condition, so that those of several l are in flight), zero past the last
+    if (c.kind == kWinds) {   // (psi, chi) -> (u cos(lat), v cos(lat)), the highest l clipped
+      const int k = c.f0 + wave;
+      const bool on = k < a.winds;
+      const float* z = a.vor + (size_t)(on ? k : 0) * per;
+      const float* d = a.div + (size_t)(on ? k : 0) * per;
+#pragma unroll 2
+      for (int i = 32 * k0 + lane; i < 32 * k1; i += 64) {
+        const bool in = on && m + i < nl - 1;
+        const int l = min(m + i, nl - 2), lm = max(l - 1, 0);
+        auto inv_lap = [&](int ll) { return ll == 0 ? 0.0f : -a.radius2 / ((float)ll * (float)(ll + 1)); };
+        const float zc = z[oc + l], zs = z[os + l], dc = d[oc + l], ds = d[os + l];
+        const float zcp = z[oc + l + 1], zsp = z[os + l + 1], dcp = d[oc + l + 1], dsp = d[os + l + 1];
+        const float zcm = z[oc + lm], zsm = z[os + lm], dcm = d[oc + lm], dsm = d[os + lm];
+        // cos(lat) d/dlat at l: (l+2) eps(l+1) x_{l+1} - (l-1) eps(l) x_{l-1}
+        const float cp = (float)(l + 2) * eps_ml(m, l + 1) * inv_lap(l + 1);
+        const float cm = -(float)(l - 1) * eps_ml(m, l) * inv_lap(lm), il = inv_lap(l), fm = (float)m;
+        const float uc = (fm * ds * il - (cp * zcp + cm * zcm)) * a.inv_radius;
+        const float vc = (fm * zs * il + (cp * dcp + cm * dcm)) * a.inv_radius;
+        const float us = (-fm * dc * il - (cp * zsp + cm * zsm)) * a.inv_radius;
+        const float vs = (-fm * zc * il + (cp * dsp + cm * dsm)) * a.inv_radius;
+        float* o = lds + (i & 1) * par1 + 4 * wave * ld + place(i >> 1) - 16 * k0;
+        o[0] = in ? uc : 0.0f;
+        o[ld] = in && m ? us : 0.0f;
+        o[2 * ld] = in ? vc : 0.0f;
+        o[3 * ld] = in && m ? vs : 0.0f;
+      }
+    } else if (c.kind == kPlain) {
+      const float* x[2];
+      bool on[2];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gm = m0 + wm + 16 * i + 4 * (lane >> 4) + r;
-        if (gm >= M) continue;
-        C[gm * c_m + gn * c_n] = acc[i][j][r];
+      for (int q = 0; q < 2; ++q) {
+        int f = c.f0 + 2 * wave + q;
+        on[q] = f < a.plain;
+        if (!on[q]) f = c.f0;
+        const int run = plain_run(a, f);
+        x[q] = a.src[run] + (size_t)f * per;
+      }
+#pragma unroll 4
+      for (int i = 32 * k0 + lane; i < 32 * k1; i += 64) {
+        const bool in = m + i < nl;
+        const int l = min(m + i, nl - 1);
+        float* o = lds + (i & 1) * par1 + 4 * wave * ld + place(i >> 1) - 16 * k0;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const float xc = x[q][oc + l], xs = x[q][os + l];
+          o[2 * q * ld] = in && on[q] ? xc : 0.0f;
+          o[(2 * q + 1) * ld] = in && on[q] && m ? xs : 0.0f;
+        }
+      }
+    } else {   // get_geopotential in modal space: waves 0 and 1 take slots 0 .. 3, 2 and 3 the others
+      const int sine = wave & 1, s0 = wave & 2 ? 4 : 0;
+      for (int i = 32 * k0 + lane; i < 32 * k1; i += 64) {
+        const bool in = m + i < nl && (m || !sine);
+        const size_t at = (sine ? os : oc) + min(m + i, nl - 1);
+        const float g0 = a.gravity * a.orography[at];
+        float acc[4] = {g0, g0, g0, g0};
+        for (int kb = 0; kb < a.kx; kb += 8) {   // eight levels' loads at a time (past kx: the last, not summed)
+          float t[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) t[k] = a.tvar[(size_t)min(kb + k, a.kx - 1) * per + at];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            if (kb + k >= a.kx) break;
+            if (at == 0) t[k] += a.reference[kb + k] * kConstCoef;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc[q] += a.geo_w[min(c.f0 + s0 + q, SPEEDY_SHT_KX_MAX - 1)][kb + k] * t[k];
+          }
+        }
+        float* o = lds + (i & 1) * par1 + (2 * s0 + sine) * ld + place(i >> 1) - 16 * k0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) o[2 * q * ld] = in ? acc[q] : 0.0f;
       }
     }
+    __syncthreads();
+    // E|O[row][j] = sum_c X[row][l(par, c)] P[c][j]: a wave takes every fourth latitude tile
+    floatx4 acc[2] = {};
+    const float* A = lds + r16 * ld + 4 * g - 16 * k0;
+    for (int jt = wave, ct = k0; jt < jts;) {
+      floatx4 p[2][kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) p[0][u] = next[0][u], p[1][u] = next[1][u];
+      const bool last = ct + kAhead >= k1;
+      const int jn = last ? jt + 4 : jt, cn = last ? k0 : ct + kAhead;
+      if (jn < jts) load(jn, cn);
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        if (ct + u >= k1) break;
+#pragma unroll
+        for (int par = 0; par < 2; ++par) {
+          const floatx4 x = *reinterpret_cast<const floatx4*>(A + par * par1 + 16 * (ct + u));
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            acc[par] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q], p[par][u][q], acc[par], 0, 0, 0);
+        }
+      }
+      if (last) {   // lane holds rows 4 g .. 4 g + 3 (two fields) of latitude 16 jt + r16
+        const int j = 16 * jt + r16;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int f = slot_field(a, c, 2 * g + q);
+          if (f >= 0 && j < h) {
+            float2* y = a.y + ((size_t)f * a.n_m + m) * a.nlat;
+            const float ec = acc[0][2 * q], es = acc[0][2 * q + 1], odc = acc[1][2 * q], ods = acc[1][2 * q + 1];
+            float2 s = make_float2((ec + odc) * scale, (es + ods) * scale);
+            float2 n = make_float2((ec - odc) * scale, (es - ods) * scale);
+            if (k0) {
+              const float2 s0 = y[j], n0 = y[a.nlat - 1 - j];
+              s.x += s0.x; s.y += s0.y;
+              n.x += n0.x; n.y += n0.y;
+            }
+            y[j] = s;
+            y[a.nlat - 1 - j] = n;
+          }
+        }
+        acc[0] = acc[1] = floatx4{};
+      }
+      jt = jn;
+      ct = cn;
+    }
+  }
+}
+
+// ZLDS: the 16 modal rows fit in LDS behind the staged ones; else they are in a.z.
+template <bool ZLDS>
+__global__ __launch_bounds__(kThreads) void legendre_analysis_kernel(LegendreArgs a) {
+  extern __shared__ __align__(16) float lds[];   // [par][16][ld], then z[16][nl]
+  const Chunk c = find_chunk(a);
+  if (c.m >= a.n_m) return;
+  const int m = c.m, nl = a.nl, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, r16 = lane & 15;
+  const int h = a.nlat >> 1, jts = (h + 15) >> 4, cts = ((nl - m + 1) / 2 + 15) >> 4;
+  const int ld = lds_row(a.kt), par1 = 16 * ld;
+  float* z = ZLDS ? lds + 2 * par1 : a.z + ((size_t)c.id * a.n_m + m) * 16 * nl;
+  // a wave takes one parity and every second c tile
+  const int par = wave & 1;
+  const floatx4* P = reinterpret_cast<const floatx4*>(a.P) + ((size_t)a.blk[m] + (size_t)par * cts * jts) * 64 + lane;
+
+  for (int k0 = 0; k0 < jts; k0 += a.kt) {
+    const int k1 = min(k0 + a.kt, jts);
+    floatx4 next[kAhead];
+    auto load = [&](int ct, int jt) {
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) next[u] = P[(size_t)(ct * jts + min(jt + u, k1 - 1)) * 64];
+    };
+    const int ct0 = wave >> 1;
+    if (ct0 < cts) load(ct0, k0);
+    if (k0) __syncthreads();
+    // even and odd halves Y_j +- Y_{nlat-1-j} of both modes
+    const float2* y[2];
+    bool on[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int f = slot_field(a, c, 2 * wave + q);
+      on[q] = f >= 0 && f < a.nfield;
+      y[q] = a.y + ((size_t)(on[q] ? f : 0) * a.n_m + m) * a.nlat;
+    }
+#pragma unroll 2
+    for (int j = 16 * k0 + lane; j < 16 * k1; j += 64) {
+      const int js = min(j, h - 1), jn = a.nlat - 1 - js;
+      float* o = lds + 4 * wave * ld + j - 16 * k0;
+#pragma unroll
+      for (int q = 0; q < 2; ++q, o += 2 * ld) {
+        const float2 s = y[q][js], n = y[q][jn];
+        const bool in = on[q] && j < h;
+        o[0] = in ? s.x + n.x : 0.0f;
+        o[ld] = in ? s.y + n.y : 0.0f;
+        o[par1] = in ? s.x - n.x : 0.0f;
+        o[par1 + ld] = in ? s.y - n.y : 0.0f;
+      }
+    }
+    __syncthreads();
+    floatx4 acc = {};
+    const float* A = lds + par * par1 + r16 * ld + 4 * g - 16 * k0;
+    for (int ct = ct0, jt = k0; ct < cts;) {
+      floatx4 p[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) p[u] = next[u];
+      const bool last = jt + kAhead >= k1;
+      const int cn = last ? ct + 2 : ct, jn = last ? k0 : jt + kAhead;
+      if (cn < cts) load(cn, jn);
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        if (jt + u >= k1) break;
+        const floatx4 x = *reinterpret_cast<const floatx4*>(A + 16 * (jt + u));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q], p[u][q], acc, 0, 0, 0);
+      }
+      if (last) {   // lane holds rows 4 g .. 4 g + 3 of c = 16 ct + r16
+        const int l = m + par + 2 * (16 * ct + r16);
+        if (l < nl) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            float* o = z + (size_t)(4 * g + q) * nl + l;
+            *o = k0 ? *o + acc[q] : acc[q];
+          }
+        }
+        acc = floatx4{};
+      }
+      ct = cn;
+      jt = jn;
+    }
+  }
+  __syncthreads();
+  // the coefficients below l = m are zero (not finite where the order's others are not)
+  auto at = [&](int row, int l) {
+    const float v = z[(size_t)row * nl + max(l, m)];
+    return l < m ? v * 0.0f + 0.0f : v;
+  };
+  const size_t per = (size_t)(2 * a.n_m - 1) * nl;
+  const size_t oc = (size_t)(m == 0 ? 0 : 2 * m - 1) * nl, os = oc + nl;
+  if (c.kind == kWinds) {
+    // (U, V) = (u, v) / cos(lat) -> vorticity and divergence, the highest l clipped:
+    // sec(lat) d/dlat cos^2(lat) at l is l eps(l+1) x_{l+1} - (l+1) eps(l) x_{l-1}
+    const int k = c.f0 + wave, ru = 4 * wave, rv = ru + 2;
+    if (k >= a.winds) return;
+    const float fm = (float)m;
+    for (int l = lane; l < nl; l += 64) {
+      float zc = 0.0f, zs = 0.0f, dc = 0.0f, ds = 0.0f;
+      if (l < nl - 1) {
+        const int lm = max(l - 1, 0);
+        const float cp = (float)l * eps_ml(m, l + 1), cm = -(float)(l + 1) * eps_ml(m, l);
+        zc = (fm * at(rv + 1, l) - (cp * at(ru, l + 1) + cm * at(ru, lm))) * a.inv_radius;
+        dc = (fm * at(ru + 1, l) + (cp * at(rv, l + 1) + cm * at(rv, lm))) * a.inv_radius;
+        zs = (-fm * at(rv, l) - (cp * at(ru + 1, l + 1) + cm * at(ru + 1, lm))) * a.inv_radius;
+        ds = (-fm * at(ru, l) + (cp * at(rv + 1, l + 1) + cm * at(rv + 1, lm))) * a.inv_radius;
+      }
+      a.vor_out[k * per + oc + l] = zc;
+      a.div_out[k * per + oc + l] = dc;
+      if (m) {
+        a.vor_out[k * per + os + l] = zs;
+        a.div_out[k * per + os + l] = ds;
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int slot = 2 * wave + q;
+    int f = c.f0 + slot;
+    if (f >= a.plain) return;
+    const int run = plain_run(a, f);
+    float* o = a.dst[run] + (size_t)f * per;
+    for (int l = lane; l < nl; l += 64) {
+      o[oc + l] = at(2 * slot, l);
+      if (m) o[os + l] = at(2 * slot + 1, l);
+    }
+  }
 }
 
 // ------------------------------------------------------------ Fourier stages
@@ -242,26 +475,19 @@ __global__ __launch_bounds__(kThreads) void sht_gemm_kernel(StageArgs a) {
 // N = n1 * n2, longitude i = i1 + n1 * i2, wavenumber k = k2 + n2 * k1):
 //   X_k = sum_i1 w^(i1 k) Z[i1][k mod n2],   Z[i1][k2] = sum_i2 x[i1 + n1 i2] w_n2^(i2 k2),
 // with w = exp(-2 pi i / N) and w_n2 = w^n1.  Z of a real line is Hermitian in
-// k2, so only k2 <= n2 / 2 is formed.  The modal coefficients are the basis's
-// projections: mode 0 = X_0 / sqrt(2 pi), mode 2k-1 = Re X_k / sqrt(pi), mode
-// 2k = -Im X_k / sqrt(pi).  Synthesis runs the same passes backwards.  About
-// 4x fewer flops than the dense contraction with the basis, and two passes of
-// length n1 and n2 instead of one of length nlon.  A workgroup takes one field
-// and `tl` latitudes (latitude fastest, as in memory); the line tile, the
-// intermediate Z or W and the N roots of unity live in LDS.
+// k2, so only k2 <= n2 / 2 is formed.  Y holds the cosine and the sine projection of
+// order k, Re X_k and -Im X_k; the basis's factors are the Legendre stages'.  Synthesis
+// runs the same passes backwards.  A workgroup takes one field and `tl` latitudes
+// (latitude fastest, as in memory); the intermediate Z or W and the N roots of unity
+// live in LDS, in the generic kernels the line tile too.
 struct FourierArgs {
   int32_t nlon, nlat, mm, n_m, n1, n2, tl, nfield;
   const float* twr;     // [nlon] cos(2 pi j / nlon)
   const float* twi;     // [nlon] -sin(2 pi j / nlon)
-  const float* w;       // [nlat] Gauss weights * 2 pi / nlon
   const float* sec;     // [nlat]
-  const float* in;      // synthesis: E / O halves [2][nfield][mm][nlat / 2]
-  float* out;           // analysis: Y [nfield][mm][nlat]
+  float2* y;            // [nfield][n_m][nlat]: cosine and sine mode, without the basis's factors
   SegTable seg;
 };
-
-constexpr float kRsqrt2Pi = 0.3989422804014327f;   // 1 / sqrt(2 pi)
-constexpr float kRsqrtPi = 0.5641895835477563f;    // 1 / sqrt(pi)
 
 __device__ __forceinline__ void load_roots(const FourierArgs& a, float* twr, float* twi) {
   for (int i = threadIdx.x; i < a.nlon; i += kThreads) {
@@ -270,7 +496,7 @@ __device__ __forceinline__ void load_roots(const FourierArgs& a, float* twr, flo
   }
 }
 
-// Y_b[mode][lat] = sum_lon F[lon][mode] * prologue(x_b[lon][lat]) for one field b
+// Y_b[m][lat] = sum_lon (cos, sin)(m lon) prologue(x_b[lon][lat]) for one field b
 // (blockIdx.y) and latitudes j0 .. j0 + tl - 1 (blockIdx.x).
 __global__ __launch_bounds__(kThreads) void fourier_analysis_generic(FourierArgs a) {
   extern __shared__ float lds[];
@@ -292,7 +518,7 @@ __global__ __launch_bounds__(kThreads) void fourier_analysis_generic(FourierArgs
       v = src[(size_t)lon * a.nlat + j];
       if (sg.op & kOpLog) v = logf(v);
       if (sg.op & kOpSubLevel) v -= lvl;
-      v *= sg.mul * a.w[j] * ((sg.op & kOpSecLat) ? a.sec[j] : 1.0f);
+      v *= sg.mul * ((sg.op & kOpSecLat) ? a.sec[j] : 1.0f);
     }
     xs[e] = v;
   }
@@ -314,7 +540,7 @@ __global__ __launch_bounds__(kThreads) void fourier_analysis_generic(FourierArgs
   }
   __syncthreads();
   // pass 2: X_k = sum_i1 w^(i1 k) Z[i1][k mod n2] for k < n_m, then the modes
-  float* Y = a.out + (size_t)b * a.mm * a.nlat;
+  float2* Y = a.y + (size_t)b * a.n_m * a.nlat;
   for (int e = threadIdx.x; e < a.n_m * tl; e += kThreads) {
     const int k = e / tl, jj = e - k * tl, j = j0 + jj;
     int k2 = k % n2;
@@ -333,57 +559,39 @@ __global__ __launch_bounds__(kThreads) void fourier_analysis_generic(FourierArgs
       q += kq;
       if (q >= N) q -= N;
     }
-    if (j < a.nlat) {
-      if (k == 0) {
-        Y[j] = re * kRsqrt2Pi;
-      } else {
-        Y[(size_t)(2 * k - 1) * a.nlat + j] = re * kRsqrtPi;
-        Y[(size_t)(2 * k) * a.nlat + j] = -im * kRsqrtPi;
-      }
-    }
+    if (j < a.nlat) Y[(size_t)k * a.nlat + j] = make_float2(re, -im);
   }
 }
 
-// out_b[lon][lat] = epilogue(sum_mode F[lon][mode] * Y_b[mode][lat]), Y_b from the
-// Legendre synthesis's even / odd halves: E + O (southern latitudes), E - O
-// (northern).
+// out_b[lon][lat] = epilogue(sum_m of both modes times (cos, sin)(m lon)), twice the
+// halves that the Legendre synthesis leaves in Y_b.
 __global__ __launch_bounds__(kThreads) void fourier_synthesis_generic(FourierArgs a) {
   extern __shared__ float lds[];
-  const int N = a.nlon, n1 = a.n1, n2 = a.n2, tl = a.tl, h = a.nlat >> 1;
+  const int N = a.nlon, n1 = a.n1, n2 = a.n2, tl = a.tl, n_m = a.n_m;
   const int b = blockIdx.y, j0 = blockIdx.x * tl;
   float* twr = lds;
   float* twi = twr + N;
-  float* ys = twi + N;             // [mm][tl]
-  float* wr = ys + a.mm * tl;      // [n1][n2][tl]
+  float* yc = twi + N;             // [n_m][tl]
+  float* ys = yc + n_m * tl;       // [n_m - 1][tl]: m >= 1
+  float* wr = ys + (n_m - 1) * tl; // [n1][n2][tl]
   float* wi = wr + N * tl;
   const Seg sg = a.seg.s[find_seg(a.seg, b)];
   load_roots(a, twr, twi);
-  const float* E = a.in + (size_t)b * a.mm * h;
-  const size_t odd = (size_t)a.nfield * a.mm * h;
-  for (int e = threadIdx.x; e < a.mm * tl; e += kThreads) {
-    const int mode = e / tl, jj = e - mode * tl, j = j0 + jj;
-    float v = 0.0f;
-    if (j < a.nlat) {
-      const float* p = E + (size_t)mode * h + (j < h ? j : a.nlat - 1 - j);
-      v = j < h ? p[0] + p[odd] : p[0] - p[odd];
-    }
-    ys[e] = v;
+  const float2* Y = a.y + (size_t)b * n_m * a.nlat;
+  for (int e = threadIdx.x; e < n_m * tl; e += kThreads) {
+    const int k = e / tl, jj = e - k * tl, j = j0 + jj;
+    float2 v = make_float2(0.0f, 0.0f);
+    if (j < a.nlat) v = Y[(size_t)k * a.nlat + j];
+    yc[e] = v.x;
+    if (k) ys[e - tl] = v.y;
   }
   __syncthreads();
-  // pass 1: W[i1][k2] = sum_{k = k2 + n2 k1 < n_m} c_k conj(w^(i1 k)),
-  // c_0 = Y_0 / sqrt(2 pi), c_k = (Y_{2k-1} - i Y_{2k}) / sqrt(pi)
+  // pass 1: W[i1][k2] = sum_{k = k2 + n2 k1 < n_m} c_k conj(w^(i1 k)), c_k = cosine - i sine of Y
   for (int e = threadIdx.x; e < N * tl; e += kThreads) {
     const int r = e / tl, jj = e - r * tl, k2 = r % n2, i1 = r / n2;
     float re = 0.0f, im = 0.0f;
     for (int k = k2; k < a.n_m; k += n2) {
-      float c_r, c_i;
-      if (k == 0) {
-        c_r = ys[jj] * kRsqrt2Pi;
-        c_i = 0.0f;
-      } else {
-        c_r = ys[(2 * k - 1) * tl + jj] * kRsqrtPi;
-        c_i = -ys[(2 * k) * tl + jj] * kRsqrtPi;
-      }
+      const float c_r = yc[k * tl + jj], c_i = k ? -ys[(k - 1) * tl + jj] : 0.0f;
       const int q = (int)(((long)i1 * k) % N);
       const float t_r = twr[q], t_i = -twi[q];
       re += c_r * t_r - c_i * t_i;
@@ -411,7 +619,7 @@ __global__ __launch_bounds__(kThreads) void fourier_synthesis_generic(FourierArg
     }
     if (j < a.nlat) {
       if (sg.op & kOpSecLat) v *= a.sec[j];
-      v = v * sg.mul;
+      v = v * (2.0f * sg.mul);
       if (sg.op & kOpAddLevel) v += lvl;
       if (sg.op & kOpExp) v = expf(v);
       dst[(size_t)lon * a.nlat + j] = v;
@@ -425,13 +633,15 @@ __global__ __launch_bounds__(kThreads) void fourier_synthesis_generic(FourierArg
 // memory directly; only the pass-1 results and the N roots of unity for the twiddles
 // w^(i1 k2) go through LDS.
 //
-// The real side of each stage uses the Hermitian symmetry in k2: a thread takes the
-// pair (k2, N2 - k2), so half the pass-1 results are exchanged and the real FFTs do
-// half the work.  Bound by latency: of the launch's single wave of workgroups at T85, of
-// the few workgroups a CU holds at T213.  With dense sums for the short DFTs (n1 and n2
-// terms per output) T85 analysis and synthesis took 8.7 and 12.3 us, now 7.3 and 11.6;
-// T213 x 41 fields synthesis 115 us, now 53; a T425 conversion of 41 fields 1977 us in
-// the generic kernels, now 617.
+// The real side of each stage uses the Hermitian symmetry in k2: half the analysis's
+// pass-1 results are formed and exchanged, and the real FFTs do half the work; on the
+// wavenumber side n_m <= nlon / 2 leaves half the inputs zero or outputs unused.  Bound
+// by latency: of the launch's single wave of workgroups at T85, of the few workgroups
+// that a CU holds at T213.  With dense sums for the short DFTs (n1 and n2 terms per
+// output) and Y as the even and odd halves of every mode, T85 analysis (32 fields) and
+// synthesis (41) took 8.7 and 12.3 us, now 5.8 and 7.2; T213 x 41 synthesis 115 us, now
+// 30.  A thread that took a pair of k2 in the synthesis, to exchange half as much, had
+// twice the chain: T85 17.4 us a conversion against 16.2, T213 69 against 56.
 constexpr double kPiD = 3.14159265358979323846;
 constexpr double ct_sin(double x) {   // |x| <= pi, Taylor series to 1e-16
   double term = x, sum = x;
@@ -467,8 +677,9 @@ struct Roots {
 constexpr int radix(int n) { return n % 4 == 0 ? 4 : n % 2 == 0 ? 2 : n % 3 == 0 ? 3 : n % 5 == 0 ? 5 : n; }
 
 // X_k = sum_j x_j w_n^(jk), in place and in natural order.  The inverse (conjugated
-// roots) is the same with real and imaginary parts exchanged: fft(im, re).
-template <int n>
+// roots) is the same with real and imaginary parts exchanged: fft(im, re).  HALF: x_j is
+// zero (and not read) for j >= n / 2, n of 2 or a multiple of 4 or n = 2 b.
+template <int n, bool HALF = false>
 __device__ __forceinline__ void fft(float (&re)[n], float (&im)[n]) {
   static_assert(n == 1 || radix(n) < n || n <= 5, "lengths of factors 2, 3 and 5");
   if constexpr (n == 2) {
@@ -513,8 +724,19 @@ __device__ __forceinline__ void fft(float (&re)[n], float (&im)[n]) {
     for (int j = 0; j < b; ++j) {
       float xr[a], xi[a];
 #pragma unroll
-      for (int i = 0; i < a; ++i) { xr[i] = re[j + b * i]; xi[i] = im[j + b * i]; }
-      fft<a>(xr, xi);
+      for (int i = 0; i < (HALF ? a / 2 : a); ++i) { xr[i] = re[j + b * i]; xi[i] = im[j + b * i]; }
+      if constexpr (!HALF) {
+        fft<a>(xr, xi);
+      } else if constexpr (a == 2) {
+        xr[1] = xr[0]; xi[1] = xi[0];
+      } else {
+        static_assert(a == 4, "half-zero transforms start with a radix of 2 or 4");
+        const float r0 = xr[0], i0 = xi[0], r1 = xr[1], i1 = xi[1];
+        xr[0] = r0 + r1; xi[0] = i0 + i1;
+        xr[1] = r0 + i1; xi[1] = i0 - r1;
+        xr[2] = r0 - r1; xi[2] = i0 - i1;
+        xr[3] = r0 - i1; xi[3] = i0 + r1;
+      }
 #pragma unroll
       for (int k = 0; k < a; ++k) {
         const float c = w.c[(j * k) % n], s = w.s[(j * k) % n];
@@ -673,315 +895,138 @@ __device__ __forceinline__ void c2r(const float (&re)[n / 2 + 1], const float (&
 }
 
 // Threads of a compiled Fourier kernel with tl latitudes: one per (i1, latitude) on the
-// longitude side and one per (pair of k2, latitude) on the wavenumber side.
-constexpr int fourier_threads(int n1, int n2, int tl) {
-  return ((n1 > n2 / 2 ? n1 : n2 / 2) * tl + 63) / 64 * 64;
+// longitude side and one per (k2, latitude) on the wavenumber side (n1 <= n2).
+constexpr int fourier_threads(int n2, int tl) { return (n2 * tl + 63) / 64 * 64; }
+
+// 32-bit byte offset from a uniform base (a field is below 2^31 / 16 bytes).
+template <typename T>
+__device__ __forceinline__ T* at(T* base, uint32_t bytes) {
+  return (T*)((char*)base + bytes);
 }
 
 template <int N1, int N2, int TL>
-__global__ __launch_bounds__(fourier_threads(N1, N2, TL)) void fourier_analysis_kernel(FourierArgs a) {
-  constexpr int N = N1 * N2, NH = N2 / 2 + 1, T = fourier_threads(N1, N2, TL);
+__global__ __launch_bounds__(fourier_threads(N2, TL)) void fourier_analysis_kernel(FourierArgs a) {
+  constexpr int N = N1 * N2, NH = N2 / 2 + 1, T = fourier_threads(N2, TL);
   __shared__ float2 tw[N], z[NH * N1 * TL];   // z: [k2][i1][lat]
   const int b = blockIdx.y, j0 = blockIdx.x * TL;
   const Seg sg = a.seg.s[find_seg(a.seg, b)];
   const float* src = sg.src + (size_t)(b - sg.first) * N * a.nlat;
-  const float lvl = sg.level ? sg.level[(b - sg.first) % sg.period] : 0.0f;
+  const float lvl = sg.op & kOpSubLevel ? sg.level[(b - sg.first) % sg.period] : 0.0f;
   const int row = threadIdx.x / TL, jj = threadIdx.x % TL, j = j0 + jj;
   const bool in = j < a.nlat;
   const int jc = in ? j : 0;
   float x[N2];
   if (row < N1) {
 #pragma unroll
-    for (int i2 = 0; i2 < N2; ++i2) x[i2] = src[(size_t)(row + N1 * i2) * a.nlat + jc];
+    for (int i2 = 0; i2 < N2; ++i2) x[i2] = *at(src, ((row + N1 * i2) * a.nlat + jc) * 4u);
   }
   for (int i = threadIdx.x; i < N; i += T) tw[i] = make_float2(a.twr[i], a.twi[i]);
   // pass 1: thread (i1, lat): Z[i1][k2] = sum_i2 x[i1 + N1 i2] w_N2^(i2 k2), k2 <= N2 / 2
   if (row < N1) {
-    const float cs = in ? sg.mul * a.w[jc] * ((sg.op & kOpSecLat) ? a.sec[jc] : 1.0f) : 0.0f;
+    const float cs = sg.mul * ((sg.op & kOpSecLat) ? a.sec[jc] : 1.0f);
 #pragma unroll
-    for (int i2 = 0; i2 < N2; ++i2) {
-      float v = x[i2];
-      if (sg.op & kOpLog) v = logf(v);
-      if (sg.op & kOpSubLevel) v -= lvl;
-      x[i2] = in ? v * cs : 0.0f;
-    }
+    for (int i2 = 0; i2 < N2; ++i2)
+      if (sg.op & kOpLog) x[i2] = logf(x[i2]);
+#pragma unroll
+    for (int i2 = 0; i2 < N2; ++i2) x[i2] = (x[i2] - lvl) * cs;
     float re[NH], im[NH];
     rfft<N2>(x, re, im);
 #pragma unroll
     for (int k2 = 0; k2 < NH; ++k2) z[(k2 * N1 + row) * TL + jj] = make_float2(re[k2], im[k2]);
   }
   __syncthreads();
-  // pass 2: thread (k2 and N2 - k2, lat): X_{k2 + N2 k1} = sum_i1 (Z[i1][k2] w^(i1 k2)) w_N1^(i1 k1);
-  // thread row 0 takes k2 = 0 and N2 / 2
-  if (row >= N2 / 2) return;
-  float* Y = a.out + (size_t)b * a.mm * a.nlat + j;
+  // pass 2: thread (k2, lat): X_{k2 + N2 k1} = sum_i1 (Z[i1][k2] w^(i1 k2)) w_N1^(i1 k1), with
+  // Z[N2 - k2] = conj(Z[k2])
+  const int k2 = row, kz = k2 <= N2 / 2 ? k2 : N2 - k2;
+  if (k2 >= N2) return;
+  const float cj = k2 <= N2 / 2 ? 1.0f : -1.0f;
+  float2* Y = a.y + (size_t)b * a.n_m * a.nlat;
+  float re[N1], im[N1];
 #pragma unroll
-  for (int side = 0; side < 2; ++side) {
-    const int k2 = side == 0 ? row : (row == 0 ? N2 / 2 : N2 - row);
-    const int kz = side == 0 || row == 0 ? k2 : row;   // the row of z: Z[N2 - k2] = conj(Z[k2])
-    const float cj = side == 0 || row == 0 ? 1.0f : -1.0f;
-    float re[N1], im[N1];
-#pragma unroll
-    for (int i1 = 0; i1 < N1; ++i1) {
-      const float2 v = z[(kz * N1 + i1) * TL + jj], t = tw[i1 * k2];
-      const float vi = cj * v.y;
-      re[i1] = v.x * t.x - vi * t.y;
-      im[i1] = v.x * t.y + vi * t.x;
-    }
-    fft<N1>(re, im);
-#pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) {
-      if (N2 * k1 >= a.n_m) break;   // uniform; k < n_m is masked per lane below
-      const int k = k2 + N2 * k1;
-      if (in && k < a.n_m) {
-        if (k == 0) {
-          Y[0] = re[k1] * kRsqrt2Pi;
-        } else {
-          Y[(size_t)(2 * k - 1) * a.nlat] = re[k1] * kRsqrtPi;
-          Y[(size_t)(2 * k) * a.nlat] = -im[k1] * kRsqrtPi;
-        }
-      }
-    }
+  for (int i1 = 0; i1 < N1; ++i1) {
+    const float2 v = z[(kz * N1 + i1) * TL + jj], t = tw[i1 * k2];
+    const float vi = cj * v.y;
+    re[i1] = v.x * t.x - vi * t.y;
+    im[i1] = v.x * t.y + vi * t.x;
   }
+  fft<N1>(re, im);
+#pragma unroll
+  for (int k1 = 0; k1 < N1 / 2; ++k1) {   // 2 n_m - 1 <= N: no wavenumber above N / 2
+    if (N2 * k1 >= a.n_m) break;          // uniform; k < n_m is masked per lane below
+    const int k = k2 + N2 * k1;
+    if (in && k < a.n_m) *at(Y, (k * a.nlat + j) * 8u) = make_float2(re[k1], -im[k1]);
+  }
+}
+
+// Y_k of one latitude (byte offset `at` in the field): zero for k >= n_m, past the
+// buffer's end.
+__device__ __forceinline__ float2 load_y(__amdgpu_buffer_rsrc_t y, int at) {
+  typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+  const uintx2 v = __builtin_amdgcn_raw_buffer_load_b64(y, at, 0, 0);
+  return make_float2(__uint_as_float(v.x), __uint_as_float(v.y));
 }
 
 template <int N1, int N2, int TL>
-__global__ __launch_bounds__(fourier_threads(N1, N2, TL)) void fourier_synthesis_kernel(FourierArgs a) {
-  constexpr int N = N1 * N2, NH = N2 / 2 + 1, T = fourier_threads(N1, N2, TL);
-  __shared__ float2 tw[N], hs[N1 * NH * TL];   // hs: [i1][k2][lat]
-  const int h = a.nlat >> 1, b = blockIdx.y, j0 = blockIdx.x * TL;
-  const Seg sg = a.seg.s[find_seg(a.seg, b)];
-  const float* E = a.in + (size_t)b * a.mm * h;
-  const size_t odd = (size_t)a.nfield * a.mm * h;
+__global__ __launch_bounds__(fourier_threads(N2, TL)) void fourier_synthesis_kernel(FourierArgs a) {
+  constexpr int N = N1 * N2, NH = N2 / 2 + 1, T = fourier_threads(N2, TL);
+  __shared__ float2 tw[N], w[N * TL];   // w: [i1][k2][lat]
+  const int b = blockIdx.y, j0 = blockIdx.x * TL;
   const int row = threadIdx.x / TL, jj = threadIdx.x % TL, j = j0 + jj;
   const bool in = j < a.nlat;
-  const int jh = !in ? 0 : (j < h ? j : a.nlat - 1 - j);
-  const float so = j < h ? 1.0f : -1.0f;
+  const __amdgpu_buffer_rsrc_t Y = __builtin_amdgcn_make_buffer_rsrc(
+      a.y + (size_t)b * a.n_m * a.nlat, 0, a.n_m * a.nlat * 8, 0x00020000);
+  // pass 1: thread (k2, lat): W[i1][k2] = conj(w^(i1 k2)) sum_k1 c_{k2 + N2 k1} conj(w_N1^(i1 k1)),
+  // c = cosine - i sine of Y, zero from k1 = N1 / 2 on
+  const int k2 = row;
+  float re[N1], im[N1];
+  if (k2 < N2) {
+    int at = (k2 * a.nlat + (in ? j : 0)) * 8;
+#pragma unroll
+    for (int k1 = 0; k1 < N1 / 2; ++k1) {
+      re[k1] = im[k1] = 0.0f;
+      if (N2 * k1 >= a.n_m) continue;   // uniform
+      const float2 y = load_y(Y, at);
+      re[k1] = y.x;
+      im[k1] = -y.y;
+      at += N2 * a.nlat * 8;
+    }
+  }
   for (int i = threadIdx.x; i < N; i += T) tw[i] = make_float2(a.twr[i], a.twi[i]);
   __syncthreads();
-  // pass 1: thread (k2 and N2 - k2, lat): W[i1][k2] = conj(w^(i1 k2)) sum_k1 c_{k2 + N2 k1} conj(w_N1^(i1 k1)),
-  // c_0 = Y_0 / sqrt(2 pi), c_k = (Y_{2k-1} - i Y_{2k}) / sqrt(pi); Y from E + O (south), E - O
-  // (north).  The line is the real part of W's transform over k2, so the Hermitian part
-  // (W[k2] + conj(W[N2 - k2])) / 2 is all that pass 2 reads; the halves are in c here.
-  if (row < N2 / 2) {
-    float re[2][N1], im[2][N1];
-#pragma unroll
-    for (int side = 0; side < 2; ++side) {
-      const int k2 = side == 0 ? row : (row == 0 ? N2 / 2 : N2 - row);
-      // the wavenumbers k = k2 + N2 k1 < n_m: k1 < ceil(n_m / N2) for every lane (a
-      // uniform bound), the last one masked per lane; loads at clamped modes (in bounds)
-#pragma unroll
-      for (int k1 = 0; k1 < N1; ++k1) {
-        re[side][k1] = im[side][k1] = 0.0f;
-        if (N2 * k1 >= a.n_m) continue;
-        const int k = k2 + N2 * k1;
-        const int kc = k < a.n_m ? k : 0;
-        const float* pc = E + (size_t)(kc == 0 ? 0 : 2 * kc - 1) * h + jh;
-        const float* ps = E + (size_t)(2 * kc) * h + jh;
-        const float y_c = pc[0] + so * pc[odd], y_s = ps[0] + so * ps[odd];
-        const bool use = in && k < a.n_m;
-        re[side][k1] = use ? y_c * (k == 0 ? 0.5f * kRsqrt2Pi : 0.5f * kRsqrtPi) : 0.0f;
-        im[side][k1] = use && k > 0 ? -y_s * (0.5f * kRsqrtPi) : 0.0f;
-      }
-    }
-#pragma unroll
-    for (int side = 0; side < 2; ++side) {
-      const int k2 = side == 0 ? row : (row == 0 ? N2 / 2 : N2 - row);
-      fft<N1>(im[side], re[side]);   // inverse
-#pragma unroll
-      for (int i1 = 0; i1 < N1; ++i1) {
-        const float2 t = tw[i1 * k2];   // conjugated below
-        const float r = re[side][i1], m = im[side][i1];
-        re[side][i1] = r * t.x + m * t.y;
-        im[side][i1] = m * t.x - r * t.y;
-      }
-    }
+  if (k2 < N2) {
+    if (k2 == 0) im[0] = 0.0f;   // m = 0 has no sine mode
+    fft<N1, true>(im, re);       // inverse
 #pragma unroll
     for (int i1 = 0; i1 < N1; ++i1) {
-      float2* o = &hs[i1 * NH * TL + jj];
-      if (row == 0) {
-        o[0] = make_float2(2.0f * re[0][i1], 0.0f);
-        o[(N2 / 2) * TL] = make_float2(2.0f * re[1][i1], 0.0f);
-      } else {
-        o[row * TL] = make_float2(re[0][i1] + re[1][i1], im[0][i1] - im[1][i1]);
-      }
+      const float2 t = tw[i1 * k2];   // conjugated
+      w[(i1 * N2 + k2) * TL + jj] = make_float2(re[i1] * t.x + im[i1] * t.y, im[i1] * t.x - re[i1] * t.y);
     }
   }
+  const Seg sg = a.seg.s[find_seg(a.seg, b)];
   __syncthreads();
-  // pass 2: thread (i1, lat): x[i1 + N1 i2] = sum_k2 H[i1][k2] conj(w_N2^(i2 k2)), then the epilogue
+  // pass 2: thread (i1, lat): the line is the real part of W's transform over k2, that is
+  // the transform of its Hermitian part H[k2] = W[k2] + conj(W[N2 - k2]) (the half is in Y):
+  // x[i1 + N1 i2] = sum_k2 H[i1][k2] conj(w_N2^(i2 k2)), then the epilogue
   if (row >= N1 || !in) return;
-  float* dst = sg.dst + (size_t)(b - sg.first) * N * a.nlat + j;
-  const float lvl = sg.level ? sg.level[(b - sg.first) % sg.period] : 0.0f;
-  const float sc = ((sg.op & kOpSecLat) ? a.sec[j] : 1.0f);
-  float re[NH], im[NH], x[N2];
+  float* dst = sg.dst + (size_t)(b - sg.first) * N * a.nlat;
+  const float lvl = sg.op & kOpAddLevel ? sg.level[(b - sg.first) % sg.period] : 0.0f;
+  const float sc = sg.mul * ((sg.op & kOpSecLat) ? a.sec[j] : 1.0f);
+  float hr[NH], hi[NH], x[N2];
 #pragma unroll
   for (int k2 = 0; k2 < NH; ++k2) {
-    const float2 v = hs[(row * NH + k2) * TL + jj];
-    re[k2] = v.x;
-    im[k2] = v.y;
+    const float2 v = w[(row * N2 + k2) * TL + jj], u = w[(row * N2 + (k2 ? N2 - k2 : 0)) * TL + jj];
+    hr[k2] = v.x + u.x;
+    hi[k2] = v.y - u.y;
   }
-  c2r<N2>(re, im, x);
+  c2r<N2>(hr, hi, x);
 #pragma unroll
-  for (int i2 = 0; i2 < N2; ++i2) {
-    float v = x[i2] * sc * sg.mul;
-    if (sg.op & kOpAddLevel) v += lvl;
-    if (sg.op & kOpExp) v = expf(v);
-    dst[(size_t)(row + N1 * i2) * a.nlat] = v;
-  }
-}
-
-// eps(m, l) = sqrt((l^2 - m^2) / (4 l^2 - 1)) for m <= l, l >= 1; else 0:
-// x P_l^m = eps(m, l+1) P_{l+1}^m + eps(m, l) P_{l-1}^m (unit-norm functions).
-__device__ __forceinline__ float eps_ml(int m, int l) {
-  if (l <= 0 || m > l) return 0.0f;
-  const float fl = (float)l, fm = (float)m;
-  return sqrtf((fl * fl - fm * fm) / (4.0f * fl * fl - 1.0f));
-}
-
-struct ModalArgs {
-  int32_t mm, nl, kx;
-  float inv_radius, radius2;
-  const float* vor;     // [kx][mm][nl]
-  const float* div;
-  const float* copy_src[4];   // modal fields copied behind the winds (null: zeros)
-  int32_t copy_count[4];
-  float* out;           // contiguous [nfield][mm][nl]
-  float* vor_out;       // post: destinations of vorticity / divergence
-  float* div_out;
-  float* copy_dst[4];
-  // geopotential rows behind the copies (winds kernel; kx rows when geo_w is set):
-  // phi_j = g orography + sum_k W[j][k] (T_var_k + reference_k as a constant)
-  const float* tvar;
-  const float* orography;
-  const float* reference;
-  float gravity;
-  int32_t geo;
-  float geo_w[SPEEDY_SHT_KX_MAX][SPEEDY_SHT_KX_MAX];
-};
-
-// Modal coefficient (mode 0, l 0) of the constant 1: 1 / (F_0 P_0^0) = 2 sqrt(pi).
-constexpr float kConstCoef = 3.5449077018110318f;
-
-__device__ __forceinline__ float d_dlon(const float* x, int mode, int m, int l, int nl) {
-  if (mode == 0) return 0.0f;
-  return (mode & 1) ? (float)m * x[(mode + 1) * nl + l] : -(float)m * x[(mode - 1) * nl + l];
-}
-
-// Modal (psi, chi) -> (u cos(lat), v cos(lat)) for every level, then copies of
-// the remaining modal inputs, into one contiguous stack (vor_div_to_uv_nodal's
-// modal half and compute_diagnostic_state's inputs).  blockIdx.y is the row:
-// rows below kx are the winds of level blockIdx.y (writing the u and v rows),
-// the others write output row blockIdx.y + kx; blockIdx.x covers the row's
-// mm x nl coefficients.
-__global__ __launch_bounds__(kThreads) void modal_winds_kernel(ModalArgs a) {
-  const int per = a.mm * a.nl;
-  const int rem = blockIdx.x * kThreads + threadIdx.x;
-  if (rem >= per) return;
-  int r = blockIdx.y;
-  if (r < a.kx) {
-    const int k = r, mode = rem / a.nl, l = rem - mode * a.nl;
-    const int m = (mode + 1) >> 1;
-    const float* z = a.vor + (size_t)k * per;
-    const float* d = a.div + (size_t)k * per;
-    float u = 0.0f, v = 0.0f;
-    if (l < a.nl - 1) {     // the highest total wavenumber is clipped
-      auto inv_lap = [&](int ll) { return ll == 0 ? 0.0f : -a.radius2 / ((float)ll * (float)(ll + 1)); };
-      // d/dlon of psi, chi at (mode, l)
-      const float psi_lon = d_dlon(z, mode, m, l, a.nl) * inv_lap(l);
-      const float chi_lon = d_dlon(d, mode, m, l, a.nl) * inv_lap(l);
-      // cos(lat) d/dlat at l: (l+2) eps(l+1) x_{l+1} - (l-1) eps(l) x_{l-1}
-      float psi_lat = 0.0f, chi_lat = 0.0f;
-      if (l + 1 < a.nl) {
-        const float c = (float)(l + 2) * eps_ml(m, l + 1) * inv_lap(l + 1);
-        psi_lat += c * z[mode * a.nl + l + 1];
-        chi_lat += c * d[mode * a.nl + l + 1];
-      }
-      if (l >= 1) {
-        const float c = -(float)(l - 1) * eps_ml(m, l) * inv_lap(l - 1);
-        psi_lat += c * z[mode * a.nl + l - 1];
-        chi_lat += c * d[mode * a.nl + l - 1];
-      }
-      u = (chi_lon - psi_lat) * a.inv_radius;
-      v = (chi_lat + psi_lon) * a.inv_radius;
-    }
-    a.out[(size_t)k * per + rem] = u;
-    a.out[(size_t)(a.kx + k) * per + rem] = v;
-    return;
-  }
-  float* dst = a.out + (size_t)(blockIdx.y + a.kx) * per + rem;
-  r -= a.kx;
-  for (int s = 0; s < 4; ++s) {
-    if (r < a.copy_count[s]) {
-      *dst = a.copy_src[s] ? a.copy_src[s][(size_t)r * per + rem] : 0.0f;
-      return;
-    }
-    r -= a.copy_count[s];
-  }
-  if (!a.geo || r >= a.kx) return;
-  // get_geopotential in modal space: the reference temperature enters the
-  // (mode 0, l 0) coefficient only.  Every level's load is issued before the
-  // sum (levels past kx re-read the last one and are not summed).
-  const int j = r;
-  float t[SPEEDY_SHT_KX_MAX];
+  for (int i2 = 0; i2 < N2; ++i2) x[i2] = x[i2] * sc + lvl;
+  if (sg.op & kOpExp) {
 #pragma unroll
-  for (int k = 0; k < SPEEDY_SHT_KX_MAX; ++k) t[k] = a.tvar[(size_t)min(k, a.kx - 1) * per + rem];
-  float acc = a.gravity * a.orography[rem];
+    for (int i2 = 0; i2 < N2; ++i2) x[i2] = expf(x[i2]);
+  }
 #pragma unroll
-  for (int k = 0; k < SPEEDY_SHT_KX_MAX; ++k) {
-    if (k < a.kx) {
-      float tk = t[k];
-      if (rem == 0) tk += a.reference[k] * kConstCoef;
-      acc += a.geo_w[j][k] * tk;
-    }
-  }
-  *dst = acc;
-}
-
-// Modal (U, V) = (u, v)/cos(lat) -> vorticity and divergence (curl_cos_lat,
-// div_cos_lat, clipped), then the remaining stacked rows to their destinations
-// (null source rows: zeros).  blockIdx.y is the row as in modal_winds_kernel:
-// rows below kx are the winds of that level, the others copy stacked row
-// blockIdx.y + kx.
-__global__ __launch_bounds__(kThreads) void modal_vordiv_kernel(ModalArgs a) {
-  const int per = a.mm * a.nl;
-  const int rem = blockIdx.x * kThreads + threadIdx.x;
-  if (rem >= per) return;
-  int r = blockIdx.y;
-  if (r < a.kx) {
-    const int k = r, mode = rem / a.nl, l = rem - mode * a.nl;
-    const int m = (mode + 1) >> 1;
-    const float* U = a.out + (size_t)k * per;
-    const float* V = a.out + (size_t)(a.kx + k) * per;
-    float z = 0.0f, d = 0.0f;
-    if (l < a.nl - 1) {
-      // sec(lat) d/dlat cos^2(lat) at l: l eps(l+1) x_{l+1} - (l+1) eps(l) x_{l-1}
-      float u_lat = 0.0f, v_lat = 0.0f;
-      if (l + 1 < a.nl) {
-        const float c = (float)l * eps_ml(m, l + 1);
-        u_lat += c * U[mode * a.nl + l + 1];
-        v_lat += c * V[mode * a.nl + l + 1];
-      }
-      if (l >= 1) {
-        const float c = -(float)(l + 1) * eps_ml(m, l);
-        u_lat += c * U[mode * a.nl + l - 1];
-        v_lat += c * V[mode * a.nl + l - 1];
-      }
-      z = (d_dlon(V, mode, m, l, a.nl) - u_lat) * a.inv_radius;
-      d = (d_dlon(U, mode, m, l, a.nl) + v_lat) * a.inv_radius;
-    }
-    a.vor_out[(size_t)k * per + rem] = z;
-    a.div_out[(size_t)k * per + rem] = d;
-    return;
-  }
-  const float* src = a.out + (size_t)(blockIdx.y + a.kx) * per + rem;
-  r -= a.kx;
-  for (int s = 0; s < 4; ++s) {
-    if (r < a.copy_count[s]) {
-      a.copy_dst[s][(size_t)r * per + rem] = a.copy_src[s] ? *src : 0.0f;
-      return;
-    }
-    r -= a.copy_count[s];
-  }
+  for (int i2 = 0; i2 < N2; ++i2) *at(dst, ((row + N1 * i2) * a.nlat + j) * 4u) = x[i2];
 }
 
 // ------------------------------------------------------------------ host side
@@ -1024,6 +1069,28 @@ int check_grid(int32_t n_m, int32_t n_l, int32_t nlon, int32_t nlat) {
   return SPEEDY_OK;
 }
 
+// The normalized P_l^m(x_j), l = 0 .. n_l - 1, of latitudes j < count: each(j, m, column).
+template <typename F>
+void legendre_columns(int32_t n_m, int32_t n_l, int32_t count, const double* x, F each) {
+  std::vector<double> col(n_l);
+  for (int j = 0; j < count; ++j) {
+    const double xj = x[j], yj = std::sqrt(1.0 - xj * xj);
+    double diag = 1.0 / std::sqrt(2.0);
+    for (int m = 0; m < n_m; ++m) {
+      if (m > 0) diag = -std::sqrt(1.0 + 1.0 / (2.0 * m)) * yj * diag;
+      std::fill(col.begin(), col.end(), 0.0);
+      col[m] = diag;
+      if (m + 1 < n_l) col[m + 1] = std::sqrt(2.0 * m + 3.0) * xj * diag;
+      for (int l = m + 2; l < n_l; ++l) {
+        const double a = std::sqrt((4.0 * l * l - 1.0) / ((double)l * l - (double)m * m));
+        const double b = std::sqrt(((l - 1.0) * (l - 1.0) - (double)m * m) / (4.0 * (l - 1.0) * (l - 1.0) - 1.0));
+        col[l] = a * (xj * col[l - 1] - b * col[l - 2]);
+      }
+      each(j, m, col.data());
+    }
+  }
+}
+
 void fill_basis(int32_t n_m, int32_t n_l, int32_t nlon, int32_t nlat, const double* x, float* fourier,
                 float* legendre) {
   const int mm = 2 * n_m - 1;
@@ -1038,50 +1105,46 @@ void fill_basis(int32_t n_m, int32_t n_l, int32_t nlon, int32_t nlat, const doub
     }
   }
   if (legendre) {
-    std::vector<double> col(n_l);
-    for (int j = 0; j < nlat; ++j) {
-      const double xj = x[j], yj = std::sqrt(1.0 - xj * xj);
-      double diag = 1.0 / std::sqrt(2.0);
-      for (int m = 0; m < n_m; ++m) {
-        if (m > 0) diag = -std::sqrt(1.0 + 1.0 / (2.0 * m)) * yj * diag;
-        std::fill(col.begin(), col.end(), 0.0);
-        col[m] = diag;
-        if (m + 1 < n_l) col[m + 1] = std::sqrt(2.0 * m + 3.0) * xj * diag;
-        for (int l = m + 2; l < n_l; ++l) {
-          const double a = std::sqrt((4.0 * l * l - 1.0) / ((double)l * l - (double)m * m));
-          const double b = std::sqrt(((l - 1.0) * (l - 1.0) - (double)m * m) / (4.0 * (l - 1.0) * (l - 1.0) - 1.0));
-          col[l] = a * (xj * col[l - 1] - b * col[l - 2]);
-        }
-        float* dst = legendre + ((size_t)m * nlat + j) * n_l;
-        for (int l = 0; l < n_l; ++l) dst[l] = (float)col[l];
-      }
-    }
+    legendre_columns(n_m, n_l, nlat, x, [&](int j, int m, const double* col) {
+      float* dst = legendre + ((size_t)m * nlat + j) * n_l;
+      for (int l = 0; l < n_l; ++l) dst[l] = (float)col[l];
+    });
   }
 }
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
+size_t y_bytes(const SpeedyShtPlan* p, int32_t nfield) {
+  return align256((size_t)nfield * p->n_m * p->nlat * sizeof(float2));
+}
+
+// LDS of the Legendre kernels: two parities of 16 staged rows, and the analysis's 16
+// modal rows where both fit kLegendreLds (two workgroups a CU; T425 takes 69 KiB).
+constexpr size_t kLegendreLds = 80 * 1024;
+constexpr int kMaxTiles = 30;   // staged at a time: 62 KiB
+size_t staged_lds(int kt) { return 2 * 16 * (size_t)lds_row(kt) * sizeof(float); }
+int tiles16(int n) { return (n + 15) / 16; }
+int analysis_kt(const SpeedyShtPlan* p) { return std::min(tiles16(p->nlat / 2), kMaxTiles); }
+int synthesis_kt(const SpeedyShtPlan* p) { return std::min(tiles16((p->n_l + 1) / 2), kMaxTiles); }
+size_t z_lds(const SpeedyShtPlan* p) { return 16 * (size_t)p->n_l * sizeof(float); }
+bool z_in_lds(const SpeedyShtPlan* p) { return staged_lds(analysis_kt(p)) + z_lds(p) <= kLegendreLds; }
+
+// The Y of a call; where the analysis's modal rows do not fit in LDS, also those of
+// every workgroup: with its zero rows a call has at most 5 / 4 nfield fields, in chunks
+// of four levels or eight fields.
 size_t ws_bytes(const SpeedyShtPlan* p, int32_t nfield) {
-  return align256((size_t)nfield * p->mm * p->nlat * 4) + align256((size_t)nfield * p->mm * p->n_l * 4);
+  const size_t z = z_in_lds(p) ? 0 : (((size_t)nfield + nfield / 4) / 8 + 2) * p->n_m * z_lds(p);
+  return y_bytes(p, nfield) + align256(z);
 }
 
-struct Ws {
-  float* y;   // [nfield][mm][nlat]: between the Fourier and Legendre stages
-  float* z;   // [nfield][mm][nl]: stacked modal fields
-};
-
-Ws carve(const SpeedyShtPlan* p, int32_t nfield, void* ws) {
-  char* b = static_cast<char*>(ws);
-  Ws r;
-  r.y = reinterpret_cast<float*>(b);
-  r.z = reinterpret_cast<float*>(b + align256((size_t)nfield * p->mm * p->nlat * 4));
-  return r;
-}
-
-StageArgs stage_args(const SpeedyShtPlan* p, int32_t nfield) {
-  StageArgs a{};
-  a.nlon = p->nlon; a.nlat = p->nlat; a.mm = p->mm; a.nl = p->n_l; a.nfield = nfield;
-  a.P = p->P;
+LegendreArgs legendre_args(const SpeedyShtPlan* p, int32_t nfield, void* ws) {
+  LegendreArgs a{};
+  a.n_m = p->n_m; a.nl = p->n_l; a.nlat = p->nlat; a.nfield = nfield;
+  a.blk = p->blk;
+  a.y = static_cast<float2*>(ws);
+  a.z = reinterpret_cast<float*>(static_cast<char*>(ws) + y_bytes(p, nfield));
+  a.inv_radius = (float)(1.0 / p->radius);
+  a.radius2 = (float)(p->radius * p->radius);
   return a;
 }
 
@@ -1089,24 +1152,27 @@ FourierArgs fourier_args(const SpeedyShtPlan* p, int32_t nfield, int32_t tl, con
   FourierArgs f{};
   f.nlon = p->nlon; f.nlat = p->nlat; f.mm = p->mm; f.n_m = p->n_m; f.n1 = p->n1; f.n2 = p->n2; f.tl = tl;
   f.nfield = nfield;
-  f.twr = p->tw; f.twi = p->tw + p->nlon; f.w = p->w; f.sec = p->sec;
+  f.twr = p->tw; f.twi = p->tw + p->nlon; f.sec = p->sec;
   f.seg = seg;
   return f;
 }
 
 // The Fourier kernels of one factor pair nlon = n1 * n2, compiled for the nlon of the
-// Grid.T<N> table, each with the latitudes a workgroup takes: 16 (64-byte rows) where
-// the exchange fits 64 KiB of LDS, which is everywhere but T340 and T425.  Other nlon
-// take the generic LDS kernels.
+// Grid.T<N> table, each with the latitudes a workgroup takes in the analysis and the
+// synthesis: 16 (64-byte rows), or 8 where a CU would hold too few (T213 conversions 56.3
+// us with 8 in the synthesis, 57.6 with 16; tendencies 41.2 with 16 in the analysis, 44.4
+// with 8; T425 272 and 229 us with 8, 302 and 261 with 4).  Other nlon take the generic
+// LDS kernels.
 typedef void (*FourierKernel)(FourierArgs);
 struct FourierPair {
-  int n1, n2, tl;
+  int n1, n2, tl_a, tl_s;
   FourierKernel analysis, synthesis;
 };
-#define SHT_PAIR(a, b, t) {a, b, t, fourier_analysis_kernel<a, b, t>, fourier_synthesis_kernel<a, b, t>}
-const FourierPair kPairs[] = {SHT_PAIR(8, 8, 16),   SHT_PAIR(8, 12, 16),  SHT_PAIR(8, 16, 16),  SHT_PAIR(16, 16, 16),
-                              SHT_PAIR(16, 20, 16), SHT_PAIR(18, 20, 16), SHT_PAIR(16, 32, 16), SHT_PAIR(20, 32, 16),
-                              SHT_PAIR(32, 32, 8),  SHT_PAIR(32, 40, 8)};
+#define SHT_PAIR(a, b, ta, ts) {a, b, ta, ts, fourier_analysis_kernel<a, b, ta>, fourier_synthesis_kernel<a, b, ts>}
+const FourierPair kPairs[] = {SHT_PAIR(8, 8, 16, 16),   SHT_PAIR(8, 12, 16, 16),  SHT_PAIR(8, 16, 16, 16),
+                              SHT_PAIR(16, 16, 16, 16), SHT_PAIR(16, 20, 16, 16), SHT_PAIR(18, 20, 16, 16),
+                              SHT_PAIR(16, 32, 16, 16), SHT_PAIR(20, 32, 16, 8),  SHT_PAIR(32, 32, 8, 8),
+                              SHT_PAIR(32, 40, 8, 8)};
 #undef SHT_PAIR
 
 const FourierPair* find_pair(int n1, int n2) {
@@ -1122,42 +1188,40 @@ size_t analysis_lds(int N, int n1, int n2, int tl) {
 }
 size_t synthesis_lds(int N, int mm, int tl) { return 4 * (2 * (size_t)N + 2 * (size_t)N * tl + (size_t)mm * tl); }
 
-int tiles(int M, int N) { return ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN); }
-
-hipError_t run_analysis(const SpeedyShtPlan* p, int32_t nfield, const SegTable& seg, float* y, float* modal_out,
-                        hipStream_t s) {
-  FourierArgs f = fourier_args(p, nfield, p->tl_a, seg);
-  f.out = y;
-  const FourierPair* fp = find_pair(p->n1, p->n2);
-  hipLaunchKernelGGL(fp ? fp->analysis : fourier_analysis_generic, dim3((p->nlat + p->tl_a - 1) / p->tl_a, nfield),
-                     dim3(fp ? fourier_threads(p->n1, p->n2, p->tl_a) : kThreads),
-                     fp ? 0 : analysis_lds(p->nlon, p->n1, p->n2, p->tl_a), s, f);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  StageArgs a = stage_args(p, nfield);
-  a.in = y;
-  a.out = modal_out;
-  hipLaunchKernelGGL(sht_gemm_kernel<kLegendreAnalysis>, dim3(tiles(nfield, (p->n_l + 1) / 2), 2 * p->mm),
-                     dim3(kThreads), 0, s, a);
+hipError_t run_fourier(const SpeedyShtPlan* p, int32_t nfield, const SegTable& seg, float2* y, bool analysis,
+                       hipStream_t s) {
+  const int tl = analysis ? p->tl_a : p->tl_s;
+  FourierArgs f = fourier_args(p, nfield, tl, seg);
+  f.y = y;
+  const dim3 grid((p->nlat + tl - 1) / tl, nfield);
+  if (const FourierPair* fp = find_pair(p->n1, p->n2))
+    hipLaunchKernelGGL(analysis ? fp->analysis : fp->synthesis, grid, dim3(fourier_threads(fp->n2, tl)),
+                       0, s, f);
+  else
+    hipLaunchKernelGGL(analysis ? fourier_analysis_generic : fourier_synthesis_generic, grid, dim3(kThreads),
+                       analysis ? analysis_lds(p->nlon, p->n1, p->n2, tl) : synthesis_lds(p->nlon, p->mm, tl), s, f);
   return hipGetLastError();
 }
 
-hipError_t run_synthesis(const SpeedyShtPlan* p, int32_t nfield, const SegTable& seg, const float* modal_in, float* y,
-                         hipStream_t s) {
-  StageArgs a = stage_args(p, nfield);
-  a.in = modal_in;
-  a.out = y;
-  hipLaunchKernelGGL(sht_gemm_kernel<kLegendreSynthesis>, dim3(tiles(nfield, p->nlat / 2), 2 * p->mm),
-                     dim3(kThreads), 0, s, a);
-  hipError_t e = hipGetLastError();
+dim3 legendre_grid(const LegendreArgs& a) { return dim3((a.n_m + 7) / 8 * 8 * chunks(a.winds, a.plain, a.geo)); }
+
+hipError_t run_analysis(const SpeedyShtPlan* p, int32_t nfield, const SegTable& seg, LegendreArgs a, hipStream_t s) {
+  const hipError_t e = run_fourier(p, nfield, seg, a.y, true, s);
   if (e != hipSuccess) return e;
-  FourierArgs f = fourier_args(p, nfield, p->tl_s, seg);
-  f.in = y;
-  const FourierPair* fp = find_pair(p->n1, p->n2);
-  hipLaunchKernelGGL(fp ? fp->synthesis : fourier_synthesis_generic, dim3((p->nlat + p->tl_s - 1) / p->tl_s, nfield),
-                     dim3(fp ? fourier_threads(p->n1, p->n2, p->tl_s) : kThreads),
-                     fp ? 0 : synthesis_lds(p->nlon, p->mm, p->tl_s), s, f);
+  a.P = p->Pa;
+  a.kt = analysis_kt(p);
+  const bool zlds = z_in_lds(p);
+  hipLaunchKernelGGL(zlds ? legendre_analysis_kernel<true> : legendre_analysis_kernel<false>, legendre_grid(a),
+                     dim3(kThreads), staged_lds(a.kt) + (zlds ? z_lds(p) : 0), s, a);
   return hipGetLastError();
+}
+
+hipError_t run_synthesis(const SpeedyShtPlan* p, int32_t nfield, const SegTable& seg, LegendreArgs a, hipStream_t s) {
+  a.P = p->Ps;
+  a.kt = synthesis_kt(p);
+  hipLaunchKernelGGL(legendre_synthesis_kernel, legendre_grid(a), dim3(kThreads), staged_lds(a.kt), s, a);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? e : run_fourier(p, nfield, seg, a.y, false, s);
 }
 
 void add_seg(SegTable& t, const float* src, float* dst, int32_t count, int32_t op, float mul,
@@ -1190,8 +1254,6 @@ int hip_result(hipError_t e) {
   return SPEEDY_OK;
 }
 
-int blocks(size_t n) { return (int)((n + kThreads - 1) / kThreads); }
-
 }  // namespace sht
 
 using namespace sht;
@@ -1220,7 +1282,7 @@ int speedy_sht_create(int32_t n_m, int32_t n_l, int32_t nlon, int32_t nlat, doub
     if (nlon % d == 0) n1 = d;
   const int n2 = nlon / n1;
   const FourierPair* fp = find_pair(n1, n2);
-  int tl_a = fp ? fp->tl : 16, tl_s = tl_a;
+  int tl_a = fp ? fp->tl_a : 16, tl_s = fp ? fp->tl_s : 16;
   if (!fp) {
     while (tl_a > 1 && analysis_lds(nlon, n1, n2, tl_a) > kFourierLds) --tl_a;
     while (tl_s > 1 && synthesis_lds(nlon, mm, tl_s) > kFourierLds) --tl_s;
@@ -1229,26 +1291,41 @@ int speedy_sht_create(int32_t n_m, int32_t n_l, int32_t nlon, int32_t nlat, doub
   }
   std::vector<double> x(nlat), w(nlat);
   gauss_nodes(nlat, x.data(), w.data());
-  std::vector<float> P((size_t)n_m * nlat * n_l), wf(nlat), sec(nlat), tw(2 * (size_t)nlon);
-  fill_basis(n_m, n_l, nlon, nlat, x.data(), nullptr, P.data());
-  for (int j = 0; j < nlat; ++j) {
-    wf[j] = (float)(w[j] * 2.0 * M_PI / nlon);
-    sec[j] = (float)(1.0 / std::sqrt(1.0 - x[j] * x[j]));
+  // operand blocks of the Legendre stages
+  const int h = nlat / 2, jts = tiles16(h);
+  std::vector<int32_t> blk(n_m);
+  int64_t nblk = 0;
+  for (int m = 0; m < n_m; ++m) {
+    blk[m] = (int32_t)nblk;
+    nblk += (int64_t)2 * tiles16((n_l - m + 1) / 2) * jts;
   }
+  std::vector<float> Ps((size_t)nblk * 256, 0.0f), Pa((size_t)nblk * 256, 0.0f), sec(nlat), tw(2 * (size_t)nlon);
+  legendre_columns(n_m, n_l, h, x.data(), [&](int j, int m, const double* col) {
+    const double f = 1.0 / std::sqrt(m == 0 ? 2.0 * M_PI : M_PI), wj = w[j] * 2.0 * M_PI / nlon;
+    const int cts = tiles16((n_l - m + 1) / 2);
+    for (int l = m; l < n_l; ++l) {
+      const int par = (l - m) & 1, c = (l - m) >> 1, ci = c & 15, ji = j & 15;
+      const size_t at = ((size_t)blk[m] + (size_t)(par * cts + c / 16) * jts + j / 16) * 256;
+      Ps[at + ((ci & 3) * 16 + ji) * 4 + (ci >> 2)] = (float)col[l];
+      Pa[at + ((ji >> 2) * 16 + ci) * 4 + (ji & 3)] = (float)(f * wj * col[l]);
+    }
+  });
+  for (int j = 0; j < nlat; ++j) sec[j] = (float)(1.0 / std::sqrt(1.0 - x[j] * x[j]));
   for (int j = 0; j < nlon; ++j) {
     tw[j] = (float)std::cos(2.0 * M_PI * j / nlon);
     tw[nlon + j] = (float)-std::sin(2.0 * M_PI * j / nlon);
   }
   SpeedyShtPlan* p = new SpeedyShtPlan{n_m, n_l, nlon, nlat, mm, radius, 0, n1, n2, tl_a, tl_s,
-                                       nullptr, nullptr, nullptr, nullptr};
+                                       nullptr, nullptr, nullptr, nullptr, nullptr};
   hipError_t e = hipGetDevice(&p->device);
-  auto up = [&](float** dst, const std::vector<float>& v) {
+  auto up = [&](auto** dst, const auto& v) {
     if (e != hipSuccess) return;
-    e = hipMalloc(reinterpret_cast<void**>(dst), v.size() * sizeof(float));
-    if (e == hipSuccess) e = hipMemcpy(*dst, v.data(), v.size() * sizeof(float), hipMemcpyHostToDevice);
+    e = hipMalloc(reinterpret_cast<void**>(dst), v.size() * sizeof(v[0]));
+    if (e == hipSuccess) e = hipMemcpy(*dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice);
   };
-  up(&p->P, P);
-  up(&p->w, wf);
+  up(&p->Ps, Ps);
+  up(&p->Pa, Pa);
+  up(&p->blk, blk);
   up(&p->sec, sec);
   up(&p->tw, tw);
   if (e != hipSuccess) {
@@ -1261,8 +1338,9 @@ int speedy_sht_create(int32_t n_m, int32_t n_l, int32_t nlon, int32_t nlat, doub
 
 int speedy_sht_destroy(SpeedyShtPlan* p) {
   if (!p) return SPEEDY_OK;
-  for (float* q : {p->P, p->w, p->sec, p->tw})
+  for (float* q : {p->Ps, p->Pa, p->sec, p->tw})
     if (q) (void)hipFree(q);
+  if (p->blk) (void)hipFree(p->blk);
   delete p;
   return SPEEDY_OK;
 }
@@ -1277,8 +1355,10 @@ int speedy_sht_to_modal(const SpeedyShtPlan* p, const float* nodal, float* modal
   if (!nodal || !modal) return fail(SPEEDY_ERR_ARG, "speedy_sht_to_modal: null field");
   SegTable seg{};
   add_seg(seg, nodal, nullptr, nfield, 0, 1.0f);
-  const Ws w = carve(p, nfield, ws);
-  return hip_result(run_analysis(p, nfield, seg, w.y, modal, static_cast<hipStream_t>(stream)));
+  LegendreArgs a = legendre_args(p, nfield, ws);
+  a.plain = a.count[0] = nfield;
+  a.dst[0] = modal;
+  return hip_result(run_analysis(p, nfield, seg, a, static_cast<hipStream_t>(stream)));
 }
 
 int speedy_sht_to_nodal(const SpeedyShtPlan* p, const float* modal, float* nodal, int32_t nfield, void* ws,
@@ -1287,8 +1367,10 @@ int speedy_sht_to_nodal(const SpeedyShtPlan* p, const float* modal, float* nodal
   if (!nodal || !modal) return fail(SPEEDY_ERR_ARG, "speedy_sht_to_nodal: null field");
   SegTable seg{};
   add_seg(seg, nullptr, nodal, nfield, 0, 1.0f);
-  const Ws w = carve(p, nfield, ws);
-  return hip_result(run_synthesis(p, nfield, seg, modal, w.y, static_cast<hipStream_t>(stream)));
+  LegendreArgs a = legendre_args(p, nfield, ws);
+  a.plain = a.count[0] = nfield;
+  a.src[0] = modal;
+  return hip_result(run_synthesis(p, nfield, seg, a, static_cast<hipStream_t>(stream)));
 }
 
 int speedy_dynamics_to_physics(const SpeedyShtPlan* p, const SpeedyDynamicsSpec* spec, const SpeedySpectralState* in,
@@ -1304,23 +1386,19 @@ int speedy_dynamics_to_physics(const SpeedyShtPlan* p, const SpeedyDynamicsSpec*
   const int nfield = 5 * kx + nsp;
   if (int rc = check_call(p, nfield, ws, wsb)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const Ws w = carve(p, nfield, ws);
-  // 1. modal (u cos, v cos), the other modal inputs and the modal geopotential,
-  //    stacked in z: rows [u kx][v kx][T_var kx][q kx][log ps nsp][phi kx]
-  ModalArgs m{};
-  m.mm = p->mm; m.nl = p->n_l; m.kx = kx;
-  m.inv_radius = (float)(1.0 / p->radius);
-  m.radius2 = (float)(p->radius * p->radius);
+  // 1. modal (u cos, v cos), the other modal inputs and the modal geopotential:
+  //    fields [u kx][v kx][T_var kx][q kx][log ps nsp][phi kx]
+  LegendreArgs m = legendre_args(p, nfield, ws);
+  m.kx = m.winds = m.geo = kx;
+  m.plain = 2 * kx + nsp;
   m.vor = in->vorticity; m.div = in->divergence;
-  m.copy_src[0] = in->temperature_variation; m.copy_count[0] = kx;
-  m.copy_src[1] = in->specific_humidity; m.copy_count[1] = kx;
-  m.copy_src[2] = in->log_surface_pressure; m.copy_count[2] = nsp;
-  m.out = w.z;
+  m.src[0] = in->temperature_variation; m.count[0] = kx;
+  m.src[1] = in->specific_humidity; m.count[1] = kx;
+  m.src[2] = in->log_surface_pressure; m.count[2] = nsp;
   m.tvar = in->temperature_variation;
   m.orography = spec->orography;
   m.reference = spec->reference_temperature;
   m.gravity = (float)spec->gravity;
-  m.geo = 1;
   // hydrostatic trapezoid on log(sigma): alpha_k = (ln s_k+1 - ln s_k)/2,
   // alpha_K-1 = -ln s_K-1; W[j][j] = alpha_j, W[j][k>j] = alpha_k + alpha_k-1
   std::vector<double> ls(kx), alpha(kx);
@@ -1330,9 +1408,6 @@ int speedy_dynamics_to_physics(const SpeedyShtPlan* p, const SpeedyDynamicsSpec*
   for (int j = 0; j < kx; ++j)
     for (int k = 0; k < kx; ++k)
       m.geo_w[j][k] = (float)(spec->gas_constant * (k < j ? 0.0 : k == j ? alpha[j] : alpha[k] + alpha[k - 1]));
-  const size_t per = (size_t)p->mm * p->n_l;
-  hipLaunchKernelGGL(modal_winds_kernel, dim3(blocks(per), nfield - kx), dim3(kThreads), 0, s, m);
-  if (int rc = hip_result(hipGetLastError())) return rc;
   // 2. synthesis with the nodal post-operations
   SegTable seg{};
   add_seg(seg, nullptr, out->u_wind, kx, kOpSecLat, 1.0f);
@@ -1341,7 +1416,7 @@ int speedy_dynamics_to_physics(const SpeedyShtPlan* p, const SpeedyDynamicsSpec*
   add_seg(seg, nullptr, out->specific_humidity, kx, 0, 1000.0f);
   add_seg(seg, nullptr, out->normalized_surface_pressure, nsp, kOpExp, 1.0f);
   add_seg(seg, nullptr, out->geopotential, kx, 0, 1.0f);
-  return hip_result(run_synthesis(p, nfield, seg, w.z, w.y, s));
+  return hip_result(run_synthesis(p, nfield, seg, m, s));
 }
 
 namespace {
@@ -1360,7 +1435,6 @@ int nodal_to_spectral(const SpeedyShtPlan* p, const SpeedyDynamicsSpec* spec, co
   const int nfield = 4 * kx + nsp_in;
   if (int rc = check_call(p, nfield, ws, wsb)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const Ws w = carve(p, nfield, ws);
   SegTable seg{};
   add_seg(seg, in->u_wind, nullptr, kx, kOpSecLat, 1.0f);
   add_seg(seg, in->v_wind, nullptr, kx, kOpSecLat, 1.0f);
@@ -1370,19 +1444,14 @@ int nodal_to_spectral(const SpeedyShtPlan* p, const SpeedyDynamicsSpec* spec, co
     add_seg(seg, in->temperature, nullptr, kx, kOpSubLevel, 1.0f, spec->reference_temperature, kx);
   add_seg(seg, in->specific_humidity, nullptr, kx, 0, 1e-3f);
   if (!tendency) add_seg(seg, in->normalized_surface_pressure, nullptr, nsp, kOpLog, 1.0f);
-  if (int rc = hip_result(run_analysis(p, nfield, seg, w.y, w.z, s))) return rc;
-  ModalArgs m{};
-  m.mm = p->mm; m.nl = p->n_l; m.kx = kx;
-  m.inv_radius = (float)(1.0 / p->radius);
-  m.radius2 = (float)(p->radius * p->radius);
-  m.out = w.z;
+  LegendreArgs m = legendre_args(p, nfield, ws);
+  m.kx = m.winds = kx;
+  m.plain = 2 * kx + nsp;
   m.vor_out = out->vorticity; m.div_out = out->divergence;
-  m.copy_src[0] = w.z; m.copy_count[0] = kx; m.copy_dst[0] = out->temperature_variation;
-  m.copy_src[1] = w.z; m.copy_count[1] = kx; m.copy_dst[1] = out->specific_humidity;
-  m.copy_src[2] = tendency ? nullptr : w.z; m.copy_count[2] = nsp; m.copy_dst[2] = out->log_surface_pressure;
-  const size_t per = (size_t)p->mm * p->n_l;
-  hipLaunchKernelGGL(modal_vordiv_kernel, dim3(blocks(per), 3 * kx + nsp), dim3(kThreads), 0, s, m);
-  return hip_result(hipGetLastError());
+  m.dst[0] = out->temperature_variation; m.count[0] = kx;
+  m.dst[1] = out->specific_humidity; m.count[1] = kx;
+  m.dst[2] = out->log_surface_pressure; m.count[2] = nsp;   // zeros for a tendency
+  return hip_result(run_analysis(p, nfield, seg, m, s));
 }
 }  // namespace
 
