@@ -1011,25 +1011,61 @@ __global__ __launch_bounds__(kBlock) void fwd_kernel(KArgs a) {
 // A batch descriptor holds one KArgs per segment and, per launch, a table of
 // (segment << 20 | block-in-segment) words; every block reads its word once and
 // then works exactly as in the single-call kernels.
+// A single call that the fused launch cannot take goes through the same kernels with no
+// table and its argument block by value, or, in the kernels that are short of registers
+// (sixteen levels, forward + VJP), in the workspace, written by the level-set launch.
+// (A launch of its own that wrote it and the tables cost 2.3 us and a gap.)
 constexpr uint32_t kSegShift = 20, kSegLocalMask = (1u << kSegShift) - 1u;
 
 template <int KX>
-__global__ __launch_bounds__(kBlock) void levelset_batch_kernel(const KArgs* __restrict__ segs,
-                                                                const uint32_t* __restrict__ table) {
+constexpr bool kByValue = KX <= 8;   // forward kernels
+
+// The workgroup's segment, and its block in it.  By value: either source is read-only
+// to the launch and read through address space 4, so that the fields are scalar loads
+// and move freely (T425 x 8 levels forward 97.8 -> 93.5 us, with the launch saved).
+// The descriptor alone, __restrict__ in the kernels' signatures: scalar loads next to
+// their use; through address space 4 they all move up and spill (64 members of T31 x
+// 16 levels forward 126.8 us against 118.2, T425 x 8 levels forward + VJP 278 against 217).
+template <int KX>
+__device__ __forceinline__ const KArgs& segment(const KArgs* segs, const uint32_t* table, uint32_t& bid) {
+  const uint32_t e = table ? __builtin_amdgcn_readfirstlane(table[blockIdx.x]) : blockIdx.x;
+  bid = e & kSegLocalMask;
+  if constexpr (kByValue<KX>) {
+    typedef const __attribute__((address_space(4))) KArgs* ConstPtr;
+    ConstPtr p = table ? (ConstPtr)segs + (e >> kSegShift) : (ConstPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    return *(const KArgs*)p;
+  } else {
+    return segs[e >> kSegShift];
+  }
+}
+
+// Copies a by-value argument block to memory, by one workgroup.
+__device__ __forceinline__ void write_desc(KArgs* dst) {
+  const auto* src = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
+  for (uint32_t w = threadIdx.x; w < (uint32_t)(sizeof(KArgs) / 4); w += kBlock)
+    gst(reinterpret_cast<uint32_t*>(dst), w, src[w]);
+}
+__global__ __launch_bounds__(kBlock) void desc_kernel(KArgs, KArgs* desc) { write_desc(desc); }
+
+// desc: where a single call's argument block goes that the next launch reads from memory.
+template <int KX>
+__global__ __launch_bounds__(kBlock) void levelset_batch_kernel(KArgs, const KArgs* segs, const uint32_t* table,
+                                                                KArgs* desc) {
   extern __shared__ uint32_t s_or[];
-  const uint32_t e = __builtin_amdgcn_readfirstlane(table[blockIdx.x]);
-  levelset_body<KX>(segs[e >> kSegShift], e & kSegLocalMask, s_or);
+  if (desc && blockIdx.x == 0) write_desc(desc);
+  uint32_t bid;
+  const KArgs& a = segment<8>(segs, table, bid);   // by value at every level count
+  levelset_body<KX>(a, bid, s_or);
 }
 
 // Forward-only segments of a batch: the forward without the adjoint's registers.
-// The descriptors are read-only and alias nothing the kernel writes
-// (__restrict__), so their fields are scalar loads and the field pointers read
-// from them are global-memory pointers.
 template <int KX>
-__global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_only_batch_kernel(const KArgs* __restrict__ segs,
-                                                                const uint32_t* __restrict__ table) {
-  const uint32_t e = __builtin_amdgcn_readfirstlane(table[blockIdx.x]);
-  fwd_body<KX, false, false, true>(segs[e >> kSegShift], e & kSegLocalMask);
+__global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_only_batch_kernel(KArgs,
+                                                                                 const KArgs* __restrict__ segs,
+                                                                                 const uint32_t* __restrict__ table) {
+  uint32_t bid;
+  const KArgs& a = segment<KX>(segs, table, bid);
+  fwd_body<KX, false, false, true>(a, bid);
 }
 
 // Forward-only segments of a batch in which none needs the verify steps or the
@@ -1038,19 +1074,22 @@ __global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_only_batch_kernel
 // levels (at most 256 registers a lane, no scratch): the second wave covers the
 // first one's stalls, 128 -> 86 us at T425 x 8 levels.
 template <int KX>
-__global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_plain_batch_kernel(const KArgs* __restrict__ segs,
-                                                                 const uint32_t* __restrict__ table) {
-  const uint32_t e = __builtin_amdgcn_readfirstlane(table[blockIdx.x]);
-  fwd_body<KX, false, false, false>(segs[e >> kSegShift], e & kSegLocalMask);
+__global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_plain_batch_kernel(KArgs,
+                                                                                  const KArgs* __restrict__ segs,
+                                                                                  const uint32_t* __restrict__ table) {
+  uint32_t bid;
+  const KArgs& a = segment<KX>(segs, table, bid);
+  fwd_body<KX, false, false, false>(a, bid);
 }
 
 // Forward-only segments that also write the PhysicsData diagnostics: single
 // calls with diagnostics that the fused launch cannot take.
 template <int KX>
-__global__ __launch_bounds__(kBlock) void fwd_diag_batch_kernel(const KArgs* __restrict__ segs,
+__global__ __launch_bounds__(kBlock) void fwd_diag_batch_kernel(KArgs, const KArgs* __restrict__ segs,
                                                                 const uint32_t* __restrict__ table) {
-  const uint32_t e = __builtin_amdgcn_readfirstlane(table[blockIdx.x]);
-  fwd_body<KX, true, false, true>(segs[e >> kSegShift], e & kSegLocalMask);
+  uint32_t bid;
+  const KArgs& a = segment<KX>(segs, table, bid);
+  fwd_body<KX, true, false, true>(a, bid);
 }
 
 // Forward + VJP segments of a batch.  Bound by VALU issue.  Built for two waves per
@@ -1059,12 +1098,12 @@ __global__ __launch_bounds__(kBlock) void fwd_diag_batch_kernel(const KArgs* __r
 // of scratch).  T425 x 8 levels: 412 -> 195 us, and 64 members of T31 x 16 levels:
 // 2710 -> 275 us, against reversing every term from a recompute of its own
 // (speedy_adjoint.hpp).  The descriptor is __restrict__, so uniforms are scalar
-// loads next to their use (without it, vector loads: 310 us at T425).  The fused
-// kernel keeps one wave per SIMD and no scratch.
+// loads next to their use (vector loads without it: 310 us at T425).  The fused kernel
+// keeps one wave per SIMD and no scratch.
 template <int KX>
 __global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_batch_kernel(const KArgs* __restrict__ segs,
-                                                                        const uint32_t* __restrict__ table) {
-  const uint32_t e = __builtin_amdgcn_readfirstlane(table[blockIdx.x]);
+                                                                            const uint32_t* __restrict__ table) {
+  const uint32_t e = table ? __builtin_amdgcn_readfirstlane(table[blockIdx.x]) : blockIdx.x;
   vjp_body<KX, false>(segs[e >> kSegShift], e & kSegLocalMask);
 }
 
@@ -1072,20 +1111,6 @@ __global__ __launch_bounds__(kBlock) void param_reduce_batch_kernel(const KArgs*
                                                                     const uint32_t* __restrict__ table) {
   const uint32_t e = __builtin_amdgcn_readfirstlane(table[blockIdx.x]);
   member_reduce_body(segs[e >> kSegShift], e & kSegLocalMask);
-}
-
-// The call's arguments as a one-segment batch in the workspace: block 0 copies the
-// argument block word by word; every thread writes one table entry (the block-,
-// level-set-block- and member-tables in turn, each counting from 0).
-__global__ __launch_bounds__(kBlock) void seg_desc_kernel(KArgs a, KArgs* dst, uint32_t* tbl, uint32_t nblk,
-                                                          uint32_t nls, uint32_t nred) {
-  if (blockIdx.x == 0) {
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(&a);
-    uint32_t* d = reinterpret_cast<uint32_t*>(dst);
-    for (uint32_t w = threadIdx.x; w < (uint32_t)(sizeof(KArgs) / 4); w += kBlock) d[w] = src[w];
-  }
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i < nblk + nls + nred) tbl[i] = i < nblk ? i : (i < nblk + nls ? i - nblk : i - nblk - nls);
 }
 
 // acc[e] += diag[e] / steps for e < n (the diagnostics' running mean): four
@@ -1174,7 +1199,7 @@ Grid make_grid(int64_t nlon, int64_t nlat, int64_t nmember) {
 }
 
 struct WsLayout {
-  size_t last_s, partial, prm, bud, desc, tbl, total;
+  size_t last_s, partial, prm, bud, desc, total;
 };
 
 WsLayout ws_layout(const Grid& g, int32_t nmember) {
@@ -1187,9 +1212,7 @@ WsLayout ws_layout(const Grid& g, int32_t nmember) {
   L.bud = L.prm + align256(sizeof(float) * nprm);
   const size_t nbud = g.ncol >= (uint32_t)kBlock ? (size_t)g.nblk * 2 * kBudParts : (size_t)g.ntot * kBudParts;
   L.desc = L.bud + align256(sizeof(double) * nbud);
-  // one-segment batch descriptor and its block tables, for grids the fused launch cannot take
-  L.tbl = L.desc + align256(sizeof(KArgs));
-  L.total = L.tbl + align256(sizeof(uint32_t) * ((size_t)g.nblk + g.ls_blocks + (size_t)nmember));
+  L.total = L.desc + align256(sizeof(KArgs));   // a single call's argument block
   return L;
 }
 
@@ -1329,48 +1352,33 @@ int launch_fwd(const KArgs& a, hipStream_t s) {
     timer_end(s, slot);
   } else {
     // Grids the fused launch cannot take (beyond one co-resident launch, members
-    // narrower than a workgroup, or a given level set) run as a one-segment batch
-    // through the batch kernels; the workspace holds the descriptor and tables.
-    if (a.nblk > kSegLocalMask || a.ls_blocks > kSegLocalMask)
+    // narrower than a workgroup, or a given level set): the batch kernels on this one
+    // call.
+    if (a.nblk > kSegLocalMask)
       return fail(SPEEDY_ERR_CAPACITY, "speedy: more than 2^20 workgroups (2^28 columns) in one call");
     const WsLayout L = ws_layout(make_grid(a.ncol, 1, a.nmember), (int32_t)a.nmember);
-    char* w = reinterpret_cast<char*>(a.gen);
-    KArgs* d_args = reinterpret_cast<KArgs*>(w + L.desc);
-    uint32_t* tbl = reinterpret_cast<uint32_t*>(w + L.tbl);
-    const uint32_t nls = a.level_set < 0 ? a.ls_blocks : 0u;
-    const uint32_t nred = (VJP || a.f.budget) ? a.nmember : 0u;
-    const uint32_t n = a.nblk + nls + nred;
-    hipLaunchKernelGGL(seg_desc_kernel, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, a, d_args, tbl, a.nblk,
-                       nls, nred);
-    if (nls) {
+    KArgs* desc = VJP || !kByValue<KX> ? reinterpret_cast<KArgs*>(reinterpret_cast<char*>(a.gen) + L.desc) : nullptr;
+    const KArgs* segs = desc;
+    const uint32_t* table = nullptr;
+    if (a.level_set < 0) {
       const int slot = timer_begin(s, 0);
-      hipLaunchKernelGGL(levelset_batch_kernel<KX>, dim3(nls), dim3(kBlock), a.jmax * sizeof(uint32_t), s,
-                         (const KArgs*)d_args, (const uint32_t*)(tbl + a.nblk));
+      hipLaunchKernelGGL(levelset_batch_kernel<KX>, dim3(a.ls_blocks), dim3(kBlock), a.jmax * sizeof(uint32_t), s, a,
+                         segs, table, desc);
       timer_end(s, slot);
+    } else if (desc) {
+      hipLaunchKernelGGL(desc_kernel, dim3(1), dim3(kBlock), 0, s, a, desc);
     }
     const int slot = timer_begin(s, kind);
     if (VJP)
-      hipLaunchKernelGGL(fwd_batch_kernel<KX>, dim3(a.nblk), dim3(kBlock), 0, s, (const KArgs*)d_args,
-                         (const uint32_t*)tbl);
+      hipLaunchKernelGGL(fwd_batch_kernel<KX>, dim3(a.nblk), dim3(kBlock), 0, s, segs, table);
     else if (DIAG)
-      hipLaunchKernelGGL(fwd_diag_batch_kernel<KX>, dim3(a.nblk), dim3(kBlock), 0, s, (const KArgs*)d_args,
-                         (const uint32_t*)tbl);
+      hipLaunchKernelGGL(fwd_diag_batch_kernel<KX>, dim3(a.nblk), dim3(kBlock), 0, s, a, segs, table);
     else if (EXTRA)
-      hipLaunchKernelGGL(fwd_only_batch_kernel<KX>, dim3(a.nblk), dim3(kBlock), 0, s, (const KArgs*)d_args,
-                         (const uint32_t*)tbl);
+      hipLaunchKernelGGL(fwd_only_batch_kernel<KX>, dim3(a.nblk), dim3(kBlock), 0, s, a, segs, table);
     else
-      hipLaunchKernelGGL(fwd_plain_batch_kernel<KX>, dim3(a.nblk), dim3(kBlock), 0, s, (const KArgs*)d_args,
-                         (const uint32_t*)tbl);
-    timer_end(s, slot);
-    if (nred) {
-      const int slot2 = timer_begin(s, 3);
-      hipLaunchKernelGGL(param_reduce_batch_kernel, dim3(nred), dim3(kBlock), 0, s, (const KArgs*)d_args,
-                         (const uint32_t*)(tbl + a.nblk + nls));
-      timer_end(s, slot2);
-    }
+      hipLaunchKernelGGL(fwd_plain_batch_kernel<KX>, dim3(a.nblk), dim3(kBlock), 0, s, a, segs, table);
     e = hipGetLastError();
-    if (e != hipSuccess) return fail(SPEEDY_ERR_HIP, std::string("speedy: launch failed: ") + hipGetErrorString(e));
-    return SPEEDY_OK;
+    timer_end(s, slot);
   }
   // Per-member sums in a second small kernel.  (Summing them in the last block to
   // finish instead, after an agent-scope fence per block, cost more than this
@@ -1590,19 +1598,22 @@ int speedy_fwd_batch(const SpeedySegment* segs, int32_t nseg, const SpeedyVertic
   // function-local static: thread-safe); a failure fails every batch call.
   static const hipError_t stack_err[3] = {
       batch_stack<7>(), batch_stack<8>(), batch_stack<16>()};
+  KArgs none;   // the kernels take a call's arguments by value or from the descriptor
+  std::memset(&none, 0, sizeof(none));
   auto launch = [&](auto ls_kernel, auto fwd_only_b, auto fwd_plain_b, auto fwd_kernel_b, int kxi) -> hipError_t {
     if (stack_err[kxi] != hipSuccess) return stack_err[kxi];
     if (nl) {
       const int slot = timer_begin(s, 0);
-      hipLaunchKernelGGL(ls_kernel, dim3(nl), dim3(kBlock), jmax * sizeof(uint32_t), s, d_args, d_ls);
+      hipLaunchKernelGGL(ls_kernel, dim3(nl), dim3(kBlock), jmax * sizeof(uint32_t), s, none, d_args, d_ls,
+                         (KArgs*)nullptr);
       timer_end(s, slot);
     }
     if (nbf) {
       const int slot = timer_begin(s, 1);
       if (fwd_extra)
-        hipLaunchKernelGGL(fwd_only_b, dim3(nbf), dim3(kBlock), 0, s, d_args, d_blk);
+        hipLaunchKernelGGL(fwd_only_b, dim3(nbf), dim3(kBlock), 0, s, none, d_args, d_blk);
       else
-        hipLaunchKernelGGL(fwd_plain_b, dim3(nbf), dim3(kBlock), 0, s, d_args, d_blk);
+        hipLaunchKernelGGL(fwd_plain_b, dim3(nbf), dim3(kBlock), 0, s, none, d_args, d_blk);
       timer_end(s, slot);
     }
     if (nbv) {
