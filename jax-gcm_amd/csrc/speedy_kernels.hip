@@ -796,14 +796,14 @@ __device__ __forceinline__ void fwd_body(const KArgs& a, uint32_t bid) {
 // shortwave reversed from their own tapes): nothing of phase B is computed twice
 // but the up sweep's transmissivities, and the tendencies are the forward
 // kernels' bit for bit.  The longwave tape lies in LDS, [slot][thread].
-template <int KX, bool FUSED>
+template <int KX, bool FUSED, bool STASH = !FUSED>
 __device__ __forceinline__ void vjp_body(const KArgs& a, uint32_t bid) {
   // Values of phase A that phase B does not read wait in LDS (tvd, qsat and, up to
   // eight levels, rh above the top level) or are read again from memory (phi, dL/ddq), in
   // the kernels whose registers are short: the batched ones (two waves per SIMD at 7 and 8
   // levels, 79 floats a column with the tape: two blocks fill a CU's 160 KB).
   constexpr int kTape = vjp_tape_floats<KX>();
-  constexpr bool kStash = !FUSED;
+  constexpr bool kStash = STASH;
   constexpr int kStashRh = KX <= 8 ? KX - 1 : 0;
   __shared__ float s_tape[(kTape + (kStash ? 2 * KX + kStashRh : 0)) * kBlock];
   LdsStore tape{s_tape + threadIdx.x};
@@ -1107,6 +1107,25 @@ __global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_batch_kernel(cons
   vjp_body<KX, false>(segs[e >> kSegShift], e & kSegLocalMask);
 }
 
+// Batches of 7 or 8 levels whose blocks are co-resident (at most 512 of them, two a CU):
+// the single-launch bodies on every segment, so the level sets are gathered in the
+// launch and forward and forward + VJP segments run side by side.  Bound by the latency
+// of its longest block, an adjoint's.  Built for two waves per SIMD as fwd_batch_kernel
+// is (a block a CU would hold T85 twice).  Six requests from T21 to T85 (346 blocks):
+// 32.5 us against 6.4 + 13.3 + 26.7 us and two gaps in the launches below, 216 -> 200 us
+// a burst; four of T85 (512 blocks) 178 -> 165, all forward 122 -> 119.  Beyond that the
+// kernels below have the higher occupancy or the leaner forward.
+template <int KX>
+__global__ __launch_bounds__(kBlock, 2) void small_batch_kernel(const KArgs* __restrict__ segs,
+                                                             const uint32_t* __restrict__ table) {
+  const uint32_t e = __builtin_amdgcn_readfirstlane(table[blockIdx.x]);
+  const KArgs& a = segs[e >> kSegShift];
+  if (a.adj.g_t)
+    vjp_body<KX, true, true>(a, e & kSegLocalMask);
+  else
+    fwd_body<KX, false, true, true>(a, e & kSegLocalMask);
+}
+
 __global__ __launch_bounds__(kBlock) void param_reduce_batch_kernel(const KArgs* __restrict__ segs,
                                                                     const uint32_t* __restrict__ table) {
   const uint32_t e = __builtin_amdgcn_readfirstlane(table[blockIdx.x]);
@@ -1315,6 +1334,11 @@ int64_t coresident_blocks(K kernel) {
   if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock, 0) != hipSuccess) return 0;
   return (int64_t)per_cu * ncu;
+}
+
+template <int KX>
+int64_t small_batch_blocks() {
+  return ensure_stack(small_batch_kernel<KX>) == hipSuccess ? coresident_blocks(small_batch_kernel<KX>) : 0;
 }
 
 // One-time set-up of a kernel family: the stack limit its kernels need and the
@@ -1549,6 +1573,17 @@ int speedy_fwd_batch(const SpeedySegment* segs, int32_t nseg, const SpeedyVertic
   uint32_t* t_blk = reinterpret_cast<uint32_t*>(h + L.blk);
   uint32_t* t_ls = reinterpret_cast<uint32_t*>(h + L.ls);
   uint32_t* t_red = reinterpret_cast<uint32_t*>(h + L.red);
+  // Co-resident, at 7 or 8 levels and with no member narrower than a workgroup: one
+  // launch of small_batch_kernel (there both sides are measured).
+  static const int64_t small_cap[2] = {small_batch_blocks<7>(), small_batch_blocks<8>()};
+  int64_t blocks = 0;
+  bool small = vert && (vert->kx == 7 || vert->kx == 8);
+  for (int32_t i = 0; i < nseg; ++i) {
+    const Grid g = make_grid(segs[i].nlon, segs[i].nlat, segs[i].nmember);
+    blocks += g.nblk;
+    small = small && g.ncol >= (uint32_t)kBlock;
+  }
+  small = small && blocks <= small_cap[vert->kx - 7];
   uint32_t nb = 0, nl = 0, nr = 0, jmax = 1;
   bool fwd_extra = false;   // a forward-only segment needs the verify steps or budgets
   std::vector<uint8_t> is_vjp((size_t)nseg, 0u);
@@ -1569,7 +1604,7 @@ int speedy_fwd_batch(const SpeedySegment* segs, int32_t nseg, const SpeedyVertic
     std::memcpy(&ha[i], &a, sizeof(KArgs));
     is_vjp[i] = nset != 0;
     if (!nset && needs_extra(a)) fwd_extra = true;
-    if (a.level_set < 0) {
+    if (a.level_set < 0 && !small) {
       for (uint32_t b = 0; b < a.ls_blocks; ++b) t_ls[nl++] = ((uint32_t)i << kSegShift) | b;
       jmax = std::max(jmax, a.jmax);
     }
@@ -1584,7 +1619,7 @@ int speedy_fwd_batch(const SpeedySegment* segs, int32_t nseg, const SpeedyVertic
   uint32_t nbf = 0;
   for (int32_t i = 0; i < nseg; ++i)
     if (!is_vjp[i]) nbf += ha[i].nblk;
-  const uint32_t nbv = nb - nbf;
+  uint32_t nbv = nb - nbf;
   g_last_error.clear();
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = hipMemcpyAsync(desc, host_staging, L.total, hipMemcpyHostToDevice, s);
@@ -1600,8 +1635,15 @@ int speedy_fwd_batch(const SpeedySegment* segs, int32_t nseg, const SpeedyVertic
       batch_stack<7>(), batch_stack<8>(), batch_stack<16>()};
   KArgs none;   // the kernels take a call's arguments by value or from the descriptor
   std::memset(&none, 0, sizeof(none));
-  auto launch = [&](auto ls_kernel, auto fwd_only_b, auto fwd_plain_b, auto fwd_kernel_b, int kxi) -> hipError_t {
+  auto launch = [&](auto ls_kernel, auto fwd_only_b, auto fwd_plain_b, auto fwd_kernel_b, auto small_b,
+                    int kxi) -> hipError_t {
     if (stack_err[kxi] != hipSuccess) return stack_err[kxi];
+    if (small) {
+      const int slot = timer_begin(s, nbv ? 2 : 1);
+      hipLaunchKernelGGL(small_b, dim3(nb), dim3(kBlock), 0, s, d_args, d_blk);
+      timer_end(s, slot);
+      nbf = nbv = 0;
+    }
     if (nl) {
       const int slot = timer_begin(s, 0);
       hipLaunchKernelGGL(ls_kernel, dim3(nl), dim3(kBlock), jmax * sizeof(uint32_t), s, none, d_args, d_ls,
@@ -1631,14 +1673,16 @@ int speedy_fwd_batch(const SpeedySegment* segs, int32_t nseg, const SpeedyVertic
   hipError_t le;
   switch (vert->kx) {
     case 7:
-      le = launch(levelset_batch_kernel<7>, fwd_only_batch_kernel<7>, fwd_plain_batch_kernel<7>, fwd_batch_kernel<7>, 0);
+      le = launch(levelset_batch_kernel<7>, fwd_only_batch_kernel<7>, fwd_plain_batch_kernel<7>, fwd_batch_kernel<7>,
+                  small_batch_kernel<7>, 0);
       break;
     case 8:
-      le = launch(levelset_batch_kernel<8>, fwd_only_batch_kernel<8>, fwd_plain_batch_kernel<8>, fwd_batch_kernel<8>, 1);
+      le = launch(levelset_batch_kernel<8>, fwd_only_batch_kernel<8>, fwd_plain_batch_kernel<8>, fwd_batch_kernel<8>,
+                  small_batch_kernel<8>, 1);
       break;
     default:
       le = launch(levelset_batch_kernel<16>, fwd_only_batch_kernel<16>, fwd_plain_batch_kernel<16>,
-                  fwd_batch_kernel<16>, 2);
+                  fwd_batch_kernel<16>, fwd_batch_kernel<16>, 2);
       break;
   }
   if (le != hipSuccess) return fail(SPEEDY_ERR_HIP, std::string("speedy_fwd_batch: stack limit: ") + hipGetErrorString(le));
