@@ -59,6 +59,8 @@ struct Divisor {          // n / d for n < 2^32 by multiply-high + one correctio
   uint32_t d, m;          // m = floor(2^32 / d) (unused when d == 1)
 };
 
+constexpr uint32_t kArrivedWord = 2, kMergedMembers = 62;   // words of the workspace's header
+
 struct KArgs {
   SpeedyFields f;
   SpeedyVertical v;
@@ -73,6 +75,8 @@ struct KArgs {
   uint32_t *gen, *err, *last_s, *partial;
   // fused forward + VJP only
   SpeedyAdjoint adj;
+  uint32_t* arrived;                 // per member: blocks whose partials are out (zero between calls)
+  uint32_t merged;                   // a fused call's members are summed in the launch (fused_sums)
   float* prm_part;                   // parameter-gradient partials (per block and member slot, or per column)
   double* bud_part;                  // float64 budget partials (same layout, kBudParts doubles each)
 };
@@ -481,6 +485,19 @@ __device__ __forceinline__ void levelset_body(const KArgs& a, uint32_t bid, uint
   for (uint32_t i = threadIdx.x; i < nm; i += kBlock) gst(a.partial, bid * a.jmax + i, s_or[i]);
 }
 
+// Where a block's columns lie and what it knows of its members' level sets.
+// Threads past the last column take the last column and do all its work, its
+// stores included (the same values to the same addresses), so no store needs a
+// branch; only the block sums leave them out.
+struct BlockPos {
+  uint32_t gid, m, c;       // global column, member and column of this thread
+  bool active, wide;        // wide: a member is at least a block, so a block spans at most two members
+  uint32_t m_first, nm;     // the block's first member and how many it spans
+  uint32_t wave;            // this wave's index in the block, as a scalar: branches on it keep all lanes on
+  uint32_t gen, tag;        // fused: the generation word and the call's tag
+  uint32_t lw0, lw1;        // two launches: this thread's share of the members' chunk words
+};
+
 // ---------------------------------------------------------------- VJP helpers
 // One column's slice of an LDS array laid out [slot][thread] (conflict-free).
 struct LdsStore {
@@ -553,30 +570,42 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
 
 // Parameter gradients of this block: a fixed-order tree sum per member slot
 // (deterministic), written to prm_part[block][slot][5].  Members narrower than
-// a block write per-column values instead (prm_part[column][5]).
-__device__ __forceinline__ void block_param_partials(const KArgs& a, uint32_t bid, uint32_t gid, bool active,
-                                                     uint32_t slot, const float prm[VJP_NPARAM]) {
-  if (a.ncol < (uint32_t)kBlock) {
-    if (active)
+// a block write per-column values instead (prm_part[column][5]).  TAGGED: as
+// tagged_word(tag, value), for the block that sums the member in the same launch.
+__device__ __forceinline__ uint64_t tagged_word(uint32_t tag, float v) {
+  return (uint64_t)tag << 32 | __builtin_bit_cast(uint32_t, v);
+}
+template <bool TAGGED>
+__device__ __forceinline__ void block_param_partials(const KArgs& a, uint32_t bid, const BlockPos& b,
+                                                     const float prm[VJP_NPARAM]) {
+  if (!TAGGED && a.ncol < (uint32_t)kBlock) {
+    if (b.active)
 #pragma unroll
-      for (int i = 0; i < VJP_NPARAM; ++i) gst(a.prm_part, (size_t)gid * VJP_NPARAM + i, prm[i]);
+      for (int i = 0; i < VJP_NPARAM; ++i) gst(a.prm_part, (size_t)b.gid * VJP_NPARAM + i, prm[i]);
     return;
   }
   __shared__ float s_red[kBlock / 64][2 * VJP_NPARAM];
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+  const uint32_t lane = threadIdx.x & 63u, slot = b.m - b.m_first;
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < 2; ++j) {
+    if (j > 0 && b.nm == 1u) break;   // uniform
 #pragma unroll
     for (int i = 0; i < VJP_NPARAM; ++i) {
-      const float v = wave_sum((active && slot == (uint32_t)j) ? prm[i] : 0.0f);
-      if (lane == 0) s_red[wave][j * VJP_NPARAM + i] = v;
+      const float v = wave_sum((b.active && slot == (uint32_t)j) ? prm[i] : 0.0f);
+      if (lane == 0) s_red[b.wave][j * VJP_NPARAM + i] = v;
     }
+  }
   __syncthreads();
-  if (threadIdx.x < 2 * VJP_NPARAM) {
+  if (threadIdx.x < b.nm * VJP_NPARAM) {
     float acc = s_red[0][threadIdx.x];
 #pragma unroll
     for (int w = 1; w < kBlock / 64; ++w) acc = acc + s_red[w][threadIdx.x];
-    gst(a.prm_part, (size_t)bid * 2 * VJP_NPARAM + threadIdx.x, acc);
+    const size_t at = (size_t)bid * 2 * VJP_NPARAM + threadIdx.x;
+    if constexpr (TAGGED)
+      __hip_atomic_store(reinterpret_cast<uint64_t*>(a.prm_part) + at, tagged_word(b.gen + 1u, acc), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    else
+      gst(a.prm_part, at, acc);
   }
 }
 
@@ -642,19 +671,6 @@ __device__ __forceinline__ auto tau_store(float* s) {
     return NoTauStore{};
 }
 
-// Where a block's columns lie and what it knows of its members' level sets.
-// Threads past the last column take the last column and do all its work, its
-// stores included (the same values to the same addresses), so no store needs a
-// branch; only the block sums leave them out.
-struct BlockPos {
-  uint32_t gid, m, c;       // global column, member and column of this thread
-  bool active, wide;        // wide: a member is at least a block, so a block spans at most two members
-  uint32_t m_first, nm;     // the block's first member and how many it spans
-  uint32_t wave;            // this wave's index in the block, as a scalar: branches on it keep all lanes on
-  uint32_t gen, tag;        // fused: the generation word and the call's tag
-  uint32_t lw0, lw1;        // two launches: this thread's share of the members' chunk words
-};
-
 // The thread's position, and the loads the level set needs, issued first so that
 // their round trip overlaps the state's: the generation word (fused), or the level-set
 // chunk words (a member wider than a block: each thread ORs its share of the
@@ -709,10 +725,26 @@ __device__ __forceinline__ void publish_level_bits(const KArgs& a, uint32_t bid,
   }
 }
 
+// Counts the block in for its members' sums (by one wave): s_last[j] becomes whether it
+// is the last of member m_first + j.
+__device__ __forceinline__ void count_in(const KArgs& a, const BlockPos& b, uint32_t* s_last) {
+  for (uint32_t j = 0; j < b.nm; ++j) {
+    const uint32_t m = b.m_first + j;
+    const uint32_t n = (m * a.ncol + a.ncol - 1u) / kBlock - (m * a.ncol) / kBlock + 1u;
+    uint32_t before = 0u;
+    if ((threadIdx.x & 63u) == 0u)
+      before = __hip_atomic_fetch_add(&a.arrived[m], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool last = __builtin_amdgcn_readfirstlane(before) == n - 1u;
+    if (last) __hip_atomic_store(&a.arrived[m], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last[j] = last;
+  }
+}
+
 // The level set of this thread's member: gathered from the published words
 // (fused) or from the chunk words (two launches), or the call's own.
-template <int KX, bool FUSED>
-__device__ __forceinline__ uint32_t gather_level_set(const KArgs& a, uint32_t bid, const BlockPos& b) {
+template <int KX, bool FUSED, bool SUMS = false>
+__device__ __forceinline__ uint32_t gather_level_set(const KArgs& a, uint32_t bid, const BlockPos& b,
+                                                     uint32_t* s_last = nullptr) {
   if (a.level_set >= 0) return (uint32_t)a.level_set;
   if (FUSED) {
     __shared__ uint32_t s_s[2];
@@ -720,6 +752,8 @@ __device__ __forceinline__ uint32_t gather_level_set(const KArgs& a, uint32_t bi
       for (uint32_t j = 0; j < b.nm; ++j) s_s[j] = collect_fused<KX>(a, b.tag, b.m_first + j);
     } else if (b.wave == 1u && bid == 0u) {
       finish_generation(a, b.gen, b.tag);   // no other block waits for this one here: it has published
+    } else if (SUMS && b.wave == 2u && a.merged) {
+      count_in(a, b, s_last);
     }
     __syncthreads();
     return s_s[b.m - b.m_first];
@@ -752,12 +786,12 @@ __device__ __forceinline__ void column_budgets(const KArgs& a, uint32_t bid, con
   block_budget_partials(a, bid, b.gid, b.active, b.m - b.m_first, v);
 }
 
-// The launch's by-value argument block, read again from the argument segment: what
-// follows loads its uniforms anew (scalar loads) where the scalar registers could not
-// hold them from kernel entry and would spill them lane by lane into vector registers.
-__device__ __forceinline__ const KArgs& reread() {
+// The argument block (the launch's own, or a descriptor) read again: what follows loads
+// its uniforms anew (scalar loads) where the scalar registers could not hold them from
+// kernel entry and would spill them lane by lane into vector registers.
+__device__ __forceinline__ const KArgs& reread(const void* args) {
   typedef const __attribute__((address_space(4))) KArgs* ConstPtr;
-  ConstPtr p = (ConstPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  ConstPtr p = (ConstPtr)args;
   asm volatile("" : "+s"(p));
   return *(const KArgs*)p;
 }
@@ -783,11 +817,136 @@ __device__ __forceinline__ void fwd_body(const KArgs& a, uint32_t bid) {
   // with every output compiled in, the uniforms of phase b2 and the stores are read
   // again (T85 with diagnostics and verify: 17.2 -> 16.2 us; the plain forward is
   // 0.4 us slower that way)
-  const KArgs& o = FUSED && DIAG && EXTRA ? reread() : a;
+  const KArgs& o = FUSED && DIAG && EXTRA ? reread((const void*)__builtin_amdgcn_kernarg_segment_ptr()) : a;
   phase_b2<float, KX, DIAG>(col, pa, S, o.p, o.v, o.u, o.flags, pb, ts);
   double colsum[2] = {0.0, 0.0};
   store_outputs<KX, DIAG, EXTRA>(o, b.m, b.c, col, pa, pb, tend_t, tend_q, colsum);
   if (EXTRA && a.f.budget) column_budgets<KX>(o, bid, b, pa, pb, colsum);
+}
+
+// Per-member parameter gradients from the partials, one block per member, in a
+// fixed order (deterministic).
+__device__ __forceinline__ void budget_reduce_body(const KArgs& a, uint32_t m) {
+  double acc[kBudParts];
+#pragma unroll
+  for (int i = 0; i < kBudParts; ++i) acc[i] = 0.0;
+  // (unrolled: several iterations' loads in flight; the order of the sums is the loop's)
+  if (a.ncol >= (uint32_t)kBlock) {
+    const uint32_t b0 = (m * a.ncol) / kBlock, b1 = (m * a.ncol + a.ncol - 1u) / kBlock;
+#pragma unroll 4
+    for (uint32_t b = b0 + threadIdx.x; b <= b1; b += kBlock) {
+      const uint32_t j = m - divq(b * kBlock, a.dcol);
+#pragma unroll
+      for (int i = 0; i < kBudParts; ++i) {
+        const double x = gld(a.bud_part, ((size_t)b * 2 + j) * kBudParts + i);
+        acc[i] = i == 5 ? fmax(acc[i], x) : acc[i] + x;
+      }
+    }
+  } else {
+#pragma unroll 4
+    for (uint32_t cc = threadIdx.x; cc < a.ncol; cc += kBlock)
+#pragma unroll
+      for (int i = 0; i < kBudParts; ++i) {
+        const double x = gld(a.bud_part, ((size_t)m * a.ncol + cc) * kBudParts + i);
+        acc[i] = i == 5 ? fmax(acc[i], x) : acc[i] + x;
+      }
+  }
+  __shared__ double s_red[kBlock / 64][kBudParts];
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+#pragma unroll
+  for (int i = 0; i < kBudParts; ++i) {
+    const double v = i == 5 ? wave_max_d(acc[i]) : wave_sum_d(acc[i]);
+    if (lane == 0) s_red[wave][i] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < kBudParts) {
+    const bool is_max = threadIdx.x == 5;
+    double t = s_red[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < kBlock / 64; ++w) t = is_max ? fmax(t, s_red[w][threadIdx.x]) : t + s_red[w][threadIdx.x];
+    s_red[0][threadIdx.x] = t;
+  }
+  __syncthreads();
+  if (threadIdx.x < SPEEDY_NBUDGET) {
+    const double wsum = s_red[0][SPEEDY_NBUDGET];
+    const double t = s_red[0][threadIdx.x];
+    gst(a.f.budget, (size_t)m * SPEEDY_NBUDGET + threadIdx.x, threadIdx.x == 5 ? t : t / wsum);
+  }
+}
+
+// One partial, once it is of this call.
+__device__ __forceinline__ float tagged_partial(const KArgs& a, size_t at, uint32_t tag) {
+  const uint64_t* p = reinterpret_cast<const uint64_t*>(a.prm_part) + at;
+  uint64_t w;
+  do w = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  while ((uint32_t)(w >> 32) != tag);
+  return __builtin_bit_cast(float, (uint32_t)w);
+}
+
+template <bool TAGGED>
+__device__ __forceinline__ void param_reduce_body(const KArgs& a, uint32_t m, uint32_t tag) {
+  float acc[VJP_NPARAM];
+#pragma unroll
+  for (int i = 0; i < VJP_NPARAM; ++i) acc[i] = 0.0f;
+  // (unrolled: several iterations' loads in flight; the order of the sums is the loop's)
+  if (a.ncol >= (uint32_t)kBlock) {
+    const uint32_t b0 = (m * a.ncol) / kBlock, b1 = (m * a.ncol + a.ncol - 1u) / kBlock;
+#pragma unroll 4
+    for (uint32_t b = b0 + threadIdx.x; b <= b1; b += kBlock) {
+      const uint32_t j = m - divq(b * kBlock, a.dcol);
+#pragma unroll
+      for (int i = 0; i < VJP_NPARAM; ++i) {
+        const size_t at = ((size_t)b * 2 + j) * VJP_NPARAM + i;
+        acc[i] += TAGGED ? tagged_partial(a, at, tag) : gld(a.prm_part, at);
+      }
+    }
+  } else {
+#pragma unroll 4
+    for (uint32_t cc = threadIdx.x; cc < a.ncol; cc += kBlock)
+#pragma unroll
+      for (int i = 0; i < VJP_NPARAM; ++i) acc[i] += gld(a.prm_part, ((size_t)m * a.ncol + cc) * VJP_NPARAM + i);
+  }
+  __shared__ float s_red[kBlock / 64][VJP_NPARAM];
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+#pragma unroll
+  for (int i = 0; i < VJP_NPARAM; ++i) {
+    const float v = wave_sum_dpp(acc[i]);
+    if (lane == 0) s_red[wave][i] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < VJP_NPARAM) {
+    float t = s_red[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < kBlock / 64; ++w) t = t + s_red[w][threadIdx.x];
+    gst(a.adj.g_params, (size_t)m * VJP_NPARAM + threadIdx.x, t);
+  }
+}
+
+// Per-member sums of a call: parameter gradients (VJP) and float64 budgets.
+__device__ __forceinline__ void member_reduce_body(const KArgs& a, uint32_t m) {
+  if (a.adj.g_params) param_reduce_body<false>(a, m, 0u);
+  if (a.f.budget) {
+    __syncthreads();
+    budget_reduce_body(a, m);
+  }
+}
+
+// Fused forward + VJP: the block's partials, and the sums of the members that it was the
+// last to be counted in for, in the order of member_reduce_body.  The count is taken
+// while the block gathers the level set, so nobody waits for it; the blocks counted
+// before are all running, and their partials carry the call's tag, so this one reads a
+// word again until it has come: no fence between blocks (fences, which write the L2
+// caches back, cost more than the launch they save).  A launch of its own took 3.9 us and
+// a gap: 27.4 -> 26.0 us a call at T85 x 8 levels, 26.6 -> 25.3 at T42; counted at the end
+// instead, T85 29.1 -> 28.8 us back to back, and 28.0 this way.
+__device__ __forceinline__ void fused_sums(const KArgs& a, uint32_t bid, const BlockPos& b, const float prm[VJP_NPARAM],
+                                           const uint32_t* s_last) {
+  block_param_partials<true>(a, bid, b, prm);
+  for (uint32_t j = 0; j < b.nm; ++j)
+    if (__builtin_amdgcn_readfirstlane(s_last[j])) {
+      param_reduce_body<true>(a, b.m_first + j, b.gen + 1u);
+      __syncthreads();
+    }
 }
 
 // Forward + VJP (all terms; the optional verify steps and budgets by run-time
@@ -838,7 +997,8 @@ __device__ __forceinline__ void vjp_body(const KArgs& a, uint32_t bid) {
       if (k > 0 && kStashRh > 0) tape.put(kTape + 2 * KX + k - 1, pa.rh[k]);
     }
   }
-  const uint32_t S = gather_level_set<KX, FUSED>(a, bid, b);
+  __shared__ uint32_t s_last[2];
+  const uint32_t S = gather_level_set<KX, FUSED, FUSED>(a, bid, b, s_last);
   phase_b2_taped<float, KX>(col, pa, S, a.p, a.v, a.u, a.flags, ct, pb, g, t);
   const bool budget = a.f.budget != nullptr;
   const double dpg = (double)col.ps * (double)(P0 / GRAV);   // p0 ps / g; times dhs_k: dp_k / g
@@ -895,103 +1055,16 @@ __device__ __forceinline__ void vjp_body(const KArgs& a, uint32_t bid) {
       g.Q[k] += sel(((limited >> k) & 1u) != 0u, -gld(a.adj.ct_dq, base3 + k * ncol) / a.u.dt_step, 0.0f);
   }
   store_grads<KX>(a, b.m, b.c, g);
-  block_param_partials(a, bid, b.gid, b.active, b.m - b.m_first, g.prm);
-}
-
-
-// Per-member parameter gradients from the partials, one block per member, in a
-// fixed order (deterministic).
-__device__ __forceinline__ void budget_reduce_body(const KArgs& a, uint32_t m) {
-  double acc[kBudParts];
-#pragma unroll
-  for (int i = 0; i < kBudParts; ++i) acc[i] = 0.0;
-  // (unrolled: several iterations' loads in flight; the order of the sums is the loop's)
-  if (a.ncol >= (uint32_t)kBlock) {
-    const uint32_t b0 = (m * a.ncol) / kBlock, b1 = (m * a.ncol + a.ncol - 1u) / kBlock;
-#pragma unroll 4
-    for (uint32_t b = b0 + threadIdx.x; b <= b1; b += kBlock) {
-      const uint32_t j = m - divq(b * kBlock, a.dcol);
-#pragma unroll
-      for (int i = 0; i < kBudParts; ++i) {
-        const double x = gld(a.bud_part, ((size_t)b * 2 + j) * kBudParts + i);
-        acc[i] = i == 5 ? fmax(acc[i], x) : acc[i] + x;
-      }
-    }
+  if (FUSED && a.merged) {
+    if constexpr (STASH)   // a descriptor: as it is (segment)
+      fused_sums(a, bid, b, g.prm, s_last);
+    else
+      fused_sums(reread(&a), bid, b, g.prm, s_last);
   } else {
-#pragma unroll 4
-    for (uint32_t cc = threadIdx.x; cc < a.ncol; cc += kBlock)
-#pragma unroll
-      for (int i = 0; i < kBudParts; ++i) {
-        const double x = gld(a.bud_part, ((size_t)m * a.ncol + cc) * kBudParts + i);
-        acc[i] = i == 5 ? fmax(acc[i], x) : acc[i] + x;
-      }
-  }
-  __shared__ double s_red[kBlock / 64][kBudParts];
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-#pragma unroll
-  for (int i = 0; i < kBudParts; ++i) {
-    const double v = i == 5 ? wave_max_d(acc[i]) : wave_sum_d(acc[i]);
-    if (lane == 0) s_red[wave][i] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < kBudParts) {
-    const bool is_max = threadIdx.x == 5;
-    double t = s_red[0][threadIdx.x];
-#pragma unroll
-    for (int w = 1; w < kBlock / 64; ++w) t = is_max ? fmax(t, s_red[w][threadIdx.x]) : t + s_red[w][threadIdx.x];
-    s_red[0][threadIdx.x] = t;
-  }
-  __syncthreads();
-  if (threadIdx.x < SPEEDY_NBUDGET) {
-    const double wsum = s_red[0][SPEEDY_NBUDGET];
-    const double t = s_red[0][threadIdx.x];
-    gst(a.f.budget, (size_t)m * SPEEDY_NBUDGET + threadIdx.x, threadIdx.x == 5 ? t : t / wsum);
+    block_param_partials<false>(a, bid, b, g.prm);
   }
 }
 
-__device__ __forceinline__ void param_reduce_body(const KArgs& a, uint32_t m) {
-  float acc[VJP_NPARAM];
-#pragma unroll
-  for (int i = 0; i < VJP_NPARAM; ++i) acc[i] = 0.0f;
-  // (unrolled: several iterations' loads in flight; the order of the sums is the loop's)
-  if (a.ncol >= (uint32_t)kBlock) {
-    const uint32_t b0 = (m * a.ncol) / kBlock, b1 = (m * a.ncol + a.ncol - 1u) / kBlock;
-#pragma unroll 4
-    for (uint32_t b = b0 + threadIdx.x; b <= b1; b += kBlock) {
-      const uint32_t j = m - divq(b * kBlock, a.dcol);
-#pragma unroll
-      for (int i = 0; i < VJP_NPARAM; ++i) acc[i] += gld(a.prm_part, ((size_t)b * 2 + j) * VJP_NPARAM + i);
-    }
-  } else {
-#pragma unroll 4
-    for (uint32_t cc = threadIdx.x; cc < a.ncol; cc += kBlock)
-#pragma unroll
-      for (int i = 0; i < VJP_NPARAM; ++i) acc[i] += gld(a.prm_part, ((size_t)m * a.ncol + cc) * VJP_NPARAM + i);
-  }
-  __shared__ float s_red[kBlock / 64][VJP_NPARAM];
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-#pragma unroll
-  for (int i = 0; i < VJP_NPARAM; ++i) {
-    const float v = wave_sum_dpp(acc[i]);
-    if (lane == 0) s_red[wave][i] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < VJP_NPARAM) {
-    float t = s_red[0][threadIdx.x];
-#pragma unroll
-    for (int w = 1; w < kBlock / 64; ++w) t = t + s_red[w][threadIdx.x];
-    gst(a.adj.g_params, (size_t)m * VJP_NPARAM + threadIdx.x, t);
-  }
-}
-
-// Per-member sums of a call: parameter gradients (VJP) and float64 budgets.
-__device__ __forceinline__ void member_reduce_body(const KArgs& a, uint32_t m) {
-  if (a.adj.g_params) param_reduce_body(a, m);
-  if (a.f.budget) {
-    __syncthreads();
-    budget_reduce_body(a, m);
-  }
-}
 
 __global__ __launch_bounds__(kBlock) void param_reduce_kernel(KArgs a) { member_reduce_body(a, blockIdx.x); }
 
@@ -1194,8 +1267,9 @@ void timer_end(hipStream_t s, int slot) {
 
 constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
-// Workspace: word [0] generation, [1] error word; from byte 256 last_s[nmember];
-// then the published level-set words (max of the fused path's two per block
+// Workspace: word [0] generation, [1] error word, from kArrivedWord the members' counts
+// of arrived blocks (zero between calls; calls on other grids may share the workspace,
+// so they are at a place of their own); from byte 256 last_s[nmember]; then the published level-set words (max of the fused path's two per block
 // and the two-kernel path's jmax per chunk).
 struct Grid {
   uint32_t ncol, ntot, nblk, ls_blocks, chunk, jmax;
@@ -1227,7 +1301,7 @@ WsLayout ws_layout(const Grid& g, int32_t nmember) {
   L.partial = L.last_s + align256(sizeof(uint32_t) * (size_t)nmember);
   const size_t npart = std::max<size_t>(2 * (size_t)g.nblk, (size_t)g.ls_blocks * g.jmax);
   L.prm = L.partial + align256(sizeof(uint32_t) * npart);
-  const size_t nprm = g.ncol >= (uint32_t)kBlock ? (size_t)g.nblk * 2 * VJP_NPARAM : (size_t)g.ntot * VJP_NPARAM;
+  const size_t nprm = g.ncol >= (uint32_t)kBlock ? (size_t)g.nblk * 4 * VJP_NPARAM : (size_t)g.ntot * VJP_NPARAM;   // tagged: 8 bytes each
   L.bud = L.prm + align256(sizeof(float) * nprm);
   const size_t nbud = g.ncol >= (uint32_t)kBlock ? (size_t)g.nblk * 2 * kBudParts : (size_t)g.ntot * kBudParts;
   L.desc = L.bud + align256(sizeof(double) * nbud);
@@ -1295,6 +1369,8 @@ int prepare(const SpeedyFields* fields, const SpeedyVertical* vert, const Speedy
   a.err = a.gen + 1;
   a.last_s = reinterpret_cast<uint32_t*>(w + L.last_s);
   a.partial = reinterpret_cast<uint32_t*>(w + L.partial);
+  a.arrived = a.gen + kArrivedWord;
+  a.merged = level_set < 0 && gr.ncol >= (uint32_t)kBlock && a.nmember <= kMergedMembers && !fields->budget;
   a.prm_part = reinterpret_cast<float*>(w + L.prm);
   a.bud_part = reinterpret_cast<double*>(w + L.bud);
   return SPEEDY_OK;
@@ -1404,10 +1480,8 @@ int launch_fwd(const KArgs& a, hipStream_t s) {
     e = hipGetLastError();
     timer_end(s, slot);
   }
-  // Per-member sums in a second small kernel.  (Summing them in the last block to
-  // finish instead, after an agent-scope fence per block, cost more than this
-  // launch: the fences write back the L2 caches.)
-  if (e == hipSuccess && (VJP || a.f.budget)) {
+  // Per-member sums in a second small kernel, where the launch has not taken them.
+  if (e == hipSuccess && ((VJP && !(fused && a.merged)) || a.f.budget)) {
     const int slot = timer_begin(s, 3);
     hipLaunchKernelGGL(param_reduce_kernel, dim3(a.nmember), dim3(kBlock), 0, s, a);
     timer_end(s, slot);
@@ -1608,7 +1682,7 @@ int speedy_fwd_batch(const SpeedySegment* segs, int32_t nseg, const SpeedyVertic
       for (uint32_t b = 0; b < a.ls_blocks; ++b) t_ls[nl++] = ((uint32_t)i << kSegShift) | b;
       jmax = std::max(jmax, a.jmax);
     }
-    if (nset || sg.fields.budget)
+    if ((nset && !(small && a.merged)) || sg.fields.budget)
       for (uint32_t m = 0; m < a.nmember; ++m) t_red[nr++] = ((uint32_t)i << kSegShift) | m;
   }
   // block table: the forward-only segments' blocks first, then the VJP segments'
