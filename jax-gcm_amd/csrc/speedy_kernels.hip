@@ -18,14 +18,13 @@
 //     waiting block itself from the state, so no block depends on another one being
 //     resident, and a plain launch is enough (a cooperative one took 20 us more).
 //     Block 0 advances the generation once every block has published.  No
-//     read-modify-write atomics: contended same-address atomics cost microseconds
-//     per call on this GPU.
+//     read-modify-write atomics in the exchange: contended same-address atomics cost
+//     microseconds per call on this GPU.  Small batches run the same bodies.
 //   two launches (larger grids, members narrower than a block, a given S, and
-//     every batch): a level-set kernel, a fixed number of blocks each covering a
+//     larger batches): a level-set kernel, a fixed number of blocks each covering a
 //     contiguous chunk of columns, writes per-(chunk, member) ORs; the forward
 //     kernel ORs the few chunks of its member, recomputes phase A and does
-//     phase B.  Single calls run this as a one-segment batch (seg_desc_kernel
-//     writes the descriptor into the workspace).
+//     phase B.
 //
 // One thread per column; the column lives in registers.  Accesses are
 // [field][level][column] with consecutive lanes on consecutive columns
@@ -44,8 +43,8 @@
 namespace speedy {
 
 constexpr int kBlock = 256;
-// Internal flag (above the public SPEEDY_FLAG_* bits): take the one-segment batch
-// route even where the fused launch could run (speedy_fwd_noalloc).
+// Internal flag (above the public SPEEDY_FLAG_* bits): take the batch kernels' route
+// even where the fused launch could run (speedy_fwd_noalloc).
 constexpr uint32_t kFlagBatchRoute = 1u << 31;
 // Polls (about 1 us each) before a block forms the words it misses itself.  In a
 // GPU without other work the words are there after one or two; each word formed
@@ -60,6 +59,7 @@ struct Divisor {          // n / d for n < 2^32 by multiply-high + one correctio
 };
 
 constexpr uint32_t kArrivedWord = 2, kMergedMembers = 62;   // words of the workspace's header
+constexpr uint32_t kMergedBlocks = 1024;   // above any co-resident grid of the fused kernels
 
 struct KArgs {
   SpeedyFields f;
@@ -1301,7 +1301,8 @@ WsLayout ws_layout(const Grid& g, int32_t nmember) {
   L.partial = L.last_s + align256(sizeof(uint32_t) * (size_t)nmember);
   const size_t npart = std::max<size_t>(2 * (size_t)g.nblk, (size_t)g.ls_blocks * g.jmax);
   L.prm = L.partial + align256(sizeof(uint32_t) * npart);
-  const size_t nprm = g.ncol >= (uint32_t)kBlock ? (size_t)g.nblk * 4 * VJP_NPARAM : (size_t)g.ntot * VJP_NPARAM;   // tagged: 8 bytes each
+  const size_t slots = g.nblk <= kMergedBlocks ? 4 : 2;   // the fused launch's tagged partials take 8 bytes each
+  const size_t nprm = g.ncol >= (uint32_t)kBlock ? g.nblk * slots * VJP_NPARAM : (size_t)g.ntot * VJP_NPARAM;
   L.bud = L.prm + align256(sizeof(float) * nprm);
   const size_t nbud = g.ncol >= (uint32_t)kBlock ? (size_t)g.nblk * 2 * kBudParts : (size_t)g.ntot * kBudParts;
   L.desc = L.bud + align256(sizeof(double) * nbud);
@@ -1370,7 +1371,8 @@ int prepare(const SpeedyFields* fields, const SpeedyVertical* vert, const Speedy
   a.last_s = reinterpret_cast<uint32_t*>(w + L.last_s);
   a.partial = reinterpret_cast<uint32_t*>(w + L.partial);
   a.arrived = a.gen + kArrivedWord;
-  a.merged = level_set < 0 && gr.ncol >= (uint32_t)kBlock && a.nmember <= kMergedMembers && !fields->budget;
+  a.merged = level_set < 0 && gr.ncol >= (uint32_t)kBlock && gr.nblk <= kMergedBlocks &&
+             a.nmember <= kMergedMembers && !fields->budget;
   a.prm_part = reinterpret_cast<float*>(w + L.prm);
   a.bud_part = reinterpret_cast<double*>(w + L.bud);
   return SPEEDY_OK;
@@ -1843,7 +1845,7 @@ const char* speedy_last_error(void) { return g_last_error.c_str(); }
 // array instead of a caller's buffer, for callers that cannot allocate.  Each GPU
 // holds its own copy for the life of the process; its device address is looked
 // up once per device (hipGetSymbolAddress) and only that address is passed to
-// kernels.  Calls take the one-segment batch route, which reads no word of the
+// kernels.  Calls take the batch kernels' route, which reads no word of the
 // workspace that the same call has not written first (descriptor, level-set
 // words, partials), so the contents left by an earlier call, of any grid, are
 // never read and nothing needs clearing.  Calls that overlap on one GPU share
