@@ -11,11 +11,11 @@ land recipe of jcm_amd.synthetic (seed 1), inputs resident in HBM.
              replay stream time them (untimed replays queued just before keep
              the GPU's clock ramp after setup out of short measurements).
   fwd_vjp    the same for compute_tendencies_vjp (fused forward + VJP w.r.t. T, q,
-             u, v, ps and five parameters, cotangents N(0,1); two launches: the
-             column kernel and the parameter-gradient sums).
+             u, v, ps and five parameters, cotangents N(0,1); one launch, which
+             also sums the parameter gradients).
   per_call   both calls made from Python one by one without graphs (the plain
-             per-call path: host overhead included), with the default
-             cooperative launch and with plain_launch=True.
+             per-call path: host overhead included), and with plain_launch=True
+             (without effect: single-launch calls are launched plainly).
   serving    a Poisson stream of requests of mixed resolution (T21, T31, T42,
              T85) and kind (forward, forward + VJP) through the continuous-
              batching loop (jcm_amd.serving) and through one call per request:
@@ -34,6 +34,7 @@ from __future__ import annotations
 
 import argparse
 import json
+import math
 import os
 import sys
 import time
@@ -358,32 +359,20 @@ def large_leg(phys, dev, reps=5):
 MFMA_FP32_PEAK_TFS = 157.3
 
 
-def _fourier_factors(nlon):
-    """nlon = n1 * n2 with n1 the largest divisor <= sqrt(nlon), as the library splits it."""
-    n1 = max(d for d in range(1, int(nlon ** 0.5) + 1) if nlon % d == 0)
-    return n1, nlon // n1
-
-
 def transform_work(g, kx):
     """(flops, bytes) of one transform step: dynamics -> physics state plus physics
     tendency -> dynamics at the grid g (5*kx+1 fields synthesised: winds,
     temperature, humidity, log surface pressure, geopotential; 4*kx analysed).
-    Flops, 2 per multiply-add, as the kernels compute them: the Legendre
-    contraction over half the latitudes (equatorial symmetry), and the Fourier
-    stages' two passes per latitude line (nlon = n1 * n2; analysis: n2-point real
-    DFTs, twiddles, n1-point DFTs for the n_m wavenumbers kept; synthesis the
-    reverse).  Bytes: modal inputs and outputs, nodal inputs and outputs, and the
-    Legendre basis and the roots of unity read once."""
+    Flops, 2 per multiply-add: the Legendre contraction over l >= m and half the
+    latitudes (equatorial symmetry), and 2.5 nlon log2(nlon) per latitude line for
+    the real FFTs.  Bytes: modal inputs and outputs, nodal inputs and outputs, and
+    the Legendre basis (l >= m, one hemisphere) and the roots of unity read once."""
     mm, nl, nlon, nlat, n_m = 2 * g.n_m - 1, g.n_l, g.nlon, g.nlat, g.n_m
-    n1, n2 = _fourier_factors(nlon)
-    nh, k1 = n2 // 2 + 1, -(-n_m // n2)
-    legendre = lambda nf: 2.0 * nf * mm * nlat * (nl / 2.0)
-    analysis_line = 4.0 * n1 * nh * n2 + 6.0 * n1 * n2 + 8.0 * n_m * n1
-    synthesis_line = n2 * n1 * (8.0 * k1 + 6.0) + 4.0 * n1 * n2 * n2
-    flops = (legendre(5 * kx + 1) + (5 * kx + 1) * nlat * synthesis_line
-             + legendre(4 * kx) + 4 * kx * nlat * analysis_line)
+    kept = sum((1 if m == 0 else 2) * (nl - m) for m in range(n_m))   # coefficients with l >= m
+    fields = 9 * kx + 1
+    flops = fields * (2.0 * kept * (nlat / 2.0) + nlat * 2.5 * nlon * math.log2(nlon))
     modal, nodal = mm * nl * 4, nlon * nlat * 4
-    bases = g.n_m * nlat * nl * 4 + nlon * 8
+    bases = sum(nl - m for m in range(n_m)) * (nlat // 2) * 4 + nlon * 8
     nbytes = ((4 * kx + 2) * modal + (5 * kx + 1) * nodal      # dynamics -> physics
               + 4 * kx * nodal + (4 * kx + 1) * modal           # tendency -> dynamics
               + 2 * bases)
@@ -450,12 +439,8 @@ def main():
     case = to_device(case_np, dev)
     kx, ix, il = case_np[2].nodal_shape
     ncol = ix * il
-    # The profile run launches every call plainly (as graph replays do): under
-    # rocprofv3, a process that made cooperative launches ends in the tool's exit
-    # handlers with SIGSEGV after the results are written.
-    plain = args.profile_only
-    phys = SpeedyPhysics(device=dev, plain_launch=plain)
-    vphys = SpeedyPhysics(parameters=synthetic.draw_vjp_parameters(2), device=dev, plain_launch=plain)
+    phys = SpeedyPhysics(device=dev)
+    vphys = SpeedyPhysics(parameters=synthetic.draw_vjp_parameters(2), device=dev)
     gen = torch.Generator(device=dev)
     gen.manual_seed(2)
     cot = PhysicsTendency(*[torch.randn(case[0].temperature.shape, device=dev, generator=gen) for _ in range(4)])
@@ -508,11 +493,9 @@ def main():
     lib.speedy_timer_disable()
     launches = {k: v[1] for k, v in tm.items() if v[1]}
 
-    # per-kernel device time of the forward + VJP call (HIP events around each of
-    # its two kernels): the VJP kernel without the parameter sums.  The calls use
-    # plain launches, as the graph replays do (a cooperative launch waits for an
-    # idle device), and queue behind ~20 ms of graph replays on the same stream, so
-    # each event pair brackets its kernel and not the host's launch gaps.
+    # device time of the forward + VJP call's kernel (HIP events around it).  The calls
+    # queue behind ~20 ms of graph replays on the same stream, so each event pair
+    # brackets its kernel and not the host's launch gaps.
     p_phys = SpeedyPhysics(device=dev, plain_launch=True)
     p_vphys = SpeedyPhysics(parameters=vphys.parameters, device=dev, plain_launch=True)
     with torch.cuda.stream(g_vjp.stream):
@@ -549,7 +532,7 @@ def main():
                      "used_bytes": {"bytes_per_column": FWD_USED_BYTES_PER_COL(kx), "achieved": used_fwd,
                                     "frac": used_fwd / HBM_PEAK_GBS}},
         "fwd_vjp": {"value": ncol / (ms_vjp * 1e-3), "unit": "columns/s", "ms_per_step": ms_vjp,
-                    "launches_per_step": 2, "kernel_ms": vjp_kernel_ms,
+                    "launches_per_step": 1, "kernel_ms": vjp_kernel_ms,
                     "roofline": {"bound": "hbm", "achieved": achieved_vjp, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                  "frac": achieved_vjp / HBM_PEAK_GBS, "algorithmic_bytes_per_step": bytes_vjp,
                                  "bytes_per_column": VJP_BYTES_PER_COL(kx),
@@ -557,13 +540,13 @@ def main():
                                                 "frac": used_vjp / HBM_PEAK_GBS},
                                  "traffic": profile_traffic("fwd_vjp_kernel_T85"),
                                  "valu": profile_valu("speedy::fwd_kernel<8, false, true, true, true>"),
-                                 "kernel": "speedy::fwd_kernel<8, false, true, true, true> + param_reduce_kernel"}},
+                                 "kernel": "speedy::fwd_kernel<8, false, true, true, true>"}},
         "launches_per_call": launches,
     }
     # ---- plain per-call path (Python, no graphs)
     pc_f = per_call_ms(fwd, args.per_call_steps)
     pc_v = per_call_ms(vjp, args.per_call_steps)
-    # the same calls with plain instead of cooperative launches (plain_launch=True)
+    # the same calls with plain_launch=True
     pc_pf = per_call_ms(lambda: p_phys.compute_tendencies(*case), args.per_call_steps)
     pc_pv = per_call_ms(lambda: p_vphys.compute_tendencies_vjp(*case, cot), args.per_call_steps)
     out["per_call"] = {"fwd_columns_per_s": ncol / (pc_f * 1e-3), "fwd_ms": pc_f,

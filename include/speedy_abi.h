@@ -181,8 +181,8 @@ int speedy_diag_names(int32_t kx, char *buf, size_t buf_len);
  * level_set < 0: the Q1 cloud-top level set (shortwave_radiation.py:63-70) is
  * computed per member over all its columns; >= 0: used as given (bit k =
  * level k), for parity tests.  A grid whose workgroups fit on the GPU at once
- * runs as one launch; other grids (and a given level set) run as a
- * one-segment batch, described in the workspace, in two to four launches.
+ * runs as one launch; other grids (and a given level set) run through the
+ * batch kernels, in one to three launches.
  * Stream-ordered and safe to capture in a HIP graph; no allocation. */
 int speedy_fwd(const SpeedyFields *fields, const SpeedyVertical *vert, const SpeedyParams *params,
                const SpeedyDate *date, int32_t nlon, int32_t nlat, int32_t nmember, uint32_t flags,
@@ -198,7 +198,7 @@ int speedy_fwd(const SpeedyFields *fields, const SpeedyVertical *vert, const Spe
  * SPEEDY_ERR_CAPACITY.  The caller passes inputs and outputs as for speedy_fwd;
  * no hipMalloc, hipFree or allocating call is made.  Every call on one GPU uses
  * that GPU's array: calls that overlap on one GPU (two streams, two threads)
- * race.  The call always runs as a one-segment batch (two to four launches),
+ * race.  The call always runs through the batch kernels (one to three launches),
  * which reads nothing an earlier call left in the array. */
 size_t speedy_noalloc_max_bytes(void);
 int speedy_fwd_noalloc(const SpeedyFields *fields, const SpeedyVertical *vert, const SpeedyParams *params,

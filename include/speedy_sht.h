@@ -10,7 +10,7 @@
  * Grid.to_modal / Grid.to_nodal with RealSphericalHarmonics, selected at
  * jcm/utils.py:28-54).  Both transform directions are a longitude Fourier
  * contraction (a truncated real DFT in two short passes) and a latitude
- * Legendre contraction (a batched fp32 MFMA GEMM) on gfx950.
+ * Legendre contraction (fp32 matrix instructions) on gfx950.
  *
  * Conventions (dinosaur RealSphericalHarmonics on a Gaussian grid):
  *   nodal field  float[nlon][nlat], latitude fastest, Gauss-Legendre latitudes
