@@ -216,6 +216,42 @@ __device__ __forceinline__ void tend_after_b1(uint32_t tm, const PhaseB<float, K
 }
 
 // at, aq: the partial sums of tend_after_a / tend_after_b1.
+// The diagnostics' rows (order of kDiag2D, then kDiag3D), stored as soon as they are
+// final, so that phase b2 runs beside the stores and their 90 values leave the registers:
+// the batch kernel then fits two waves per SIMD at 7 and 8 levels.  With all 140 rows
+// stored at the end T213 took 62.9 us a call, now 49.1; T85 x 16 levels 39.8, now 34.4; T85
+// x 8 18.0, now 17.7.  The fused kernels store after the level-set gather, whose loads
+// would wait for the stores (T85 0.75 us slower before it).
+template <int KX>
+__device__ __forceinline__ float* diag_column(const KArgs& a, uint32_t m, uint32_t c) {
+  return a.f.diag + (size_t)m * diag_rows(KX) * a.ncol + c;
+}
+template <int KX>
+__device__ __forceinline__ void store_diag_a(const KArgs& a, uint32_t m, uint32_t c, const ColumnIn<float, KX>& col,
+                                             const PhaseA<float, KX>& pa) {
+  float* dg = diag_column<KX>(a, m, c);
+  auto W = [&](int row, float x) { gst(dg, (size_t)row * a.ncol, x); };
+  W(0, (float)pa.iptop); W(1, pa.cbmf); W(2, pa.precnv); W(3, pa.precls);
+  W(4, (float)pa.icltop); W(5, pa.cloudc); W(6, pa.clstr); W(7, pa.qcloud); W(8, pa.gse);
+  W(12, col.fsol); W(13, col.ozupp); W(14, col.ozone); W(15, col.zenit); W(16, col.stratz);
+#pragma unroll
+  for (int k = 0; k < KX; ++k) {
+    W(kN2D + k, pa.qsat[k]); W(kN2D + KX + k, pa.rh[k]); W(kN2D + 2 * KX + k, pa.se[k]);
+  }
+}
+template <int KX>
+__device__ __forceinline__ void store_diag_b1(const KArgs& a, uint32_t m, uint32_t c, const PhaseB<float, KX>& pb) {
+  float* dg = diag_column<KX>(a, m, c);
+  auto W = [&](int row, float x) { gst(dg, (size_t)row * a.ncol, x); };
+  W(18, pb.albsfc); W(19, pb.alb_l); W(20, pb.alb_s); W(21, pb.snowc);
+#pragma unroll
+  for (int k = 0; k < KX; ++k) {
+    W(kN2D + 5 * KX + k, pb.st4a0[k]); W(kN2D + 6 * KX + k, pb.st4a1[k]);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) W(kN2D + (7 + b) * KX + k, pb.tauL[k][b]);
+  }
+}
+
 template <int KX, bool DIAG, bool EXTRA>
 __device__ __forceinline__ void store_outputs(const KArgs& a, uint32_t m, uint32_t c,
                                               const ColumnIn<float, KX>& col, const PhaseA<float, KX>& pa,
@@ -265,41 +301,21 @@ __device__ __forceinline__ void store_outputs(const KArgs& a, uint32_t m, uint32
     }
   }
   if (DIAG) {
-    float* dg = a.f.diag + (size_t)m * diag_rows(KX) * ncol + c;
-    int r = 0;
-    auto W = [&](float x) { gst(dg, (size_t)(r++) * ncol, x); };
-    W((float)pa.iptop); W(pa.cbmf); W(pa.precnv); W(pa.precls);
-    W((float)pa.icltop); W(pa.cloudc); W(pa.clstr); W(pa.qcloud); W(pa.gse);
-    W(pb.rsds); W(pb.rsns); W(pb.ftop_sw);
-    W(col.fsol); W(col.ozupp); W(col.ozone); W(col.zenit); W(col.stratz);
-    W(pb.ftop_lw); W(pb.albsfc); W(pb.alb_l); W(pb.alb_s); W(pb.snowc);
-    W(pb.stratc0); W(pb.stratc1);
-    for (int i = 0; i < 4; ++i) W(pb.flux_out[i]);
-    for (int i = 0; i < 3; ++i) W(pb.ustr[i]);
-    for (int i = 0; i < 3; ++i) W(pb.vstr[i]);
-    for (int i = 0; i < 3; ++i) W(pb.shf[i]);
-    for (int i = 0; i < 3; ++i) W(pb.evap[i]);
-    for (int i = 0; i < 3; ++i) W(pb.rlus[i]);
-    W(pb.rlds); W(pb.rlns); W(pb.hfluxn[0]); W(pb.hfluxn[1]);
-    W(pb.tsfc); W(pb.tskin); W(pb.u0); W(pb.v0); W(pb.t0);
+    float* dg = diag_column<KX>(a, m, c);
+    auto W = [&](int row, float x) { gst(dg, (size_t)row * ncol, x); };
+    W(9, pb.rsds); W(10, pb.rsns); W(11, pb.ftop_sw); W(17, pb.ftop_lw);
+    W(22, pb.stratc0); W(23, pb.stratc1);
+    for (int i = 0; i < 4; ++i) W(24 + i, pb.flux_out[i]);
+    for (int i = 0; i < 3; ++i) {
+      W(28 + i, pb.ustr[i]); W(31 + i, pb.vstr[i]); W(34 + i, pb.shf[i]); W(37 + i, pb.evap[i]); W(40 + i, pb.rlus[i]);
+    }
+    W(43, pb.rlds); W(44, pb.rlns); W(45, pb.hfluxn[0]); W(46, pb.hfluxn[1]);
+    W(47, pb.tsfc); W(48, pb.tskin); W(49, pb.u0); W(50, pb.v0); W(51, pb.t0);
 #pragma unroll
-    for (int k = 0; k < KX; ++k) W(pa.qsat[k]);
-#pragma unroll
-    for (int k = 0; k < KX; ++k) W(pa.rh[k]);
-#pragma unroll
-    for (int k = 0; k < KX; ++k) W(pa.se[k]);
-#pragma unroll
-    for (int k = 0; k < KX; ++k) W(pb.dfabs_sw[k]);
-#pragma unroll
-    for (int k = 0; k < KX; ++k) W(pb.dfl[k]);
-#pragma unroll
-    for (int k = 0; k < KX; ++k) W(pb.st4a0[k]);
-#pragma unroll
-    for (int k = 0; k < KX; ++k) W(pb.st4a1[k]);
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-      for (int k = 0; k < KX; ++k) W(pb.tauL[k][b]);
+    for (int k = 0; k < KX; ++k) {
+      W(kN2D + 3 * KX + k, pb.dfabs_sw[k]);
+      W(kN2D + 4 * KX + k, pb.dfl[k]);
+    }
   }
 }
 
@@ -810,14 +826,23 @@ __device__ __forceinline__ void fwd_body(const KArgs& a, uint32_t bid) {
   float tend_t[KX], tend_q[KX];
   tend_after_a<KX>(a.term_mask, pa, tend_t, tend_q);
   if (FUSED && a.level_set < 0) publish_level_bits(a, bid, b, pa.icltop, KX);
+  if (DIAG && !FUSED) store_diag_a<KX>(a, b.m, b.c, col, pa);
   PhaseB<float, KX> pb;
   phase_b1<float, KX>(col, pa, a.p, a.v, a.u, pb, ts);
+  if (DIAG && !FUSED) store_diag_b1<KX>(a, b.m, b.c, pb);
   tend_after_b1<KX>(a.term_mask, pb, tend_q);
   const uint32_t S = gather_level_set<KX, FUSED>(a, bid, b);
   // with every output compiled in, the uniforms of phase b2 and the stores are read
   // again (T85 with diagnostics and verify: 17.2 -> 16.2 us; the plain forward is
   // 0.4 us slower that way)
-  const KArgs& o = FUSED && DIAG && EXTRA ? reread((const void*)__builtin_amdgcn_kernarg_segment_ptr()) : a;
+  if (DIAG && FUSED) {
+    store_diag_a<KX>(a, b.m, b.c, col, pa);
+    store_diag_b1<KX>(a, b.m, b.c, pb);
+  }
+  const KArgs& o = !(DIAG && EXTRA) ? a
+                   : FUSED          ? reread((const void*)__builtin_amdgcn_kernarg_segment_ptr())
+                   : KX <= 8        ? reread(&a)
+                                    : a;
   phase_b2<float, KX, DIAG>(col, pa, S, o.p, o.v, o.u, o.flags, pb, ts);
   double colsum[2] = {0.0, 0.0};
   store_outputs<KX, DIAG, EXTRA>(o, b.m, b.c, col, pa, pb, tend_t, tend_q, colsum);
@@ -1156,9 +1181,10 @@ __global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_plain_batch_kerne
 }
 
 // Forward-only segments that also write the PhysicsData diagnostics: single
-// calls with diagnostics that the fused launch cannot take.
+// calls with diagnostics that the fused launch cannot take.  Two waves per SIMD as
+// in the kernels above (T213 59.7 -> 49.1 us).
 template <int KX>
-__global__ __launch_bounds__(kBlock) void fwd_diag_batch_kernel(KArgs, const KArgs* __restrict__ segs,
+__global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_diag_batch_kernel(KArgs, const KArgs* __restrict__ segs,
                                                                 const uint32_t* __restrict__ table) {
   uint32_t bid;
   const KArgs& a = segment<KX>(segs, table, bid);
