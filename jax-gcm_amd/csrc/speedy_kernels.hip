@@ -252,7 +252,7 @@ __device__ __forceinline__ void store_diag_b1(const KArgs& a, uint32_t m, uint32
   }
 }
 
-template <int KX, bool DIAG, bool EXTRA>
+template <int KX, bool DIAG, bool EXTRA, bool FUSED>
 __device__ __forceinline__ void store_outputs(const KArgs& a, uint32_t m, uint32_t c,
                                               const ColumnIn<float, KX>& col, const PhaseA<float, KX>& pa,
                                               const PhaseB<float, KX>& pb, const float at[KX], const float aq[KX],
@@ -265,6 +265,16 @@ __device__ __forceinline__ void store_outputs(const KArgs& a, uint32_t m, uint32
   const uint32_t tm = a.term_mask;
   const size_t ncol = a.ncol;
   const size_t base3 = (size_t)m * KX * ncol + c;
+  // verify: the unclamped q again (L2), all levels ahead of the stores: a load between
+  // them waits for the store before it (T425 with verify 107.2 -> 100.4 us a call, 64
+  // members of T31 x 16 levels 136.6 -> 128.3, T85 16.9 -> 16.2).  The batched diagnostics
+  // at 7 and 8 levels have no registers left for it.
+  const bool verify = EXTRA && (a.flags & SPEEDY_FLAG_VERIFY_TENDENCIES) != 0u;
+  constexpr bool kAhead = !DIAG || FUSED || KX > 8;
+  float q_raw[KX];
+  if (verify && kAhead)
+#pragma unroll
+    for (int k = 0; k < KX; ++k) q_raw[k] = gld(a.f.q, base3 + k * ncol);
 #pragma unroll
   for (int k = 0; k < KX; ++k) {
     float t = 0.0f, q = 0.0f, du = 0.0f, dv = 0.0f;
@@ -284,9 +294,9 @@ __device__ __forceinline__ void store_outputs(const KArgs& a, uint32_t m, uint32
       t = t + pb.tvd[k];
       if (!kEarlySums<KX> || k == KX - 1) q = q + pb.qvd[k];   // early sums: the levels above took it already
     }
-    if (EXTRA && (a.flags & SPEEDY_FLAG_VERIFY_TENDENCIES)) {
+    if (verify) {
       bool lim;
-      q = verify_dq(gld(a.f.q, base3 + k * ncol), q, a.u.dt_step, lim);   // the unclamped q (re-read, L2)
+      q = verify_dq(kAhead ? q_raw[k] : gld(a.f.q, base3 + k * ncol), q, a.u.dt_step, lim);
     }
     if (k == KX - 1) {   // the levels above were zeroed by store_uv_zeros
       gst(a.f.du, base3 + k * ncol, du);
@@ -845,7 +855,7 @@ __device__ __forceinline__ void fwd_body(const KArgs& a, uint32_t bid) {
                                     : a;
   phase_b2<float, KX, DIAG>(col, pa, S, o.p, o.v, o.u, o.flags, pb, ts);
   double colsum[2] = {0.0, 0.0};
-  store_outputs<KX, DIAG, EXTRA>(o, b.m, b.c, col, pa, pb, tend_t, tend_q, colsum);
+  store_outputs<KX, DIAG, EXTRA, FUSED>(o, b.m, b.c, col, pa, pb, tend_t, tend_q, colsum);
   if (EXTRA && a.f.budget) column_budgets<KX>(o, bid, b, pa, pb, colsum);
 }
 
