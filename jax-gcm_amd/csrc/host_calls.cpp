@@ -310,7 +310,8 @@ bool set_item(PyObject* tuple, Py_ssize_t i, const at::Tensor& t) {
 PyObject* fwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
   long term_mask, level_set;
   if (n != 13 || !p_fwd || !as_long(args[10], &term_mask) || !as_long(args[11], &level_set)) return general();
-  const bool diagnostics = args[12] == Py_True;
+  const int diagnostics = PyObject_IsTrue(args[12]);   // any object, as the general path takes it
+  if (diagnostics < 0) return general();
   try {
     PhysicsCall c;
     if (!c.read(args)) return general();

@@ -382,7 +382,7 @@ class SpeedyPhysics(Physics):
         if _native.host is not None and not budgets and not self.check_barrier:
             r = _native.host.fwd(self._consts, self._workspaces, self.parameters, *self._where(), state, forcing, geometry,
                                  date, (VERIFY_FLAGS if verify else 0) | self._launch_flags, term_mask, level_set,
-                                 self.with_diagnostics is True)
+                                 self.with_diagnostics)
             if r.__class__ is tuple:
                 data = None
                 if r[4] is not None:
