@@ -194,7 +194,8 @@ int speedy_fwd(const SpeedyFields *fields, const SpeedyVertical *vert, const Spe
  * tight serving loops, harnesses that forbid hipMalloc).  The same forward and
  * the same results as speedy_fwd, with the workspace taken from a static device
  * array of speedy_noalloc_max_bytes() (4 MiB) per GPU, held until the process
- * ends; a grid whose speedy_workspace_bytes exceeds it is rejected with
+ * ends; a grid that needs more (speedy_workspace_bytes less the words of the single
+ * launch, which it never takes) is rejected with
  * SPEEDY_ERR_CAPACITY.  The caller passes inputs and outputs as for speedy_fwd;
  * no hipMalloc, hipFree or allocating call is made.  Every call on one GPU uses
  * that GPU's array: calls that overlap on one GPU (two streams, two threads)

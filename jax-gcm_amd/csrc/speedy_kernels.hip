@@ -39,10 +39,12 @@
 #include <vector>
 
 #include "speedy_adjoint.hpp"
+#include "speedy_workspace.hpp"
 
 namespace speedy {
 
-constexpr int kBlock = 256;
+static_assert(kParamParts == VJP_NPARAM && kBudParts == SPEEDY_NBUDGET + 1, "partials");
+
 // Internal flag (above the public SPEEDY_FLAG_* bits): take the batch kernels' route
 // even where the fused launch could run (speedy_fwd_noalloc).
 constexpr uint32_t kFlagBatchRoute = 1u << 31;
@@ -57,9 +59,6 @@ constexpr uint32_t kSpinLimit = 1u << 31;
 struct Divisor {          // n / d for n < 2^32 by multiply-high + one correction step
   uint32_t d, m;          // m = floor(2^32 / d) (unused when d == 1)
 };
-
-constexpr uint32_t kArrivedWord = 2, kMergedMembers = 62;   // words of the workspace's header
-constexpr uint32_t kMergedBlocks = 1024;   // above any co-resident grid of the fused kernels
 
 struct KArgs {
   SpeedyFields f;
@@ -78,10 +77,9 @@ struct KArgs {
   uint32_t* arrived;                 // per member: blocks whose partials are out (zero between calls)
   uint32_t merged;                   // a fused call's members are summed in the launch (fused_sums)
   float* prm_part;                   // parameter-gradient partials (per block and member slot, or per column)
-  double* bud_part;                  // float64 budget partials (same layout, kBudParts doubles each)
+  double* bud_part;                  // float64 budget partials, kBudParts each (at block + member, or per column)
+  void* desc;                        // a single call's argument block in its workspace
 };
-
-constexpr int kBudParts = SPEEDY_NBUDGET + 1;   // the budgets and the weight sum
 
 // ---------------------------------------------------------------- diagnostics
 // Names follow Physics.data_struct_to_dict (physics_interface.py:157-194):
@@ -344,10 +342,6 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t v) {
   return __builtin_amdgcn_readlane(v, 63);
 }
 
-__device__ __forceinline__ uint32_t gen_tag(uint32_t g) { return (g & 0x7fffu) | 0x8000u; }
-
-
-
 __device__ __forceinline__ uint32_t clip_bit(int icl, int kx) {
   return 1u << (icl < 0 ? 0 : (icl > kx - 1 ? kx - 1 : icl));
 }
@@ -379,6 +373,15 @@ __device__ __forceinline__ uint32_t block_level_bits(const KArgs& a, uint32_t b,
   return bits;   // the member's last column is one of its own: its bit belongs to S
 }
 
+// The single launch's tagged words (speedy_workspace.hpp), per block and member slot:
+// level bits, and partials of the parameter gradients (kParamParts each).
+__device__ __forceinline__ uint64_t* level_words(const KArgs& a) {
+  return reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(a.gen) + kHeaderBytes);
+}
+__device__ __forceinline__ uint64_t* param_words(const KArgs& a) {
+  return reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(a.gen) + kHeaderBytes + kWordBytes);
+}
+
 // One poll of the published words of the blocks covering member m: the OR of their
 // level bits, and whether any word is not of this call yet.  By one wave, all lanes
 // active throughout: lanes past the last word read it again (OR is idempotent).
@@ -390,9 +393,9 @@ __device__ __forceinline__ uint32_t poll_words(const KArgs& a, uint32_t tag, uin
   for (uint32_t bb = b0; bb <= b1; bb += 64u) {
     const uint32_t b = min(bb + lane, b1);
     const uint32_t j = m - divq(b * kBlock, a.dcol);
-    const uint32_t w = __hip_atomic_load(&a.partial[2u * b + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    stale |= (w >> 16) != tag;
-    acc |= w & 0xffffu;
+    const uint64_t w = __hip_atomic_load(&level_words(a)[2u * b + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    stale |= (uint32_t)(w >> 32) != tag;
+    acc |= (uint32_t)w;
   }
   missing = __any(stale);
   return wave_or(acc);
@@ -414,10 +417,9 @@ __device__ __forceinline__ uint32_t collect_fused(const KArgs& a, uint32_t tag, 
   uint32_t acc = 0u;
   for (uint32_t b = b0; b <= b1; ++b) {   // uniform: every lane reads the same word
     const uint32_t j = m - divq(b * kBlock, a.dcol);
-    const uint32_t w = __builtin_amdgcn_readfirstlane(
-        __hip_atomic_load(&a.partial[2u * b + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    if ((w >> 16) == tag && patience != 0u)
-      acc |= w & 0xffffu;
+    const uint64_t w = __hip_atomic_load(&level_words(a)[2u * b + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane((uint32_t)(w >> 32)) == tag && patience != 0u)
+      acc |= (uint32_t)w;
     else
       acc |= block_level_bits<KX>(a, b, m);
   }
@@ -441,7 +443,7 @@ __device__ __forceinline__ void finish_generation(const KArgs& a, uint32_t gen, 
     }
     gst(a.last_s, m, v);
   }
-  __hip_atomic_store(a.gen, gen + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(a.gen, next_generation(gen), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Two-kernel path: member m's word of level-set chunk b (levelset_batch_kernel output).
@@ -520,7 +522,7 @@ struct BlockPos {
   bool active, wide;        // wide: a member is at least a block, so a block spans at most two members
   uint32_t m_first, nm;     // the block's first member and how many it spans
   uint32_t wave;            // this wave's index in the block, as a scalar: branches on it keep all lanes on
-  uint32_t gen, tag;        // fused: the generation word and the call's tag
+  uint32_t gen, tag;        // fused: the generation word and its tag (call_tag)
   uint32_t lw0, lw1;        // two launches: this thread's share of the members' chunk words
 };
 
@@ -596,11 +598,8 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
 
 // Parameter gradients of this block: a fixed-order tree sum per member slot
 // (deterministic), written to prm_part[block][slot][5].  Members narrower than
-// a block write per-column values instead (prm_part[column][5]).  TAGGED: as
-// tagged_word(tag, value), for the block that sums the member in the same launch.
-__device__ __forceinline__ uint64_t tagged_word(uint32_t tag, float v) {
-  return (uint64_t)tag << 32 | __builtin_bit_cast(uint32_t, v);
-}
+// a block write per-column values instead (prm_part[column][5]).  TAGGED: tagged words
+// (param_words), for the block that sums the member in the same launch.
 template <bool TAGGED>
 __device__ __forceinline__ void block_param_partials(const KArgs& a, uint32_t bid, const BlockPos& b,
                                                      const float prm[VJP_NPARAM]) {
@@ -628,7 +627,7 @@ __device__ __forceinline__ void block_param_partials(const KArgs& a, uint32_t bi
     for (int w = 1; w < kBlock / 64; ++w) acc = acc + s_red[w][threadIdx.x];
     const size_t at = (size_t)bid * 2 * VJP_NPARAM + threadIdx.x;
     if constexpr (TAGGED)
-      __hip_atomic_store(reinterpret_cast<uint64_t*>(a.prm_part) + at, tagged_word(b.gen + 1u, acc), __ATOMIC_RELAXED,
+      __hip_atomic_store(param_words(a) + at, tagged_word(b.tag, __builtin_bit_cast(uint32_t, acc)), __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
     else
       gst(a.prm_part, at, acc);
@@ -647,15 +646,18 @@ __device__ __forceinline__ double wave_max_d(double v) {
   return v;
 }
 
-// Float64 budget partials of this block per member slot (layout as the
-// parameter partials, kBudParts doubles): weighted sums, the largest column
-// water residual, and the weight sum.
-__device__ __forceinline__ void block_budget_partials(const KArgs& a, uint32_t bid, uint32_t gid, bool active,
-                                                      uint32_t slot, const double v[kBudParts]) {
+// Float64 budget partials of this block per member slot: weighted sums, the largest
+// column water residual, and the weight sum.  Block b's of member m are at place b + m
+// (the next block of a member, and the next member of a block, are both one further on).
+// Members narrower than a block write per-column values instead.
+__device__ __forceinline__ void block_budget_partials(const KArgs& a, uint32_t bid, const BlockPos& b,
+                                                      const double v[kBudParts]) {
+  // (formed again: the scalar registers are short at the end of a kernel)
+  const uint32_t m_first = divq(bid * kBlock, a.dcol), slot = b.m - m_first;
   if (a.ncol < (uint32_t)kBlock) {
-    if (active)
+    if (b.active)
 #pragma unroll
-      for (int i = 0; i < kBudParts; ++i) gst(a.bud_part, (size_t)gid * kBudParts + i, v[i]);
+      for (int i = 0; i < kBudParts; ++i) gst(a.bud_part, (size_t)b.gid * kBudParts + i, v[i]);
     return;
   }
   __shared__ double s_bud[kBlock / 64][2 * kBudParts];
@@ -664,17 +666,18 @@ __device__ __forceinline__ void block_budget_partials(const KArgs& a, uint32_t b
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int i = 0; i < kBudParts; ++i) {
-      const bool mine = active && slot == (uint32_t)j;
+      const bool mine = b.active && slot == (uint32_t)j;
       const double x = i == 5 ? wave_max_d(mine ? v[i] : 0.0) : wave_sum_d(mine ? v[i] : 0.0);
       if (lane == 0) s_bud[wave][j * kBudParts + i] = x;
     }
   __syncthreads();
-  if (threadIdx.x < 2 * kBudParts) {
+  const uint32_t nm = divq(min(bid * kBlock + kBlock, a.ntot) - 1u, a.dcol) - m_first + 1u;
+  if (threadIdx.x < nm * kBudParts) {
     const bool is_max = (threadIdx.x % kBudParts) == 5;
     double acc = s_bud[0][threadIdx.x];
 #pragma unroll
     for (int w = 1; w < kBlock / 64; ++w) acc = is_max ? fmax(acc, s_bud[w][threadIdx.x]) : acc + s_bud[w][threadIdx.x];
-    gst(a.bud_part, (size_t)bid * 2 * kBudParts + threadIdx.x, acc);
+    gst(a.bud_part, (size_t)(bid + m_first) * kBudParts + threadIdx.x, acc);
   }
 }
 
@@ -718,7 +721,7 @@ __device__ __forceinline__ BlockPos block_pos(const KArgs& a, uint32_t bid) {
   const bool need_s = a.level_set < 0;
   if (FUSED && need_s) {
     b.gen = __hip_atomic_load(a.gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    b.tag = gen_tag(b.gen);
+    b.tag = call_tag(b.gen);
   }
   if (!FUSED && need_s) {
     if (b.wide) {
@@ -746,7 +749,7 @@ __device__ __forceinline__ void publish_level_bits(const KArgs& a, uint32_t bid,
       uint32_t w = 0u;
 #pragma unroll
       for (int i = 0; i < kBlock / 64; ++i) w |= s_wor[i][j];
-      __hip_atomic_store(&a.partial[2u * bid + j], (b.tag << 16) | w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&level_words(a)[2u * bid + j], tagged_word(b.tag, w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
 }
@@ -809,7 +812,7 @@ __device__ __forceinline__ void column_budgets(const KArgs& a, uint32_t bid, con
   const double E = (double)pb.evap2, P = (double)pa.precnv + (double)pa.precls;
   const double res = colsum[1] - (E - P);
   const double v[kBudParts] = {w * colsum[0], w * colsum[1], w * E, w * P, w * res, fabs(res), w};
-  block_budget_partials(a, bid, b.gid, b.active, b.m - b.m_first, v);
+  block_budget_partials(a, bid, b, v);
 }
 
 // The argument block (the launch's own, or a descriptor) read again: what follows loads
@@ -869,14 +872,12 @@ __device__ __forceinline__ void budget_reduce_body(const KArgs& a, uint32_t m) {
   if (a.ncol >= (uint32_t)kBlock) {
     const uint32_t b0 = (m * a.ncol) / kBlock, b1 = (m * a.ncol + a.ncol - 1u) / kBlock;
 #pragma unroll 4
-    for (uint32_t b = b0 + threadIdx.x; b <= b1; b += kBlock) {
-      const uint32_t j = m - divq(b * kBlock, a.dcol);
+    for (uint32_t b = b0 + threadIdx.x; b <= b1; b += kBlock)
 #pragma unroll
       for (int i = 0; i < kBudParts; ++i) {
-        const double x = gld(a.bud_part, ((size_t)b * 2 + j) * kBudParts + i);
+        const double x = gld(a.bud_part, (size_t)(b + m) * kBudParts + i);
         acc[i] = i == 5 ? fmax(acc[i], x) : acc[i] + x;
       }
-    }
   } else {
 #pragma unroll 4
     for (uint32_t cc = threadIdx.x; cc < a.ncol; cc += kBlock)
@@ -911,9 +912,8 @@ __device__ __forceinline__ void budget_reduce_body(const KArgs& a, uint32_t m) {
 
 // One partial, once it is of this call.
 __device__ __forceinline__ float tagged_partial(const KArgs& a, size_t at, uint32_t tag) {
-  const uint64_t* p = reinterpret_cast<const uint64_t*>(a.prm_part) + at;
   uint64_t w;
-  do w = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  do w = __hip_atomic_load(param_words(a) + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   while ((uint32_t)(w >> 32) != tag);
   return __builtin_bit_cast(float, (uint32_t)w);
 }
@@ -979,7 +979,7 @@ __device__ __forceinline__ void fused_sums(const KArgs& a, uint32_t bid, const B
   block_param_partials<true>(a, bid, b, prm);
   for (uint32_t j = 0; j < b.nm; ++j)
     if (__builtin_amdgcn_readfirstlane(s_last[j])) {
-      param_reduce_body<true>(a, b.m_first + j, b.gen + 1u);
+      param_reduce_body<true>(a, b.m_first + j, b.tag);
       __syncthreads();
     }
 }
@@ -1301,51 +1301,6 @@ void timer_end(hipStream_t s, int slot) {
   (void)hipEventRecord(g_timer.ev[2 * slot + 1], s);
 }
 
-constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
-
-// Workspace: word [0] generation, [1] error word, from kArrivedWord the members' counts
-// of arrived blocks (zero between calls; calls on other grids may share the workspace,
-// so they are at a place of their own); from byte 256 last_s[nmember]; then the published level-set words (max of the fused path's two per block
-// and the two-kernel path's jmax per chunk).
-struct Grid {
-  uint32_t ncol, ntot, nblk, ls_blocks, chunk, jmax;
-};
-
-Grid make_grid(int64_t nlon, int64_t nlat, int64_t nmember) {
-  Grid g;
-  g.ncol = (uint32_t)(nlon * nlat);
-  g.ntot = (uint32_t)(nlon * nlat * nmember);
-  g.nblk = (g.ntot + kBlock - 1) / kBlock;
-  // At most 512 level-set chunks (~2 blocks per CU): the forward + VJP kernels
-  // gather a member's chunk words in one wave, one round trip per 64 chunks, and at
-  // T425 512 chunks cost that gather 20 us less than 1024 (fwd+VJP 892 vs 912 us)
-  // while the level-set pass itself stays at 25 us (256 chunks: 33 us).
-  const uint32_t lsb = g.nblk < 512u ? g.nblk : 512u;
-  g.chunk = ((g.ntot + lsb - 1) / lsb + kBlock - 1) / kBlock * kBlock;
-  g.ls_blocks = (g.ntot + g.chunk - 1) / g.chunk;
-  g.jmax = (g.chunk - 1) / g.ncol + 2;
-  return g;
-}
-
-struct WsLayout {
-  size_t last_s, partial, prm, bud, desc, total;
-};
-
-WsLayout ws_layout(const Grid& g, int32_t nmember) {
-  WsLayout L;
-  L.last_s = 256;
-  L.partial = L.last_s + align256(sizeof(uint32_t) * (size_t)nmember);
-  const size_t npart = std::max<size_t>(2 * (size_t)g.nblk, (size_t)g.ls_blocks * g.jmax);
-  L.prm = L.partial + align256(sizeof(uint32_t) * npart);
-  const size_t slots = g.nblk <= kMergedBlocks ? 4 : 2;   // the fused launch's tagged partials take 8 bytes each
-  const size_t nprm = g.ncol >= (uint32_t)kBlock ? g.nblk * slots * VJP_NPARAM : (size_t)g.ntot * VJP_NPARAM;
-  L.bud = L.prm + align256(sizeof(float) * nprm);
-  const size_t nbud = g.ncol >= (uint32_t)kBlock ? (size_t)g.nblk * 2 * kBudParts : (size_t)g.ntot * kBudParts;
-  L.desc = L.bud + align256(sizeof(double) * nbud);
-  L.total = L.desc + align256(sizeof(KArgs));   // a single call's argument block
-  return L;
-}
-
 constexpr uint32_t kMaxJ = 16384;   // LDS words of the level-set kernel's per-member ORs
 
 Divisor make_divisor(uint32_t d) {
@@ -1366,7 +1321,8 @@ int check_fields(const SpeedyFields* f) {
 
 int prepare(const SpeedyFields* fields, const SpeedyVertical* vert, const SpeedyParams* params,
             const SpeedyDate* date, int32_t nlon, int32_t nlat, int32_t nmember, uint32_t flags,
-            uint32_t term_mask, int32_t level_set, void* workspace, size_t workspace_bytes, KArgs& a) {
+            uint32_t term_mask, int32_t level_set, void* workspace, size_t workspace_bytes, KArgs& a,
+            size_t tag_bytes = kTagBytes) {
   if (!fields || !vert || !params || !date) return fail(SPEEDY_ERR_ARG, "speedy: NULL struct argument");
   if (nlon <= 0 || nlat <= 0 || nmember <= 0) return fail(SPEEDY_ERR_ARG, "speedy: nlon, nlat, nmember must be > 0");
   if (vert->kx != 7 && vert->kx != 8 && vert->kx != 16)
@@ -1384,7 +1340,7 @@ int prepare(const SpeedyFields* fields, const SpeedyVertical* vert, const Speedy
   if (gr.jmax > kMaxJ) return fail(SPEEDY_ERR_CAPACITY, "speedy: too many members per column chunk");
   if (gr.ls_blocks > kChunkLoads * kBlock)   // chunk_share's reach (make_grid keeps it <= 512)
     return fail(SPEEDY_ERR_CAPACITY, "speedy: too many level-set chunks");
-  const WsLayout L = ws_layout(gr, nmember);
+  const WsLayout L = ws_layout(gr, nmember, sizeof(KArgs), tag_bytes);
   if (!workspace) return fail(SPEEDY_ERR_WORKSPACE, "speedy: workspace is NULL");
   if (workspace_bytes < L.total)
     return fail(SPEEDY_ERR_WORKSPACE, "speedy: workspace too small (need " + std::to_string(L.total) + " bytes)");
@@ -1406,8 +1362,9 @@ int prepare(const SpeedyFields* fields, const SpeedyVertical* vert, const Speedy
   a.err = a.gen + 1;
   a.last_s = reinterpret_cast<uint32_t*>(w + L.last_s);
   a.partial = reinterpret_cast<uint32_t*>(w + L.partial);
+  a.desc = w + L.desc;
   a.arrived = a.gen + kArrivedWord;
-  a.merged = level_set < 0 && gr.ncol >= (uint32_t)kBlock && gr.nblk <= kMergedBlocks &&
+  a.merged = level_set < 0 && gr.ncol >= (uint32_t)kBlock && gr.nblk <= kFusedBlocks &&
              a.nmember <= kMergedMembers && !fields->budget;
   a.prm_part = reinterpret_cast<float*>(w + L.prm);
   a.bud_part = reinterpret_cast<double*>(w + L.bud);
@@ -1440,14 +1397,15 @@ hipError_t batch_stack() {
   return e;
 }
 
-// Largest grid that is co-resident on the current device for a kernel.
+// Largest grid that is co-resident on the current device for a kernel, as far as the
+// workspace has words for it.
 template <typename K>
 int64_t coresident_blocks(K kernel) {
   int dev = 0, ncu = 0, per_cu = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 0;
   if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock, 0) != hipSuccess) return 0;
-  return (int64_t)per_cu * ncu;
+  return std::min<int64_t>((int64_t)per_cu * ncu, kFusedBlocks);
 }
 
 template <int KX>
@@ -1494,8 +1452,7 @@ int launch_fwd(const KArgs& a, hipStream_t s) {
     // call.
     if (a.nblk > kSegLocalMask)
       return fail(SPEEDY_ERR_CAPACITY, "speedy: more than 2^20 workgroups (2^28 columns) in one call");
-    const WsLayout L = ws_layout(make_grid(a.ncol, 1, a.nmember), (int32_t)a.nmember);
-    KArgs* desc = VJP || !kByValue<KX> ? reinterpret_cast<KArgs*>(reinterpret_cast<char*>(a.gen) + L.desc) : nullptr;
+    KArgs* desc = VJP || !kByValue<KX> ? static_cast<KArgs*>(a.desc) : nullptr;
     const KArgs* segs = desc;
     const uint32_t* table = nullptr;
     if (a.level_set < 0) {
@@ -1584,7 +1541,7 @@ int speedy_abi_version(void) { return SPEEDY_ABI_VERSION; }
 size_t speedy_workspace_bytes(int32_t nlon, int32_t nlat, int32_t nmember) {
   if (nlon <= 0 || nlat <= 0 || nmember <= 0) return 0;
   if ((int64_t)nlon * nlat * nmember >= ((int64_t)1 << 31) - kBlock) return 0;
-  return ws_layout(make_grid(nlon, nlat, nmember), nmember).total;
+  return ws_layout(make_grid(nlon, nlat, nmember), nmember, sizeof(KArgs)).total;
 }
 
 int speedy_workspace_init(void* workspace, size_t workspace_bytes, void* stream) {
@@ -1813,9 +1770,10 @@ size_t speedy_batch_desc_bytes(const SpeedySegment* segs, int32_t nseg) {
 int speedy_read_level_sets(const void* workspace, size_t workspace_bytes, int32_t nmember, uint32_t* out,
                            void* stream) {
   if (!workspace || !out || nmember <= 0) return fail(SPEEDY_ERR_ARG, "speedy: bad arguments");
-  if (workspace_bytes < 256 + align256(sizeof(uint32_t) * (size_t)nmember))
+  const size_t at = kHeaderBytes + kTagBytes;   // WsLayout::last_s of every grid
+  if (workspace_bytes < at + align256(sizeof(uint32_t) * (size_t)nmember))
     return fail(SPEEDY_ERR_WORKSPACE, "speedy: workspace too small");
-  hipError_t e = hipMemcpyAsync(out, static_cast<const char*>(workspace) + 256, sizeof(uint32_t) * nmember,
+  hipError_t e = hipMemcpyAsync(out, static_cast<const char*>(workspace) + at, sizeof(uint32_t) * nmember,
                                 hipMemcpyDeviceToHost, (hipStream_t)stream);
   if (e == hipSuccess) e = hipStreamSynchronize((hipStream_t)stream);
   if (e != hipSuccess) return fail(SPEEDY_ERR_HIP, std::string("speedy: copy failed: ") + hipGetErrorString(e));
@@ -1900,8 +1858,8 @@ extern "C" size_t speedy_noalloc_max_bytes(void) { return kNoAllocScratchBytes; 
 extern "C" int speedy_fwd_noalloc(const SpeedyFields* fields, const SpeedyVertical* vert, const SpeedyParams* params,
                                   const SpeedyDate* date, int32_t nlon, int32_t nlat, int32_t nmember, uint32_t flags,
                                   uint32_t term_mask, int32_t level_set, void* stream) {
-  const size_t need = speedy_workspace_bytes(nlon, nlat, nmember);
-  if (need == 0) return fail(SPEEDY_ERR_ARG, "speedy_fwd_noalloc: bad grid");
+  if (speedy_workspace_bytes(nlon, nlat, nmember) == 0) return fail(SPEEDY_ERR_ARG, "speedy_fwd_noalloc: bad grid");
+  const size_t need = ws_layout(make_grid(nlon, nlat, nmember), nmember, sizeof(KArgs), 0).total;
   if (need > kNoAllocScratchBytes)
     return fail(SPEEDY_ERR_CAPACITY, "speedy_fwd_noalloc: the call needs " + std::to_string(need) +
                                          " bytes of workspace, above the " + std::to_string(kNoAllocScratchBytes) +
@@ -1924,7 +1882,7 @@ extern "C" int speedy_fwd_noalloc(const SpeedyFields* fields, const SpeedyVertic
   }
   KArgs a;
   if (int rc = prepare(fields, vert, params, date, nlon, nlat, nmember, flags, term_mask, level_set, ws,
-                       kNoAllocScratchBytes, a))
+                       kNoAllocScratchBytes, a, 0))
     return rc;
   a.flags |= kFlagBatchRoute;
   g_last_error.clear();
