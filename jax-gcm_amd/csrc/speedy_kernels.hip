@@ -53,8 +53,6 @@ constexpr uint32_t kFlagBatchRoute = 1u << 31;
 // takes one wave about 10 us, so waiting out a short kernel of another stream is
 // cheaper than replacing the blocks it holds up.
 constexpr uint32_t kHelpAfter = 256;
-// Bound of block 0's wait for the last block to publish (hours: a wave always exits).
-constexpr uint32_t kSpinLimit = 1u << 31;
 
 struct Divisor {          // n / d for n < 2^32 by multiply-high + one correction step
   uint32_t d, m;          // m = floor(2^32 / d) (unused when d == 1)
@@ -382,6 +380,17 @@ __device__ __forceinline__ uint64_t* param_words(const KArgs& a) {
   return reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(a.gen) + kHeaderBytes + kWordBytes);
 }
 
+// The call's results are invalid (speedy_workspace_status).
+__device__ __forceinline__ void set_error(const KArgs& a) {
+  __hip_atomic_store(a.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Between two polls of a wait: about 4 us, in short ones nothing to speak of.
+__device__ __forceinline__ void poll_pause(bool brief) {
+  if (brief) __builtin_amdgcn_s_sleep(1);
+  else __builtin_amdgcn_s_sleep(100);
+}
+
 // One poll of the published words of the blocks covering member m: the OR of their
 // level bits, and whether any word is not of this call yet.  By one wave, all lanes
 // active throughout: lanes past the last word read it again (OR is idempotent).
@@ -429,16 +438,16 @@ __device__ __forceinline__ uint32_t collect_fused(const KArgs& a, uint32_t tag, 
 // Block 0: every member's S to last_s (speedy_read_level_sets), then the next
 // generation, once every block of the call has published (and so read this one).
 __device__ __forceinline__ void finish_generation(const KArgs& a, uint32_t gen, uint32_t tag) {
+  uint32_t spins = 0;
   for (uint32_t m = 0; m < a.nmember; ++m) {
     bool missing;
     uint32_t v = poll_words(a, tag, m, missing);
-    for (uint32_t spins = 0; missing; ++spins) {
+    while (missing) {
       if (spins >= kSpinLimit) {
-        __hip_atomic_store(a.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        set_error(a);
         break;
       }
-      if (spins < kHelpAfter) __builtin_amdgcn_s_sleep(1);
-      else __builtin_amdgcn_s_sleep(100);
+      poll_pause(spins++ < kShortPolls);
       v = poll_words(a, tag, m, missing);
     }
     gst(a.last_s, m, v);
@@ -763,8 +772,10 @@ __device__ __forceinline__ void count_in(const KArgs& a, const BlockPos& b, uint
     uint32_t before = 0u;
     if ((threadIdx.x & 63u) == 0u)
       before = __hip_atomic_fetch_add(&a.arrived[m], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const bool last = __builtin_amdgcn_readfirstlane(before) == n - 1u;
+    before = __builtin_amdgcn_readfirstlane(before);
+    const bool last = before == n - 1u;
     if (last) __hip_atomic_store(&a.arrived[m], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (before >= n) set_error(a);   // more than there are: calls overlap on this workspace
     s_last[j] = last;
   }
 }
@@ -910,12 +921,18 @@ __device__ __forceinline__ void budget_reduce_body(const KArgs& a, uint32_t m) {
   }
 }
 
-// One partial, once it is of this call.
-__device__ __forceinline__ float tagged_partial(const KArgs& a, size_t at, uint32_t tag) {
-  uint64_t w;
-  do w = __hip_atomic_load(param_words(a) + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  while ((uint32_t)(w >> 32) != tag);
-  return __builtin_bit_cast(float, (uint32_t)w);
+// A block's partials of the parameter gradients, once they are of this call; NaN, and the
+// error word set, if they do not come.
+__device__ __forceinline__ void tagged_partials(const KArgs& a, size_t at, uint32_t tag, uint32_t& left,
+                                                float x[VJP_NPARAM]) {
+  uint64_t w[VJP_NPARAM];
+  const bool here = await_words(
+      tag, left,
+      [&](int i) { return __hip_atomic_load(param_words(a) + at + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); },
+      [](bool brief) { poll_pause(brief); }, w);
+  if (!here) set_error(a);
+#pragma unroll
+  for (int i = 0; i < VJP_NPARAM; ++i) x[i] = here ? __builtin_bit_cast(float, (uint32_t)w[i]) : __builtin_nanf("");
 }
 
 template <bool TAGGED>
@@ -923,17 +940,25 @@ __device__ __forceinline__ void param_reduce_body(const KArgs& a, uint32_t m, ui
   float acc[VJP_NPARAM];
 #pragma unroll
   for (int i = 0; i < VJP_NPARAM; ++i) acc[i] = 0.0f;
-  // (unrolled: several iterations' loads in flight; the order of the sums is the loop's)
-  if (a.ncol >= (uint32_t)kBlock) {
+  if constexpr (TAGGED) {
+    uint32_t left = kSpinLimit;
+    const uint32_t b0 = (m * a.ncol) / kBlock, b1 = (m * a.ncol + a.ncol - 1u) / kBlock;
+#pragma unroll 1
+    for (uint32_t b = b0 + threadIdx.x; b <= b1; b += kBlock) {   // twice at most (kFusedBlocks)
+      const uint32_t j = m - divq(b * kBlock, a.dcol);
+      float x[VJP_NPARAM];
+      tagged_partials(a, ((size_t)b * 2 + j) * VJP_NPARAM, tag, left, x);
+#pragma unroll
+      for (int i = 0; i < VJP_NPARAM; ++i) acc[i] += x[i];
+    }
+  } else if (a.ncol >= (uint32_t)kBlock) {
+    // (unrolled: several iterations' loads in flight; the order of the sums is the loop's)
     const uint32_t b0 = (m * a.ncol) / kBlock, b1 = (m * a.ncol + a.ncol - 1u) / kBlock;
 #pragma unroll 4
     for (uint32_t b = b0 + threadIdx.x; b <= b1; b += kBlock) {
       const uint32_t j = m - divq(b * kBlock, a.dcol);
 #pragma unroll
-      for (int i = 0; i < VJP_NPARAM; ++i) {
-        const size_t at = ((size_t)b * 2 + j) * VJP_NPARAM + i;
-        acc[i] += TAGGED ? tagged_partial(a, at, tag) : gld(a.prm_part, at);
-      }
+      for (int i = 0; i < VJP_NPARAM; ++i) acc[i] += gld(a.prm_part, ((size_t)b * 2 + j) * VJP_NPARAM + i);
     }
   } else {
 #pragma unroll 4

@@ -41,6 +41,27 @@ constexpr uint32_t call_tag(uint32_t gen) { return gen + 1u; }
 constexpr uint32_t next_generation(uint32_t gen) { return gen + 2u == 0u ? 0u : gen + 1u; }
 constexpr uint64_t tagged_word(uint32_t tag, uint32_t value) { return (uint64_t)tag << 32 | value; }
 
+// Polls of a wait inside a launch, for the whole of it, before the call gives up and sets
+// the error word: about a minute, nearly all of them 4 us apart.  Other work may hold the
+// GPU that long before a call's last block runs; a wait that lasts longer waits for a word
+// that cannot come (calls that overlap on one workspace).
+constexpr uint32_t kSpinLimit = 1u << 24;
+constexpr uint32_t kShortPolls = 256;   // the first ones: about 1 us apart
+
+// The N words w[i] = load(i), all read again until each carries `tag`.  Takes its polls from
+// `left`; with none left it reads them once and returns false where one has not come.
+template <int N, typename Load, typename Pause>
+constexpr bool await_words(uint32_t tag, uint32_t& left, Load load, Pause pause, uint64_t (&w)[N]) {
+  for (;;) {
+    for (int i = 0; i < N; ++i) w[i] = load(i);
+    uint32_t stale = 0u;
+    for (int i = 0; i < N; ++i) stale |= (uint32_t)(w[i] >> 32) ^ tag;
+    if (!stale) return true;
+    if (left == 0u) return false;
+    pause(kSpinLimit - left-- < kShortPolls);
+  }
+}
+
 struct Grid {
   uint32_t ncol, ntot, nblk, ls_blocks, chunk, jmax;
 };

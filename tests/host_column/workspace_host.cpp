@@ -26,4 +26,20 @@ uint32_t ws_call_tag(uint32_t gen) { return call_tag(gen); }
 uint32_t ws_next_generation(uint32_t gen) { return next_generation(gen); }
 uint64_t ws_tagged_word(uint32_t tag, uint32_t value) { return tagged_word(tag, value); }
 
+
+// await_words on three words, the middle one of which carries `tag` from its polls-th
+// second read on: {came, reads, short pauses, polls left}
+void ws_await(uint32_t tag, uint32_t left, uint64_t polls, uint64_t* out) {
+  uint64_t reads = 0, brief = 0, w[3] = {};
+  const bool came = await_words(
+      tag, left,
+      [&](int i) {
+        if (i == 0) ++reads;
+        return tagged_word(i == 1 && reads <= polls ? tag - 1u : tag, 7u);
+      },
+      [&](bool b) { brief += b; }, w);
+  out[0] = came; out[1] = reads; out[2] = brief; out[3] = left;
+}
+uint32_t ws_spin_limit() { return kSpinLimit; }
+
 }  // extern "C"

@@ -132,3 +132,27 @@ def test_budgets_of_blocks_on_two_members(nlon, nlat, nmember):
         alone = phys.last_budgets.cpu().numpy()[0]
         # the tendencies of the two routes differ in their last float32 bits
         assert np.all(np.abs(got[m] - alone) <= 2e-5 * np.abs(alone) + 2e-5 * np.abs(got[m]).max())
+
+
+@pytest.mark.parametrize("kx", [7, 8])
+def test_counts_out_of_step_are_reported(kx):
+    """Calls that overlap on one workspace can leave the count of arrived blocks where no
+    block is the last; such a call ends, and the workspace's status says that its
+    results are invalid.  The count is set from the host here."""
+    import torch
+    from jcm_amd.speedy_physics import SpeedyPhysics
+    run = Calls(SpeedyPhysics())
+    case = synthetic.make_case(128, 64, kx, seed=68, land=True)
+    cot = _cot(case, 69)
+    ws = run.workspace((128, 64, 1))
+    words = ws.view(torch.int32)
+    fresh = run(ws, case, cot)
+    status = lambda: (_native.check(run.lib.speedy_workspace_status(  # noqa: E731
+        ws.data_ptr(), ws.numel(), ctypes.byref(st), run.phys._stream()), "status"), int(st.value))[1]
+    st = ctypes.c_uint32(0)
+    assert status() == 0 and int(words[2]) == 0
+    words[2] = 32                        # as many as the grid has blocks
+    run(ws, case, cot)
+    assert status() == 1
+    _same(run(ws, case, cot), fresh)     # the query reset the workspace
+    assert status() == 0

@@ -99,3 +99,22 @@ def test_tags_return_only_after_every_other(ws):
     for tag, bits in ((1, 0xFFFF), (0x8001, 0xFC), ((1 << 32) - 1, 0)):
         w = ws.ws_tagged_word(tag, bits)
         assert w >> 32 == tag and w & 0xFFFFFFFF == bits
+
+
+def test_a_wait_ends(ws):
+    """A wait for a word that does not come gives up, and the waits after it look only
+    once: a launch always ends."""
+    ws.ws_await.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint64, ctypes.POINTER(ctypes.c_uint64)]
+    limit = ws.ws_spin_limit()
+    assert limit * 4e-6 < 120.0     # seconds: 4 us a poll
+
+    def wait(left, polls):
+        out = (ctypes.c_uint64 * 4)()
+        ws.ws_await(9, left, polls, out)
+        return tuple(out)
+
+    assert wait(limit, 0) == (1, 1, 0, limit)
+    assert wait(limit, 3) == (1, 4, 3, limit - 3)
+    assert wait(limit, 1 << 40) == (0, limit + 1, 256, 0)
+    assert wait(0, 1 << 40) == (0, 1, 0, 0)
+    assert wait(0, 0) == (1, 1, 0, 0)
