@@ -19,9 +19,11 @@
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstring>
+#include <exception>
 #include <string>
 #include <vector>
 
@@ -78,6 +80,13 @@ PyObject* attr(PyObject* o, PyObject* name) { return PyObject_GetAttr(o, name); 
 PyObject* general() {
   PyErr_Clear();
   Py_RETURN_NONE;
+}
+
+// The exception in flight (an allocation that failed, a tensor torch objects to) as the
+// Python exception that torch's own functions raise for it: torch.OutOfMemoryError stays one.
+PyObject* raised() {
+  torch::translate_exception_to_python(std::current_exception());
+  return nullptr;
 }
 
 bool modes_active() {
@@ -345,9 +354,8 @@ PyObject* fwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
     PyObject* r = t.p;
     t.p = nullptr;
     return r;
-  } catch (const std::exception& e) {   // an allocation that failed, a tensor torch objects to
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
+  } catch (...) {
+    return raised();
   }
 }
 
@@ -397,9 +405,8 @@ PyObject* fwd_vjp(PyObject*, PyObject* const* args, Py_ssize_t n) {
     PyObject* r = t.p;
     t.p = nullptr;
     return r;
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
+  } catch (...) {
+    return raised();
   }
 }
 
@@ -515,9 +522,8 @@ PyObject* dynamics_to_physics(PyObject*, PyObject* const* args, Py_ssize_t n) {
     PyObject* r = t.p;
     t.p = nullptr;
     return r;
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
+  } catch (...) {
+    return raised();
   }
 }
 
@@ -566,9 +572,8 @@ PyObject* to_dynamics(PyObject*, PyObject* const* args, Py_ssize_t n) {
     PyObject* res = r.p;
     r.p = nullptr;
     return res;
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
+  } catch (...) {
+    return raised();
   }
 }
 

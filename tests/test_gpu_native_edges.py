@@ -17,3 +17,54 @@ def test_diagnostics_are_asked_for_by_truth_value(value):
     for _ in range(3):   # the first call makes the workspace, the others are native
         _, data = phys.compute_tendencies(st, fo, ge, da)
         assert (data is not None) == bool(value)
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("call", ["fwd", "vjp", "d2p", "t2d"])
+def test_out_of_memory_keeps_its_type(call, native, monkeypatch):
+    """A caller that catches torch.OutOfMemoryError, to free something or to go on with
+    fewer members, still can.  The allocator's own limit stands in for a full card."""
+    import torch
+    from jcm_amd import _native
+    from jcm_amd import transforms as T
+    from jcm_amd.physics_interface import PhysicsTendency
+    from jcm_amd.speedy_physics import SpeedyPhysics
+    if call in ("fwd", "vjp"):   # fields of 16 MiB
+        st, fo, ge, da, cot = _case(nmember=128, nlon=64, nlat=64)
+        phys = SpeedyPhysics()
+        run = ((lambda: phys.compute_tendencies(st, fo, ge, da)) if call == "fwd" else
+               (lambda: phys.compute_tendencies_vjp(st, fo, ge, da, cot)))
+    else:
+        grid = T.SpectralGrid.truncation(213)
+        z = lambda *s: torch.zeros(s, device="cuda")  # noqa: E731
+        dyn = T.PrimitiveEquations(z(16) + 250.0, z(*grid.modal_shape),
+                                   T.CoordinateSystem(grid, T.SigmaCoordinates(np.linspace(0, 1, 17))))
+        if call == "d2p":
+            m = z(16, *grid.modal_shape)
+            state = T.DynamicsState(m, m, m, z(*grid.modal_shape), {"specific_humidity": m})
+            run = lambda: T.dynamics_state_to_physics_state(state, dyn)  # noqa: E731
+        else:
+            x = z(16, *grid.nodal_shape)
+            tend = PhysicsTendency(x, x, x, x)
+            run = lambda: T.physics_tendency_to_dynamics_tendency(tend, dyn)  # noqa: E731
+    run()                               # workspaces and plans
+    torch.cuda.synchronize()
+    if not native:
+        monkeypatch.setattr(_native, "host", None)
+        monkeypatch.setattr(T, "host", None)
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
+    held = []
+    try:
+        for size in (4 << 20, (1 << 20) + 512):   # what the allocator still has
+            with pytest.raises(torch.OutOfMemoryError):
+                while True:
+                    held.append(torch.empty(size, dtype=torch.uint8, device="cuda"))
+        with pytest.raises(torch.OutOfMemoryError):
+            run()
+    finally:
+        del held
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    run()
+    torch.cuda.synchronize()
