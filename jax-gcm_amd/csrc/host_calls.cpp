@@ -42,12 +42,14 @@ decltype(&speedy_dynamics_to_physics) p_d2p = nullptr;
 decltype(&speedy_physics_to_dynamics) p_p2d = nullptr;
 decltype(&speedy_physics_tendency_to_dynamics) p_t2d = nullptr;
 
-// One parameter of SpeedyParams: its group (index into the group names), name and place.
+// One parameter of SpeedyParams: its group (index into the group names), name, place and
+// kind.  A flag is a bool: Parameters.to_abi refuses any other value for one.
+enum ParamKind { kFloat = 0, kFlag = 1, kInt = 2 };
 struct ParamSlot {
   int group;
   PyObject* name;
   size_t offset;
-  bool is_int;
+  int kind;
 };
 std::vector<PyObject*> g_groups;
 std::vector<ParamSlot> g_params;
@@ -165,9 +167,9 @@ bool pack_params(PyObject* parameters, SpeedyParams* p) {
     PyObject* v = PyDict_GetItemWithError(dicts[s.group], s.name);
     if (!v) return false;
     char* dst = reinterpret_cast<char*>(p) + s.offset;
-    if (s.is_int) {
+    if (s.kind != kFloat) {
       long x;
-      if (!as_long(v, &x)) return false;
+      if ((s.kind == kFlag && !PyBool_Check(v)) || !as_long(v, &x)) return false;
       const int32_t y = (int32_t)x;
       std::memcpy(dst, &y, sizeof(y));
     } else {
@@ -578,17 +580,17 @@ PyObject* to_dynamics(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // ---------------------------------------------------------------- module
-// bind_physics(fwd, fwd_vjp, diag_rows, groups, [(group index, name, offset, is_int)])
+// bind_physics(fwd, fwd_vjp, diag_rows, groups, [(group index, name, offset, kind)])
 PyObject* bind_physics(PyObject*, PyObject* args) {
   PyObject *a, *b, *c, *groups, *slots;
   if (!PyArg_ParseTuple(args, "OOOO!O!", &a, &b, &c, &PyTuple_Type, &groups, &PyList_Type, &slots)) return nullptr;
   std::vector<ParamSlot> ps;
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(slots); ++i) {
-    int g, is_int;
+    int g, kind;
     Py_ssize_t off;
     const char* name;
-    if (!PyArg_ParseTuple(PyList_GET_ITEM(slots, i), "isnp", &g, &name, &off, &is_int)) return nullptr;
-    ps.push_back({g, PyUnicode_InternFromString(name), (size_t)off, is_int != 0});
+    if (!PyArg_ParseTuple(PyList_GET_ITEM(slots, i), "isni", &g, &name, &off, &kind)) return nullptr;
+    ps.push_back({g, PyUnicode_InternFromString(name), (size_t)off, kind});
   }
   g_groups.clear();
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(groups); ++i) {

@@ -109,8 +109,9 @@ def address(fn) -> int:
 def _bind_host(lib):
     from .params import _GROUPS, Parameters
     p = Parameters.default()
-    ints = {n for n, t in SpeedyParams._fields_ if t is ctypes.c_int32}
-    slots = [(g, n, getattr(SpeedyParams, n).offset, n in ints)
+    # 0 a float, 1 a flag, 2 an integer
+    kinds = {n: 0 if t is not ctypes.c_int32 else 2 if n == "co2_year_ref" else 1 for n, t in SpeedyParams._fields_}
+    slots = [(g, n, getattr(SpeedyParams, n).offset, kinds[n])
              for g, grp in enumerate(_GROUPS) for n in vars(getattr(p, grp))]
     host.bind_physics(address(lib.speedy_fwd), address(lib.speedy_fwd_vjp), address(lib.speedy_diag_rows), _GROUPS, slots)
 

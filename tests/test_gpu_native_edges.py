@@ -68,3 +68,22 @@ def test_out_of_memory_keeps_its_type(call, native, monkeypatch):
         torch.cuda.set_per_process_memory_fraction(1.0)
     run()
     torch.cuda.synchronize()
+
+
+def test_parameter_types_are_judged_alike_on_every_call():
+    """A flag that is not a bool is refused by Parameters.to_abi, so also once the grid's
+    workspace exists; values that it converts are taken."""
+    from jcm_amd import Parameters
+    from jcm_amd.speedy_physics import SpeedyPhysics
+    st, fo, ge, da, _ = _case()
+    for group, name, value in [("surface_flux", "lscasym", 1), ("surface_flux", "lskineb", 0),
+                               ("forcing", "increase_co2", 1)]:
+        phys = SpeedyPhysics(parameters=Parameters.default().replace(**{group: {name: value}}))
+        for _ in range(3):
+            with pytest.raises(TypeError):
+                phys.compute_tendencies(st, fo, ge, da)
+    for group, name, value in [("forcing", "co2_year_ref", 1960.0), ("forcing", "co2_year_ref", True),
+                               ("convection", "rhbl", 1), ("convection", "rhbl", True), ("convection", "rhbl", "0.9")]:
+        phys = SpeedyPhysics(parameters=Parameters.default().replace(**{group: {name: value}}))
+        for _ in range(2):
+            phys.compute_tendencies(st, fo, ge, da)
