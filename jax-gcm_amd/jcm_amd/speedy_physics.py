@@ -297,11 +297,8 @@ class SpeedyPhysics(Physics):
         hit = self._consts.get(key)
         if hit is not None and hit[0] is arr:
             return hit[1]
-        t = _device(arr, self.device)
-        if len(self._consts) > 256:
-            self._consts.clear()
-        self._consts[key] = (arr, t)
-        return t
+        t = self._consts[key] = (arr, _device(arr, self.device))
+        return t[1]
 
     def _fields(self, state: PhysicsState, forcing: ForcingData, geometry: Geometry, date: DateData,
                 keep: list):
@@ -337,6 +334,11 @@ class SpeedyPhysics(Physics):
         hit = self._fg.get(key)
         if hit is not None and hit[0] is forcing and hit[1] is geometry:
             return hit[2]
+        if len(self._consts) > 246:   # a call's eleven arrays at most are added below
+            # _fg goes with it: what it holds is not looked up here again, and the native
+            # calls take a NumPy field by its entry in _consts
+            self._consts.clear()
+            self._fg.clear()
         out, by_identity = [], True
         fmap = dict(zip(FORCING_FIELDS, ("alb0", "sice_am", "snowc_am", "soilw_am", "stl_am", "sst")))
         srcs = [(dst, getattr(forcing, src)) for src, dst in fmap.items()]

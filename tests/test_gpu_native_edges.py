@@ -87,3 +87,26 @@ def test_parameter_types_are_judged_alike_on_every_call():
         phys = SpeedyPhysics(parameters=Parameters.default().replace(**{group: {name: value}}))
         for _ in range(2):
             phys.compute_tendencies(st, fo, ge, da)
+
+
+def test_device_copies_given_back_are_made_again():
+    """The cache of device copies of NumPy fields is bounded; after it was emptied, a
+    forcing and geometry known from before find their copies again."""
+    from jcm_amd import _native, synthetic
+    from jcm_amd.speedy_physics import SpeedyPhysics
+    st, fo, ge, da, _ = _case()
+    fo = fo.copy(**{k: getattr(fo, k).cpu().numpy() for k in ("alb0", "sice_am", "snowc_am", "soilw_am", "stl_am",
+                                                              "sea_surface_temperature")})
+    phys = SpeedyPhysics()
+    native = lambda: _native.host.fwd(phys._consts, phys._workspaces, phys.parameters, *phys._where(), st, fo, ge, da, 0,  # noqa: E731,E501
+                                      _native.TERMS_ALL, -1, False)
+    phys.compute_tendencies(st, fo, ge, da)
+    assert isinstance(native(), tuple)
+    keep = []
+    for i in range(30):                  # 11 fields each
+        other = synthetic.make_case(4, 6, 8, seed=i, land=True)
+        keep.append(other)
+        phys.compute_tendencies(*other)
+        assert len(phys._consts) <= 257
+        phys.compute_tendencies(st, fo, ge, da)
+        assert isinstance(native(), tuple)
