@@ -231,6 +231,10 @@ struct PhysicsCall {
   c10::DeviceIndex dev = 0;
 
   // args: consts, workspaces, parameters, device index, stream, state, forcing, geometry, date, flags
+  //
+  // In the order of what the general path is most often taken for: a call that is refused
+  // has cost little (a climatology or a new NumPy array, the first field or two; a new
+  // grid, no packing of levels and parameters).
   bool read(PyObject* const* args) {
     std::memset(&f, 0, sizeof(f));
     long device, fl;
@@ -245,12 +249,8 @@ struct PhysicsCall {
         !as_long(PyTuple_GET_ITEM(shape.p, 0), &kx) || !as_long(PyTuple_GET_ITEM(shape.p, 1), &ix) ||
         !as_long(PyTuple_GET_ITEM(shape.p, 2), &il) || kx < 1 || kx > SPEEDY_KX_MAX)
       return false;
-    if (!pack_vertical(geometry, (int)kx, &v) || !pack_date(args[8], &d) || !pack_params(args[2], &p)) return false;
-    Ref lfl(attr(forcing, s_lfluxland));
-    const int land = lfl ? PyObject_IsTrue(lfl.p) : -1;
-    if (land < 0) return false;
-    if (land) flags |= SPEEDY_FLAG_LFLUXLAND;
     keep.reserve(24);
+    if (!read_shared(args[0], forcing, geometry)) return false;
     PyObject* const names[5] = {s_temperature, s_u_wind, s_v_wind, s_specific_humidity, s_geopotential};
     const float** const dst[5] = {&f.t, &f.u, &f.v, &f.q, &f.phi};
     for (int i = 0; i < 5; ++i) {
@@ -274,6 +274,19 @@ struct PhysicsCall {
     keep.push_back(THPVariable_Unpack(ps.p));
     if (keep.back().numel() != nmember * ix * il) return false;
     f.ps = cptr(keep.back());
+    Ref key(Py_BuildValue("(lllO)", ix, il, (long)nmember, args[4]));
+    PyObject* w = key ? PyDict_GetItemWithError(args[1], key.p) : nullptr;
+    if (!w || !THPVariable_Check(w)) return false;
+    ws = THPVariable_Unpack(w);
+    Ref lfl(attr(forcing, s_lfluxland));
+    const int land = lfl ? PyObject_IsTrue(lfl.p) : -1;
+    if (land < 0) return false;
+    if (land) flags |= SPEEDY_FLAG_LFLUXLAND;
+    return pack_vertical(geometry, (int)kx, &v) && pack_date(args[8], &d) && pack_params(args[2], &p);
+  }
+
+  // the forcing's and the geometry's fields
+  bool read_shared(PyObject* consts, PyObject* forcing, PyObject* geometry) {
     PyObject* const two[9] = {s_alb0, s_sice_am, s_snowc_am, s_soilw_am, s_stl_am, s_sea_surface_temperature,
                               s_fmask, s_orog, s_phis0};
     const float** const dst2[9] = {&f.alb0, &f.sice_am, &f.snowc_am, &f.soilw_am, &f.stl_am, &f.sst,
@@ -281,21 +294,17 @@ struct PhysicsCall {
     for (int i = 0; i < 9; ++i) {
       Ref o(attr(i < 6 ? forcing : geometry, two[i]));
       at::Tensor t;
-      if (!shared_field(o.p, args[0], dev, {ix, il}, &t)) return false;
+      if (!shared_field(o.p, consts, dev, {ix, il}, &t)) return false;
       *dst2[i] = cptr(t);
       keep.push_back(std::move(t));
     }
     for (int i = 0; i < 2; ++i) {
       Ref o(attr(geometry, i ? s_coa : s_sia));
       at::Tensor t;
-      if (!shared_field(o.p, args[0], dev, {il}, &t)) return false;
+      if (!shared_field(o.p, consts, dev, {il}, &t)) return false;
       (i ? f.coa : f.sia) = cptr(t);
       keep.push_back(std::move(t));
     }
-    Ref key(Py_BuildValue("(lllO)", ix, il, (long)nmember, args[4]));
-    PyObject* w = key ? PyDict_GetItemWithError(args[1], key.p) : nullptr;
-    if (!w || !THPVariable_Check(w)) return false;
-    ws = THPVariable_Unpack(w);
     return true;
   }
 
