@@ -150,6 +150,12 @@ SPD_HD void qsat_grad(R ta, R q, R& dq_dt, R& ps_dq_dps) {
   ps_dq_dps = -gq;
 }
 
+// acc += a * b where `on`.  The choice is made on the sum and not on a factor: a term that
+// is off adds nothing, whatever its other factor is (a level whose humidity is not finite
+// must not reach the gradients of the levels beside it through terms that are off).
+template <typename R>
+SPD_HD void add_if(bool on, R& acc, R a, R b) { acc = sel(on, acc + a * b, acc); }
+
 // Adjoint of radset4 (longwave_radiation.py:216-225): returns d/d temp of
 // sum_b a_fb[b] * fb[b].  jnp.clip(temp, 200, 320) = min(max(temp, 200), 320).
 template <typename R>
@@ -517,11 +523,12 @@ SPD_HD void surface_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const 
     a_den1 += a_Dn * s.chl * (R(CP) + R(ALHC) * t.qs1);
     a_qs1 += a_Dn * s.chl * t.den1 * R(ALHC);
     {
-      const R a_qs1p = sel(t.evap0a > R(0.0), a_qs1 * c.soilw, R(0.0));
-      a_qsat00 += -a_qs1p;
+      const bool wet = t.evap0a > R(0.0);
+      const R a_qs1p = a_qs1 * c.soilw;
+      a_qsat00 += sel(wet, -a_qs1p, R(0.0));
       qsat_grad(t.tskin0 + R(1.0), t.qs1p, dqt, dqp);
-      a_tskin += a_qs1p * dqt;
-      a_psq += a_qs1p * dqp;
+      add_if(wet, a_tskin, a_qs1p, dqt);
+      add_if(wet, a_psq, a_qs1p, dqp);
     }
     a_hfl0 += a_hflc;
     a_tskin += -a_hflc * t.clamb;
@@ -652,7 +659,7 @@ SPD_HD void shortwave_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, cons
   const bool csw = u.compute_sw != 0u;
   R a_dfabs[KX];
 #pragma unroll
-  for (int k = 0; k < KX; ++k) a_dfabs[k] = sel(csw, ct.dt[k], R(0.0)) * v.grdscp[k] * rps;
+  for (int k = 0; k < KX; ++k) a_dfabs[k] = sel(csw, ct.dt[k] * v.grdscp[k] * rps, R(0.0));
   R a_tau0[KX], a_tau1[KX], a_f1[KX], a_f2[KX], a_Rf[KX], a_fu[KX], a_t22[KX];
 #pragma unroll
   for (int k = 0; k < KX; ++k) {
@@ -764,9 +771,9 @@ SPD_HD void vdiff_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const Sp
   for (int k = 2; k < KX - 2; ++k) {
     const R d = a.rh[k + 1] - a.rh[k];
     const bool on = (d >= u.vd_drh0[k]) & (((u.vd_on >> k) & 1u) != 0u);
-    const R a_fq = sel(on, ct.dq[k] * u.rsig[k] - ct.dq[k + 1] * u.rsig[k + 1], R(0.0));
-    g.qsat[k] += a_fq * u.vd_fq[k] * d;
-    const R a_d = a_fq * u.vd_fq[k] * a.qsat[k];
+    const R a_fq = (ct.dq[k] * u.rsig[k] - ct.dq[k + 1] * u.rsig[k + 1]) * u.vd_fq[k];
+    add_if(on, g.qsat[k], a_fq, d);
+    const R a_d = sel(on, a_fq * a.qsat[k], R(0.0));
     g.rh[k + 1] += a_d;
     g.rh[k] += -a_d;
   }
@@ -778,11 +785,11 @@ SPD_HD void vdiff_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, const Sp
   const R rsA = u.rsig[NL1 - 1], rsB = u.rsig[KX - 1];
   const R a_fq2 = ct.dq[NL1 - 1] * rsA - ct.dq[KX - 1] * rsB;
   const R a_dmse = sel(up, (ct.dt[NL1 - 1] * rsA - ct.dt[KX - 1] * rsB) * fcnv * u.fshcse, R(0.0));
-  const R a_up = sel(up & (drh >= R(0.0)), a_fq2 * fcnv * u.fshcq, R(0.0));
-  const R a_dn = sel(!up & (drh > u.drh0), a_fq2 * u.fvdiq2, R(0.0));
-  g.qsat[KX - 1] += a_up * drh;
-  g.qsat[NL1 - 1] += a_dn * drh;
-  const R a_drh = a_up * a.qsat[KX - 1] + a_dn * a.qsat[NL1 - 1];
+  const bool mix_up = up & (drh >= R(0.0)), mix_dn = !up & (drh > u.drh0);
+  const R a_up = a_fq2 * fcnv * u.fshcq, a_dn = a_fq2 * u.fvdiq2;
+  add_if(mix_up, g.qsat[KX - 1], a_up, drh);
+  add_if(mix_dn, g.qsat[NL1 - 1], a_dn, drh);
+  const R a_drh = sel(mix_up, a_up * a.qsat[KX - 1], sel(mix_dn, a_dn * a.qsat[NL1 - 1], R(0.0)));
   g.se[KX - 1] += a_dmse;
   g.se[NL1 - 1] += -a_dmse;
   g.Q[KX - 1] += a_dmse * R(ALHC);
@@ -862,7 +869,7 @@ SPD_HD void condensation_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, c
     const R a_dqa = sel(on, a_dq * u.rtlsc, R(0.0));
     g.qsat[k] += a_dqa * u.rhref[k];
     g.Q[k] += -a_dqa;
-    g.prm[VJP_RHLSC] += a_dqa * a.qsat[k] * u.rhref_d[k];
+    add_if(on, g.prm[VJP_RHLSC], a_dqa * a.qsat[k], u.rhref_d[k]);
   }
   g.ps += a_psa2 * R(2.0) * ps;
 }
@@ -925,9 +932,10 @@ SPD_HD void convection_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, con
 #pragma unroll
   for (int k = 0; k < KX - 1; ++k) {
     const R a_fsq = a_dfqa[k] - a_dfqa[KX - 1];
-    const R a_s = sel(t.delq[k] > R(0.0), a_fsq * p.smf, R(0.0));
-    a_cbmf += a_s * t.delq[k];
-    const R a_delq = a_s * a.cbmf;
+    const bool dry = t.delq[k] > R(0.0);
+    const R a_s = a_fsq * p.smf;
+    add_if(dry, a_cbmf, a_s, t.delq[k]);
+    const R a_delq = sel(dry, a_s * a.cbmf, R(0.0));
     g.qsat[k] += a_delq * p.rhil;
     g.Q[k] += -a_delq;
     const R as = sel(k >= iptop, a_dfse[k], R(0.0)), aq = sel(k >= iptop, a_dfqa[k], R(0.0));
@@ -960,9 +968,9 @@ SPD_HD void convection_adj(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, con
       g.se[j] += pS * t.en[j];
       g.Q[j] += pQ * t.en[j];
       if (j >= 1 && j <= KX - 2) {
-        const R ae = sel(j >= iptop, a_en * u.entr[j], R(0.0));
-        g.ps += ae * a.cbmf;
-        a_cbmf += ae * ps;
+        const R ae = a_en * u.entr[j];
+        add_if(j >= iptop, g.ps, ae, a.cbmf);
+        add_if(j >= iptop, a_cbmf, ae, ps);
       }
     }
     a_fmass += pm;
@@ -1091,7 +1099,7 @@ SPD_HD void phase_b2_taped(const ColumnIn<R, KX>& c, const PhaseA<R, KX>& a, uin
   shortwave<R, KX, false>(c, a, S, p, v, u, b, flux_h, t.sw);
 #pragma unroll
   for (int k = 0; k < KX; ++k)   // tsw[k] = dfabs[k] grdscp[k] / ps
-    g.rps += sel(u.compute_sw != 0u, ct.dt[k], R(0.0)) * t.sw.dfabs[k] * v.grdscp[k];
+    add_if(u.compute_sw != 0u, g.rps, ct.dt[k] * t.sw.dfabs[k], R(v.grdscp[k]));
   R tsfc;
   surface<R, KX, false>(c, a, p, v, u, flags, b, tsfc, t.sf);
   b.flux_h[0] = flux_h[0]; b.flux_h[1] = flux_h[1]; b.rlus2 = t.sf.rlus2; b.tsfc = tsfc;
