@@ -157,18 +157,21 @@ typedef struct {
 int speedy_abi_version(void);
 
 /* Bytes of device workspace a call on this grid needs (0 if unsupported).  A
- * workspace may be reused by later calls of the same or a smaller grid. */
+ * workspace may be reused by later calls of the same or a smaller grid, one after
+ * the other: it holds the words that the workgroups of a single launch exchange,
+ * so calls that overlap need workspaces of their own. */
 size_t speedy_workspace_bytes(int32_t nlon, int32_t nlat, int32_t nmember);
 
 /* Zero a fresh workspace once (a fill kernel on `stream`); later calls leave it
  * ready for the next call. */
 int speedy_workspace_init(void *workspace, size_t workspace_bytes, void *stream);
 
-/* Status of a workspace: bit 0 is set if a call's grid barrier gave up
- * waiting (that call's results are invalid).  Reading a set bit clears it and
- * re-zeroes the whole workspace (a fill kernel on `stream`): a failed wait
- * leaves late blocks' level-set words and the generation word out of step, and
- * the next call then starts from a clean workspace. */
+/* Status of a workspace: bit 0 is set if a wait inside a call's single launch gave
+ * up (after about a minute: other work held the GPU that long, or calls overlapped
+ * on the workspace) or its count of workgroups was out of step (the latter).  That
+ * call's results are invalid.  Reading a set bit clears it and re-zeroes the whole
+ * workspace (a fill kernel on `stream`): the words and the generation may be out of
+ * step then, and the next call starts from a clean workspace. */
 int speedy_workspace_status(void *workspace, size_t workspace_bytes, uint32_t *status, void *stream);
 
 /* Rows of the diagnostic output for kx levels, and their names as a
@@ -195,8 +198,7 @@ int speedy_fwd(const SpeedyFields *fields, const SpeedyVertical *vert, const Spe
  * the same results as speedy_fwd, with the workspace taken from a static device
  * array of speedy_noalloc_max_bytes() (4 MiB) per GPU, held until the process
  * ends; a grid that needs more (speedy_workspace_bytes less the words of the single
- * launch, which it never takes) is rejected with
- * SPEEDY_ERR_CAPACITY.  The caller passes inputs and outputs as for speedy_fwd;
+ * launch, which it never takes) is rejected with SPEEDY_ERR_CAPACITY.  The caller passes inputs and outputs as for speedy_fwd;
  * no hipMalloc, hipFree or allocating call is made.  Every call on one GPU uses
  * that GPU's array: calls that overlap on one GPU (two streams, two threads)
  * race.  The call always runs through the batch kernels (one to three launches),
@@ -215,7 +217,8 @@ int speedy_fwd_noalloc(const SpeedyFields *fields, const SpeedyVertical *vert, c
  * differentiation.  g_u and g_v are zero below level kx-1 (only the surface
  * stress depends on the winds).  fields->diag must be NULL.  The parameter
  * gradients are summed over each member's columns in a fixed order
- * (deterministic), by a second small kernel on the same stream. */
+ * (deterministic): inside the launch where the grid runs as one (up to 62 members,
+ * no budgets), else by a small kernel after it on the same stream. */
 int speedy_fwd_vjp(const SpeedyFields *fields, const SpeedyAdjoint *adj, const SpeedyVertical *vert,
                    const SpeedyParams *params, const SpeedyDate *date, int32_t nlon, int32_t nlat,
                    int32_t nmember, uint32_t flags, int32_t level_set, void *workspace,
@@ -224,7 +227,9 @@ int speedy_fwd_vjp(const SpeedyFields *fields, const SpeedyAdjoint *adj, const S
 /* One request of a batched call (speedy_fwd_batch): its own grid, members,
  * fields, date and kind.  All adjoint pointers NULL: forward only; all set:
  * forward + VJP.  The workspace is the segment's own (speedy_workspace_bytes of
- * its grid, initialised once by speedy_workspace_init). */
+ * its grid, initialised once by speedy_workspace_init): a batch that runs as one
+ * launch exchanges the segment's words and counts through it, so two segments of
+ * a batch, or of batches that overlap, never share one. */
 typedef struct {
   SpeedyFields fields;          /* fields.diag must be NULL */
   SpeedyAdjoint adj;
@@ -250,9 +255,12 @@ size_t speedy_batch_desc_bytes(const SpeedySegment *segs, int32_t nseg);
  * serves continuous batching.  Writes the descriptor to host_staging (pinned
  * host memory of speedy_batch_desc_bytes, not to be reused until this call's
  * copy has completed on `stream`), copies it to `desc` (device memory of the
- * same size) and launches, in stream order: the level sets of every segment,
- * one column kernel over all segments' columns, and the parameter-gradient sums
- * of the VJP segments.  No allocation. */
+ * same size) and launches.  A batch of 7 or 8 levels whose workgroups fit on the GPU
+ * at once and whose members are at least a workgroup wide runs as one launch (and a
+ * second one for budgets, or for the sums of more than 62 members or a given level
+ * set).  Others, in stream order: the level sets of every segment, a column kernel
+ * over all forward segments' columns, one over the VJP segments', and the sums of
+ * the parameter gradients and budgets.  No allocation. */
 int speedy_fwd_batch(const SpeedySegment *segs, int32_t nseg, const SpeedyVertical *vert,
                      const SpeedyParams *params, void *desc, size_t desc_bytes, void *host_staging,
                      void *stream);

@@ -211,7 +211,6 @@ __device__ __forceinline__ void tend_after_b1(uint32_t tm, const PhaseB<float, K
   }
 }
 
-// at, aq: the partial sums of tend_after_a / tend_after_b1.
 // The diagnostics' rows (order of kDiag2D, then kDiag3D), stored as soon as they are
 // final, so that phase b2 runs beside the stores and their 90 values leave the registers:
 // the batch kernel then fits two waves per SIMD at 7 and 8 levels.  With all 140 rows
@@ -248,6 +247,7 @@ __device__ __forceinline__ void store_diag_b1(const KArgs& a, uint32_t m, uint32
   }
 }
 
+// at, aq: the partial sums of tend_after_a / tend_after_b1.
 template <int KX, bool DIAG, bool EXTRA, bool FUSED>
 __device__ __forceinline__ void store_outputs(const KArgs& a, uint32_t m, uint32_t c,
                                               const ColumnIn<float, KX>& col, const PhaseA<float, KX>& pa,
@@ -690,8 +690,8 @@ __device__ __forceinline__ void block_budget_partials(const KArgs& a, uint32_t b
   }
 }
 
-// The forward.  FUSED: single launch with the split grid barrier (all blocks
-// co-resident); otherwise S comes from the level-set kernel of the same batch.
+// The forward.  FUSED: single launch with the level-set exchange; otherwise S comes
+// from the level-set kernel of the same call or batch.
 // EXTRA: the optional verify steps and float64 budgets are compiled in (their
 // flags and pointers are then read at run time); the plain forward omits them.
 // The batched forward kernels up to eight levels keep the longwave
@@ -995,8 +995,9 @@ __device__ __forceinline__ void member_reduce_body(const KArgs& a, uint32_t m) {
 // last to be counted in for, in the order of member_reduce_body.  The count is taken
 // while the block gathers the level set, so nobody waits for it; the blocks counted
 // before are all running, and their partials carry the call's tag, so this one reads a
-// word again until it has come: no fence between blocks (fences, which write the L2
-// caches back, cost more than the launch they save).  A launch of its own took 3.9 us and
+// block's words again until they have come: no fence between blocks (fences, which write
+// the L2 caches back, cost more than the launch they save).  The five words of a block are
+// read together; one after the other took T85 23.6 -> 25.2 us in graph replays.  A launch of its own took 3.9 us and
 // a gap: 27.4 -> 26.0 us a call at T85 x 8 levels, 26.6 -> 25.3 at T42; counted at the end
 // instead, T85 29.1 -> 28.8 us back to back, and 28.0 this way.
 __device__ __forceinline__ void fused_sums(const KArgs& a, uint32_t bid, const BlockPos& b, const float prm[VJP_NPARAM],
@@ -1228,7 +1229,7 @@ __global__ __launch_bounds__(kBlock, KX <= 8 ? 2 : 1) void fwd_diag_batch_kernel
 
 // Forward + VJP segments of a batch.  Bound by VALU issue.  Built for two waves per
 // SIMD at 7 and 8 levels (at most 256 registers a lane; 56 B of scratch at 8 levels,
-// none at 7; 80 KB of LDS a block), one at 16 (512 registers, 156 KB of LDS, 232 B
+// none at 7; 80 KB of LDS a block), one at 16 (512 registers, 156 KB of LDS, 212 B
 // of scratch).  T425 x 8 levels: 412 -> 195 us, and 64 members of T31 x 16 levels:
 // 2710 -> 275 us, against reversing every term from a recompute of its own
 // (speedy_adjoint.hpp).  The descriptor is __restrict__, so uniforms are scalar
@@ -1864,8 +1865,8 @@ const char* speedy_last_error(void) { return g_last_error.c_str(); }
 // array instead of a caller's buffer, for callers that cannot allocate.  Each GPU
 // holds its own copy for the life of the process; its device address is looked
 // up once per device (hipGetSymbolAddress) and only that address is passed to
-// kernels.  Calls take the batch kernels' route, which reads no word of the
-// workspace that the same call has not written first (descriptor, level-set
+// kernels.  Calls take the batch kernels' route, which has no tagged words and reads no
+// word of the workspace that the same call has not written first (descriptor, chunk
 // words, partials), so the contents left by an earlier call, of any grid, are
 // never read and nothing needs clearing.  Calls that overlap on one GPU share
 // the array and race.

@@ -10,9 +10,9 @@ T31, T42, T85, ...).  The loop:
     outputs plus the call workspace; states are already resident) fits in the
     budget beside every request on the device, and while the batch stays under
     a column and a segment limit;
-  * launches each admitted group as ONE batched call (``speedy_fwd_batch``:
-    level sets, one column kernel over all of the batch's columns, parameter
-    sums) on one of ``n_streams`` HIP streams, so a batch can start while the
+  * launches each admitted group as ONE batched call (``speedy_fwd_batch``: one
+    launch where the batch's workgroups fit on the GPU at once, else level sets,
+    column kernels and parameter sums) on one of ``n_streams`` HIP streams, so a batch can start while the
     previous one still runs and their work overlaps on the device;
   * completes a request when its batch's event has fired, releasing its budget
     so that waiting requests are admitted into the next batch.

@@ -504,7 +504,8 @@ class SpeedyPhysics(Physics):
         _native.check(self._lib.speedy_workspace_status(ws.data_ptr(), ws.numel(), ctypes.byref(st), stream),
                       "speedy_workspace_status")
         if st.value:
-            raise _native.SpeedyError("the call's level-set exchange gave up (a workgroup never started); "
+            raise _native.SpeedyError("the call's level-set exchange gave up (a workgroup never started, or calls "
+                                      "overlapped on its workspace); "
                                       "its results are invalid and the workspace has been reset")
 
     def level_sets(self, nlon: int, nlat: int, nmember: int = 1) -> list:
@@ -518,7 +519,7 @@ class SpeedyPhysics(Physics):
     def barrier_status(self, nlon: int, nlat: int, nmember: int = 1) -> int:
         # (a set flag also re-zeroes the workspace: see speedy_workspace_status)
         """Nonzero if a call on this grid and the current stream since the last query
-        gave up waiting for the level set (its results are invalid); reading clears
+        gave up a wait inside its launch (its results are invalid); reading clears
         the flag."""
         ws = self.workspace(nlon, nlat, nmember)
         st = ctypes.c_uint32(0)
